@@ -297,8 +297,9 @@ struct Engine {
   DBuf<cx> dCaus;
   DBuf<int2> dSeeds;
   DBuf<int> dPoolBase, dPoolCount, dPoolOwner;
-  DBuf<cx> dPoolZeta, dPoolCoef, dSlots;
-  DBuf<cx> dPolyScratch;  // polynomials of the disk samples / point-source positions
+  DBuf<cx> dPoolZeta, dPoolFresh, dSlots;
+  DBuf<double> dPoolRec;
+  DBuf<cx> dPolyScratch;  // polynomials of the disk samples
   DBuf<double> dPtCausD2;
   std::vector<int2> hSeeds;  // host copy of the last seed search's seed table
   DBuf<unsigned long long> dPoolCursor;
@@ -405,6 +406,25 @@ struct Engine {
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, ev0, ev1));
     return ms;
+  }
+
+  // a pool of `cap` solves for nPts points, and its arguments
+  void solve_pool(TrialArgs& ta, int nPts, size_t cap) {
+    dPoolBase.ensure(nPts);
+    dPoolCount.ensure(nPts);
+    dPoolCursor.ensure(1);
+    dPoolZeta.ensure(cap);
+    dPoolOwner.ensure(cap);
+    dPoolRec.ensure((cap + 1) * kRecSize);
+    dPoolFresh.ensure((cap + 1) * 10);
+    ta.pool.base = dPoolBase.p;
+    ta.pool.count = dPoolCount.p;
+    ta.pool.zeta = dPoolZeta.p;
+    ta.pool.owner = dPoolOwner.p;
+    ta.pool.rec = dPoolRec.p;
+    ta.pool.fresh = dPoolFresh.p;
+    ta.pool.cursor = dPoolCursor.p;
+    ta.pool.cap = (int)cap;
   }
 
   void run(Job& job);
@@ -683,25 +703,13 @@ void Engine::run(Job& job) {
     ta.ptPos = dPtPos.p;
     dPtCausD2.ensure(nPts);
     ta.ptCausD2 = dPtCausD2.p;
-    dPoolBase.ensure(nPts);
-    dPoolCount.ensure(nPts);
-    dPoolCursor.ensure(1);
+    ta.trig = dTrig.p;
     size_t cap = std::max<size_t>(dPoolZeta.n, 2 * (size_t)nPts + 1024);
     HIPCHK(hipEventRecord(evTrial0, sstream));
     unsigned long long used = 0;
     for (int attempt = 0;; attempt++) {
       if (cap > (size_t)INT32_MAX) throw std::runtime_error("solve pool exceeds 2^31 entries");
-      dPoolZeta.ensure(cap);
-      dPoolOwner.ensure(cap);
-      dPoolCoef.ensure(cap * 11);
-      ta.pool.base = dPoolBase.p;
-      ta.pool.count = dPoolCount.p;
-      ta.pool.zeta = dPoolZeta.p;
-      ta.pool.owner = dPoolOwner.p;
-      ta.pool.coef = dPoolCoef.p;
-      ta.pool.cursor = dPoolCursor.p;
-      ta.pool.cap = (int)cap;
-      HIPCHK((hipError_t)launch_clear_u64(dPoolCursor.p, 1, 0, sstream));
+      solve_pool(ta, nPts, cap);
       HIPCHK((hipError_t)launch_trials(ta, sstream));
       HIPCHK(hipMemcpyAsync(&used, dPoolCursor.p, sizeof(used), hipMemcpyDeviceToHost, sstream));
       HIPCHK(hipStreamSynchronize(sstream));
@@ -709,7 +717,7 @@ void Engine::run(Job& job) {
       if (attempt >= 2) throw std::runtime_error("solve pool sizing did not converge");
       cap = (size_t)used + 1024;
     }
-    HIPCHK((hipError_t)launch_trial_polys(ta, (int)used, sstream));
+    HIPCHK((hipError_t)launch_solve_prep(ta, (int)used, sstream));
     HIPCHK(hipEventRecord(evTrial1, sstream));
     stats.solves = (double)used;
     SeedArgs sa;
@@ -1163,10 +1171,19 @@ void Engine::point_lc(Curve& c, cx s, cx e) {
   dCurves.ensure(1);
   dChain.ensure(1);
   dPointLC.ensure(c.lcLength);
-  dPolyScratch.ensure((size_t)c.lcLength * 11);
+  const size_t words = ((size_t)c.lcLength + 1) / 2;  // the points' curve, 0, as 64-bit words
+  dPtCurve.ensure(2 * words);
   HIPCHK(hipMemcpyAsync(dCurves.p, &d, sizeof(CurveDev), hipMemcpyHostToDevice, stream));
-  HIPCHK((hipError_t)launch_point_lc(dCurves.p, 1, (int)c.lcLength, dTrig.p, dPointLC.p, dChain.p,
-                                     dPolyScratch.p, stream));
+  HIPCHK((hipError_t)launch_clear_u64(reinterpret_cast<unsigned long long*>(dPtCurve.p), words, 0,
+                                      stream));
+  TrialArgs ta;
+  std::memset(&ta, 0, sizeof(ta));
+  ta.curves = dCurves.p;
+  ta.ptCurve = dPtCurve.p;
+  ta.nPts = (int)c.lcLength;
+  ta.trig = dTrig.p;
+  solve_pool(ta, ta.nPts, std::max<size_t>(dPoolZeta.n, c.lcLength));
+  HIPCHK((hipError_t)launch_point_lc(ta, 1, dPointLC.p, dChain.p, stream));
   HIPCHK(hipStreamSynchronize(stream));
   HIPCHK(hipMemcpy(c.lcVec.data(), dPointLC.p, c.lcLength * sizeof(double), hipMemcpyDeviceToHost));
   HIPCHK(hipMemcpy(&c.chain, dChain.p, sizeof(RootChain), hipMemcpyDeviceToHost));

@@ -75,15 +75,27 @@ struct alignas(16) Task {
 
 // The source positions each light-curve point solves for, in the order the
 // reference solves them (lcirs.cc:123-165): its centre, then the caustic
-// trial points.  Written by trial_kernel for every point at once (they do
-// not depend on the root chain), with the image polynomial of every solve.
+// trial points, points in order.  Written for every point at once (they do
+// not depend on the root chain), with everything of each solve that the
+// chain does not decide.
+//
+// One solve's record, in doubles:
+constexpr int kRecCoef = 0;    // the image polynomial's 11 coefficients (image_poly)
+constexpr int kRecDefl = 22;   // ... deflated by the first root of a chained solve: 10
+constexpr int kRecRoot = 42;   // that root (Laguerre from 0 on the full polynomial)
+constexpr int kRecZeta = 44;   // the source position
+constexpr int kRecFlags = 46;  // an integer: image mask of the fresh solve (bits 0-9), and
+constexpr int kRecOobFirst = 1 << 16;  // whether the first step, or the fresh solve, reached
+constexpr int kRecOobFresh = 1 << 17;  // Laguerre step 64 (kFlagKickTable)
+constexpr int kRecSize = 48;
 struct SolvePool {
   int* base;          // [point] first solve in the pool
   int* count;         // [point] solves (1 + caustic trials)
   cx* zeta;           // [solve] source position
   int* owner;         // [solve] the point it belongs to
-  cx* coef;           // [solve * 11 + k] coefficient of z^k (image_poly)
-  unsigned long long* cursor;  // solves handed out (may exceed cap: then rerun bigger)
+  double* rec;        // [solve * kRecSize] the record; cap + 1 of them (a chain loads one ahead)
+  cx* fresh;          // [solve * 10 + k] roots of the solve that does not use the chain; cap + 1
+  unsigned long long* cursor;  // solves of all points (may exceed cap: then rerun bigger)
   int cap;            // pool capacity in solves
 };
 
@@ -92,6 +104,7 @@ struct TrialArgs {
   const int* ptCurve;  // global point -> curve
   int nPts;
   const cx* caustics;
+  const TrigTable* trig;
   double2* ptPos;      // source position of every point
   double* ptCausD2;    // squared distance to the nearest caustic sample
   SolvePool pool;
@@ -213,8 +226,9 @@ struct FillArgs {
 
 // Host-side launchers (tl_kernels.hip).  All return hipError_t as int.
 int launch_trials(const TrialArgs& a, hipStream_t s);
-// The polynomials of the first nSolves solves of the pool (after launch_trials).
-int launch_trial_polys(const TrialArgs& a, int nSolves, hipStream_t s);
+// The records and fresh roots of the first nSolves solves of the pool (after
+// launch_trials).
+int launch_solve_prep(const TrialArgs& a, int nSolves, hipStream_t s);
 int launch_seed(const SeedArgs& a, hipStream_t s);
 // Rounds of the verified speculative chain (SpecArgs), with a.maxSplit and
 // the curves' split set to the pieces: round 1, the repair chains, and the
@@ -249,11 +263,11 @@ int launch_fill_reset(const FillArgs& a, hipStream_t s);
 int launch_resolve(const FillArgs& a, int nLabels, unsigned long long* ptCount,
                    unsigned long long* ptSum, hipStream_t s);
 // Point-source light curves (LightCurveBase::getLC): curve k writes
-// lcLength values at out[curves[k].pointBase ...].
-// nTotal: the largest pointBase + lcLength of the curves; coef: nTotal * 11
-// values of scratch for the positions' polynomials.
-int launch_point_lc(const CurveDev* curves, int nCurves, int nTotal, const TrigTable* trig,
-                    double* out, RootChain* chainOut, cx* coef, hipStream_t s);
+// lcLength values at out[curves[k].pointBase ...].  a.nPts: the largest
+// pointBase + lcLength; the pool holds at least that many solves (its fields
+// but `cursor` are used).
+int launch_point_lc(const TrialArgs& a, int nCurves, double* out, RootChain* chainOut,
+                    hipStream_t s);
 
 // Fixed-point brightness sum: each pixel's A + B sqrt(1 - r^2) is rounded to
 // a multiple of 1/scale and summed as an integer, which makes the sum

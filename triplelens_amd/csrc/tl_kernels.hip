@@ -19,6 +19,7 @@
 // same IEEE values as the reference's irsSIMD.
 #include <hip/hip_runtime.h>
 #include "tl_engine.h"
+#include "tl_roots.h"
 
 namespace tl {
 
@@ -113,9 +114,6 @@ __device__ double point_amp_term(const Lens& L, cx z) {
 // caustic-segment tests) run on separate lanes.  Values and their order are
 // those of the serial code in tl_math.h, operation for operation.
 
-// Laguerre's fractional kicks (laguerre.cc:22), read modulo 8 as lag_iter does.
-__constant__ double kLagFrac[8] = {0.5, 0.23, 0.73, 0.13, 0.37, 0.61, 0.89, 1.0};
-
 __device__ __forceinline__ double rl(double v, int k) {
   const long long b = __double_as_longlong(v);
   const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, k);
@@ -123,259 +121,207 @@ __device__ __forceinline__ double rl(double v, int k) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 __device__ __forceinline__ cx rlc(const cx& v, int k) { return mk(rl(v.re, k), rl(v.im, k)); }
-// One part of the quotient n / d as cdiv_sel forms it (part 0: real, 1:
-// imaginary), for this lane's numerator and part: lanes that need the
-// quotients of several numerators over one denominator share one division
-// sequence.
-__device__ __forceinline__ double smith_part(cx n, cx d, int part) {
-  const double a = n.re, b = n.im, c = d.re, e = d.im;
-  const bool ce = fabs(c) < fabs(e);
-  const double num = ce ? c : e, den = ce ? e : c;
-  const double ratio = num / den;
-  const double denom = (num * ratio) + den;
-  const double ar = a * ratio, br = b * ratio;
-  const double xn = ce ? ar + b : br + a;
-  const double yn = ce ? br - a : b - ar;
-  return (part ? yn : xn) / denom;
-}
-
-// Laguerre::laguerre (laguerre.cc:18-99) for an x held by every lane; the
-// polynomial's coefficient j is lane j of pv, and M is its degree.  The
-// coefficients are read once per call (the degree is a template argument,
-// so every lane index is a constant and the loops unroll), not once per
-// iteration.  The Horner recurrence runs on all lanes and lane j keeps b_j;
-// independent scalar steps of the reference run on separate lanes in one
-// instruction sequence: the moduli |b_j|, |p_m| and |x|, the four parts of
-// f/b and 2s/b, the moduli of the two candidate denominators and the two
-// parts of m/g.  Every value is the one the serial code computes.
-template <int M>
-__device__ __forceinline__ bool wl_lag(const cx& pv, cx* xp, const TrigTable* trig, bool& oob) {
-  const int ln = __lane_id();
-  cx x = *xp;
-  const double md = (double)M;
-  if constexpr (M == 1) {
-    const cx p0 = rlc(pv, 0), p1 = rlc(pv, 1);
-    if (cabs_sel(p1) != 0.0) {
-      *xp = cdiv_sel(cneg(p0), p1);
-      return true;
-    }
-    *xp = mk(999.0, 999.0);
-    return false;
-  } else {
-    cx p[M + 1];
-#pragma unroll
-    for (int j = 0; j <= M; j++) p[j] = rlc(pv, j);
-    for (int i = 1; i <= kLagMaxIt; i++) {
-      const cx pm = p[M];
-      cx b = pm;
-      cx s = mk(0.0, 0.0), f = mk(0.0, 0.0);
-      // lanes past M + 1 carry 1 + i, whose modulus (unused) takes the
-      // branch-free path of cabs_sel: with 0 there they would send the wave
-      // through the general routine as well
-      cx mine = ln == M ? pm : (ln == M + 1 ? x : mk(1.0, 1.0));
-#pragma unroll
-      for (int j = M - 1; j >= 0; j--) {
-        s = cadd(cmul(x, s), f);
-        f = cadd(cmul(x, f), b);
-        b = cadd(cmul(x, b), p[j]);
-        if (ln == j) mine = b;
-      }
-      // lane j < M: |b_j|; lane M: |p_M| (the error bound's start); lane M+1: |x|
-      const double mabs = cabs_sel(mine);
-      const double ax = rl(mabs, M + 1);
-      double err = rl(mabs, M);
-#pragma unroll
-      for (int j = M - 1; j >= 0; j--) err = rl(mabs, j) + ax * err;
-      err *= kLagEps;
-      if (rl(mabs, 0) <= err) {
-        *xp = x;
-        return true;
-      }
-      // g = f / b (lanes 0, 1) and 2s / b (lanes 2, 3)
-      const double qv = smith_part(ln < 2 ? f : cscale(s, 2.0), b, ln & 1);
-      const cx g = mk(rl(qv, 0), rl(qv, 1));
-      const cx h = csub(cmul(g, g), mk(rl(qv, 2), rl(qv, 3)));
-      const cx rad = cscale(csub(cscale(h, md), cmul(g, g)), md - 1.0);
-      const cx sq = csqrt_sel(rad);
-      cx gp = cadd(g, sq);
-      const cx gm = csub(g, sq);
-      // |gp| (lane 0) and |gm| (lane 1)
-      const double av = cabs_sel(ln == 0 ? gp : gm);
-      double agp = rl(av, 0);
-      const double agm = rl(av, 1);
-      if (agp < agm) {
-        gp = gm;
-        agp = agm;
-      }
-      cx dx;
-      if (agp > 0.0) {
-        const double dv = smith_part(mk(md, 0.0), gp, ln & 1);
-        dx = mk(rl(dv, 0), rl(dv, 1));
-      } else {
-        dx = cscale(mk(trig->c[i], trig->s[i]), 1.0 + ax);
-      }
-      cx x1 = csub(x, dx);
-      if (x.re == x1.re && x.im == x1.im) {
-        *xp = x;
-        return true;
-      }
-      if (i % kLagMT) {
-        x = x1;
-      } else {
-        oob |= i / kLagMT >= 8;
-        x = csub(x, cmul(mk(kLagFrac[(i / kLagMT) & 7], 0.0), dx));
-      }
-    }
-    *xp = x;
-    return false;
-  }
-}
-
-// Laguerre::laguerre with a different x on every lane (the polishing step):
-// the coefficients are the lanes of pv (degree M), read once per call and
-// used in the same order by all lanes.
-template <int M>
-__device__ __forceinline__ bool wl_lag_lanes(const cx& pv, cx* xp, const TrigTable* trig,
-                                             bool& oob) {
-  cx x = *xp;
-  const double md = (double)M;
-  cx p[M + 1];
-#pragma unroll
-  for (int j = 0; j <= M; j++) p[j] = rlc(pv, j);
-  for (int i = 1; i <= kLagMaxIt; i++) {
-    cx b = p[M];
-    double err = cabs_sel(b);
-    const double ax = cabs_sel(x);
-    cx s = mk(0.0, 0.0), f = mk(0.0, 0.0);
-#pragma unroll
-    for (int j = M - 1; j >= 0; j--) {
-      s = cadd(cmul(x, s), f);
-      f = cadd(cmul(x, f), b);
-      b = cadd(cmul(x, b), p[j]);
-      err = cabs_sel(b) + ax * err;
-    }
-    err *= kLagEps;
-    if (cabs_sel(b) <= err) {
-      *xp = x;
-      return true;
-    }
-    cx g = cdiv_sel(f, b);
-    cx h = csub(cmul(g, g), cdiv_sel(cscale(s, 2.0), b));
-    cx rad = cscale(csub(cscale(h, md), cmul(g, g)), md - 1.0);
-    cx sq = csqrt_sel(rad);
-    cx gp = cadd(g, sq);
-    cx gm = csub(g, sq);
-    // the moduli are taken once: |gp| after the choice is the chosen one's,
-    // and |x| is ax
-    double agp = cabs_sel(gp);
-    const double agm = cabs_sel(gm);
-    if (agp < agm) {
-      gp = gm;
-      agp = agm;
-    }
-    cx dx;
-    if (agp > 0.0) dx = cdiv_rc_sel(md, gp);
-    else dx = cscale(mk(trig->c[i], trig->s[i]), 1.0 + ax);
-    cx x1 = csub(x, dx);
-    if (x.re == x1.re && x.im == x1.im) {
-      *xp = x;
-      return true;
-    }
-    if (i % kLagMT) {
-      x = x1;
-    } else {
-      oob |= i / kLagMT >= 8;
-      x = csub(x, cmul(mk(kLagFrac[(i / kLagMT) & 7], 0.0), dx));
-    }
-  }
-  *xp = x;
-  return false;
-}
-
-// The deflation steps J..1 of Laguerre::solveRoots (laguerre.cc:103-167):
-// every lane holds the step's root, the deflated coefficients stay on the
-// lanes of tmp, and the root of step J goes to lane 10 - J of rootv.
+// The deflation steps J..1 of Laguerre::solveRoots (laguerre.cc:103-167) on
+// a wavefront whose lanes all hold the same polynomial p and the same x: the
+// root of step J goes to lane 10 - J of rootv.  initv's lane j seeds the
+// search of step j.  The accepted x's Horner sums are the next polynomial.
 template <int J>
-__device__ __forceinline__ void wl_deflate(cx& tmp, cx& rootv, bool init, const cx& initv,
+__device__ __forceinline__ void wl_deflate(const cx (&p)[J + 1], cx& rootv, const cx& initv,
                                            const TrigTable* trig, bool& oob) {
-  if constexpr (J >= 1) {
-    const int ln = __lane_id();
-    cx x = init ? rlc(initv, J) : mk(kLagEps, kLagEps);
-    if (!wl_lag<J>(tmp, &x, trig, oob) && init) x = mk(kLagEps, kLagEps);
-    if (ln == 10 - J) rootv = x;
-    cx b = rlc(tmp, J);
-#pragma unroll
-    for (int jj = J - 1; jj >= 0; jj--) {
-      const cx c = rlc(tmp, jj);
-      if (ln == jj) tmp = b;
-      b = cadd(cmul(x, b), c);
+  const int ln = __lane_id();
+  cx x = rlc(initv, J);
+  if constexpr (J == 1) {
+    // a root step that fails restarts from (eps, eps), which is what it then
+    // leaves as the root (laguerre.cc:120-128)
+    if (p[1].re != 0.0 || p[1].im != 0.0) x = cdiv_sel(cneg(p[0]), p[1]);
+    else x = mk(kLagEps, kLagEps);
+    if (ln == 9) rootv = x;
+  } else {
+    cx b[J + 1];
+    if (!lag_fast<J, true>(p, x, b, trig, oob)) {
+      x = mk(kLagEps, kLagEps);
+      horner_sums<J>(p, x, b);
     }
-    wl_deflate<J - 1>(tmp, rootv, init, initv, trig, oob);
+    if (ln == 10 - J) rootv = x;
+    cx q[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) q[j] = b[j + 1];
+    wl_deflate<J - 1>(q, rootv, initv, trig, oob);
   }
 }
 
-// Laguerre::solveRoots for the degree-10 image polynomial (coefficients on
-// lanes 0..10 of cv): the deflation, then lane r polishes root r on the
-// full polynomial.  Returns root r on lane r (r < 10; 0 elsewhere).  With
-// init, initv's lane j seeds the search of step j (j = 10..1).
-__device__ __forceinline__ cx wl_solve10(const cx& cv, bool init, const cx& initv,
-                                         const TrigTable* trig, bool& oob) {
-  const int ln = __lane_id();
-  cx tmp = cv;
-  cx rootv = mk(0.0, 0.0);
-  wl_deflate<10>(tmp, rootv, init, initv, trig, oob);
-  bool laneOob = false;
-  if (ln < 10) wl_lag_lanes<10>(cv, &rootv, trig, laneOob);
-  oob |= __ballot(laneOob) != 0;
-  return rootv;
+// v of the lane n places further round its row of 16 lanes.
+template <int N>
+__device__ __forceinline__ double row_ror(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + N, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + N, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+template <int N>
+__device__ __forceinline__ cx row_times(const cx& v) {
+  return cmul(v, mk(row_ror<N>(v.re), row_ror<N>(v.im)));
 }
 
-// Laguerre::checkRoots (laguerre.cc:188-198) on roots held one per lane.
-__device__ __forceinline__ bool wl_check(const cx& cv, const cx& rootv) {
-  cx c0 = rlc(cv, 10);
+// Laguerre::checkRoots (laguerre.cc:188-198) on roots held one per lane, as
+// written (the product in root order).
+__device__ __forceinline__ bool wl_check_exact(cx c10, cx a0, const cx& rootv) {
+  cx c0 = c10;
   for (int j = 0; j < 10; j++) c0 = cmul(c0, cneg(rlc(rootv, j)));
-  const cx a0 = rlc(cv, 0);
-  if (cabs_sel(a0) > 1.0e-8) return (1.0 - cabs_sel(cdiv_sel(c0, a0))) < 1.0e-5;
-  return cabs_sel(csub(c0, a0)) < 1.0e-10;
+  if (cabs_(a0) > 1.0e-8) return (1.0 - cabs_(cdiv_sel(c0, a0))) < 1.0e-5;
+  return cabs_(csub(c0, a0)) < 1.0e-10;
 }
 
-// getRootsPrecalculated + getImages (imgpoint.cc:160-274) on a wavefront,
-// for the polynomial whose coefficient k is lane k of cv.  chainv holds
-// tempRoots[k] on lane k (lane 10 is the slot the reference reads past the
-// end of its vector: 0 here, or a recorded value the caller put there).
-// Returns the mask of the roots accepted as images (bit k: root k on lane k
-// of chainv).
-__device__ __forceinline__ unsigned long long wl_get_images(const Lens& L, const cx& cv,
-                                                            cx& chainv, int& have, cx zeta,
+// checkRoots decided from the product taken in any order (a tree over the
+// lanes, good to a few units in the last place) where |c0 / a0| is not within
+// 1e-9 of its threshold 1 - 1e-5; ten sign changes cancel.
+__device__ __forceinline__ bool wl_check(cx c10, cx a0, const cx& rootv) {
+  const int ln = __lane_id();
+  cx v = ln < 10 ? rootv : mk(1.0, 0.0);
+  v = row_times<8>(v);
+  v = row_times<4>(v);
+  v = row_times<2>(v);
+  v = row_times<1>(v);
+  const double A = cnorm(cmul(c10, v)), T = cnorm(a0) * ((1.0 - 1.0e-5) * (1.0 - 1.0e-5));
+  const bool big = T > 1.0001e-16 && A < 1e300;
+  const unsigned long long yes = __ballot(big && A > T * (1.0 + 1e-9));
+  if (yes & 1ull) return true;
+  const unsigned long long no = __ballot(big && A < T * (1.0 - 1e-9));
+  if (no & 1ull) return false;
+  return wl_check_exact(c10, a0, rootv);
+}
+
+// img_check (imgpoint.cc:72-90) on every lane's root: the residual of the
+// lens equation with fused arithmetic, its error bounded by 1e-14 of the sum
+// of its terms' magnitudes; where that leaves the comparison with the
+// threshold 1e-6 open on some lane below 10, all lanes run img_check itself.
+__device__ __forceinline__ bool wl_img_check(const Lens& L, const cx& z, cx zeta) {
+  double wr = z.re - zeta.re, wi = z.im - zeta.im;
+  double S = fabs(z.re) + fabs(z.im) + fabs(zeta.re) + fabs(zeta.im);
+  auto term = [&](double m, const cx& zk) {
+    const double dr = z.re - zk.re, di = z.im - zk.im;
+    const double r = m * rcp_near(fma(dr, dr, di * di));
+    wr = fma(-dr, r, wr);
+    wi = fma(-di, r, wi);
+    S = fma(fabs(dr) + fabs(di), fabs(r), S);
+  };
+  term(L.m1, L.z1);
+  term(L.m2, L.z2);
+  term(L.m3, L.z3);
+  const double n = fma(wr, wr, wi * wi), e = 1e-14 * S;
+  const bool yes = e < 5e-7 && n < (1e-6 - e) * (1e-6 - e);
+  const bool no = n > (1e-6 + e) * (1e-6 + e);
+  if (__ballot(!yes && !no && __lane_id() < 10) == 0) return yes;
+  return img_check(L, z, zeta, 1.0e-6);
+}
+
+// getRootsPrecalculated + getImages (imgpoint.cc:160-274) on a wavefront for
+// one solve of the pool: v is lane k's element k of its record (SolvePool),
+// freshv the roots of its fresh solve (root r on lane r).  chainv holds
+// tempRoots[k] on lane k.  With `slot`, the chained solve's first step starts
+// from tempRoots[10] on lane 10 of chainv (a recorded value of the slot the
+// reference reads past the end of its vector) instead of 0.  Returns the mask
+// of the roots accepted as images (bit k: root k on lane k of chainv).
+//
+// The reference's sequence (imgpoint.cc:181-206,262-270): a solve from the
+// chain's roots (when it has some), replaced by a fresh solve when the roots
+// fail checkRoots; then, if the image count is invalid, one more fresh solve.
+// A fresh solve depends on the polynomial alone, and so does the chained
+// solve's first step (it starts from 0): solve_prep_kernel has done both for
+// every solve of the run, and the chain only runs the deflation steps 9..1,
+// the polish and the tests.
+template <bool TRACED>
+__device__ __forceinline__ unsigned long long wl_get_images(const Lens& L, double v, cx freshv,
+                                                            bool slot, cx& chainv, int& have,
                                                             const TrigTable* trig, bool binImg,
                                                             bool& oob) {
   const int ln = __lane_id();
-  // The reference's sequence (imgpoint.cc:181-206,262-270): a solve from the
-  // chain's roots (when it has some), replaced by a fresh solve when the
-  // roots fail checkRoots; then, if the image count is invalid, one more
-  // fresh solve.  A fresh solve of the same coefficients gives the same
-  // roots, so the second one is skipped when the first solve was fresh.
-  bool withInit = have != 0;
-  bool second = false;
-  while (true) {
-    const cx r = wl_solve10(cv, withInit, chainv, trig, oob);
-    if (withInit && !wl_check(cv, r)) {
-      withInit = false;
-      continue;
+  const int fl = (int)rl(v, kRecFlags);
+  if (have) {
+    cx c[11];
+#pragma unroll
+    for (int j = 0; j <= 10; j++) c[j] = mk(rl(v, 2 * j), rl(v, 2 * j + 1));
+    cx p[10];
+#pragma unroll
+    for (int j = 0; j < 10; j++) p[j] = mk(rl(v, kRecDefl + 2 * j), rl(v, kRecDefl + 2 * j + 1));
+    cx rootv = mk(rl(v, kRecRoot), rl(v, kRecRoot + 1));
+    bool firstOob = (fl & kRecOobFirst) != 0;
+    if constexpr (TRACED) {
+      if (slot) {
+        firstOob = false;
+        cx x = rlc(chainv, 10), b[11];
+        if (!lag_fast<10, true>(c, x, b, trig, firstOob)) {
+          x = mk(kLagEps, kLagEps);
+          horner_sums<10>(c, x, b);
+        }
+        rootv = x;
+#pragma unroll
+        for (int j = 0; j < 10; j++) p[j] = b[j + 1];
+      }
     }
-    chainv = ln < 10 ? r : mk(0.0, 0.0);
-    have = 1;
-    const bool ok = ln < 10 && img_check(L, chainv, zeta, 1.0e-6);
-    const unsigned long long m = __ballot(ok);
-    const int n = __builtin_popcountll(m);
-    // a valid count: even and at least 4, or for the binary lens odd and at
-    // least 3 (imgpoint.cc:236-237)
-    const bool bad = binImg ? (n % 2 != 1 || n < 3) : (n % 2 != 0 || n < 4);
-    if (!bad || second || !withInit) return m;
-    second = true;
-    withInit = false;
+    oob |= firstOob;
+    wl_deflate<9>(p, rootv, chainv, trig, oob);
+    // root r is polished on lane r; the other lanes repeat root 0
+    bool laneOob = false;
+    cx b[11];
+    lag_fast<10, false>(c, rootv, b, trig, laneOob);
+    oob |= __ballot(laneOob) != 0;
+    if (wl_check(c[10], c[0], rootv)) {
+      const bool ok = wl_img_check(L, rootv, mk(rl(v, kRecZeta), rl(v, kRecZeta + 1))) && ln < 10;
+      const unsigned long long m = __ballot(ok);
+      const int n = __builtin_popcountll(m);
+      // a valid count: even and at least 4, or for the binary lens odd and at
+      // least 3 (imgpoint.cc:236-237)
+      if (binImg ? (n % 2 == 1 && n >= 3) : (n % 2 == 0 && n >= 4)) {
+        chainv = ln < 10 ? rootv : mk(0.0, 0.0);
+        return m;
+      }
+    }
   }
+  chainv = ln < 10 ? freshv : mk(0.0, 0.0);
+  have = 1;
+  oob |= (fl & kRecOobFresh) != 0;
+  return (unsigned long long)(fl & 0x3ff);
 }
+
+// Walks a curve's solves in order (the pool holds them so): the record and
+// the fresh roots of the coming solve are loaded one solve ahead, and the
+// solve counts 64 positions at a time, so that the chain does not wait for
+// memory.
+struct SolveWalk {
+  const SolvePool& P;
+  int p, pEnd, k, cnt;
+  size_t sid;
+  double v;
+  cx f;
+  __device__ __forceinline__ SolveWalk(const SolvePool& pool, int p0, int end)
+      : P(pool), p(p0), pEnd(end), k(64), cnt(0) {
+    sid = (size_t)uni(P.base[p0]);
+    fetch();
+  }
+  __device__ __forceinline__ void fetch() {
+    const int ln = __lane_id();
+    v = ln < kRecSize ? P.rec[sid * kRecSize + ln] : 0.0;
+    f = ln < 10 ? P.fresh[sid * 10 + ln] : mk(0.0, 0.0);
+  }
+  // solves of the next position
+  __device__ __forceinline__ int position() {
+    if (k == 64) {
+      const int q = p + __lane_id();
+      cnt = q < pEnd ? P.count[q] : 0;
+      k = 0;
+    }
+    p++;
+    return __builtin_amdgcn_readlane(cnt, k++);
+  }
+  // the next solve's record and fresh roots
+  __device__ __forceinline__ void next(double& rv, cx& fv) {
+    rv = v;
+    fv = f;
+    sid++;
+    fetch();
+  }
+};
 
 __device__ __forceinline__ double wave_sum_d(double v) {
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -430,16 +376,14 @@ __device__ __forceinline__ void scan_trials(const CurveDev& C, cx pos, const cx*
 }
 
 // Everything of a light-curve point that does not depend on the root chain,
-// one wavefront per point, all points at once: its source position, the
-// distance to the nearest caustic sample, and the list of positions the
-// chain will solve for (the centre, then the caustic trial points).  The
-// list goes to the pool at a place taken with one atomic add; when the pool
-// is too small, the cursor still advances and nothing is written, and the
-// host runs the kernel again with a bigger pool.  The solves' polynomials
-// are computed afterwards by trial_poly_kernel, one lane per solve (that
-// evaluation needs many registers; kept apart, this kernel stays small and
-// many of its wavefronts share each SIMD).
-__global__ void __launch_bounds__(64) trial_kernel(TrialArgs a) {
+// all points at once: its source position, the distance to the nearest
+// caustic sample, and the list of positions the chain will solve for (the
+// centre, then the caustic trial points).  One wavefront per point counts
+// the solves, one workgroup turns the counts into places in the pool (point
+// order, so that a chain finds its next solve behind the last one), and one
+// wavefront per point writes the list.  When the pool is too small nothing is
+// written and the host runs the kernels again with a bigger pool.
+__global__ void __launch_bounds__(64) trial_count_kernel(TrialArgs a) {
   const int p = blockIdx.x;
   if (p >= a.nPts) return;
   const int ln = __lane_id();
@@ -463,20 +407,50 @@ __global__ void __launch_bounds__(64) trial_kernel(TrialArgs a) {
   }
   int n = 1;
   scan_trials(C, pos, caus, [&](unsigned long long f, const cx&) { n += __builtin_popcountll(f); });
-  int base = 0;
-  if (ln == 0) base = (int)atomicAdd(a.pool.cursor, (unsigned long long)n);
-  base = __shfl(base, 0, 64);
-  if (ln == 0) {
-    a.pool.base[p] = base;
-    a.pool.count[p] = n;
+  if (ln == 0) a.pool.count[p] = n;
+}
+
+// Exclusive prefix sum of the points' solve counts (one workgroup; every
+// thread sums a contiguous share), and their total in *cursor.
+constexpr int kScanThreads = 1024;
+__global__ void __launch_bounds__(kScanThreads) pool_scan_kernel(SolvePool P, int nPts) {
+  __shared__ int part[kScanThreads];
+  const int t = threadIdx.x;
+  const int per = (nPts + kScanThreads - 1) / kScanThreads;
+  const int lo = t * per < nPts ? t * per : nPts, hi = lo + per < nPts ? lo + per : nPts;
+  int sum = 0;
+  for (int p = lo; p < hi; p++) sum += P.count[p];
+  part[t] = sum;
+  __syncthreads();
+  for (int o = 1; o < kScanThreads; o <<= 1) {
+    const int v = t >= o ? part[t - o] : 0;
+    __syncthreads();
+    part[t] += v;
+    __syncthreads();
   }
-  if ((long long)base + n > a.pool.cap) return;
-  if (ln == 0) {
-    a.pool.zeta[base] = pos;
-    a.pool.owner[base] = p;
+  int at = part[t] - sum;
+  for (int p = lo; p < hi; p++) {
+    P.base[p] = at;
+    at += P.count[p];
   }
-  int next = base + 1;
-  scan_trials(C, pos, caus, [&](unsigned long long f, const cx& trial) {
+  if (t == kScanThreads - 1) *P.cursor = (unsigned long long)part[t];
+}
+
+__global__ void __launch_bounds__(64) trial_list_kernel(TrialArgs a) {
+  const int p = blockIdx.x;
+  if (p >= a.nPts || *a.pool.cursor > (unsigned long long)a.pool.cap) return;
+  const int ln = __lane_id();
+  const CurveDev& C = a.curves[a.ptCurve[p]];
+  const double2 pp = a.ptPos[p];
+  const cx pos = mk(pp.x, pp.y);
+  int next = a.pool.base[p];
+  if (ln == 0) {
+    a.pool.zeta[next] = pos;
+    a.pool.owner[next] = p;
+  }
+  next++;
+  if (a.pool.count[p] == 1) return;
+  scan_trials(C, pos, a.caustics + C.causticBase, [&](unsigned long long f, const cx& trial) {
     if ((f >> ln) & 1ull) {
       const int sid = next + __builtin_popcountll(f & ((1ull << ln) - 1ull));
       a.pool.zeta[sid] = trial;
@@ -493,19 +467,100 @@ __global__ void __launch_bounds__(64) trial_poly_kernel(TrialArgs a, int nSolves
   if (sid >= nSolves) return;
   const CurveDev& C = a.curves[a.ptCurve[a.pool.owner[sid]]];
   cx c[11];
-  image_poly(C.L, C.fixedPoly, a.pool.zeta[sid], c);
-  for (int k = 0; k < 11; k++) a.pool.coef[(size_t)sid * 11 + k] = c[k];
+  const cx zeta = a.pool.zeta[sid];
+  image_poly(C.L, C.fixedPoly, zeta, c);
+  cx* rec = reinterpret_cast<cx*>(a.pool.rec + (size_t)sid * kRecSize);
+  for (int k = 0; k < 11; k++) rec[k] = c[k];
+  rec[kRecZeta / 2] = zeta;
+}
+
+// The root solver for one lane per solve, every array in registers (the
+// degree is a template argument).
+// The deflation steps J..1 of Laguerre::solveRoots (laguerre.cc:103-167): the
+// root found at step J goes to roots[10 - J].
+template <int J>
+__device__ __forceinline__ void lane_deflate(const cx (&p)[J + 1], const cx* init, bool withInit,
+                                             cx* roots, const TrigTable* trig, bool& oob) {
+  cx x = withInit ? init[J] : mk(kLagEps, kLagEps);
+  if constexpr (J == 1) {
+    if (p[1].re != 0.0 || p[1].im != 0.0) x = cdiv(cneg(p[0]), p[1]);
+    else x = withInit ? mk(kLagEps, kLagEps) : mk(999.0, 999.0);
+    roots[9] = x;
+  } else {
+    cx b[J + 1];
+    if (!lag_fast<J, false>(p, x, b, trig, oob) && withInit) {
+      x = mk(kLagEps, kLagEps);
+      horner_sums<J>(p, x, b);
+    }
+    roots[10 - J] = x;
+    cx q[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) q[j] = b[j + 1];
+    lane_deflate<J - 1>(q, init, withInit, roots, trig, oob);
+  }
+}
+// solveRoots: the deflation, then each root polished on the full polynomial
+// in root order (the roots rotate through roots[0], so one copy of the
+// polishing code serves all of them).
+__device__ __forceinline__ void lane_solve(const cx (&c)[11], const cx* init, bool withInit,
+                                           cx* roots, const TrigTable* trig, bool& oob) {
+  lane_deflate<10>(c, init, withInit, roots, trig, oob);
+#pragma unroll 1
+  for (int j = 0; j < 10; j++) {
+    cx x = roots[0], b[11];
+    lag_fast<10, false>(c, x, b, trig, oob);
+#pragma unroll
+    for (int k = 0; k < 9; k++) roots[k] = roots[k + 1];
+    roots[9] = x;
+  }
+}
+
+// What a solve of the chain needs that does not depend on the chain, one lane
+// per solve: the first deflation step of a chained solve (root and deflated
+// polynomial) and the fresh solve (roots and image mask).
+__global__ void __launch_bounds__(64) solve_prep_kernel(TrialArgs a, int nSolves) {
+  const int sid = blockIdx.x * blockDim.x + threadIdx.x;
+  if (sid >= nSolves) return;
+  const Lens L = a.curves[a.ptCurve[a.pool.owner[sid]]].L;
+  cx* rec = reinterpret_cast<cx*>(a.pool.rec + (size_t)sid * kRecSize);
+  cx c[11];
+#pragma unroll
+  for (int k = 0; k < 11; k++) c[k] = rec[k];
+  const cx zeta = rec[kRecZeta / 2];
+  cx x = mk(0.0, 0.0), b[11];
+  bool oob = false;
+  if (!lag_fast<10, false>(c, x, b, a.trig, oob)) {
+    x = mk(kLagEps, kLagEps);
+    horner_sums<10>(c, x, b);
+  }
+#pragma unroll
+  for (int k = 0; k < 10; k++) rec[kRecDefl / 2 + k] = b[k + 1];
+  rec[kRecRoot / 2] = x;
+  int fl = oob ? kRecOobFirst : 0;
+  cx roots[10];
+  oob = false;
+  lane_solve(c, nullptr, false, roots, a.trig, oob);
+  if (oob) fl |= kRecOobFresh;
+#pragma unroll
+  for (int k = 0; k < 10; k++) {
+    a.pool.fresh[(size_t)sid * 10 + k] = roots[k];
+    if (img_check(L, roots[k], zeta, 1.0e-6)) fl |= 1 << k;
+  }
+  rec[kRecFlags / 2] = mk((double)fl, 0.0);
 }
 
 int launch_trials(const TrialArgs& a, hipStream_t s) {
   if (a.nPts <= 0) return 0;
-  hipLaunchKernelGGL(trial_kernel, dim3(a.nPts), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(trial_count_kernel, dim3(a.nPts), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(pool_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, a.pool, a.nPts);
+  hipLaunchKernelGGL(trial_list_kernel, dim3(a.nPts), dim3(64), 0, s, a);
   return (int)hipGetLastError();
 }
 
-int launch_trial_polys(const TrialArgs& a, int nSolves, hipStream_t s) {
+int launch_solve_prep(const TrialArgs& a, int nSolves, hipStream_t s) {
   if (nSolves <= 0) return 0;
   hipLaunchKernelGGL(trial_poly_kernel, dim3((nSolves + 63) / 64), dim3(64), 0, s, a, nSolves);
+  hipLaunchKernelGGL(solve_prep_kernel, dim3((nSolves + 63) / 64), dim3(64), 0, s, a, nSolves);
   return (int)hipGetLastError();
 }
 
@@ -535,6 +590,7 @@ int launch_image_poly(const Lens& L, const cx* fixedPoly, const cx* zeta, int n,
 // fresh solve.  Each position's solves (centre, then caustic trial points)
 // and their polynomials come from trial_kernel's pool, so the chain itself
 // only runs the root solves, the image tests and the seed output.
+template <bool TRACED>
 __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
   const int c = blockIdx.x / a.maxSplit, q = blockIdx.x % a.maxSplit;
   if (c >= a.nCurves) return;
@@ -560,27 +616,30 @@ __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
     have = C.chainHave;
     calls = C.chainCalls;
   }
-  const bool traced = q == 0 && a.slotTrace && C.slotCount > 0;
+  const bool traced = TRACED && q == 0 && C.slotCount > 0;
   const long long n = (long long)C.lcLength + 1;
   const long long cBegin = n * a.chunk / a.nChunks, cEnd = n * (a.chunk + 1) / a.nChunks;
   const unsigned iBegin = (unsigned)(cBegin + (cEnd - cBegin) * q / C.split);
   const unsigned iEnd = (unsigned)(cBegin + (cEnd - cBegin) * (q + 1) / C.split);
+  if (iBegin < iEnd) {
+  SolveWalk W(a.pool, C.pointBase + (int)iBegin, C.pointBase + (int)iEnd);
   for (unsigned i = iBegin; i < iEnd; i++) {
     const int p = C.pointBase + (int)i;
-    const int base = a.pool.base[p], nSolve = a.pool.count[p];
+    const int nSolve = W.position();
     int cnt = 0;
     uint32_t fl = 0;
     int2* out = a.seeds + (size_t)p * kMaxSeeds;
     double amp = 0.0;
     for (int sIdx = 0; sIdx < nSolve; sIdx++) {
-      const size_t sid = (size_t)base + sIdx;
-      const cx cv = ln <= 10 ? a.pool.coef[sid * 11 + (ln <= 10 ? ln : 0)] : mk(0.0, 0.0);
-      const cx zeta = a.pool.zeta[sid];
-      if (traced && have && calls < C.slotCount && ln == 10)
-        chainv = a.slotTrace[C.slotBase + calls];
+      double rv;
+      cx fv;
+      W.next(rv, fv);
+      const bool slot = traced && have && calls < C.slotCount;
+      if (slot && ln == 10) chainv = a.slotTrace[C.slotBase + calls];
       calls++;
       bool oob = false;
-      const unsigned long long m = wl_get_images(L, cv, chainv, have, zeta, a.trig, C.binImg, oob);
+      const unsigned long long m =
+          wl_get_images<TRACED>(L, rv, fv, slot, chainv, have, a.trig, C.binImg, oob);
       if (oob) fl |= kFlagKickTable;
       emit_seeds(C, chainv, m, out, cnt, fl);
       if (sIdx == 0) {
@@ -627,6 +686,7 @@ __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
       a.cost[p] = (float)(amp * 3.141592653589793 * C.ppr * C.ppr);
     }
   }
+  }
   if (q == C.split - 1) {
     if (ln <= 10) a.chainOut[c].tempRoots[ln] = chainv;
     if (ln == 0) {
@@ -637,30 +697,25 @@ __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
 }
 
 // ---- verified speculative chain (SpecArgs) ---------------------------------
-// The chain's solves of position p (centre, then caustic trial points), as
-// seed_kernel runs them, without output.
+// The chain's solves of the walk's next position (centre, then caustic trial
+// points), as seed_kernel runs them, without output.
 __device__ __forceinline__ void chain_step(const SeedArgs& a, const CurveDev& C, const Lens& L,
-                                           int p, cx& chainv, int& have) {
-  const int ln = __lane_id();
-  const int base = a.pool.base[p], nSolve = a.pool.count[p];
+                                           SolveWalk& W, cx& chainv, int& have) {
+  const int nSolve = W.position();
   for (int sIdx = 0; sIdx < nSolve; sIdx++) {
-    const size_t sid = (size_t)base + sIdx;
-    const cx cv = ln <= 10 ? a.pool.coef[sid * 11 + (ln <= 10 ? ln : 0)] : mk(0.0, 0.0);
+    double rv;
+    cx fv;
+    W.next(rv, fv);
     bool oob = false;
-    wl_get_images(L, cv, chainv, have, a.pool.zeta[sid], a.trig, C.binImg, oob);
+    wl_get_images<false>(L, rv, fv, false, chainv, have, a.trig, C.binImg, oob);
   }
 }
 
 // The chain state (roots 0..9 on lanes 0..9) equals the stored one, bit for bit.
-__device__ __forceinline__ bool state_equal(const cx& chainv, const cx* st) {
-  const int ln = __lane_id();
-  bool eq = true;
-  if (ln < 10) {
-    const cx v = st[ln];
-    eq = __double_as_longlong(v.re) == __double_as_longlong(chainv.re) &&
-         __double_as_longlong(v.im) == __double_as_longlong(chainv.im);
-  }
-  return __ballot(!eq) == 0;
+__device__ __forceinline__ bool state_equal(const cx& chainv, const cx& st) {
+  const bool eq = __double_as_longlong(st.re) == __double_as_longlong(chainv.re) &&
+                  __double_as_longlong(st.im) == __double_as_longlong(chainv.im);
+  return __ballot(!eq && __lane_id() < 10) == 0;
 }
 
 __device__ __forceinline__ void piece_range(const CurveDev& C, int q, int& b, int& e) {
@@ -692,9 +747,11 @@ __global__ void __launch_bounds__(64) spec_round1_kernel(SeedArgs a, SpecArgs sp
     piece_range(C, q + 1, b2, e2);
     stop = e + sp.overlap < e2 ? e + sp.overlap : e2;
   }
+  if (b >= stop) return;
+  SolveWalk W(a.pool, C.pointBase + b, C.pointBase + stop);
   for (int i = b; i < stop; i++) {
     const int p = C.pointBase + i;
-    chain_step(a, C, L, p, chainv, have);
+    chain_step(a, C, L, W, chainv, have);
     cx* dst = (i < e ? sp.own : sp.ext) + (size_t)p * 10;
     if (ln < 10) dst[ln] = chainv;
   }
@@ -717,9 +774,12 @@ __global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp
   bool agree = false;
   for (int i = b; i < lim && !agree; i++) {
     const size_t p = (size_t)C.pointBase + i;
-    cx v = mk(0.0, 0.0);
-    if (ln < 10) v = sp.ext[p * 10 + ln];
-    agree = state_equal(v, sp.own + p * 10);
+    cx v = mk(0.0, 0.0), o = v;
+    if (ln < 10) {
+      v = sp.ext[p * 10 + ln];
+      o = sp.own[p * 10 + ln];
+    }
+    agree = state_equal(v, o);
   }
   if (ln == 0) sp.merged[gq] = agree ? 1 : 0;
   if (agree) return;
@@ -729,6 +789,8 @@ __global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp
   int have = 1;
   int qq = q, qb = b, qe = e;  // the piece the chain is in
   const long long n = (long long)C.lcLength + 1;
+  if (b >= n) return;
+  SolveWalk W(a.pool, C.pointBase + b, C.pointBase + (int)n);
   for (int i = b; i < n; i++) {
     if (i == qe) {
       // entering piece qq + 1: the chain's state before its first position
@@ -743,8 +805,12 @@ __global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp
       if (ln < 10) sp.repState[((size_t)gq * sp.depth + j) * 10 + ln] = chainv;
     }
     const int p = C.pointBase + i;
-    chain_step(a, C, L, p, chainv, have);
-    if (qq > q && i < qb + sp.overlap && state_equal(chainv, sp.own + (size_t)p * 10)) {
+    // the piece's own state, loaded before the solve that it is compared with
+    const bool mayJoin = qq > q && i < qb + sp.overlap;
+    cx own = mk(0.0, 0.0);
+    if (mayJoin && ln < 10) own = sp.own[(size_t)p * 10 + ln];
+    chain_step(a, C, L, W, chainv, have);
+    if (mayJoin && state_equal(chainv, own)) {
       if (ln == 0) sp.repTarget[gq] = qq;
       return;
     }
@@ -793,7 +859,7 @@ int launch_spec(const SeedArgs& a, const SpecArgs& sp, hipStream_t s) {
     return (int)hipErrorInvalidValue;
   if (!sp.pieceBase || !sp.own || !sp.ext || !sp.merged || !sp.repState || !sp.repTarget ||
       !sp.start || !sp.failed || sp.overlap < 1 || sp.depth < 1 || !a.curves || !a.trig ||
-      !a.pool.base || !a.pool.count || !a.pool.coef || !a.pool.zeta)
+      !a.pool.base || !a.pool.count || !a.pool.rec || !a.pool.fresh)
     return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(spec_round1_kernel, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a, sp);
   hipLaunchKernelGGL(spec_repair_kernel, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a, sp);
@@ -805,27 +871,22 @@ int launch_spec(const SeedArgs& a, const SpecArgs& sp, hipStream_t s) {
 // t = i/(lcLength-1), magnification sum over images (in root order) of
 // 1/|1 - |sum m/(z-z_k)^2|^2| (the squares as products; the reference uses
 // std::pow(z, 2.0)).  One wavefront per curve, as the seed search.
-// The image polynomial at every position of the point-source curves (one
-// lane per position), for point_lc_kernel: coef[(pointBase + i) * 11 + k].
-__global__ void __launch_bounds__(64) point_poly_kernel(const CurveDev* curves, int nCurves,
-                                                        int nTotal, cx* coef) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= nTotal) return;
-  int c = 0;
-  while (c + 1 < nCurves && curves[c + 1].pointBase <= g) c++;
-  const CurveDev& C = curves[c];
-  const int i = g - C.pointBase;
-  if (i < 0 || i >= (int)C.lcLength) return;
+// The point-source curve's positions as a pool of one solve each.
+__global__ void point_list_kernel(TrialArgs a) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= a.nPts) return;
+  const CurveDev& C = a.curves[a.ptCurve[p]];
+  const int i = p - C.pointBase;
   const cx s = mk(C.sx, C.sy), e = mk(C.ex, C.ey);
-  const cx pos = cadd(s, cscale(csub(e, s), i / (C.lcLength - 1.0)));
-  cx cf[11];
-  image_poly(C.L, C.fixedPoly, pos, cf);
-  for (int k = 0; k < 11; k++) coef[(size_t)g * 11 + k] = cf[k];
+  a.pool.zeta[p] = cadd(s, cscale(csub(e, s), i / (C.lcLength - 1.0)));
+  a.pool.owner[p] = p;
+  a.pool.base[p] = p;
+  a.pool.count[p] = 1;
 }
 
 __global__ void __launch_bounds__(64) point_lc_kernel(const CurveDev* curves, int nCurves,
                                                       const TrigTable* trig, double* out,
-                                                      RootChain* chainOut, const cx* coef) {
+                                                      RootChain* chainOut, SolvePool pool) {
   const int c = blockIdx.x;
   if (c >= nCurves) return;
   const int ln = __lane_id();
@@ -833,13 +894,14 @@ __global__ void __launch_bounds__(64) point_lc_kernel(const CurveDev* curves, in
   const Lens L = C.L;
   cx chainv = ln <= 10 ? C.chain[ln <= 10 ? ln : 0] : mk(0.0, 0.0);
   int have = C.chainHave;
-  const cx s = mk(C.sx, C.sy), e = mk(C.ex, C.ey);
+  SolveWalk W(pool, C.pointBase, C.pointBase + (int)C.lcLength);
   for (unsigned i = 0; i < C.lcLength; i++) {
-    const cx pos = cadd(s, cscale(csub(e, s), i / (C.lcLength - 1.0)));
-    const size_t g = (size_t)C.pointBase + i;
-    const cx cv = ln <= 10 ? coef[g * 11 + (ln <= 10 ? ln : 0)] : mk(0.0, 0.0);
+    double rv;
+    cx fv;
+    W.next(rv, fv);
     bool oob = false;
-    unsigned long long m = wl_get_images(L, cv, chainv, have, pos, trig, C.binImg, oob);
+    unsigned long long m = wl_get_images<false>(L, rv, fv, false, chainv, have, trig, C.binImg,
+                                                oob);
     const double term = ((m >> ln) & 1ull) ? point_amp_term(L, chainv) : 0.0;
     double amp = 0.0;
     while (m) {
@@ -856,13 +918,14 @@ __global__ void __launch_bounds__(64) point_lc_kernel(const CurveDev* curves, in
   }
 }
 
-int launch_point_lc(const CurveDev* curves, int nCurves, int nTotal, const TrigTable* trig,
-                    double* out, RootChain* chainOut, cx* coef, hipStream_t s) {
-  if (nCurves <= 0 || nTotal <= 0) return 0;
-  hipLaunchKernelGGL(point_poly_kernel, dim3((nTotal + 63) / 64), dim3(64), 0, s, curves, nCurves,
-                     nTotal, coef);
-  hipLaunchKernelGGL(point_lc_kernel, dim3(nCurves), dim3(64), 0, s, curves, nCurves, trig, out,
-                     chainOut, coef);
+int launch_point_lc(const TrialArgs& a, int nCurves, double* out, RootChain* chainOut,
+                    hipStream_t s) {
+  if (nCurves <= 0 || a.nPts <= 0) return 0;
+  hipLaunchKernelGGL(point_list_kernel, dim3((a.nPts + 255) / 256), dim3(256), 0, s, a);
+  const int rc = launch_solve_prep(a, a.nPts, s);
+  if (rc) return rc;
+  hipLaunchKernelGGL(point_lc_kernel, dim3(nCurves), dim3(64), 0, s, a.curves, nCurves, a.trig,
+                     out, chainOut, a.pool);
   return (int)hipGetLastError();
 }
 
@@ -905,111 +968,6 @@ __global__ void __launch_bounds__(64) ring_poly_kernel(const CurveDev* curves, c
   if (smp == 0) cross[p] = 0;
 }
 
-// The serial Laguerre routines of tl_math.h for one lane with every array in
-// registers: the degree is a template argument, so no array is indexed at
-// run time (tl_math.h's run-time degree puts them in scratch memory, which
-// made the disk samples several times slower).  The same operations in the
-// same order, so the same values.
-// lag_iter (laguerre.cc:18-99) for a polynomial of degree M.
-template <int M>
-__device__ __forceinline__ bool lag_iter_reg(const cx* poly, cx& xp, const TrigTable* trig) {
-  if constexpr (M == 1) {
-    if (cabs_(poly[1]) != 0.0) {
-      xp = cdiv(cneg(poly[0]), poly[1]);
-      return true;
-    }
-    xp = mk(999.0, 999.0);
-    return false;
-  } else {
-    const double frac[8] = {0.5, 0.23, 0.73, 0.13, 0.37, 0.61, 0.89, 1.0};
-    cx x = xp;
-    const double md = (double)M;
-    for (int i = 1; i <= kLagMaxIt; i++) {
-      cx b = poly[M];
-      double err = cabs_(b);
-      const double ax = cabs_(x);
-      cx s = mk(0.0, 0.0), f = mk(0.0, 0.0);
-#pragma unroll
-      for (int j = M - 1; j >= 0; j--) {
-        s = cadd(cmul(x, s), f);
-        f = cadd(cmul(x, f), b);
-        b = cadd(cmul(x, b), poly[j]);
-        err = cabs_(b) + ax * err;
-      }
-      err *= kLagEps;
-      if (cabs_(b) <= err) {
-        xp = x;
-        return true;
-      }
-      cx g = cdiv(f, b);
-      cx h = csub(cmul(g, g), cdiv(cscale(s, 2.0), b));
-      cx rad = cscale(csub(cscale(h, md), cmul(g, g)), md - 1.0);
-      cx sq = csqrt_(rad);
-      cx gp = cadd(g, sq);
-      cx gm = csub(g, sq);
-      // each modulus taken once (|x| is ax)
-      double agp = cabs_(gp);
-      const double agm = cabs_(gm);
-      if (agp < agm) {
-        gp = gm;
-        agp = agm;
-      }
-      cx dx;
-      if (agp > 0.0) dx = cdiv_rc(md, gp);
-      else dx = cscale(mk(trig->c[i], trig->s[i]), 1.0 + ax);
-      cx x1 = csub(x, dx);
-      if (x.re == x1.re && x.im == x1.im) {
-        xp = x;
-        return true;
-      }
-      if (i % kLagMT) x = x1;
-      else x = csub(x, cmul(mk(frac[(i / kLagMT) & 7], 0.0), dx));
-    }
-    xp = x;
-    return false;
-  }
-}
-
-// lag_solve's deflation steps J..1 (laguerre.cc:103-167): the root found at
-// step J goes to roots[DEG - J].
-template <int DEG, int J>
-__device__ __forceinline__ void lag_deflate_reg(cx* tmp, const cx* init, bool withInit, cx* roots,
-                                                const TrigTable* trig) {
-  if constexpr (J >= 1) {
-    cx x = withInit ? init[J] : mk(kLagEps, kLagEps);
-    if (!lag_iter_reg<J>(tmp, x, trig) && withInit) x = mk(kLagEps, kLagEps);
-    roots[DEG - J] = x;
-    cx b = tmp[J];
-#pragma unroll
-    for (int jj = J - 1; jj >= 0; jj--) {
-      cx c = tmp[jj];
-      tmp[jj] = b;
-      b = cadd(cmul(x, b), c);
-    }
-    lag_deflate_reg<DEG, J - 1>(tmp, init, withInit, roots, trig);
-  }
-}
-
-// lag_solve: the deflation, then each root polished on the full polynomial
-// in root order (the roots rotate through roots[0], so one copy of the
-// polishing code serves all of them).
-template <int DEG>
-__device__ __forceinline__ void lag_solve_reg(const cx* coeffs, const cx* init, bool withInit,
-                                              cx* roots, const TrigTable* trig) {
-  cx tmp[DEG + 1];
-#pragma unroll
-  for (int i = 0; i <= DEG; i++) tmp[i] = coeffs[i];
-  lag_deflate_reg<DEG, DEG>(tmp, init, withInit, roots, trig);
-#pragma unroll 1
-  for (int j = 0; j < DEG; j++) {
-    cx x = roots[0];
-    lag_iter_reg<DEG>(coeffs, x, trig);
-#pragma unroll
-    for (int k = 0; k < DEG - 1; k++) roots[k] = roots[k + 1];
-    roots[DEG - 1] = x;
-  }
-}
-
 // lag_check (laguerre.cc:188-198)
 template <int DEG>
 __device__ __forceinline__ bool lag_check_reg(const cx* coeffs, const cx* roots) {
@@ -1045,12 +1003,13 @@ __device__ __forceinline__ double lane_amp(const Lens& L, const cx* roots, unsig
 // 0): the sequence wl_get_images runs on a wavefront, with the Laguerre
 // routines above (the same values).  Leaves the roots in chain[0..9] and
 // returns the mask of the accepted images among them.
-__device__ __forceinline__ unsigned lane_images(const Lens& L, const cx* cf, cx* chain, cx zeta,
-                                                const TrigTable* trig, bool binImg) {
+__device__ __forceinline__ unsigned lane_images(const Lens& L, const cx (&cf)[11], cx* chain,
+                                                cx zeta, const TrigTable* trig, bool binImg) {
   bool withInit = true, second = false;
   while (true) {
     cx roots[10];
-    lag_solve_reg<10>(cf, chain, withInit, roots, trig);
+    bool oob = false;
+    lane_solve(cf, chain, withInit, roots, trig, oob);
     if (withInit && !lag_check_reg<10>(cf, roots)) {
       withInit = false;
       continue;
@@ -1159,7 +1118,10 @@ int launch_seed(const SeedArgs& a, hipStream_t s) {
   if (a.maxSplit < 1 || (long long)a.nCurves * a.maxSplit > (1ll << 30))
     return (int)hipErrorInvalidValue;
   if (a.pieceStart && !a.pieceBase) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(seed_kernel, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a);
+  if (a.slotTrace)
+    hipLaunchKernelGGL(seed_kernel<true>, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a);
+  else
+    hipLaunchKernelGGL(seed_kernel<false>, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a);
   return (int)hipGetLastError();
 }
 

@@ -1,0 +1,243 @@
+// Root solver of the image polynomial on the GPU: Laguerre's iteration of the
+// reference (laguerre.cc:18-198) with the same bits in every root, at a
+// fraction of the instructions the operation-by-operation restatement in
+// tl_math.h takes.
+//
+// What the reference's iteration computes falls in two kinds:
+//   * values that enter x (the Horner sums, the quotients f/b and 2s/b, the
+//     square root, the step m/g): these are computed with the reference's
+//     rounding, operation for operation;
+//   * values that are only compared (the error bound of |p(x)|, which of
+//     g + sq and g - sq is larger, the product check of the roots, the image
+//     test's residual): these are bracketed by cheap bounds, and the
+//     reference's own expressions are evaluated only where a comparison falls
+//     inside the bracket.
+// The moduli of the second kind (14 correctly rounded hypots per iteration)
+// were most of the chain's instructions.
+//
+// Quotients and square roots of operands in a safe range are taken without
+// the pre-scaling and special-value fix-up of the IEEE sequences, and a
+// square root hands its reciprocal on to the divisions by it (modulus
+// correction, csqrt).  Operands outside the range, signed zeros, kicks and
+// everything else unusual go through the general iteration.
+#pragma once
+
+#include "tl_math.h"
+
+namespace tl {
+
+// ---- in-range arithmetic ---------------------------------------------------
+// Reciprocal of b within about half a unit in the last place, for
+// 2^-900 <= |b| <= 2^900: the hardware estimate r0 (e = 1 - b r0, |e| below
+// 2^-22) and one third-order correction r0 (1 + e + e^2).
+__device__ __forceinline__ double rcp_near(double b) {
+  const double r0 = __builtin_amdgcn_rcp(b);
+  const double e = fma(-b, r0, 1.0);
+  const double p = fma(e, e, e);
+  return fma(r0, p, r0);
+}
+// a / b rounded to nearest from r = rcp_near(b), one correction by the exact
+// residual (Markstein), for operands and quotients within 2^-900 .. 2^900.
+__device__ __forceinline__ double quot_near(double a, double b, double r) {
+  const double q = a * r;
+  return fma(fma(-b, q, a), r, q);
+}
+// s = sqrt(a) rounded to nearest and h close to 1 / (2 s), for
+// 2^-600 <= a <= 2^600: the hardware reciprocal root y, s0 = a y, h0 = y/2 with
+// h0 s0 = 1/2 - e, one third-order step (1 - 2e)^-1/2 = 1 + e + 3/2 e^2, and the
+// exact residual.
+__device__ __forceinline__ void sqrt_near(double a, double& s, double& h) {
+  const double y = __builtin_amdgcn_rsq(a);
+  const double s0 = a * y, h0 = 0.5 * y;
+  const double e = fma(-h0, s0, 0.5);
+  const double p = e * fma(1.5, e, 1.0);
+  const double s1 = fma(s0, p, s0);
+  h = fma(h0, p, h0);
+  s = fma(fma(-s1, s1, a), h, s1);
+}
+// hyp_sel for 2^-240 <= ay <= ax <= 2^240 and ay > ax 2^-54.
+__device__ __forceinline__ double hyp_near(double ax, double ay) {
+  double h, hi;
+  sqrt_near(ax * ax + ay * ay, h, hi);
+  const double w = 2.0 * h;
+  const double r = fma(hi, fma(-w, hi, 1.0), hi);  // 1 / w
+  const double d1 = h - ay;
+  const double t1a = ax * (2.0 * d1 - ax);
+  const double t2a = (d1 - 2.0 * (ax - ay)) * d1;
+  const double d2 = h - ax;
+  const double t1b = 2.0 * d2 * (ax - 2.0 * ay);
+  const double t2b = (4.0 * d2 - ay) * ay + d2 * d2;
+  const bool lo = h <= 2.0 * ay;
+  const double t = lo ? t1a + t2a : t1b + t2b;
+  return h - quot_near(t, w, r);
+}
+__device__ __forceinline__ bool hyp_in_range(double ax, double ay) {
+  return ay >= 0x1p-240 && ax <= 0x1p+240 && ay > ax * 0x1p-54;
+}
+// csqrt_sel for re, im with hyp_in_range(max, min) of their magnitudes.
+__device__ __forceinline__ cx csqrt_near(double re, double im) {
+  const double fr = fabs(re), fi = fabs(im);
+  const double d = hyp_near(fmax(fr, fi), fmin(fr, fi));
+  double q, h;
+  sqrt_near(0.5 * (d + fr), q, h);
+  h = 2.0 * h;
+  const double w = 0.5 * quot_near(im, q, fma(h, fma(-q, h, 1.0), h));
+  const bool pos = re > 0.0;
+  return mk(pos ? q : fabs(w), copysign(pos ? w : q, im));
+}
+
+constexpr double kTinyOp = 0x1p-300, kHugeOp = 0x1p+300;
+
+// ---- Laguerre --------------------------------------------------------------
+// Horner sums of p at x: b[0] = p(x), and b[j + 1] is coefficient j of the
+// polynomial deflated by x (laguerre.cc:133-139).
+template <int M>
+__device__ __forceinline__ void horner_sums(const cx (&p)[M + 1], cx x, cx (&b)[M + 1]) {
+  b[M] = p[M];
+#pragma unroll
+  for (int j = M - 1; j >= 0; j--) b[j] = cadd(cmul(x, b[j + 1]), p[j]);
+}
+
+// The reference's iteration i at x, every value as laguerre.cc computes it;
+// b holds the Horner sums at x.  Returns true when x is accepted (and left
+// unchanged), else x is the next point.
+template <int M>
+__device__ __forceinline__ bool lag_general(const cx (&b)[M + 1], cx& x, int i,
+                                            const TrigTable* trig, bool& oob) {
+  cx f = mk(0.0, 0.0), s = mk(0.0, 0.0);
+#pragma unroll
+  for (int j = M - 1; j >= 0; j--) {
+    s = cadd(cmul(x, s), f);
+    f = cadd(cmul(x, f), b[j + 1]);
+  }
+  const double md = (double)M;
+  double err = cabs_(b[M]);
+  const double ax = cabs_(x);
+  double ab = err;
+#pragma unroll
+  for (int j = M - 1; j >= 0; j--) {
+    ab = cabs_(b[j]);
+    err = ab + ax * err;
+  }
+  if (ab <= err * kLagEps) return true;
+  const cx g = cdiv_sel(f, b[0]);
+  const cx h = csub(cmul(g, g), cdiv_sel(cscale(s, 2.0), b[0]));
+  const cx rad = cscale(csub(cscale(h, md), cmul(g, g)), md - 1.0);
+  const cx sq = csqrt_(rad);
+  cx gp = cadd(g, sq);
+  const cx gm = csub(g, sq);
+  double agp = cabs_(gp);
+  const double agm = cabs_(gm);
+  if (agp < agm) {
+    gp = gm;
+    agp = agm;
+  }
+  cx dx;
+  if (agp > 0.0) dx = cdiv_rc_sel(md, gp);
+  else dx = cscale(mk(trig->c[i], trig->s[i]), 1.0 + ax);
+  const cx x1 = csub(x, dx);
+  if (x.re == x1.re && x.im == x1.im) return true;
+  if (i % kLagMT) {
+    x = x1;
+  } else {
+    // Laguerre's fractional kicks (laguerre.cc:22), read modulo 8
+    const int k = (i / kLagMT) & 7;
+    const double frac = k == 0 ? 0.5 : k == 1 ? 0.23 : k == 2 ? 0.73 : k == 3 ? 0.13
+                      : k == 4 ? 0.37 : k == 5 ? 0.61 : k == 6 ? 0.89 : 1.0;
+    oob |= i / kLagMT >= 8;
+    x = csub(x, cmul(mk(frac, 0.0), dx));
+  }
+  return false;
+}
+
+// Laguerre::laguerre for a polynomial of degree M >= 2 held in registers.
+// Every lane runs its own x, or all lanes run the same one (UNI: the branches
+// are then taken on the whole wave).  Leaves the Horner sums at the returned
+// x in b, which are the coefficients of the deflated polynomial
+// (b[j + 1] = coefficient j, laguerre.cc:133-139).
+//
+// An iteration first runs the b recurrence alone: the one that accepts x (one
+// in two to three) needs no derivative.  The error bound sum |b_j| |x|^j is
+// bracketed by its 1-norm form E1: E1 / sqrt 2 <= E <= E1 (|x| from the
+// hardware root, good to 1e-7; the bracket is widened by 1e-5).
+template <int M, bool UNI>
+__device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M + 1],
+                                         const TrigTable* trig, bool& oob) {
+  constexpr double md = (double)M;
+  auto all = [](bool c) { return UNI ? __ballot(!c) == 0 : c; };
+  for (int i = 1; i <= kLagMaxIt; i++) {
+    const double n = cnorm(x);
+    // |x|, or NaN (which leaves every comparison undecided) where its square
+    // may have lost digits
+    const double ax = n > 1e-280 ? __builtin_amdgcn_sqrt(n) : __builtin_nan("");
+    b[M] = p[M];
+    double e1 = fabs(p[M].re) + fabs(p[M].im);
+#pragma unroll
+    for (int j = M - 1; j >= 0; j--) {
+      b[j] = cadd(cmul(x, b[j + 1]), p[j]);
+      e1 = fma(ax, e1, fabs(b[j].re) + fabs(b[j].im));
+    }
+    const double nb = cnorm(b[0]);
+    const double el = kLagEps * e1;
+    const double e2 = el * el;
+    if (all(nb < e2 * 0.49999 && e2 > 1e-250)) return true;
+    cx f = b[M], s = mk(0.0, 0.0);
+    // the recurrences' first step, from s = f = 0, leaves s = 0 and f = b[M]
+    // (up to the sign of a zero, which the range check below sends to
+    // lag_general wherever it could matter)
+    const bool far = nb > e2 * 1.0001 && nb > 1e-250;
+#pragma unroll
+    for (int j = M - 2; j >= 0; j--) {
+      s = cadd(cmul(x, s), f);
+      f = cadd(cmul(x, f), b[j + 1]);
+    }
+    // g = f / b and 2 s / b by Smith's quotient over one denominator
+    const cx B = b[0];
+    const bool ce = fabs(B.re) < fabs(B.im);
+    const double num = ce ? B.re : B.im, den = ce ? B.im : B.re;
+    const double ratio = quot_near(num, den, rcp_near(den));
+    const double denom = (num * ratio) + den;
+    const double rd = rcp_near(denom);
+    const cx s2 = cscale(s, 2.0);
+    const double far_ = f.re * ratio, fbr = f.im * ratio;
+    const double sar = s2.re * ratio, sbr = s2.im * ratio;
+    const double xf = ce ? far_ + f.im : fbr + f.re, yf = ce ? fbr - f.re : f.im - far_;
+    const double xs = ce ? sar + s2.im : sbr + s2.re, ys = ce ? sbr - s2.re : s2.im - sar;
+    const cx g = mk(quot_near(xf, denom, rd), quot_near(yf, denom, rd));
+    const cx g2 = cmul(g, g);
+    const cx h = csub(g2, mk(quot_near(xs, denom, rd), quot_near(ys, denom, rd)));
+    const cx rad = cscale(csub(cscale(h, md), g2), md - 1.0);
+    const cx sq = csqrt_near(rad.re, rad.im);
+    const cx gp = cadd(g, sq), gm = csub(g, sq);
+    const double np = cnorm(gp), nm = cnorm(gm);
+    const bool minus = np < nm;
+    const cx d = mk(minus ? gm.re : gp.re, minus ? gm.im : gp.im);
+    // the step m / d: Smith's quotient of a real numerator
+    const bool ce2 = fabs(d.re) < fabs(d.im);
+    const double num2 = ce2 ? d.re : d.im, den2 = ce2 ? d.im : d.re;
+    const double ratio2 = quot_near(num2, den2, rcp_near(den2));
+    const double denom2 = (num2 * ratio2) + den2;
+    const double rd2 = rcp_near(denom2);
+    const double mr = md * ratio2;
+    const double qa = quot_near(mr, denom2, rd2), qb = quot_near(md, denom2, rd2);
+    const cx x1 = mk(x.re - (ce2 ? qa : qb), x.im + (ce2 ? qb : qa));
+    // everything in range, every comparison decided, x moved, no kick
+    const double lo = fmin(fmin(fmin(fabs(xf), fabs(yf)), fmin(fabs(xs), fabs(ys))),
+                           fmin(fabs(num), fabs(num2)));
+    const double hi = fmax(fmax(fmax(fabs(f.re), fabs(f.im)), fmax(fabs(s2.re), fabs(s2.im))),
+                           fmax(fabs(den), fabs(den2)));
+    const double rx = fmax(fabs(rad.re), fabs(rad.im)), ry = fmin(fabs(rad.re), fabs(rad.im));
+    const bool ok = far && lo >= kTinyOp && hi <= kHugeOp && hyp_in_range(rx, ry) &&
+                    fmin(np, nm) < fmax(np, nm) * (1.0 - 1e-12) &&
+                    (x.re != x1.re || x.im != x1.im) && i % kLagMT != 0;
+    if (all(ok)) {
+      x = x1;
+      continue;
+    }
+    if (lag_general<M>(b, x, i, trig, oob)) return true;
+  }
+  horner_sums<M>(p, x, b);  // not converged: the sums where it stopped
+  return false;
+}
+
+}  // namespace tl
