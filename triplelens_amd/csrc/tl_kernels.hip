@@ -230,25 +230,33 @@ __device__ __forceinline__ bool wl_img_check(const Lens& L, const cx& z, cx zeta
 // solve's first step (it starts from 0): solve_prep_kernel has done both for
 // every solve of the run, and the chain only runs the deflation steps 9..1,
 // the polish and the tests.
+//
+// The record goes through LDS (`rec`, the wave's own 64 doubles): reading it
+// back, every lane gets every element by broadcast, 128 bits at a time.
 template <bool TRACED>
 __device__ __forceinline__ unsigned long long wl_get_images(const Lens& L, double v, cx freshv,
-                                                            bool slot, cx& chainv, int& have,
-                                                            const TrigTable* trig, bool binImg,
-                                                            bool& oob) {
+                                                            double* rec, bool slot, cx& chainv,
+                                                            int& have, const TrigTable* trig,
+                                                            bool binImg, bool& oob) {
   const int ln = __lane_id();
   const int fl = (int)rl(v, kRecFlags);
   if (have) {
-    cx c[11];
+    rec[ln] = v;
+    const double2* r2 = reinterpret_cast<const double2*>(rec);
+    auto get = [&](int k) {
+      const double2 e = r2[k / 2];
+      return mk(e.x, e.y);
+    };
+    cx c[11], p[10];
 #pragma unroll
-    for (int j = 0; j <= 10; j++) c[j] = mk(rl(v, 2 * j), rl(v, 2 * j + 1));
-    cx p[10];
-#pragma unroll
-    for (int j = 0; j < 10; j++) p[j] = mk(rl(v, kRecDefl + 2 * j), rl(v, kRecDefl + 2 * j + 1));
-    cx rootv = mk(rl(v, kRecRoot), rl(v, kRecRoot + 1));
+    for (int j = 0; j < 10; j++) p[j] = get(kRecDefl + 2 * j);
+    cx rootv = get(kRecRoot);
     bool firstOob = (fl & kRecOobFirst) != 0;
     if constexpr (TRACED) {
       if (slot) {
         firstOob = false;
+#pragma unroll
+        for (int j = 0; j <= 10; j++) c[j] = get(kRecCoef + 2 * j);
         cx x = rlc(chainv, 10), b[11];
         if (!lag_fast<10, true>(c, x, b, trig, firstOob)) {
           x = mk(kLagEps, kLagEps);
@@ -262,12 +270,14 @@ __device__ __forceinline__ unsigned long long wl_get_images(const Lens& L, doubl
     oob |= firstOob;
     wl_deflate<9>(p, rootv, chainv, trig, oob);
     // root r is polished on lane r; the other lanes repeat root 0
+#pragma unroll
+    for (int j = 0; j <= 10; j++) c[j] = get(kRecCoef + 2 * j);
     bool laneOob = false;
     cx b[11];
     lag_fast<10, false>(c, rootv, b, trig, laneOob);
     oob |= __ballot(laneOob) != 0;
     if (wl_check(c[10], c[0], rootv)) {
-      const bool ok = wl_img_check(L, rootv, mk(rl(v, kRecZeta), rl(v, kRecZeta + 1))) && ln < 10;
+      const bool ok = wl_img_check(L, rootv, get(kRecZeta)) && ln < 10;
       const unsigned long long m = __ballot(ok);
       const int n = __builtin_popcountll(m);
       // a valid count: even and at least 4, or for the binary lens odd and at
@@ -284,31 +294,47 @@ __device__ __forceinline__ unsigned long long wl_get_images(const Lens& L, doubl
   return (unsigned long long)(fl & 0x3ff);
 }
 
+// The lens as wave-uniform values (a copy that no store of the kernel can
+// alias, so that it is not read again at every position).
+__device__ __forceinline__ Lens uni_lens(const Lens& g) {
+  Lens L;
+  L.m1 = unid(g.m1); L.m2 = unid(g.m2); L.m3 = unid(g.m3);
+  L.z1 = mk(unid(g.z1.re), unid(g.z1.im));
+  L.z2 = mk(unid(g.z2.re), unid(g.z2.im));
+  L.z3 = mk(unid(g.z3.re), unid(g.z3.im));
+  return L;
+}
+
 // Walks a curve's solves in order (the pool holds them so): the record and
 // the fresh roots of the coming solve are loaded one solve ahead, and the
 // solve counts 64 positions at a time, so that the chain does not wait for
 // memory.
 struct SolveWalk {
-  const SolvePool& P;
+  const int* count;
+  const double* rec;  // this lane's element of the coming solve's record
+  const cx* fresh;
   int p, pEnd, k, cnt;
-  size_t sid;
   double v;
   cx f;
   __device__ __forceinline__ SolveWalk(const SolvePool& pool, int p0, int end)
-      : P(pool), p(p0), pEnd(end), k(64), cnt(0) {
-    sid = (size_t)uni(P.base[p0]);
+      : count(pool.count), p(p0), pEnd(end), k(64), cnt(0) {
+    const int ln = __lane_id();
+    const size_t sid = (size_t)uni(pool.base[p0]);
+    rec = pool.rec + sid * kRecSize + (ln < kRecSize ? ln : 0);
+    fresh = pool.fresh + sid * 10 + (ln < 10 ? ln : 0);
     fetch();
   }
   __device__ __forceinline__ void fetch() {
-    const int ln = __lane_id();
-    v = ln < kRecSize ? P.rec[sid * kRecSize + ln] : 0.0;
-    f = ln < 10 ? P.fresh[sid * 10 + ln] : mk(0.0, 0.0);
+    v = *rec;
+    f = *fresh;
+    rec += kRecSize;
+    fresh += 10;
   }
   // solves of the next position
   __device__ __forceinline__ int position() {
     if (k == 64) {
       const int q = p + __lane_id();
-      cnt = q < pEnd ? P.count[q] : 0;
+      cnt = q < pEnd ? count[q] : 0;
       k = 0;
     }
     p++;
@@ -318,7 +344,6 @@ struct SolveWalk {
   __device__ __forceinline__ void next(double& rv, cx& fv) {
     rv = v;
     fv = f;
-    sid++;
     fetch();
   }
 };
@@ -592,12 +617,14 @@ int launch_image_poly(const Lens& L, const cx* fixedPoly, const cx* zeta, int n,
 // only runs the root solves, the image tests and the seed output.
 template <bool TRACED>
 __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
+  __shared__ __align__(16) double rec[64];
   const int c = blockIdx.x / a.maxSplit, q = blockIdx.x % a.maxSplit;
   if (c >= a.nCurves) return;
   const int ln = __lane_id();
   const CurveDev& C = a.curves[c];
   if (q >= C.split) return;
-  const Lens L = C.L;
+  const Lens L = uni_lens(C.L);
+  const bool binImg = uni(C.binImg) != 0;
   cx chainv = mk(0.0, 0.0);
   int have = 0, calls = 0;
   if (q > 0) {
@@ -639,7 +666,7 @@ __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
       calls++;
       bool oob = false;
       const unsigned long long m =
-          wl_get_images<TRACED>(L, rv, fv, slot, chainv, have, a.trig, C.binImg, oob);
+          wl_get_images<TRACED>(L, rv, fv, rec, slot, chainv, have, a.trig, binImg, oob);
       if (oob) fl |= kFlagKickTable;
       emit_seeds(C, chainv, m, out, cnt, fl);
       if (sIdx == 0) {
@@ -675,7 +702,7 @@ __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
           a.ptCen[p] = make_double2(sx / amp, sy / amp);
           const double dist = sqrt(a.ptCausD2[p]);
           // inside a caustic: more images than the 4 (binary: 3) outside
-          a.ptCaus[p] = __builtin_popcountll(m) > (C.binImg ? 3 : 4) ? -dist : dist;
+          a.ptCaus[p] = __builtin_popcountll(m) > (binImg ? 3 : 4) ? -dist : dist;
           a.ptPair[p] = amp > 0.0 ? (t1 + t2) / amp : 0.0;
         }
       }
@@ -699,15 +726,15 @@ __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
 // ---- verified speculative chain (SpecArgs) ---------------------------------
 // The chain's solves of the walk's next position (centre, then caustic trial
 // points), as seed_kernel runs them, without output.
-__device__ __forceinline__ void chain_step(const SeedArgs& a, const CurveDev& C, const Lens& L,
-                                           SolveWalk& W, cx& chainv, int& have) {
+__device__ __forceinline__ void chain_step(const Lens& L, bool binImg, const TrigTable* trig,
+                                           SolveWalk& W, double* rec, cx& chainv, int& have) {
   const int nSolve = W.position();
   for (int sIdx = 0; sIdx < nSolve; sIdx++) {
     double rv;
     cx fv;
     W.next(rv, fv);
     bool oob = false;
-    wl_get_images<false>(L, rv, fv, false, chainv, have, a.trig, C.binImg, oob);
+    wl_get_images<false>(L, rv, fv, rec, false, chainv, have, trig, binImg, oob);
   }
 }
 
@@ -727,12 +754,15 @@ __device__ __forceinline__ void piece_range(const CurveDev& C, int q, int& b, in
 // Round 1: piece q from a fresh solve (piece 0 from the curve's chain state),
 // on into the next piece for sp.overlap positions.
 __global__ void __launch_bounds__(64) spec_round1_kernel(SeedArgs a, SpecArgs sp) {
+  __shared__ __align__(16) double rec[64];
   const int c = blockIdx.x / a.maxSplit, q = blockIdx.x % a.maxSplit;
   if (c >= a.nCurves) return;
   const int ln = __lane_id();
   const CurveDev& C = a.curves[c];
   if (q >= C.split) return;
-  const Lens L = C.L;
+  const Lens L = uni_lens(C.L);
+  const bool binImg = uni(C.binImg) != 0;
+  const int pointBase = uni(C.pointBase);
   cx chainv = mk(0.0, 0.0);
   int have = 0;
   if (q == 0) {
@@ -750,8 +780,8 @@ __global__ void __launch_bounds__(64) spec_round1_kernel(SeedArgs a, SpecArgs sp
   if (b >= stop) return;
   SolveWalk W(a.pool, C.pointBase + b, C.pointBase + stop);
   for (int i = b; i < stop; i++) {
-    const int p = C.pointBase + i;
-    chain_step(a, C, L, W, chainv, have);
+    const int p = pointBase + i;
+    chain_step(L, binImg, a.trig, W, rec, chainv, have);
     cx* dst = (i < e ? sp.own : sp.ext) + (size_t)p * 10;
     if (ln < 10) dst[ln] = chainv;
   }
@@ -762,6 +792,7 @@ __global__ void __launch_bounds__(64) spec_round1_kernel(SeedArgs a, SpecArgs sp
 // the following pieces until its state equals a piece's own at one of that
 // piece's first sp.overlap positions.
 __global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp) {
+  __shared__ __align__(16) double rec[64];
   const int c = blockIdx.x / a.maxSplit, q = blockIdx.x % a.maxSplit;
   if (c >= a.nCurves) return;
   const int ln = __lane_id();
@@ -771,32 +802,39 @@ __global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp
   int b, e;
   piece_range(C, q, b, e);
   const int lim = e < b + sp.overlap ? e : b + sp.overlap;
+  const int pointBase = uni(C.pointBase);
+  // six positions at a time, one root to a lane
   bool agree = false;
-  for (int i = b; i < lim && !agree; i++) {
-    const size_t p = (size_t)C.pointBase + i;
-    cx v = mk(0.0, 0.0), o = v;
-    if (ln < 10) {
-      v = sp.ext[p * 10 + ln];
-      o = sp.own[p * 10 + ln];
+  const int r = ln % 10, k = ln / 10;
+  for (int i = b; i < lim && !agree; i += 6) {
+    bool eq = false;
+    if (k < 6 && i + k < lim) {
+      const size_t at = ((size_t)pointBase + i + k) * 10 + r;
+      const cx v = sp.ext[at], o = sp.own[at];
+      eq = __double_as_longlong(v.re) == __double_as_longlong(o.re) &&
+           __double_as_longlong(v.im) == __double_as_longlong(o.im);
     }
-    agree = state_equal(v, o);
+    const unsigned long long m = __ballot(eq);
+    for (int j = 0; j < 6; j++) agree |= ((m >> (10 * j)) & 0x3ffull) == 0x3ffull;
   }
   if (ln == 0) sp.merged[gq] = agree ? 1 : 0;
   if (agree) return;
-  const Lens L = C.L;
+  const Lens L = uni_lens(C.L);
+  const bool binImg = uni(C.binImg) != 0;
   cx chainv = mk(0.0, 0.0);
-  if (ln < 10) chainv = sp.own[((size_t)C.pointBase + b - 1) * 10 + ln];
+  if (ln < 10) chainv = sp.own[((size_t)pointBase + b - 1) * 10 + ln];
   int have = 1;
   int qq = q, qb = b, qe = e;  // the piece the chain is in
-  const long long n = (long long)C.lcLength + 1;
+  const long long n = (long long)uni((int)C.lcLength) + 1;
+  const int split = uni(C.split);
   if (b >= n) return;
-  SolveWalk W(a.pool, C.pointBase + b, C.pointBase + (int)n);
+  SolveWalk W(a.pool, pointBase + b, pointBase + (int)n);
   for (int i = b; i < n; i++) {
     if (i == qe) {
       // entering piece qq + 1: the chain's state before its first position
       qq++;
       qb = qe;
-      piece_range(C, qq, qb, qe);
+      qe = (int)(n * (qq + 1) / split);
       const int j = qq - q - 1;
       if (j >= sp.depth) {
         if (ln == 0) sp.repTarget[gq] = -2;
@@ -804,12 +842,12 @@ __global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp
       }
       if (ln < 10) sp.repState[((size_t)gq * sp.depth + j) * 10 + ln] = chainv;
     }
-    const int p = C.pointBase + i;
+    const int p = pointBase + i;
     // the piece's own state, loaded before the solve that it is compared with
     const bool mayJoin = qq > q && i < qb + sp.overlap;
     cx own = mk(0.0, 0.0);
     if (mayJoin && ln < 10) own = sp.own[(size_t)p * 10 + ln];
-    chain_step(a, C, L, W, chainv, have);
+    chain_step(L, binImg, a.trig, W, rec, chainv, have);
     if (mayJoin && state_equal(chainv, own)) {
       if (ln == 0) sp.repTarget[gq] = qq;
       return;
@@ -887,21 +925,23 @@ __global__ void point_list_kernel(TrialArgs a) {
 __global__ void __launch_bounds__(64) point_lc_kernel(const CurveDev* curves, int nCurves,
                                                       const TrigTable* trig, double* out,
                                                       RootChain* chainOut, SolvePool pool) {
+  __shared__ __align__(16) double rec[64];
   const int c = blockIdx.x;
   if (c >= nCurves) return;
   const int ln = __lane_id();
   const CurveDev& C = curves[c];
-  const Lens L = C.L;
+  const Lens L = uni_lens(C.L);
+  const bool binImg = uni(C.binImg) != 0;
+  const int pointBase = uni(C.pointBase), len = uni((int)C.lcLength);
   cx chainv = ln <= 10 ? C.chain[ln <= 10 ? ln : 0] : mk(0.0, 0.0);
   int have = C.chainHave;
-  SolveWalk W(pool, C.pointBase, C.pointBase + (int)C.lcLength);
-  for (unsigned i = 0; i < C.lcLength; i++) {
+  SolveWalk W(pool, pointBase, pointBase + len);
+  for (int i = 0; i < len; i++) {
     double rv;
     cx fv;
     W.next(rv, fv);
     bool oob = false;
-    unsigned long long m = wl_get_images<false>(L, rv, fv, false, chainv, have, trig, C.binImg,
-                                                oob);
+    unsigned long long m = wl_get_images<false>(L, rv, fv, rec, false, chainv, have, trig, binImg, oob);
     const double term = ((m >> ln) & 1ull) ? point_amp_term(L, chainv) : 0.0;
     double amp = 0.0;
     while (m) {
@@ -909,7 +949,7 @@ __global__ void __launch_bounds__(64) point_lc_kernel(const CurveDev* curves, in
       m &= m - 1;
       amp += rl(term, k);
     }
-    if (ln == 0) out[C.pointBase + (int)i] = amp;
+    if (ln == 0) out[pointBase + i] = amp;
   }
   if (ln <= 10) chainOut[c].tempRoots[ln] = chainv;
   if (ln == 0) {

@@ -26,6 +26,24 @@
 
 namespace tl {
 
+// Smaller and larger magnitude, one instruction each (fmin and fmax of the
+// language quiet signalling NaNs first; a NaN operand here gives the other one
+// or a NaN, and every caller compares the result so that a NaN in any of its
+// operands is seen by another comparison).
+__device__ __forceinline__ double min_abs(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double max_abs(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// Keeps both sides of a select computed (the compiler would otherwise branch
+// around the shorter one: a taken branch costs one wavefront about 50 cycles).
+__device__ __forceinline__ void keep(double& a) { asm volatile("" : "+v"(a)); }
+
 // ---- in-range arithmetic ---------------------------------------------------
 // Reciprocal of b within about half a unit in the last place, for
 // 2^-900 <= |b| <= 2^900: the hardware estimate r0 (e = 1 - b r0, |e| below
@@ -62,22 +80,20 @@ __device__ __forceinline__ double hyp_near(double ax, double ay) {
   const double w = 2.0 * h;
   const double r = fma(hi, fma(-w, hi, 1.0), hi);  // 1 / w
   const double d1 = h - ay;
-  const double t1a = ax * (2.0 * d1 - ax);
-  const double t2a = (d1 - 2.0 * (ax - ay)) * d1;
+  double ta = ax * (2.0 * d1 - ax) + (d1 - 2.0 * (ax - ay)) * d1;
   const double d2 = h - ax;
-  const double t1b = 2.0 * d2 * (ax - 2.0 * ay);
-  const double t2b = (4.0 * d2 - ay) * ay + d2 * d2;
-  const bool lo = h <= 2.0 * ay;
-  const double t = lo ? t1a + t2a : t1b + t2b;
-  return h - quot_near(t, w, r);
+  double tb = 2.0 * d2 * (ax - 2.0 * ay) + ((4.0 * d2 - ay) * ay + d2 * d2);
+  keep(ta);
+  keep(tb);
+  return h - quot_near(h <= 2.0 * ay ? ta : tb, w, r);
 }
 __device__ __forceinline__ bool hyp_in_range(double ax, double ay) {
-  return ay >= 0x1p-240 && ax <= 0x1p+240 && ay > ax * 0x1p-54;
+  return (ay >= 0x1p-240) & (ax <= 0x1p+240) & (ay > ax * 0x1p-54);
 }
 // csqrt_sel for re, im with hyp_in_range(max, min) of their magnitudes.
 __device__ __forceinline__ cx csqrt_near(double re, double im) {
-  const double fr = fabs(re), fi = fabs(im);
-  const double d = hyp_near(fmax(fr, fi), fmin(fr, fi));
+  const double fr = fabs(re);
+  const double d = hyp_near(max_abs(re, im), min_abs(re, im));
   double q, h;
   sqrt_near(0.5 * (d + fr), q, h);
   h = 2.0 * h;
@@ -96,6 +112,15 @@ __device__ __forceinline__ void horner_sums(const cx (&p)[M + 1], cx x, cx (&b)[
   b[M] = p[M];
 #pragma unroll
   for (int j = M - 1; j >= 0; j--) b[j] = cadd(cmul(x, b[j + 1]), p[j]);
+}
+
+// The step dx from x with Laguerre's fractional kick (laguerre.cc:22) of
+// iteration i, a multiple of kLagMT; the table is read modulo 8.
+__device__ __forceinline__ cx lag_kick(cx x, cx dx, int i) {
+  const int k = (i / kLagMT) & 7;
+  const double frac = k == 0 ? 0.5 : k == 1 ? 0.23 : k == 2 ? 0.73 : k == 3 ? 0.13
+                    : k == 4 ? 0.37 : k == 5 ? 0.61 : k == 6 ? 0.89 : 1.0;
+  return csub(x, cmul(mk(frac, 0.0), dx));
 }
 
 // The reference's iteration i at x, every value as laguerre.cc computes it;
@@ -140,12 +165,8 @@ __device__ __forceinline__ bool lag_general(const cx (&b)[M + 1], cx& x, int i,
   if (i % kLagMT) {
     x = x1;
   } else {
-    // Laguerre's fractional kicks (laguerre.cc:22), read modulo 8
-    const int k = (i / kLagMT) & 7;
-    const double frac = k == 0 ? 0.5 : k == 1 ? 0.23 : k == 2 ? 0.73 : k == 3 ? 0.13
-                      : k == 4 ? 0.37 : k == 5 ? 0.61 : k == 6 ? 0.89 : 1.0;
     oob |= i / kLagMT >= 8;
-    x = csub(x, cmul(mk(frac, 0.0), dx));
+    x = lag_kick(x, dx, i);
   }
   return false;
 }
@@ -159,12 +180,15 @@ __device__ __forceinline__ bool lag_general(const cx (&b)[M + 1], cx& x, int i,
 // An iteration first runs the b recurrence alone: the one that accepts x (one
 // in two to three) needs no derivative.  The error bound sum |b_j| |x|^j is
 // bracketed by its 1-norm form E1: E1 / sqrt 2 <= E <= E1 (|x| from the
-// hardware root, good to 1e-7; the bracket is widened by 1e-5).
+// hardware root, good to 1e-7; the bracket is widened by 1e-5).  One
+// evaluation in a hundred falls inside it and gets moduli from the hardware
+// root, which leave a bracket of 1e-4.
 template <int M, bool UNI>
 __device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M + 1],
                                          const TrigTable* trig, bool& oob) {
   constexpr double md = (double)M;
   auto all = [](bool c) { return UNI ? __ballot(!c) == 0 : c; };
+  auto any = [](bool c) { return UNI ? __ballot(c) != 0 : c; };
   for (int i = 1; i <= kLagMaxIt; i++) {
     const double n = cnorm(x);
     // |x|, or NaN (which leaves every comparison undecided) where its square
@@ -180,14 +204,25 @@ __device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M 
     const double nb = cnorm(b[0]);
     const double el = kLagEps * e1;
     const double e2 = el * el;
-    if (all(nb < e2 * 0.49999 && e2 > 1e-250)) return true;
-    cx f = b[M], s = mk(0.0, 0.0);
-    // the recurrences' first step, from s = f = 0, leaves s = 0 and f = b[M]
-    // (up to the sign of a zero, which the range check below sends to
-    // lag_general wherever it could matter)
-    const bool far = nb > e2 * 1.0001 && nb > 1e-250;
+    bool far = nb > e2 * 1.0001;  // nb above 1e-250 follows from lo below
+    if (__builtin_expect(!all(far), 0)) {
+      if (all((nb < e2 * 0.49999) & (e2 > 1e-250))) return true;
+      if (any(!far)) {
+        // inside the bracket: the sum with moduli from the hardware root
+        double e = __builtin_amdgcn_sqrt(cnorm(b[M]));
 #pragma unroll
-    for (int j = M - 2; j >= 0; j--) {
+        for (int j = M - 1; j >= 0; j--) e = fma(ax, e, __builtin_amdgcn_sqrt(cnorm(b[j])));
+        const double eh = kLagEps * e;
+        if (all((nb < eh * eh * 0.9999) & (eh * eh > 1e-250))) return true;
+        far = nb > eh * eh * 1.0001;
+      }
+    }
+    // the recurrences' first two steps, from s = f = 0, leave s = b[M] and
+    // f = x b[M] + b[M - 1] (up to the sign of a zero, which the range check
+    // below sends to lag_general wherever it could matter)
+    cx s = b[M], f = cadd(cmul(x, b[M]), b[M - 1]);
+#pragma unroll
+    for (int j = M - 3; j >= 0; j--) {
       s = cadd(cmul(x, s), f);
       f = cadd(cmul(x, f), b[j + 1]);
     }
@@ -221,19 +256,25 @@ __device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M 
     const double mr = md * ratio2;
     const double qa = quot_near(mr, denom2, rd2), qb = quot_near(md, denom2, rd2);
     const cx x1 = mk(x.re - (ce2 ? qa : qb), x.im + (ce2 ? qb : qa));
-    // everything in range, every comparison decided, x moved, no kick
-    const double lo = fmin(fmin(fmin(fabs(xf), fabs(yf)), fmin(fabs(xs), fabs(ys))),
-                           fmin(fabs(num), fabs(num2)));
-    const double hi = fmax(fmax(fmax(fabs(f.re), fabs(f.im)), fmax(fabs(s2.re), fabs(s2.im))),
-                           fmax(fabs(den), fabs(den2)));
-    const double rx = fmax(fabs(rad.re), fabs(rad.im)), ry = fmin(fabs(rad.re), fabs(rad.im));
-    const bool ok = far && lo >= kTinyOp && hi <= kHugeOp && hyp_in_range(rx, ry) &&
-                    fmin(np, nm) < fmax(np, nm) * (1.0 - 1e-12) &&
-                    (x.re != x1.re || x.im != x1.im) && i % kLagMT != 0;
-    if (all(ok)) {
-      x = x1;
+    // everything in range, every comparison decided, x moved.  (lo bounds den
+    // and den2 from below as well; f, s, g and den2 too large for the
+    // quotients leave rad out of its range.)
+    const double lo = min_abs(min_abs(min_abs(xf, yf), min_abs(xs, ys)), min_abs(num, num2));
+    const bool ok = far & (lo >= kTinyOp) & (fabs(den) <= kHugeOp) &
+                    hyp_in_range(max_abs(rad.re, rad.im), min_abs(rad.re, rad.im)) &
+                    (min_abs(np, nm) < max_abs(np, nm) * (1.0 - 1e-12)) &
+                    ((x.re != x1.re) | (x.im != x1.im));
+    if (__builtin_expect(all(ok), 1)) {
+      if (__builtin_expect(i % kLagMT == 0, 0)) {
+        oob |= i / kLagMT >= 8;
+        x = lag_kick(x, mk(ce2 ? qa : qb, ce2 ? -qb : -qa), i);
+      } else {
+        x = x1;
+      }
       continue;
     }
+    keep(x.re);  // the general iteration shares nothing with the code above
+    keep(x.im);
     if (lag_general<M>(b, x, i, trig, oob)) return true;
   }
   horner_sums<M>(p, x, b);  // not converged: the sums where it stopped
