@@ -763,3 +763,19 @@ def test_autotuner_keeps_results(E, tmp_path):
     finally:
         for n, v in autotune.DEFAULTS.items():
             E.set_option(n, v)
+
+
+@pytest.mark.parametrize("n", [1, 2, 1025, 2049, 7200])
+def test_critical_curves_batch_sizes(E, n):
+    """tl_ccc_batch at the sizes where its layout changes (one geometry per
+    wavefront up to 1024, more beyond, a last wavefront that is not full):
+    every geometry's curves equal those of a batch of its own."""
+    rng = np.random.default_rng(n)
+    base = np.array([[1.0, 0.8, 1.1, 0.1, 0.1], [0.7, 1.6, 4.0, 1e-3, 0.2],
+                     [1.1, 1.0, 1.0, 1e-3, 0.0], [2.5, 0.4, 2.0, 0.3, 1e-4]])
+    rows = base[rng.integers(0, len(base), n)]
+    cc, ca = E.ccc_batch(rows)
+    for r in base:
+        one_cc, one_ca = E.ccc_batch(r[None])
+        at = np.nonzero((rows == r).all(axis=1))[0]
+        assert (cc[at] == one_cc).all() and (ca[at] == one_ca).all()

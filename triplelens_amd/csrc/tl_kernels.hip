@@ -501,27 +501,27 @@ __global__ void __launch_bounds__(64) trial_poly_kernel(TrialArgs a, int nSolves
 
 // The root solver for one lane per solve, every array in registers (the
 // degree is a template argument).
-// The deflation steps J..1 of Laguerre::solveRoots (laguerre.cc:103-167): the
-// root found at step J goes to roots[10 - J].
-template <int J>
+// The deflation steps J..1 of Laguerre::solveRoots (laguerre.cc:103-167) for a
+// polynomial of degree DEG: the root found at step J goes to roots[DEG - J].
+template <int DEG, int J>
 __device__ __forceinline__ void lane_deflate(const cx (&p)[J + 1], const cx* init, bool withInit,
                                              cx* roots, const TrigTable* trig, bool& oob) {
   cx x = withInit ? init[J] : mk(kLagEps, kLagEps);
   if constexpr (J == 1) {
     if (p[1].re != 0.0 || p[1].im != 0.0) x = cdiv(cneg(p[0]), p[1]);
     else x = withInit ? mk(kLagEps, kLagEps) : mk(999.0, 999.0);
-    roots[9] = x;
+    roots[DEG - 1] = x;
   } else {
     cx b[J + 1];
     if (!lag_fast<J, false>(p, x, b, trig, oob) && withInit) {
       x = mk(kLagEps, kLagEps);
       horner_sums<J>(p, x, b);
     }
-    roots[10 - J] = x;
+    roots[DEG - J] = x;
     cx q[J];
 #pragma unroll
     for (int j = 0; j < J; j++) q[j] = b[j + 1];
-    lane_deflate<J - 1>(q, init, withInit, roots, trig, oob);
+    lane_deflate<DEG, J - 1>(q, init, withInit, roots, trig, oob);
   }
 }
 // solveRoots: the deflation, then each root polished on the full polynomial
@@ -529,7 +529,7 @@ __device__ __forceinline__ void lane_deflate(const cx (&p)[J + 1], const cx* ini
 // polishing code serves all of them).
 __device__ __forceinline__ void lane_solve(const cx (&c)[11], const cx* init, bool withInit,
                                            cx* roots, const TrigTable* trig, bool& oob) {
-  lane_deflate<10>(c, init, withInit, roots, trig, oob);
+  lane_deflate<10, 10>(c, init, withInit, roots, trig, oob);
 #pragma unroll 1
   for (int j = 0; j < 10; j++) {
     cx x = roots[0], b[11];
@@ -1134,22 +1134,96 @@ int launch_clear_flag_bits(uint32_t* flags, const int* pts, int n, uint32_t bits
   return (int)hipGetLastError();
 }
 
-// Critical curves and caustics of many geometries, one per lane: the host
-// routine (critical_curves_into) with the host's step table, so every value
-// is the host's, and the reference's, to the bit.
-__global__ void __launch_bounds__(64) ccc_kernel(const Lens* lenses, int n, const CccTable* tab,
-                                                 const TrigTable* trig, cx* cc, cx* ca) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= n) return;
-  const size_t off = (size_t)g * 6 * kCccSteps;
-  critical_curves_into(lenses[g], *tab, trig, cc + off, ca + off);
+// Critical curves of many geometries: critical_curves_into with the host's
+// step table, every value the host's, and the reference's, to the bit.  The
+// 500 steps are a chain (each polishes the last one's roots), but the six
+// roots of a step are independent: eight lanes hold a geometry, lane r < 6
+// its root r.  A wavefront holds perWave geometries (1 while the launch then
+// has at most one wavefront per SIMD, up to 8 beyond).  One lane per geometry
+// with the unbracketed iteration took 40 ms for any number of geometries up
+// to a few thousand; the chain is bound by its instruction count.
+template <int CTRL>
+__device__ __forceinline__ cx dpp_times(const cx& v) {
+  auto mv = [](double x) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                            (unsigned)lo));
+  };
+  return cmul(v, mk(mv(v.re), mv(v.im)));
+}
+
+__global__ void __launch_bounds__(64) ccc_kernel(const Lens* lenses, int n, int perWave,
+                                                 const CccTable* tab, const TrigTable* trig,
+                                                 cx* cc) {
+  const int ln = __lane_id(), r = ln & 7;
+  const int slot = ln >> 3;
+  // lanes without a geometry of their own repeat the wavefront's last one
+  const int first = blockIdx.x * perWave;
+  int g = first + (slot < perWave ? slot : perWave - 1);
+  if (g >= n) g = n - 1;
+  const Lens L = lenses[g];
+  const bool mine = r < 6 && slot < perWave && first + slot < n;
+  const CccPoly st = ccc_poly_static(L);
+  cx* out = cc + (size_t)g * 6 * kCccSteps + (size_t)(r < 6 ? r : 0) * kCccSteps;
+  cx x = mk(0.0, 0.0);
+  bool oob = false;
+  for (int j = 0; j < kCccSteps; j++) {
+    cx p[7], b[7];
+    ccc_poly(L, st, tab->e[j], p);
+    bool fresh = j == 0;
+    if (!fresh) {
+      lag_fast<6, false>(p, x, b, trig, oob);
+      // Laguerre::checkRoots (laguerre.cc:188-198): the product of the roots,
+      // taken in any order where it decides (see wl_check), else in root order
+      cx v = r < 6 ? x : mk(1.0, 0.0);
+      v = dpp_times<0xB1>(v);   // lanes 1, 0, 3, 2
+      v = dpp_times<0x4E>(v);   // lanes 2, 3, 0, 1
+      v = dpp_times<0x141>(v);  // lanes 7 .. 0
+      const double A = cnorm(cmul(p[6], v));
+      const double T = cnorm(p[0]) * ((1.0 - 1.0e-5) * (1.0 - 1.0e-5));
+      const bool big = T > 1.0001e-16 && A < 1e300;
+      const bool yes = big && A > T * (1.0 + 1e-9), no = big && A < T * (1.0 - 1e-9);
+      fresh = no;
+      if (__ballot(!yes && !no)) {
+        cx roots[6];
+#pragma unroll
+        for (int k = 0; k < 6; k++)
+          roots[k] = mk(__shfl(x.re, (ln & ~7) + k, 64), __shfl(x.im, (ln & ~7) + k, 64));
+        if (!yes && !no) fresh = !lag_check_reg<6>(p, roots);
+      }
+    }
+    if (__ballot(fresh)) {
+      cx roots[6];
+      lane_deflate<6, 6>(p, nullptr, false, roots, trig, oob);
+      cx y = roots[0];
+#pragma unroll
+      for (int k = 1; k < 6; k++)
+        if (r == k) y = roots[k];
+      lag_fast<6, false>(p, y, b, trig, oob);
+      if (fresh) x = y;
+    }
+    if (mine) out[j] = x;
+  }
+}
+
+__global__ void caustic_kernel(const Lens* lenses, int n, const cx* cc, cx* ca) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  const size_t per = 6 * kCccSteps;
+  if (i < (size_t)n * per) ca[i] = caustic_point(lenses[i / per], cc[i]);
 }
 
 int launch_ccc(const Lens* lenses, int n, const CccTable* tab, const TrigTable* trig, cx* cc,
                cx* ca, hipStream_t s) {
   if (n <= 0) return 0;
-  hipLaunchKernelGGL(ccc_kernel, dim3((n + 63) / 64), dim3(64), 0, s, lenses, n, tab, trig, cc,
-                     ca);
+  int perWave = (n + 1023) / 1024;
+  if (perWave > 8) perWave = 8;
+  hipLaunchKernelGGL(ccc_kernel, dim3((n + perWave - 1) / perWave), dim3(64), 0, s, lenses, n,
+                     perWave, tab, trig, cc);
+  const size_t all = (size_t)n * 6 * kCccSteps;
+  hipLaunchKernelGGL(caustic_kernel, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, s, lenses,
+                     n, cc, ca);
   return (int)hipGetLastError();
 }
 

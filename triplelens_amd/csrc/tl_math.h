@@ -345,48 +345,57 @@ struct CccTable { cx e[kCccSteps]; };
 // its CriticalCurveCaustic from a LensPar (lcirs.cc:16), a constructor that
 // leaves the binary flag unset (ccc.cc:28-39), so this triple-lens form
 // also serves m3 = 0: two of its branches then sit at the massless z3.
+struct CccPoly {
+  cx p0, p1, z2pz3;
+};
+TL_HD CccPoly ccc_poly_static(const Lens& L) {
+  CccPoly s;
+  s.z2pz3 = cadd(L.z2, L.z3);
+  s.p1 = cscale(cmul(cmul(cscale(L.z2, 2.0), L.z3), s.z2pz3), L.m2 + L.m3 - 1.0);
+  s.p0 = cscale(cmul(cmul(cmul(cneg(L.z2), L.z2), L.z3), L.z3), L.m2 + L.m3 - 1.0);
+  return s;
+}
+// The polynomial at the step whose exp(i phi) is e.
+TL_HD void ccc_poly(const Lens& L, const CccPoly& st, cx e, cx* p) {
+  const cx z2 = L.z2, z3 = L.z3;
+  const double m2 = L.m2, m3 = L.m3;
+  p[0] = st.p0;
+  p[1] = st.p1;
+  p[6] = cneg(e);
+  p[5] = cmul(cscale(e, 2.0), st.z2pz3);
+  const cx q4 = cmul(e, cadd(cadd(cmul(z2, z2), cmul(z3, z3)), cmul(cscale(z2, 4.0), z3)));
+  p[4] = mk(1.0 - q4.re, -q4.im);
+  p[3] = cadd(cadd(cmul(cmul(cmul(cscale(e, 2.0), z2), z3), st.z2pz3),
+                   cscale(cscale(z2, 2.0), m2 - 1.0)),
+              cscale(cscale(z3, 2.0), m3 - 1.0));
+  const cx t1 = cmul(cmul(cmul(cmul(cneg(e), z2), z2), z3), z3);
+  const cx t2 = cmul(cscale(z2, 4.0 * (1.0 - m3 - m2)), z3);
+  const cx t3 = cscale(cmul(z2, z2), m2 - 1.0);
+  const cx t4 = cscale(cmul(z3, z3), m3 - 1.0);
+  p[2] = csub(csub(cadd(t1, t2), t3), t4);
+}
+// The caustic point of critical point s.
+TL_HD cx caustic_point(const Lens& L, cx s) {
+  cx v = csub(s, cdiv_rc(L.m1, cconj(csub(s, L.z1))));
+  v = csub(v, cdiv_rc(L.m2, cconj(csub(s, L.z2))));
+  return csub(v, cdiv_rc(L.m3, cconj(csub(s, L.z3))));
+}
 TL_HD void critical_curves_into(const Lens& L, const CccTable& tab, const TrigTable* trig,
                                 cx* cc, cx* ca) {
   const int len = kCccSteps;
-  const cx z2 = L.z2, z3 = L.z3;
-  const double m2 = L.m2, m3 = L.m3;
-  cx p[7];
-  const cx z2pz3 = cadd(z2, z3);
-  p[1] = cscale(cmul(cmul(cscale(z2, 2.0), z3), z2pz3), m2 + m3 - 1.0);
-  p[0] = cscale(cmul(cmul(cmul(cneg(z2), z2), z3), z3), m2 + m3 - 1.0);
-  cx roots[6];
-  bool have = false;
+  const CccPoly st = ccc_poly_static(L);
+  cx p[7], roots[6];
   for (int j = 0; j < len; j++) {
-    const cx e = tab.e[j];
-    p[6] = cneg(e);
-    p[5] = cmul(cscale(e, 2.0), z2pz3);
-    const cx q4 = cmul(e, cadd(cadd(cmul(z2, z2), cmul(z3, z3)), cmul(cscale(z2, 4.0), z3)));
-    p[4] = mk(1.0 - q4.re, -q4.im);
-    p[3] = cadd(cadd(cmul(cmul(cmul(cscale(e, 2.0), z2), z3), z2pz3),
-                     cscale(cscale(z2, 2.0), m2 - 1.0)),
-                cscale(cscale(z3, 2.0), m3 - 1.0));
-    const cx t1 = cmul(cmul(cmul(cmul(cneg(e), z2), z2), z3), z3);
-    const cx t2 = cmul(cscale(z2, 4.0 * (1.0 - m3 - m2)), z3);
-    const cx t3 = cscale(cmul(z2, z2), m2 - 1.0);
-    const cx t4 = cscale(cmul(z3, z3), m3 - 1.0);
-    p[2] = csub(csub(cadd(t1, t2), t3), t4);
-    if (!have) {
+    ccc_poly(L, st, tab.e[j], p);
+    if (j == 0) {
       lag_solve<6>(p, nullptr, roots, trig);
-      have = true;
     } else {
       lag_polish<6>(p, roots, trig);
       if (!lag_check<6>(p, roots)) lag_solve<6>(p, nullptr, roots, trig);
     }
     for (int k = 0; k < 6; k++) cc[k * len + j] = roots[k];
   }
-  for (int k = 0; k < 6; k++)
-    for (int j = 0; j < len; j++) {
-      const cx s = cc[k * len + j];
-      cx v = csub(s, cdiv_rc(L.m1, cconj(csub(s, L.z1))));
-      v = csub(v, cdiv_rc(L.m2, cconj(csub(s, L.z2))));
-      v = csub(v, cdiv_rc(L.m3, cconj(csub(s, L.z3))));
-      ca[k * len + j] = v;
-    }
+  for (int i = 0; i < 6 * len; i++) ca[i] = caustic_point(L, cc[i]);
 }
 
 // ImgPoint::imgCheck (imgpoint.cc:72-90)
