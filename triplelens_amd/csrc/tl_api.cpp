@@ -316,6 +316,7 @@ struct Engine {
   DBuf<unsigned long long> dGrp;  // run-table slices: group bases, then masks
   DBuf<unsigned long long> dLSum, dPtSum;  // split sums (hi * 2^32 + lo): 2 words each
   DBuf<Task> dQBuf;
+  DBuf<double> dPoints;  // records of a fill's batch points
   DBuf<RootChain> dChain;
   DBuf<double> dPointLC;
   DBuf<Lens> dLenses;
@@ -489,7 +490,6 @@ CurveDev to_dev(const Curve& c, cx s, cx e, int pointBase, int causticBase) {
   d.rho2pow = c.rho2pow;
   d.ldA = c.ldA;
   d.ldB = c.ldB;
-  d.sumScale = sum_scale_for(c.ldA, c.ldB);
   d.blx = c.blx;
   d.bly = c.bly;
   d.step = c.step;
@@ -787,7 +787,7 @@ void Engine::run(Job& job) {
   }
 
   std::vector<uint64_t> ptRays(nPts, 0);
-  std::vector<double> ptSumAll(nPts, 0.0);  // brightness sums in fixed-point units
+  std::vector<double> ptSumAll(nPts, 0.0);  // root sums in units of 1 / kSumScale
   // amoeba print-out: the runs of every point of the curves that asked for it
   bool wantAmoebae = false;
   for (auto* c : job.curves) wantAmoebae |= c->amoebaOut && job.runSeeds;
@@ -859,6 +859,7 @@ void Engine::run(Job& job) {
       for (int k = 0; k < nSeeds[gp]; k++) seedTasks.push_back(make_int2(b, k));
     }
     dBatchPts.ensure(nb);
+    dPoints.ensure((size_t)nb * kPointRec);
     dSeedTasks.ensure(seedTasks.size());
     dPtCount.ensure(nb);
     dPtSum.ensure(2 * (size_t)nb);
@@ -901,6 +902,7 @@ void Engine::run(Job& job) {
       fa.ptPos = dPtPos.p;
       fa.batchPts = dBatchPts.p;
       fa.nBatch = nb;
+      fa.points = dPoints.p;
       fa.seedTasks = dSeedTasks.p;
       fa.nSeedTasks = (int)seedTasks.size();
       fa.seeds = dSeeds.p;
@@ -959,6 +961,7 @@ void Engine::run(Job& job) {
           int rc = launch_fill_reset(fa, stream);
           if (!rc) rc = launch_clear_u64(dPtCount.p, nb, 0, stream);
           if (!rc) rc = launch_clear_u64(dPtSum.p, 2 * (unsigned long long)nb, 0, stream);
+          if (!rc) rc = launch_fill_points(fa, stream);
           if (!rc) rc = launch_fill(fa, nWg, stream);
           if (!rc) rc = launch_resolve(fa, labelCap, dPtCount.p, dPtSum.p, stream);
           const hipError_t ec = hipStreamEndCapture(stream, &graph);
@@ -982,6 +985,7 @@ void Engine::run(Job& job) {
         HIPCHK((hipError_t)launch_fill_reset(fa, stream));
         HIPCHK((hipError_t)launch_clear_u64(dPtCount.p, nb, 0, stream));
         HIPCHK((hipError_t)launch_clear_u64(dPtSum.p, 2 * (unsigned long long)nb, 0, stream));
+        HIPCHK((hipError_t)launch_fill_points(fa, stream));
         HIPCHK(hipEventRecord(ev0, stream));
         HIPCHK((hipError_t)launch_fill(fa, nWg, stream));
         HIPCHK(hipEventRecord(ev1, stream));
@@ -1099,7 +1103,7 @@ void Engine::run(Job& job) {
     for (int i = 0; i < n; i++) {
       const int p = pointBase[k] + i;
       c.rays[i] = ptRays[p];
-      c.full[i] = (ptSumAll[p] / hc[k].sumScale) * c.ampScale;
+      c.full[i] = (c.ldA * (double)ptRays[p] + c.ldB * (ptSumAll[p] / kSumScale)) * c.ampScale;
       c.flags[i] = flags[p];
     }
     if (job.runSeeds) {

@@ -42,7 +42,6 @@ struct CurveDev {
   cx fixedPoly[11];            // ImgPoint::getCoeffsOptNoZ of the lens (image_poly_static)
   double rho, rho2, rho2pow;   // rho, rho*rho (ray test), pow(rho, 2.0) (intersection test)
   double ldA, ldB;             // limb-darkening profile A + B sqrt(1 - r^2)
-  double sumScale;             // fixed-point scale of the brightness sum (sum_scale_for)
   double blx, bly, step, Ldbl, Nd;
   long long N;
   double sx, sy, ex, ey;       // trajectory
@@ -170,12 +169,15 @@ struct SpecArgs {
   int* failed;           // set when some curve could not be resolved
 };
 
+constexpr int kPointRec = 32;    // doubles of a batch point's record
+
 struct FillArgs {
   const CurveDev* curves;
   const int* ptCurve;         // global point -> curve
   const double2* ptPos;       // global point -> source position
   const int* batchPts;        // batch point -> global point
   int nBatch;
+  double* points;             // [batch point * kPointRec + k] constants (fill_points_kernel)
   const int2* seedTasks;      // (batch point, seed slot) in processing order
   int nSeedTasks;
   const int2* seeds;
@@ -190,7 +192,7 @@ struct FillArgs {
   int* lparent;
   int* lpoint;
   unsigned long long* lcount;
-  unsigned long long* lsum;   // 2 words per label: brightness total hi * 2^32 + lo (add_split)
+  unsigned long long* lsum;   // 2 words per label: root total hi * 2^32 + lo (flush_acc)
   int* labelNext;
   int labelCap;
   // shared queue (tasks handed between waves) and termination
@@ -253,6 +255,8 @@ int launch_ring_amp(const CurveDev* curves, const int* ptCurve, const double2* p
                     cx* coef, hipStream_t s);
 int launch_ccc(const Lens* lenses, int n, const CccTable* tab, const TrigTable* trig, cx* cc,
                cx* ca, hipStream_t s);
+// The batch points' records (before launch_fill).
+int launch_fill_points(const FillArgs& a, hipStream_t s);
 int launch_fill(const FillArgs& a, int nWorkgroups, hipStream_t s);
 int fill_resident_workgroups();
 int launch_clear_flag_bits(uint32_t* flags, const int* pts, int n, uint32_t bits, hipStream_t s);
@@ -269,21 +273,14 @@ int launch_resolve(const FillArgs& a, int nLabels, unsigned long long* ptCount,
 int launch_point_lc(const TrialArgs& a, int nCurves, double* out, RootChain* chainOut,
                     hipStream_t s);
 
-// Fixed-point brightness sum: each pixel's A + B sqrt(1 - r^2) is rounded to
-// a multiple of 1/scale and summed as an integer, which makes the sum
-// independent of the order in which pixels are visited.  The scale is 2^34
-// (rounding below 3e-11 of a pixel's value) for profiles whose brightness
-// stays within 2 (every linear profile with 0 <= u <= 1, and the default),
-// halved per doubling beyond, so that one pixel never exceeds 2^35 units and
-// one run (at most 2^25 pixels) 2^60.  Wave-local totals are flushed before
-// they pass 2^61; label and point totals are kept in two 64-bit words, the
-// low 32 bits of every addition and the rest, so that they do not wrap.
-constexpr double kSumScale = 17179869184.0;  // 2^34
-inline double sum_scale_for(double ldA, double ldB) {
-  const double peak = fabs(ldA) + fabs(ldB);
-  double s = kSumScale;
-  while (peak * s > 2.0 * kSumScale && s > 1.0) s *= 0.5;
-  return s;
-}
+// Fixed-point brightness sum: of each counted pixel's brightness A + B r,
+// r = sqrt(1 - distance^2 / rho^2), the root r is rounded to a multiple of
+// 1/kSumScale and summed as an integer, which makes the sum independent of
+// the order in which pixels are visited; a point's magnification is then
+// (A pixels + B sum / kSumScale) ampScale.  One pixel adds at most 2^36 units
+// and one run (at most 2^25 pixels) 2^61; label and point totals are kept in
+// two 64-bit words, the low 32 bits of every addition and the rest, so that
+// they do not wrap.
+constexpr double kSumScale = 68719476736.0;  // 2^36
 
 }  // namespace tl

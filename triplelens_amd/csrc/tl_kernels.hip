@@ -6,6 +6,8 @@
 //  seed_kernel    per light curve, the reference's seed sequence: point images
 //                 with the root-reuse chain, then the images of caustic trial
 //                 points (src/LightCurves/lcirs.cc:116-165), as pixel seeds.
+//  solve_prep_kernel  what a solve of the chain needs that does not depend on
+//                 the chain (its first deflation step, its fresh solve).
 //  fill_kernel    one persistent, work-stealing launch that grows the image
 //                 "amoebae" of a batch of source positions: wavefronts pop
 //                 row-check tasks, evaluate 64 pixels per step with the FP64
@@ -43,13 +45,6 @@ __device__ __forceinline__ bool acas(unsigned long long* p, unsigned long long* 
                                               __ATOMIC_RELAXED, AGENT);
 }
 __device__ __forceinline__ int aldi(int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, AGENT); }
-__device__ __forceinline__ bool acasi(int* p, int* expected, int desired) {
-  return __hip_atomic_compare_exchange_strong(p, expected, desired, __ATOMIC_RELAXED,
-                                              __ATOMIC_RELAXED, AGENT);
-}
-__device__ __forceinline__ long long afaddl(long long* p, long long v) {
-  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, AGENT);
-}
 __device__ __forceinline__ void mem_order() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0);
@@ -60,9 +55,6 @@ __device__ __forceinline__ long long wave_sum(long long v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
-
-template <typename T>
-__device__ __forceinline__ T bcast0(T v) { return __shfl(v, 0, 64); }
 
 // Wave-uniform values in scalar registers (the first active lane's value;
 // used where every lane holds the same value or lane 0 holds the result).
@@ -1255,79 +1247,163 @@ __device__ __forceinline__ unsigned long long run_key(int b, int row, int xl) {
   return ((unsigned long long)(row + 1) << 39) | ((unsigned long long)(unsigned)xl << 14) |
          (unsigned long long)(b & (kGroupPoints - 1));
 }
-// Entry of probe i from hash h in batch point b's slice.
-__device__ __forceinline__ unsigned long long run_slot(const FillArgs& A, int b,
-                                                       unsigned long long h, int i) {
-  const int g = b >> 14;
-  return A.grpBase[g] + ((h + (unsigned long long)i) & A.grpMask[g]);
+// Start of a run's probe sequence in its slice: 32-bit multiplicative mixing
+// of the key's halves (scalar instructions; the runs of an image differ in
+// row and column by small steps, which the two multipliers spread).
+__device__ __forceinline__ unsigned hash_run(unsigned long long key) {
+  unsigned h = (unsigned)key * 0x9E3779B1u + (unsigned)(key >> 32) * 0x85EBCA77u;
+  h ^= h >> 15;
+  h *= 0xC2B2AE3Du;
+  return h ^ (h >> 13);
 }
-__device__ __forceinline__ unsigned long long hash_run(unsigned long long key) {
-  unsigned long long h = key;
-  h ^= h >> 33;
-  h *= 0xff51afd7ed558ccdull;
-  h ^= h >> 33;
-  h *= 0xc4ceb9fe1a85ec53ull;
-  h ^= h >> 33;
-  return h;
+
+// A wave-uniform value the compiler knows nothing about.  What a task's rare
+// cases need is derived from such copies where they arise: the compiler would
+// otherwise compute all of it ahead of the row loop, for every task, and spill
+// it.
+__device__ __forceinline__ int opq(int x) {
+  x = uni(x);
+  asm volatile("" : "+s"(x));
+  return x;
+}
+// The launch's arguments, read where they are used (scalar loads from the
+// kernel's argument segment) instead of being held in registers: FillArgs is
+// the fill kernel's only argument.
+typedef const __attribute__((address_space(4))) FillArgs* ArgPtr;
+__device__ __forceinline__ ArgPtr opq(ArgPtr a) {
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
+// ---- single-lane memory operations of a wavefront ---------------------------
+// A worker's shared-state updates are made by lane 0 alone, with the
+// execution mask set around the instruction instead of a branch on the lane
+// number: a divergent branch inside the task loop makes the compiler turn
+// the loop's uniform branches into masked flow.  Each returning operation
+// waits for its result in the same block.
+__device__ __forceinline__ unsigned long long cas64_lane0(unsigned long long* p,
+                                                          unsigned long long expected,
+                                                          unsigned long long desired) {
+  typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+  const u64x2 d = {desired, expected};
+  unsigned long long old, save;
+  asm volatile(
+      "s_mov_b64 %1, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "global_atomic_cmpswap_x2 %0, %2, %3, off sc0\n\t"
+      "s_waitcnt vmcnt(0)\n\t"
+      "s_mov_b64 exec, %1"
+      : "=&v"(old), "=&s"(save)
+      : "v"(p), "v"(d)
+      : "memory");
+  return (unsigned long long)uni64((long long)old);
+}
+__device__ __forceinline__ int cas32_lane0(int* p, int expected, int desired) {
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  const i32x2 d = {desired, expected};
+  int old;
+  unsigned long long save;
+  asm volatile(
+      "s_mov_b64 %1, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "global_atomic_cmpswap %0, %2, %3, off sc0\n\t"
+      "s_waitcnt vmcnt(0)\n\t"
+      "s_mov_b64 exec, %1"
+      : "=&v"(old), "=&s"(save)
+      : "v"(p), "v"(d)
+      : "memory");
+  return uni(old);
+}
+__device__ __forceinline__ int add32_lane0(int* p, int v) {
+  int old;
+  unsigned long long save;
+  asm volatile(
+      "s_mov_b64 %1, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "global_atomic_add %0, %2, %3, off sc0\n\t"
+      "s_waitcnt vmcnt(0)\n\t"
+      "s_mov_b64 exec, %1"
+      : "=&v"(old), "=&s"(save)
+      : "v"(p), "v"(v)
+      : "memory");
+  return uni(old);
+}
+__device__ __forceinline__ void add64_lane0(unsigned long long* p, unsigned long long v) {
+  unsigned long long save;
+  asm volatile(
+      "s_mov_b64 %0, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "global_atomic_add_x2 %1, %2, off\n\t"
+      "s_mov_b64 exec, %0"
+      : "=&s"(save)
+      : "v"(p), "v"(v)
+      : "memory");
+}
+__device__ __forceinline__ void or32_lane0(uint32_t* p, uint32_t v) {
+  unsigned long long save;
+  asm volatile(
+      "s_mov_b64 %0, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "global_atomic_or %1, %2, off\n\t"
+      "s_mov_b64 exec, %0"
+      : "=&s"(save)
+      : "v"(p), "v"(v)
+      : "memory");
+}
+__device__ __forceinline__ void store64_lane0(unsigned long long* p, unsigned long long v) {
+  unsigned long long save;
+  asm volatile(
+      "s_mov_b64 %0, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "global_store_dwordx2 %1, %2, off sc1\n\t"
+      "s_mov_b64 exec, %0"
+      : "=&s"(save)
+      : "v"(p), "v"(v)
+      : "memory");
+}
+__device__ __forceinline__ void store32_lane0(int* p, int v) {
+  unsigned long long save;
+  asm volatile(
+      "s_mov_b64 %0, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "global_store_dword %1, %2, off sc1\n\t"
+      "s_mov_b64 exec, %0"
+      : "=&s"(save)
+      : "v"(p), "v"(v)
+      : "memory");
 }
 
 enum { kInsNew = 1, kInsDup = 0, kInsFull = -1 };
 
-// Records run (b, row, xl, xr) with `label` (lane 0 works, the result is
-// broadcast).  Returns kInsNew, kInsFull, or kInsDup with the stored label in
-// the upper half: (label << 8) | kInsDup.  The slow path probes from the
-// run's home slot on.
-__device__ __forceinline__ int insert_run_slow(const FillArgs& A, int b, int row, int xl, int xr,
-                                            int label) {
-  int res = kInsFull;
-  if (__lane_id() == 0) {
-    const unsigned long long key = run_key(b, row, xl);
-    const unsigned long long w1 =
-        ((unsigned long long)(unsigned)label << 32) | (unsigned long long)(unsigned)xr;
-    const unsigned long long h = hash_run(key);
-    for (int i = 0; i < A.probeLimit; i++) {
-      const unsigned long long idx = run_slot(A, b, h, i);
-      unsigned long long expected = 0;
-      if (acas(&A.htab[2 * idx], &expected, key)) {
-        ast(&A.htab[2 * idx + 1], w1);
-        res = kInsNew;
-        break;
-      }
-      if (expected == key) {
-        // the winner writes word1 right after its compare-and-swap
-        unsigned long long v = ald(&A.htab[2 * idx + 1]);
-        for (int spin = 0; spin < (1 << 20) && v == kEmpty1; spin++) {
-          __builtin_amdgcn_s_sleep(2);
-          v = ald(&A.htab[2 * idx + 1]);
-        }
-        const int dl = v == kEmpty1 ? -1 : (int)(v >> 32);
-        res = dl < 0 ? kInsFull : ((dl << 8) | kInsDup);
-        break;
-      }
+// Records run (b, row, xl, xr) with `label` in the slice of mask + 1 entries
+// at tab.  Returns kInsNew, kInsFull, or kInsDup with the label stored by the
+// run's first finder in `other`.
+__device__ __forceinline__ int insert_run(unsigned long long* tab, unsigned mask, ArgPtr args,
+                                          int b, int row, int xl, int xr, int label, int& other) {
+  const unsigned long long key = run_key(b, row, xl);
+  unsigned idx = hash_run(key) & mask;
+  for (int i = 0;;) {
+    unsigned long long* e = tab + 2 * (size_t)idx;
+    const unsigned long long old = cas64_lane0(e, 0, key);
+    if (__builtin_expect(old == 0, 1)) {
+      store64_lane0(e + 1, ((unsigned long long)(unsigned)label << 32) |
+                               (unsigned long long)(unsigned)xr);
+      return kInsNew;
     }
-  }
-  return uni(res);
-}
-
-// Fast path: the run's home slot is free (the common case at load <= 1/2).
-__device__ __forceinline__ int insert_run(const FillArgs& A, int b, int row, int xl, int xr,
-                                          int label) {
-  int res = -2;
-  if (__lane_id() == 0) {
-    const unsigned long long key = run_key(b, row, xl);
-    const unsigned long long idx = run_slot(A, b, hash_run(key), 0);
-    unsigned long long expected = 0;
-    if (acas(&A.htab[2 * idx], &expected, key)) {
-      ast(&A.htab[2 * idx + 1],
-          ((unsigned long long)(unsigned)label << 32) | (unsigned long long)(unsigned)xr);
-      res = kInsNew;
+    if (old == key) {
+      // the winner writes word1 right after its compare-and-swap
+      unsigned long long v = (unsigned long long)uni64((long long)ald(e + 1));
+      for (int spin = 0; spin < (1 << 20) && v == kEmpty1; spin++) {
+        __builtin_amdgcn_s_sleep(2);
+        v = (unsigned long long)uni64((long long)ald(e + 1));
+      }
+      other = (int)(v >> 32);
+      return v == kEmpty1 || other < 0 ? kInsFull : kInsDup;
     }
+    idx = (idx + 1) & mask;
+    if (++i >= opq(args)->probeLimit) return kInsFull;
   }
-  res = uni(res);
-  if (res == -2) res = insert_run_slow(A, b, row, xl, xr, label);
-  return res;
 }
-
 
 // ---------------------------------------------------------------------------
 // Labels: union-find over flood labels; label b (< nBatch) is the class of
@@ -1342,15 +1418,21 @@ __device__ __forceinline__ int find_root(int* parent, int x) {
   return x;
 }
 
-__device__ __forceinline__ void unite(const FillArgs& A, int a, int b) {
-  if (__lane_id() == 0 && a >= 0 && b >= 0 && a != b) {
-    for (int it = 0; it < (1 << 16); it++) {
-      const int ra = find_root(A.lparent, a), rb = find_root(A.lparent, b);
-      if (ra == rb) break;
-      const int hi = ra > rb ? ra : rb, lo = ra > rb ? rb : ra;
-      int expected = hi;
-      if (acasi(&A.lparent[hi], &expected, lo)) break;
-    }
+__device__ __forceinline__ int uni_root(int* parent, int x) {
+  for (int it = 0; it < (1 << 20); it++) {
+    const int p = uni(aldi(&parent[x]));
+    if (p == x) return x;
+    x = p;
+  }
+  return x;
+}
+
+__device__ __forceinline__ void unite(int* parent, int a, int b) {
+  for (int it = 0; it < (1 << 16) && a != b; it++) {
+    const int ra = uni_root(parent, a), rb = uni_root(parent, b);
+    if (ra == rb) break;
+    const int hi = ra > rb ? ra : rb, lo = ra > rb ? rb : ra;
+    if (cas32_lane0(&parent[hi], hi, lo) == hi) break;
   }
 }
 
@@ -1381,104 +1463,46 @@ __device__ __forceinline__ Task words_task(const unsigned long long (&w)[4]) {
   return t;
 }
 
-__device__ __forceinline__ bool q_push(const FillArgs& A, const Task& t) {
-  int ok = 0;
-  if (__lane_id() == 0) {
-    unsigned long long pos = ald(A.qtail);
-    for (int it = 0; it < (1 << 20); it++) {
-      const unsigned long long idx = pos & (A.qcap - 1);
-      const unsigned long long seq = ald(&A.qseq[idx]);
-      const long long dif = (long long)(seq - pos);
-      if (dif == 0) {
-        if (acas(A.qtail, &pos, pos + 1)) {
-          unsigned long long w[4];
-          task_words(t, w);
-          unsigned long long* dst = reinterpret_cast<unsigned long long*>(&A.qbuf[idx]);
-          ast(&dst[0], w[0]);
-          ast(&dst[1], w[1]);
-          ast(&dst[2], w[2]);
-          ast(&dst[3], w[3]);
-          mem_order();
-          ast(&A.qseq[idx], pos + 1);
-          ok = 1;
-          break;
-        }
-      } else if (dif < 0) {
-        break;  // full
-      } else {
-        pos = ald(A.qtail);
+__device__ __forceinline__ bool q_push(ArgPtr args, const Task& t) {
+  const ArgPtr a = opq(args);
+  unsigned long long* const qtail = a->qtail;
+  unsigned long long* const qseq = a->qseq;
+  const unsigned long long qcap = a->qcap;
+  unsigned long long pos = (unsigned long long)uni64((long long)ald(qtail));
+  for (int it = 0; it < (1 << 20); it++) {
+    const unsigned long long idx = pos & (qcap - 1);
+    const unsigned long long seq = (unsigned long long)uni64((long long)ald(&qseq[idx]));
+    const long long dif = (long long)(seq - pos);
+    if (dif < 0) return false;  // full
+    if (dif == 0) {
+      const unsigned long long old = cas64_lane0(qtail, pos, pos + 1);
+      if (old == pos) {
+        unsigned long long w[4];
+        task_words(t, w);
+        unsigned long long* dst = reinterpret_cast<unsigned long long*>(&a->qbuf[idx]);
+        for (int k = 0; k < 4; k++) store64_lane0(dst + k, w[k]);
+        mem_order();
+        store64_lane0(&qseq[idx], pos + 1);
+        return true;
       }
+      pos = old;
+    } else {
+      pos = (unsigned long long)uni64((long long)ald(qtail));
     }
   }
-  return bcast0(ok) != 0;
+  return false;
 }
 
-__device__ __forceinline__ void flag_point(const FillArgs& A, int gp, uint32_t f) {
-  if (__lane_id() == 0) atomicOr(&A.flags[gp], f);
+__device__ __forceinline__ void flag_point(ArgPtr args, int gp, uint32_t f) {
+  or32_lane0(opq(args)->flags + opq(gp), f);
 }
 
 __device__ __forceinline__ void afaddi(int* p, int v) {
   __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, AGENT);
 }
 
-// ---------------------------------------------------------------------------
-// Row scanning
-// ---------------------------------------------------------------------------
-// Everything the ray test of one row needs, held by value so that it stays
-// in registers across the scan.
-struct RowCtx {
-  Lens L;
-  double blx, bly, step, rho2, invRho2, ldA, ldB, sumScale;
-  double y, px, py;
-  int N;
-  int map;      // ray map of the row: kMapInRange, kMapTriple or kMapBinary
-  int inRange;  // the position's lens and grid allow kMapInRange rows
-};
-constexpr int kMapInRange = 0;  // irsSIMD with the in-range division
-constexpr int kMapTriple = 1;   // irsSIMD with IEEE division
-constexpr int kMapBinary = 2;   // irsBinary (m3 = 0)
-
-// a / b rounded to nearest, for 2^-500 <= |a| <= 2^10 and
-// 2^-500 <= |b| <= 2^500: the hardware reciprocal estimate, two
-// Newton-Raphson refinements, the quotient estimate and one correction by
-// the residual a - b q computed exactly with a fused multiply-add
-// (Markstein's correctly rounded division).  This is the IEEE double
-// division sequence without its operand pre-scaling and special-value
-// fix-up, which leave operands and results unchanged in that range (every
-// intermediate value stays normal), so the quotient is the IEEE quotient
-// to the bit.
-__device__ __forceinline__ double div_in_range(double a, double b) {
-  double r = __builtin_amdgcn_rcp(b);
-  double t = fma(-b, r, 1.0);
-  r = fma(r, t, r);
-  t = fma(-b, r, 1.0);
-  r = fma(r, t, r);
-  const double q = a * r;
-  const double e = fma(-b, q, a);
-  return fma(e, r, q);
-}
-
-// irs_ray (the irsSIMD lane order, lcirs.cc:290-341) with its three
-// quotients m_k / |z - z_k|^2 taken by div_in_range: the same value to the
-// bit on rows where every |z - z_k|^2 lies in [2^-500, 2^500] and every
-// mass in [2^-500, 2^10] (row_in_range checks this per row).
-__device__ __forceinline__ double irs_ray_in_range(const Lens& L, double x, double y, double sx,
-                                                   double sy) {
-  double dr3 = L.z3.re - x, dr2 = L.z2.re - x, dr1 = L.z1.re - x, drs = sx - x;
-  double di3 = L.z3.im - y, di2 = L.z2.im - y, di1 = L.z1.im - y, dis = sy - y;
-  double q3 = dr3 * dr3 + di3 * di3;
-  double q2 = dr2 * dr2 + di2 * di2;
-  double q1 = dr1 * dr1 + di1 * di1;
-  double c3 = div_in_range(L.m3, q3), c2 = div_in_range(L.m2, q2), c1 = div_in_range(L.m1, q1);
-  double tr3 = dr3 * c3, tr2 = dr2 * c2, tr1 = dr1 * c1, trs = -drs;
-  double ti3 = di3 * c3, ti2 = di2 * c2, ti1 = di1 * c1, tis = -dis;
-  double r0 = tr3 + tr1, r1 = tr2 + trs;
-  double i0 = ti3 + ti1, i1 = ti2 + tis;
-  return (r0 + r1) * (r0 + r1) + (i0 + i1) * (i0 + i1);
-}
-
-// Self-test of div_in_range against IEEE division on n operand pairs drawn
-// from its range: random sign, exponent and mantissa (one pair in two), the
+// Self-test of the in-range quotient (quot_near) and square root (sqrt_near)
+// against the IEEE operations on n operand pairs drawn from their range: random sign, exponent and mantissa (one pair in two), the
 // ends of the range, and numerators built as the rounded product of the
 // denominator and a quotient half an ulp above a random double (the
 // quotients nearest a rounding boundary).  bad counts the pairs whose
@@ -1519,8 +1543,14 @@ __global__ void div_check_kernel(long long n, unsigned long long seed, unsigned 
       b = ends[(r1 % 3) * 2 + ((r1 >> 4) & 1)] * ((r1 >> 8) & 1 ? -1.0 : 1.0);
       if (kind == 7) b = make(r1, -500, 499);
     }
-    const double x = div_in_range(a, b), y = a / b;
+    const double x = quot_near(a, b, rcp_near(b)), y = a / b;
     cnt += __double_as_longlong(x) != __double_as_longlong(y) ? 1 : 0;
+    if (kind < 4) {
+      // the ends of the range hold the two mantissas sqrt_near leaves out
+      double r, h;
+      sqrt_near(fabs(b), r, h);
+      cnt += __double_as_longlong(r) != __double_as_longlong(sqrt(fabs(b))) ? 1 : 0;
+    }
   }
   if (cnt) atomicAdd(bad, cnt);
 }
@@ -1535,104 +1565,374 @@ int launch_div_check(long long n, unsigned long long seed, unsigned long long* b
   return (int)hipGetLastError();
 }
 
-// Whether a position's lens and pixel grid keep every row's squared lens
-// distances below 2^500 and its masses in [2^-500, 2^10]: lens and pixel
-// coordinates at most 2^200 in magnitude.
-__device__ __forceinline__ bool lens_in_range(const Lens& L, double blx, double bly, double step,
-                                              int N) {
-  const double lim = 0x1p200, mlo = 0x1p-500, mhi = 0x1p10;
-  const double ext = step * (double)N;
-  const bool grid = fabs(blx) + ext <= lim && fabs(bly) + ext <= lim;
-  const bool pos = fabs(L.z1.re) <= lim && fabs(L.z1.im) <= lim && fabs(L.z2.re) <= lim &&
-                   fabs(L.z2.im) <= lim && fabs(L.z3.re) <= lim && fabs(L.z3.im) <= lim;
-  const bool mass = L.m1 >= mlo && L.m1 <= mhi && L.m2 >= mlo && L.m2 <= mhi && L.m3 >= mlo &&
-                    L.m3 <= mhi;
-  return grid && pos && mass;
+// ---------------------------------------------------------------------------
+// Row scanning
+// ---------------------------------------------------------------------------
+// What a fill needs of one batch point, one record of 32 doubles
+// (fill_points_kernel): a worker loads it with lane k holding element k and
+// reads elements from the lanes, so that a change of position costs one
+// dependent load.
+enum {
+  kPcM1, kPcM2, kPcM3, kPcX1, kPcY1, kPcX2, kPcY2, kPcX3, kPcY3,  // lens
+  kPcBlx, kPcBly, kPcStep,  // pixel grid
+  kPcPx, kPcPy,             // source position
+  kPcRho, kPcRho2, kPcInv,  // radius, its square, 1 / square
+  kPcExt,                   // bound of the coordinates' magnitudes (fast rows)
+  kPcLo, kPcHi,             // rho^2 -+ the band of rows far from the lenses
+  kPcN, kPcGp,              // grid size; global point
+  kPcFlags                  // kPt* bits
+};
+constexpr int kPtBinary = 1;  // irsBinary (m3 = 0)
+constexpr int kPtFast = 2;    // lens and grid allow fast rows
+constexpr int kPtLimb = 4;    // the profile's square-root term is not zero
+constexpr int kPtHeavy = 8;   // predicted rays reach shareRays
+
+// Half-width of the undecided band of the squared distance about rho^2 for
+// rays whose terms' magnitudes sum to at most E (see Ray).
+__device__ __forceinline__ double ray_band(double E, double rho) {
+  const double delta = 0x1p-46 * E;
+  return 2.0 * delta * (2.0 * rho + delta);
+}
+constexpr double kFarRow = 0x1p-10;
+
+__global__ void fill_points_kernel(FillArgs A) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= A.nBatch) return;
+  const int gp = A.batchPts[b];
+  const CurveDev& C = A.curves[A.ptCurve[gp]];
+  double* r = A.points + (size_t)b * kPointRec;
+  const Lens& L = C.L;
+  const double2 pos = A.ptPos[gp];
+  r[kPcM1] = L.m1; r[kPcM2] = L.m2; r[kPcM3] = L.m3;
+  r[kPcX1] = L.z1.re; r[kPcY1] = L.z1.im;
+  r[kPcX2] = L.z2.re; r[kPcY2] = L.z2.im;
+  r[kPcX3] = L.z3.re; r[kPcY3] = L.z3.im;
+  r[kPcBlx] = C.blx; r[kPcBly] = C.bly; r[kPcStep] = C.step;
+  r[kPcPx] = pos.x; r[kPcPy] = pos.y;
+  r[kPcRho] = C.rho; r[kPcRho2] = C.rho2; r[kPcInv] = 1.0 / C.rho2;
+  const double ext = fabs(C.blx) + fabs(C.bly) + 2.0 * C.step * (double)C.N + fabs(pos.x) +
+                     fabs(pos.y) + fabs(L.z2.re) + fabs(L.z2.im) + fabs(L.z3.re) +
+                     fabs(L.z3.im) + fabs(L.z1.re) + fabs(L.z1.im);
+  r[kPcExt] = ext;
+  r[kPcN] = (double)C.N;
+  r[kPcGp] = (double)gp;
+  const bool bin = C.binIrs != 0;
+  auto mass = [](double m) { return m >= 0x1p-200 && m <= 0x1p10; };
+  // E of the rows at least kFarRow from every lens
+  const double band =
+      ray_band(ext + (fabs(L.m1) + fabs(L.m2) + fabs(L.m3)) * (1.0 / kFarRow), C.rho);
+  r[kPcLo] = C.rho2 - band;
+  r[kPcHi] = C.rho2 + band;
+  const bool fast = band <= 0x1p-10 * C.rho2 && ext <= 0x1p40 && C.rho2 >= 0x1p-200 && C.rho2 <= 0x1p40 && mass(L.m1) &&
+                    mass(L.m2) && (bin || mass(L.m3));
+  r[kPcFlags] = (double)((bin ? kPtBinary : 0) | (fast ? kPtFast : 0) |
+                         (C.ldB != 0.0 ? kPtLimb : 0) |
+                         (A.shareRays > 0.0f && A.ptCost[gp] >= A.shareRays ? kPtHeavy : 0));
 }
 
-// Whether row y keeps every |z - z_k|^2 at least 2^-500: |y - y_k| >= 2^-250
-// for the three lenses (|z - z_k|^2 >= (y - y_k)^2 for every pixel z of the
-// row, and the rounded squares and sums keep that order).
-__device__ __forceinline__ bool row_in_range(const Lens& L, double y) {
-  const double lo = 0x1p-250;
-  return fabs(L.z1.im - y) >= lo && fabs(L.z2.im - y) >= lo && fabs(L.z3.im - y) >= lo;
+int launch_fill_points(const FillArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(fill_points_kernel, dim3((a.nBatch + 255) / 256), dim3(256), 0, s, a);
+  return (int)hipGetLastError();
 }
 
-// sqrt(a) for 0 <= a <= 1 within a few units in the last place: the
-// hardware reciprocal square root and two Goldschmidt refinements (the
-// brightness term only feeds the fixed-point magnification sum, whose
-// rounding is 2^-34 of a pixel).  a = 0 gives 0.
-__device__ __forceinline__ double sqrt_unit(double a) {
-  const double y = __builtin_amdgcn_rsq(a);
-  double s = a * y, h = 0.5 * y;
-  double r = fma(-s, h, 0.5);
-  s = fma(s, r, s);
-  h = fma(h, r, h);
-  r = fma(-s, s, a);
-  s = fma(r, h, s);
-  return a > 0.0 ? s : 0.0;
+// The rays of one row of one position: the position's constants (wave-uniform)
+// and the row's.
+//
+// Fast rows.  A pixel counts when its ray's squared distance from the source,
+// computed by the reference's operations (irs_ray, irs_binary), is below
+// rho^2.  Nearly every pixel is far from that boundary, so the distance is
+// first formed with fused operations and one reciprocal for the three
+// quotients (about 30 instructions instead of 80), and the reference's own
+// operations decide only where it lies within [lo, hi].  Both forms use the
+// same rounded pixel coordinates and lens distances; from there on each
+// rounds at most 20 times, to a relative 2^-53 of the sum of the terms'
+// magnitudes, which a row bounds by E = sum m_k / |y - y_k| + ext.  So the
+// rays differ by at most delta = 2^-46 E (128 roundings), the squared
+// distances near the boundary by 2 rho delta + delta^2, and lo, hi lie twice
+// that from rho^2.  Rows at least kFarRow from every lens share one band per
+// position; a row closer to one gets its own, and one whose band would exceed
+// 2^-10 rho^2, or that passes within 2^-50 of a lens, is evaluated with the
+// reference's operations throughout (kRowExact).
+//
+// A pixel's brightness always comes from the row's own form of the distance
+// (never from the one that decided), so its value does not depend on which
+// task evaluated it.
+constexpr int kRowTriple = 0, kRowBinary = 1, kRowExact = 2;
+struct Ray {
+  double m1, m2, m3, x1, x2, x3, blx, step, px, inv;
+  double f1, f2, f3, e1, e2, e3, ys, lo, hi;
+  double pc;  // lane k: element k of the position's record
+  int row, mode;
+};
+
+// Per-position constants of set_row, in vector registers.
+struct RowBase {
+  double y1, y2, y3, bly, step, py, lo, hi;
+};
+__device__ __forceinline__ double to_vgpr(double v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ RowBase row_base(const Ray& R) {
+  RowBase B;
+  B.y1 = to_vgpr(rl(R.pc, kPcY1));
+  B.y2 = to_vgpr(rl(R.pc, kPcY2));
+  B.y3 = to_vgpr(rl(R.pc, kPcY3));
+  B.bly = to_vgpr(rl(R.pc, kPcBly));
+  B.step = to_vgpr(rl(R.pc, kPcStep));
+  B.py = to_vgpr(rl(R.pc, kPcPy));
+  B.lo = to_vgpr(rl(R.pc, kPcLo));
+  B.hi = to_vgpr(rl(R.pc, kPcHi));
+  return B;
+}
+// Sets the row of a position whose lens and grid allow fast rows (kPtFast) and
+// returns whether the row lies far from every lens; else near_row has to
+// follow.
+__device__ __forceinline__ bool far_row(Ray& R, const RowBase& B, int row) {
+  R.row = row;
+  const double y = B.bly + B.step * (double)row;
+  R.f1 = y - B.y1;
+  R.f2 = y - B.y2;
+  R.f3 = y - B.y3;
+  R.e1 = R.f1 * R.f1;
+  R.e2 = R.f2 * R.f2;
+  R.e3 = R.f3 * R.f3;
+  R.ys = y - B.py;
+  R.lo = B.lo;
+  R.hi = B.hi;
+  return __ballot(min_abs(min_abs(R.f1, R.f2), R.f3) >= kFarRow) != 0;
+}
+// The row's own band; false when it has to be evaluated exactly.
+__device__ __forceinline__ bool near_row(Ray& R, bool bin) {
+  const double g1 = fabs(R.f1), g2 = fabs(R.f2), g3 = bin ? 1.0 : fabs(R.f3);
+  // the hardware reciprocal's 2^-24 is well inside the factor two
+  const double E = rl(R.pc, kPcExt) + R.m1 * __builtin_amdgcn_rcp(g1) +
+                   R.m2 * __builtin_amdgcn_rcp(g2) + fabs(R.m3) * __builtin_amdgcn_rcp(g3);
+  const double rho2 = rl(R.pc, kPcRho2), band = ray_band(E, rl(R.pc, kPcRho));
+  R.lo = rho2 - band;
+  R.hi = rho2 + band;
+  const bool ok = g1 >= 0x1p-50 && g2 >= 0x1p-50 && g3 >= 0x1p-50 && band <= 0x1p-10 * rho2;
+  return __ballot(!ok) == 0;
+}
+__device__ __forceinline__ void set_row(Ray& R, int flags, int row) {
+  const RowBase B = row_base(R);
+  const bool bin = (flags & kPtBinary) != 0;
+  const bool fast = (far_row(R, B, row) || near_row(R, bin)) && (flags & kPtFast);
+  R.mode = fast ? (bin ? kRowBinary : kRowTriple) : kRowExact;
 }
 
-// Ray test of pixel x of the row (lcirs.cc:400-402) and its brightness
-// A + B sqrt(1 - r^2) (lcirs.cc:406-407, limbdarkeningmodel.cc:45-49) as a
-// multiple of 1/sumScale.  The test is the reference's to the bit (irsSIMD,
-// or irsBinary for m3 = 0).  The brightness is rounded to the nearest
-// integer multiple by adding 1.5 * 2^52 (exact for |value| below 2^51,
-// either sign); its r^2 / rho^2 and square root are within a few units in
-// the last place of the IEEE operations, far below that rounding.
-// MAP is the row's ray map (R.map), fixed at compile time for the scan's
-// inner loop; eval_px dispatches on R.map.
-template <int MAP>
-__device__ __forceinline__ bool eval_px_map(const RowCtx& R, int x, long long& val) {
-  const double xx = R.blx + R.step * (double)x;
-  const double rsq = MAP == kMapInRange ? irs_ray_in_range(R.L, xx, R.y, R.px, R.py)
-                     : MAP == kMapTriple ? irs_ray(R.L, xx, R.y, R.px, R.py)
-                                         : irs_binary(R.L, xx, R.y, R.px, R.py);
-  if (!(rsq < R.rho2)) return false;
-  const double v = R.ldA + R.ldB * sqrt_unit(1.0 - rsq * R.invRho2);
-  const double t = fma(v, R.sumScale, 6755399441055744.0);  // 1.5 * 2^52
-  val = __double_as_longlong(t) - 0x4338000000000000ll;
-  return true;
+// Squared distance in the reference's operations (irsSIMD, lcirs.cc:290-341;
+// irsBinary, lcirs.cc:345-353), from y as set_row formed it.
+template <bool BIN>
+__device__ __forceinline__ double ray_exact(const Ray& R, double x) {
+  Lens L;
+  L.m1 = R.m1; L.m2 = R.m2; L.m3 = R.m3;
+  L.z1 = mk(R.x1, rl(R.pc, kPcY1));
+  L.z2 = mk(R.x2, rl(R.pc, kPcY2));
+  L.z3 = mk(R.x3, rl(R.pc, kPcY3));
+  const double y = rl(R.pc, kPcBly) + rl(R.pc, kPcStep) * (double)R.row, py = rl(R.pc, kPcPy);
+  return BIN ? irs_binary(L, x, y, R.px, py) : irs_ray(L, x, y, R.px, py);
 }
 
-__device__ __forceinline__ bool eval_px(const RowCtx& R, int x, long long& val) {
-  return R.map == kMapInRange ? eval_px_map<kMapInRange>(R, x, val)
-         : R.map == kMapTriple ? eval_px_map<kMapTriple>(R, x, val)
-                               : eval_px_map<kMapBinary>(R, x, val);
+template <int MODE>
+__device__ __forceinline__ double ray_fast(const Ray& R, double x) {
+  const double a1 = x - R.x1, a2 = x - R.x2;
+  const double q1 = fma(a1, a1, R.e1), q2 = fma(a2, a2, R.e2);
+  double nr, ni, Q;
+  if (MODE == kRowTriple) {
+    const double a3 = x - R.x3;
+    const double q3 = fma(a3, a3, R.e3);
+    const double q12 = q1 * q2;
+    const double w1 = R.m1 * (q2 * q3), w2 = R.m2 * (q1 * q3), w3 = R.m3 * q12;
+    Q = q12 * q3;
+    nr = fma(w1, a1, fma(w2, a2, w3 * a3));
+    ni = fma(w1, R.f1, fma(w2, R.f2, w3 * R.f3));
+  } else {
+    const double w1 = R.m1 * q2, w2 = R.m2 * q1;
+    Q = q1 * q2;
+    nr = fma(w1, a1, w2 * a2);
+    ni = fma(w1, R.f1, w2 * R.f2);
+  }
+  const double r = rcp_near(Q);
+  const double re = fma(-nr, r, x - R.px), im = fma(-ni, r, R.ys);
+  return fma(re, re, im * im);
 }
 
-// Follows a run leftwards from column `from` until its first miss or column
-// 0; returns the run's first column and adds the pixels taken in to acc
-// (lane-local) and cnt.
-__device__ __forceinline__ int extend_left(const RowCtx& R, int from, long long& acc,
-                                           unsigned long long& cnt, unsigned long long& evals) {
+// sqrt(t) for 0 < t <= 1 within a few units in the last place (the hardware
+// reciprocal root and one third-order step), as a multiple of 1/kSumScale
+// plus kMagic: rounded to the nearest integer multiple by adding 1.5 * 2^52,
+// the sum's bits are those of kMagic plus the integer.
+constexpr long long kMagicBits = 0x4338000000000000ll;  // the bits of 1.5 * 2^52
+__device__ __forceinline__ long long root_bits(double t) {
+  const double y = __builtin_amdgcn_rsq(t);
+  const double s0 = t * y, h = 0.5 * y;
+  const double e = fma(-s0, h, 0.5);
+  const double s = fma(s0, fma(1.5 * e, e, e), s0);
+  return __double_as_longlong(fma(s, kSumScale, 6755399441055744.0));
+}
+
+// The same for any t, 0 where t is not positive.
+__device__ __forceinline__ long long root_bits_or_0(double t) {
+  const bool pos = t > 0.0;
+  return root_bits(pos ? t : 1.0) - (pos ? 0 : (long long)kSumScale);
+}
+
+// Evaluates the pixels of columns c .. c + 63 (lane l: column c + l): the hit
+// mask, and (LIMB) every hit lane's square root of 1 - r^2/rho^2 as bits.
+template <int MODE, bool LIMB>
+__device__ __forceinline__ unsigned long long eval_block(const Ray& R, int c, long long& bits) {
   const int ln = __lane_id();
-  int xcur = from;
+  const double x = R.blx + R.step * (double)(c + ln);
+  if (MODE == kRowExact) {
+    const double rsq =
+        (int)rl(R.pc, kPcFlags) & kPtBinary ? ray_exact<true>(R, x) : ray_exact<false>(R, x);
+    if (LIMB) bits = root_bits_or_0(1.0 - rsq * R.inv);
+    return __ballot(rsq < rl(R.pc, kPcRho2));
+  }
+  const double rsq = ray_fast<MODE>(R, x);
+  unsigned long long hit = __ballot(rsq < R.lo);
+  const unsigned long long miss = __ballot(rsq > R.hi);
+  double t = fma(-rsq, R.inv, 1.0);
+  if (__builtin_expect(~(hit | miss) != 0, 0)) {
+    hit |= ~(hit | miss) & __ballot(ray_exact<MODE == kRowBinary>(R, x) < rl(R.pc, kPcRho2));
+    if (LIMB) {
+      bits = root_bits_or_0(t);
+      return hit;
+    }
+  }
+  if (LIMB) bits = root_bits(t);
+  return hit;
+}
+
+__device__ __forceinline__ unsigned long long low_bits(int n) {
+  return n >= 64 ? ~0ull : (1ull << n) - 1ull;
+}
+
+// The maximal hit runs of one row that meet [s, e], left to right.  The row is
+// evaluated in steps of 64 pixels over a window that pads [s, e] to whole
+// steps on the sides where runs may continue (extL, extR); elsewhere the
+// pixel next to [s, e] is a known miss.  A run that reaches the window's right
+// edge is followed past it; one that reaches its left edge is left to
+// extend_left.
+struct RunScan {
+  int s, e, ws, we, hi;    // interval, window, last column of the scan
+  int c;                   // first column of the current step
+  unsigned long long m;    // its hits not yet handed out
+  bool extL, extR;
+  long long bits;          // (lane) brightness of the step's pixel
+  // the run found
+  int xl, xr;
+  unsigned cnt;
+  long long acc;           // (lane) brightness bits of its pixels
+  unsigned steps;          // steps evaluated
+};
+
+__device__ __forceinline__ void scan_begin(RunScan& Q, int N, int s, int e, bool extL, bool extR) {
+  const int len = e - s + 1;
+  const int extra = ((len + 63) & ~63) - len;
+  const int padL = extL ? (extR ? extra / 2 : extra) : 0;
+  const int padR = extR ? extra - padL : 0;
+  Q.s = s;
+  Q.e = e;
+  Q.ws = s - padL < 0 ? 0 : s - padL;
+  Q.we = e + padR > N - 1 ? N - 1 : e + padR;
+  Q.hi = Q.we;
+  Q.c = Q.ws - 64;
+  Q.m = 0;
+  Q.extL = extL;
+  Q.extR = extR;
+}
+
+// The next run, or false.  Whole steps inside a run cost their ray tests and
+// one accumulation.
+template <int MODE, bool LIMB>
+__device__ __forceinline__ bool scan_next(const Ray& R, int N, RunScan& Q) {
+  const int ln = __lane_id();
   while (true) {
-    if (xcur < 0) return 0;
-    // lane l looks at xcur - l
-    const int x = xcur - ln;
-    const bool valid = x >= 0;
-    long long val = 0;
-    const bool hit = valid && eval_px(R, x, val);
-    const int nb = xcur + 1 < 64 ? xcur + 1 : 64;
-    evals += (unsigned long long)nb;
-    const unsigned long long m = __ballot(hit);
-    const int z = ~m == 0 ? 64 : __builtin_ctzll(~m);  // hits counted from lane 0
-    if (ln < z) acc += val;
-    cnt += (unsigned long long)z;
-    if (z < 64) return xcur - (z - 1);
-    xcur -= 64;
+    while (Q.m == 0) {
+      Q.c += 64;
+      if (Q.c > Q.e || Q.c > Q.hi) return false;  // no later run can meet [s, e]
+      const int nb = Q.hi - Q.c + 1;
+      Q.m = eval_block<MODE, LIMB>(R, Q.c, Q.bits) & low_bits(nb);
+      Q.steps++;
+    }
+    const int t = __builtin_ctzll(Q.m);
+    Q.xl = Q.c + t;
+    if (Q.xl > Q.e) return false;
+    unsigned long long inv = ~(Q.m >> t);
+    int z = inv ? __builtin_ctzll(inv) : 64;
+    if (z > 64 - t) z = 64 - t;
+    unsigned long long take = low_bits(z) << t;
+    if (LIMB) Q.acc = (take >> ln) & 1ull ? Q.bits : 0;
+    Q.cnt = (unsigned)z;
+    Q.xr = Q.xl + z - 1;
+    Q.m &= ~take;
+    // follow the run through whole steps
+    bool followed = false;
+    while (Q.xr == Q.c + 63 || Q.xr == Q.hi) {
+      if (Q.xr == Q.hi) {
+        if (!(Q.hi == Q.we && Q.extR && Q.we < N - 1)) break;  // its end is known
+        Q.hi = N - 1;
+        Q.c = Q.we - 63;
+        followed = true;
+      }
+      Q.c += 64;
+      const int nb = Q.hi - Q.c + 1;
+      Q.m = eval_block<MODE, LIMB>(R, Q.c, Q.bits) & low_bits(nb);
+      Q.steps++;
+      if (Q.m == ~0ull) {
+        if (LIMB) Q.acc += Q.bits;
+        Q.cnt += 64;
+        Q.xr += 64;
+        Q.m = 0;
+        continue;
+      }
+      z = __builtin_ctzll(~Q.m);
+      take = low_bits(z);
+      if (LIMB) Q.acc += (take >> ln) & 1ull ? Q.bits : 0;
+      Q.cnt += (unsigned)z;
+      Q.xr += z;
+      Q.m &= ~take;
+      if (z == 0) break;
+    }
+    if (followed) Q.m = 0;  // nothing beyond the followed run meets [s, e]
+    if (Q.xr >= Q.s) return true;
   }
 }
 
-// A look-back recorded while a row is scanned, processed after the scan:
-// row `row` over [xa, xb] (the new run's extent) without the known pixels
-// [k1, k2] (the run it was reached from and its two bounding misses).
-struct LookBack {
-  int row, xa, xb, k1, k2, dir, label;
-};
-constexpr int kMaxLookBacks = 2;  // kept in two named slots (no indexed array)
+// Follows a run leftwards from column `from` until its first miss or column
+// 0; returns the run's first column and adds the pixels taken in.
+template <int MODE, bool LIMB>
+__device__ __forceinline__ int extend_left(const Ray& R, int from, RunScan& Q) {
+  const int ln = __lane_id();
+  while (from >= 0) {
+    const int c = from - 63;  // the step's columns end at `from`
+    long long bits = 0;
+    unsigned long long m = eval_block<MODE, LIMB>(R, c, bits);
+    if (c < 0) m &= ~low_bits(-c);
+    Q.steps++;
+    const int z = m == ~0ull ? 64 : __builtin_clzll(~m);  // hits counted from `from` down
+    if (LIMB) Q.acc += ln >= 64 - z ? bits : 0;
+    Q.cnt += (unsigned)z;
+    if (z < 64) return from - z + 1;
+    from -= 64;
+  }
+  return 0;
+}
+
+template <int MODE, bool LIMB>
+__device__ __forceinline__ bool next_run_in(const Ray& R, int N, RunScan& Q) {
+  if (!scan_next<MODE, LIMB>(R, N, Q)) return false;
+  if (Q.xl == Q.ws && Q.extL && Q.ws > 0) Q.xl = extend_left<MODE, LIMB>(R, Q.ws - 1, Q);
+  return true;
+}
+__device__ __forceinline__ bool next_run(const Ray& R, int N, bool limb, RunScan& Q) {
+  if (R.mode == kRowTriple)
+    return limb ? next_run_in<kRowTriple, true>(R, N, Q) : next_run_in<kRowTriple, false>(R, N, Q);
+  if (R.mode == kRowBinary)
+    return limb ? next_run_in<kRowBinary, true>(R, N, Q) : next_run_in<kRowBinary, false>(R, N, Q);
+  return next_run_in<kRowExact, true>(R, N, Q);
+}
 
 // ---------------------------------------------------------------------------
 // Workgroup task pool (LDS)
@@ -1691,29 +1991,80 @@ __device__ __forceinline__ void pool_unlock(GroupPool* G) {
   lds_st(&G->lock, 0);
 }
 
-__device__ __forceinline__ Task uni_task(const Task& t) {
-  Task u;
-  u.b = uni(t.b); u.row = uni(t.row); u.xa = uni(t.xa); u.xb = uni(t.xb);
-  u.label = uni(t.label); u.kd = uni(t.kd); u.f1 = uni(t.f1); u.f2 = uni(t.f2);
-  return u;
+// A worker's tasks.  A task at rest is eight ints of LDS; a worker moves it
+// with lane k < 8 holding int k (the other lanes read and write a scratch
+// area, so that no access is under a branch) and reads the fields from the
+// lanes.
+template <int K>
+__device__ __forceinline__ void write_lane(int& v, int x) {
+  asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(uni(x)), "n"(K));
+}
+__device__ __forceinline__ int task_lanes(const Task& t) {
+  int v = 0;
+  write_lane<0>(v, t.b);
+  write_lane<1>(v, t.row);
+  write_lane<2>(v, t.xa);
+  write_lane<3>(v, t.xb);
+  write_lane<4>(v, t.label);
+  write_lane<5>(v, t.kd);
+  write_lane<6>(v, t.f1);
+  write_lane<7>(v, t.f2);
+  return v;
+}
+__device__ __forceinline__ Task lanes_task(int v) {
+  Task t;
+  t.b = __builtin_amdgcn_readlane(v, 0);
+  t.row = __builtin_amdgcn_readlane(v, 1);
+  t.xa = __builtin_amdgcn_readlane(v, 2);
+  t.xb = __builtin_amdgcn_readlane(v, 3);
+  t.label = __builtin_amdgcn_readlane(v, 4);
+  t.kd = __builtin_amdgcn_readlane(v, 5);
+  t.f1 = __builtin_amdgcn_readlane(v, 6);
+  t.f2 = __builtin_amdgcn_readlane(v, 7);
+  return t;
+}
+// This lane's int of the task at `slot`; lanes 8.. get a place of their own in
+// `spare` (64 ints per wave).
+__device__ __forceinline__ int* task_int(Task* slot, int* spare) {
+  const int ln = __lane_id();
+  return ln < 8 ? reinterpret_cast<int*>(slot) + ln : spare + ln;
+}
+
+// Takes and releases the pool lock (the whole wave; lane 0's exchange).
+__device__ __forceinline__ int lds_cas_lane0(int* p, int expected, int desired) {
+  int old;
+  unsigned long long save;
+  const unsigned at = (unsigned)(unsigned long long)(__attribute__((address_space(3))) int*)p;
+  asm volatile(
+      "s_mov_b64 %1, exec\n\t"
+      "s_mov_b64 exec, 1\n\t"
+      "ds_cmpst_rtn_b32 %0, %2, %3, %4\n\t"
+      "s_waitcnt lgkmcnt(0)\n\t"
+      "s_mov_b64 exec, %1"
+      : "=&v"(old), "=&s"(save)
+      : "v"(at), "v"(expected), "v"(desired)
+      : "memory");
+  return uni(old);
+}
+__device__ __forceinline__ void wave_lock(GroupPool* G) {
+  while (lds_cas_lane0(&G->lock, 0, 1) != 0) __builtin_amdgcn_s_sleep(1);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
 // A worker that holds work adds the (wave-uniform) task t; false when the
 // pool is full.
-__device__ __forceinline__ bool pool_push(GroupPool* G, const Task& t) {
-  int ok = 0;
-  if (__lane_id() == 0) {
-    pool_lock(G);
-    const int c = lds_ld(&G->count);
-    if (c < kPoolCap) {
-      G->slot[(lds_ld(&G->head) + c) & (kPoolCap - 1)] = t;
-      lds_st(&G->count, c + 1);
-      lds_st(&G->pending, lds_ld(&G->pending) + 1);
-      ok = 1;
-    }
-    pool_unlock(G);
+__device__ __forceinline__ bool pool_push(GroupPool* G, const Task& t, int* spare) {
+  const int v = task_lanes(t);
+  wave_lock(G);
+  const int c = uni(lds_ld(&G->count));
+  const bool ok = c < kPoolCap;
+  if (ok) {
+    *task_int(&G->slot[(uni(lds_ld(&G->head)) + c) & (kPoolCap - 1)], spare) = v;
+    lds_st(&G->count, c + 1);
+    lds_st(&G->pending, uni(lds_ld(&G->pending)) + 1);
   }
-  return uni(ok) != 0;
+  pool_unlock(G);
+  return ok;
 }
 
 // A worker takes a task of the pool: the newest (newest = true) or the
@@ -1725,29 +2076,21 @@ __device__ __forceinline__ bool pool_push(GroupPool* G, const Task& t) {
 // just opened (on the images still growing) before older ones: the
 // surrogate's fallback fill of the C2 curve takes ~3% less time with it,
 // the heaviest 41 positions ~5% less, C3's fill the same.
-__device__ __forceinline__ bool pool_take(GroupPool* G, Task& t, bool busy, bool newest) {
-  int ok = 0;
-  Task got = t;
-  if (__lane_id() == 0) {
-    pool_lock(G);
-    const int c = lds_ld(&G->count);
-    if (c > 0) {
-      const int h = lds_ld(&G->head);
-      if (newest) {
-        got = G->slot[(h + c - 1) & (kPoolCap - 1)];
-      } else {
-        got = G->slot[h];
-        lds_st(&G->head, (h + 1) & (kPoolCap - 1));
-      }
-      lds_st(&G->count, c - 1);
-      ok = 1;
-    }
-    if (busy) lds_st(&G->pending, lds_ld(&G->pending) - 1);
-    pool_unlock(G);
+__device__ __forceinline__ bool pool_take(GroupPool* G, Task& t, bool busy, bool newest,
+                                          int* spare) {
+  wave_lock(G);
+  const int c = uni(lds_ld(&G->count));
+  int v = 0;
+  if (c > 0) {
+    const int h = uni(lds_ld(&G->head));
+    v = *task_int(&G->slot[newest ? (h + c - 1) & (kPoolCap - 1) : h], spare);
+    if (!newest) lds_st(&G->head, (h + 1) & (kPoolCap - 1));
+    lds_st(&G->count, c - 1);
   }
-  ok = uni(ok);
-  if (ok) t = uni_task(got);
-  return ok != 0;
+  if (busy) lds_st(&G->pending, uni(lds_ld(&G->pending)) - 1);
+  pool_unlock(G);
+  if (c > 0) t = lanes_task(v);
+  return c > 0;
 }
 
 // Manager: adds the tasks held by lanes [lo, hi) (pending + their number).
@@ -1915,79 +2258,96 @@ __device__ __forceinline__ int claim_seeds(const FillArgs& A, Task& t, int n) {
   return k;
 }
 
-// State of the task being processed (uniform across the wave).
-struct TaskState {
-  const FillArgs* A;
-  Task t;
-  int curB;                 // batch point whose constants R holds (-1: none)
-  bool heavy;               // its predicted rays reach shareRays
-  RowCtx R;
-  int kind, dir, gp, N;
-  int xa, xb;               // the known run next to the scanned row (kind 0:
-                            // the parent, kind 3: the child)
-  Task cont;                // follow-up kept by this wave (the next sweep step)
-  bool haveCont;
+// A worker wave's state (uniform across the wave where not marked).
+struct Worker {
+  ArgPtr A;
+  int scoutRows;            // (a hot argument)
   GroupPool* G;             // the workgroup's shared pool
+  Task* ring;               // this wave's ring of waiting tasks in LDS:
+  int lhead, lcount;        // lcount tasks from lhead on
+  Task* out;                // its tasks for the pool: nOut of them
+  int nOut;
+  Task* back;               // the look-backs recorded by the row's scan: nBack of them
   int nBack;
-  LookBack back0, back1;
-  int accLabel;             // totals of new runs, credited to accLabel when
-  long long accSum;         // the label changes or the sweep ends
-  unsigned long long accCnt;
-  unsigned long long evals, nIns, nDup, insTicks;
-  unsigned long long nScout, nScoutRuns;  // scout tasks taken, runs they found
+  int* spare;               // 64 ints of LDS for the lanes without a task int
+  Task t;                   // the task in hand
+  bool haveCont;            // t is the follow-up kept by this wave
+  bool general;             // t is for process_task
+  // the position whose constants R holds
+  int curB, gp, N, flags;
+  unsigned long long* tab;  // its run-table slice
+  unsigned tabMask;
+  Ray R;
+  // totals of new runs, credited to accLabel when the label changes or the
+  // wave runs out of work
+  int accLabel;
+  unsigned accCnt;
+  long long accBits;        // (lane) brightness bits, kMagicBits included per pixel
+  unsigned nTasks, nIns, nDup, nScout, nScoutRuns, steps;
   bool landed;              // the scout task found a run (new or known)
-  // this wave's ring of waiting tasks in LDS: lcount tasks from lhead on
-  Task* ring;
-  int lhead, lcount;
 };
 
 // Task hand-off.  Follow-ups a worker does not continue with go to its own
 // ring in LDS (no atomics: one owner); the newest is taken next (depth
-// first).  While other workers of the group are idle, a worker moves its
-// oldest waiting tasks to the group's pool; a full ring spills its oldest
-// task there too, and a full pool into the global ring.
-__device__ __forceinline__ bool ring_donate(TaskState& S) {
-  const Task t = S.ring[S.lhead];
-  if (!pool_push(S.G, t) && !q_push(*S.A, t)) return false;
-  S.lhead = (S.lhead + 1) & (kLocalCap - 1);
-  S.lcount--;
-  return true;
+// first).  Tasks for the group's pool at once wait in the wave's out buffer
+// until the row's scan step is done.  While other workers of the group are
+// idle, a worker moves its oldest waiting tasks to the pool; a ring that is
+// nearly full spills there too, and a full pool into the global ring.
+__device__ __forceinline__ void ring_put(Worker& W, const Task& f) {
+  *task_int(&W.ring[(W.lhead + W.lcount) & (kLocalCap - 1)], W.spare) = task_lanes(f);
+  W.lcount++;
 }
 
-__device__ __forceinline__ void ring_push(TaskState& S, const Task& f) {
-  if (S.lcount == kLocalCap && !ring_donate(S)) {
-    flag_point(*S.A, S.gp, kFlagQueueFull);  // everything full: the task is lost
-    return;
+__device__ __forceinline__ Task ring_pop(Worker& W) {
+  W.lcount--;
+  return lanes_task(*task_int(&W.ring[(W.lhead + W.lcount) & (kLocalCap - 1)], W.spare));
+}
+
+// Empties the out buffer into the pool (the ring where the pool is full) and
+// moves `give` of the ring's oldest tasks, and as many as make room for the
+// next runs' follow-ups, to the pool or the global ring.
+constexpr int kOutCap = 8;     // out buffer: a run adds at most 3
+constexpr int kRoom = 16;      // ring places kept free (out buffer and a run's follow-ups)
+__device__ __forceinline__ void hand_off(Worker& W, int give) {
+  while (W.nOut > 0 || give > 0 || W.lcount > kLocalCap - kRoom) {
+    const bool out = W.nOut > 0;
+    if (!out && W.lcount == 0) break;
+    const Task t = lanes_task(
+        *task_int(out ? &W.out[W.nOut - 1] : &W.ring[W.lhead], W.spare));
+    const bool pooled = pool_push(W.G, t, W.spare);
+    if (out) {
+      W.nOut--;
+      if (!pooled) ring_put(W, t);
+      continue;
+    }
+    if (!pooled && !q_push(W.A, t)) {
+      if (W.lcount < kLocalCap - 4) break;  // still room: keep the rest
+      flag_point(W.A, W.gp, kFlagQueueFull);  // everything full: the task is lost
+    }
+    W.lhead = (W.lhead + 1) & (kLocalCap - 1);
+    W.lcount--;
+    give--;
   }
-  const int slot = (S.lhead + S.lcount) & (kLocalCap - 1);
-  if (__lane_id() == 0) S.ring[slot] = f;
-  S.lcount++;
 }
 
-__device__ __forceinline__ Task ring_pop(TaskState& S) {
-  S.lcount--;
-  return S.ring[(S.lhead + S.lcount) & (kLocalCap - 1)];
-}
-
-// Adds the signed value v to a split total (p[0], p[1]) that stands for
-// p[1] * 2^32 + p[0]: p[0] sums the low 32 bits of every value added (as an
-// unsigned number) and p[1] the rest (v >> 32, arithmetic).  Both adds need
-// no result, so they are issued and not waited for, and any number of
-// concurrent adds sums exactly as long as fewer than 2^32 values are added
-// to one total.
-__device__ __forceinline__ void add_split(unsigned long long* p, long long v) {
-  atomicAdd(p, (unsigned long long)(v & 0xFFFFFFFFll));
-  const long long hi = v >> 32;
-  if (hi) atomicAdd(p + 1, (unsigned long long)hi);
-}
-
-__device__ __forceinline__ void flush_acc(TaskState& S) {
-  if (S.accCnt && __lane_id() == 0) {
-    atomicAdd(&S.A->lcount[S.accLabel], S.accCnt);
-    add_split(&S.A->lsum[2 * (size_t)S.accLabel], S.accSum);
+// The totals go to the label as the count and, in two words, the sum of the
+// pixels' integers: words (p[0], p[1]) stand for p[1] * 2^32 + p[0], p[0]
+// summing the low 32 bits of every value added and p[1] the rest, so that no
+// total wraps as long as fewer than 2^32 values are added to it.
+__device__ __forceinline__ void flush_acc(Worker& W) {
+  if (W.accCnt) {
+    const ArgPtr A = opq(W.A);
+    add64_lane0(&A->lcount[W.accLabel], W.accCnt);
+    if (W.flags & kPtLimb) {
+      const unsigned long long v = (unsigned long long)uni64(wave_sum(W.accBits)) -
+                                   (unsigned long long)W.accCnt * (unsigned long long)kMagicBits;
+      unsigned long long* p = &A->lsum[2 * (size_t)W.accLabel];
+      add64_lane0(p, v & 0xFFFFFFFFull);
+      if (v >> 32) add64_lane0(p + 1, v >> 32);
+    }
   }
-  S.accCnt = 0;
-  S.accSum = 0;
+  W.accCnt = 0;
+  W.accBits = 0;
 }
 
 __device__ __forceinline__ Task make_task(int b, int row, int xa, int xb, int label, int kind,
@@ -1999,22 +2359,33 @@ __device__ __forceinline__ Task make_task(int b, int row, int xa, int xb, int la
   return f;
 }
 
-constexpr int kQueueOnly = 8;  // kd flag: never kept by the wave
-constexpr int kShare = 16;     // kd flag: to the group's pool at once (the wave's
+constexpr int kQueueOnly = 8;  // follow-up flag: never kept by the wave
+constexpr int kShare = 16;     // follow-up flag: to the group's pool at once (the wave's
                                // ring when the pool is full)
 
 // A follow-up of a run, dispatched as soon as it is made: the first one that
 // may stay with the wave becomes its next step, tasks marked kShare go to the
-// group's pool, the others to the wave's ring.  (Collecting them first made
-// the compiler keep them in a scratch array.)
-__device__ __forceinline__ void follow(TaskState& S, Task f) {
-  const bool queueOnly = (f.kd & kQueueOnly) != 0, share = (f.kd & kShare) != 0;
-  f.kd &= ~(kQueueOnly | kShare);
-  if (!queueOnly && !share && !S.haveCont) {
-    S.cont = f;
-    S.haveCont = true;
-  } else if (!(share && pool_push(S.G, f))) {
-    ring_push(S, f);
+// group's pool, the others to the wave's ring.
+__device__ __forceinline__ void follow(Worker& W, const Task& f, int where) {
+  if (where == 0 && !W.haveCont) {
+    W.t = f;
+    W.haveCont = true;
+  } else if (where & kShare) {
+    *task_int(&W.out[W.nOut], W.spare) = task_lanes(f);
+    W.nOut++;
+  } else {
+    ring_put(W, f);
+  }
+}
+
+// A look-back, kept for the end of the row's scan, or queued when two are
+// already waiting.
+__device__ __forceinline__ void put_back(Worker& W, const Task& f) {
+  if (W.nBack < 2) {
+    *task_int(&W.back[W.nBack], W.spare) = task_lanes(f);
+    W.nBack++;
+  } else {
+    ring_put(W, f);
   }
 }
 
@@ -2025,460 +2396,413 @@ __device__ __forceinline__ void follow(TaskState& S, Task f) {
 // jump it was sent with in the high half of f2 (the low half counts the
 // scouts of its chain since the last leap).
 constexpr int kMinJump = 16;
-__device__ __forceinline__ int scout_jump_for(const FillArgs& A, int w) {
-  if (A.scoutWidth <= 0 || w <= A.scoutWidth) return A.scoutJump;
-  const long long j = (long long)A.scoutJump * A.scoutWidth / w;
-  const int lo = kMinJump < A.scoutJump ? kMinJump : A.scoutJump;
+__device__ __forceinline__ int scout_jump_for(ArgPtr A, int w) {
+  const int jump = A->scoutJump, width = A->scoutWidth;
+  if (width <= 0 || w <= width) return jump;
+  // below 2^15 and 2^25: the quotient in 64 bits, by the hardware reciprocal
+  // would round; the integer division is rare (one run in kMinJump at most)
+  const long long j = (long long)jump * width / w;
+  const int lo = kMinJump < jump ? kMinJump : jump;
   return j < lo ? lo : (int)j;
 }
 
-// A maximal hit run [xl, xr] of the row being scanned was found: record it,
-// credit its pixels to its label and schedule the neighbouring rows.
-__device__ __forceinline__ void handle_run(TaskState& S, int xl, int xr, long long sum,
-                                           unsigned long long cnt) {
-  const FillArgs& A = *S.A;
-  const Task& t = S.t;
-  int label = t.label;
-  if (S.kind == 2) {
-    S.landed = true;
+// What a task scans: a row between columns, in one or two pieces around known
+// pixels.
+struct Scan {
+  int kind, dir, row, label;
+  int xa, xb;  // the interval: the known run next to the row (kind 0: the
+               // parent, kind 3: the child)
+  int k1, k2;  // known pixels within it (none if k1 > k2)
+};
+
+// A maximal hit run [xl, xr] of the scan's row was found (cnt pixels, their
+// brightness bits per lane in acc): record it, credit its pixels to its label
+// and schedule the neighbouring rows.  f1, f2: those of the task in hand (they
+// drive sweeps and scouts).  Returns whether a look-back is due: at the row
+// the run was reached from, where it reaches past that row's known run and
+// its two bounding misses.
+__device__ __forceinline__ bool handle_run(Worker& W, const Scan& S, int f1, int f2, int xl, int xr,
+                                           unsigned cnt, long long acc, int& labelOut) {
+  const int b = W.curB, row = opq(S.row), N = opq(W.N), d = opq(S.dir), kind = opq(S.kind);
+  f1 = opq(f1);
+  f2 = opq(f2);
+  int label = S.label;
+  if (__builtin_expect(kind == 2, 0)) {
+    W.landed = true;
     // a scout run starts a class of its own
-    int nl = 0;
-    if (__lane_id() == 0) nl = atomicAdd(A.labelNext, 1);
-    nl = uni(nl);
-    if (nl >= A.labelCap) {
-      flag_point(A, S.gp, kFlagLabelFull);
-      return;
+    const ArgPtr A = opq(W.A);
+    label = add32_lane0(A->labelNext, 1);
+    if (label >= A->labelCap) {
+      flag_point(W.A, W.gp, kFlagLabelFull);
+      return false;
     }
-    if (__lane_id() == 0) A.lpoint[nl] = t.b;
-    label = nl;
+    store32_lane0(&A->lpoint[label], b);
   }
-  const unsigned long long ti0 = __builtin_amdgcn_s_memrealtime();
-  const int ins = insert_run(A, t.b, t.row, xl, xr, label);
-  S.insTicks += __builtin_amdgcn_s_memrealtime() - ti0;
-  if (ins == kInsFull) {
-    flag_point(A, S.gp, kFlagHashFull);
-    return;
-  }
-  if ((ins & 0xFF) == kInsDup) {
-    S.nDup++;
-    if (S.kind != 2) unite(A, label, ins >> 8);
-    return;
-  }
-  S.nIns++;
-  S.nScoutRuns += S.kind == 2 ? 1 : 0;
-  if (xl <= 1 || xr >= S.N - 2) flag_point(A, S.gp, kFlagEdge);
-  // a run adds at most 2^60 units: flushing from 2^61 on keeps the total
-  // within 2^62
-  if (label != S.accLabel || S.accSum > (1ll << 61) || S.accSum < -(1ll << 61)) {
-    flush_acc(S);
-    S.accLabel = label;
-  }
-  S.accCnt += cnt;
-  S.accSum += sum;
-  const int row = t.row, N = S.N, center = (int)(((long long)xl + xr) / 2);
-  const int d = S.dir;  // direction of travel
-  if (S.kind == 1) {
-    if (row + 1 < N) follow(S, make_task(t.b, row + 1, xl, xr, label, 0, 1, center, 0));
-    if (row - 1 >= 0) follow(S, make_task(t.b, row - 1, xl, xr, label, 0, -1, center, 0));
-  } else if (S.kind == 2) {
-    // A scout landed (t.f1: the column of the run it was sent from, one jump
-    // back; t.f2: that jump's length and the scouts in its chain since the
-    // last leap).  The wave sends the next scout straight on at once, with
-    // the shift measured over the last jump, and keeps it as its next step, so that the scouts run ahead
-    // one task per jump; every leapEvery-th scout also sends a leap scout
-    // leapJumps jumps ahead to the shared queue, which starts a chain of its
-    // own, so that long images get many chains.  The two sweeps of the new
-    // class go to the shared queue for idle waves; they start as if they had
-    // just sent a scout.
-    const int count = t.f2 & 0xFFFF, prevJump = (int)((unsigned)t.f2 >> 16);
-    const int J = scout_jump_for(A, xr - xl + 1);
-    // the shift over the last jump, rescaled to this jump
-    const long long shift = ((long long)center - t.f1) * J / (prevJump > 0 ? prevJump : J);
-    const long long ash = shift < 0 ? -shift : shift;
-    for (int leap = 0; leap < 2 && A.scoutRows > 0; leap++) {
-      if (leap == 1 && (A.leapEvery <= 0 || (count + 1) % A.leapEvery != 0)) break;
-      const long long k = leap ? A.leapJumps : 1;
-      const long long rt = (long long)row + (long long)d * J * k;
-      if (rt < 0 || rt >= N) continue;
-      const long long pc = center + shift * k;
-      const long long hw = ((long long)xr - xl) / 2 + ash * k / 4 + 32 * k;
-      long long sa = pc - hw, sb = pc + hw;
-      if (sa < 0) sa = 0;
-      if (sb > N - 1) sb = N - 1;
-      if (sa > sb) continue;
-      Task f = make_task(t.b, (int)rt, (int)sa, (int)sb, -1, 2, d, center,
-                         (J << 16) | (leap ? 0 : (count + 1) & 0xFFFF));
-      if (leap) {
-        // the leap's chain measures its next shift from the column expected
-        // one jump before its landing row
-        f.f1 = (int)(center + shift * (A.leapJumps - 1));
-        f.kd |= kQueueOnly | kShare;
-      }
-      follow(S, f);
+  labelOut = label;
+  int other = 0;
+  const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, xl, xr, label, other);
+  if (__builtin_expect(ins != kInsNew, 0)) {
+    if (ins == kInsFull) {
+      flag_point(W.A, W.gp, kFlagHashFull);
+    } else {
+      W.nDup++;
+      if (kind != 2) unite(opq(W.A)->lparent, label, other);
     }
-    Task up = make_task(t.b, row + 1, xl, xr, label, 0, 1, center, -1);
-    Task dn = make_task(t.b, row - 1, xl, xr, label, 0, -1, center, -1);
-    up.kd |= kShare;
-    dn.kd |= kShare;
-    if (row + 1 < N) follow(S, up);
-    if (row - 1 >= 0) follow(S, dn);
-  } else if (S.kind == 3) {
-    // a run found looking back: sweep on away from the run it was reached
-    // from, and look back towards that run's row where this one reaches past it
-    if (row + d >= 0 && row + d < N)
-      follow(S, make_task(t.b, row + d, xl, xr, label, 0, d, center, 0));
-    if (row - d >= 0 && row - d < N && (xl < S.xa - 1 || xr > S.xb + 1)) {
-      Task f = make_task(t.b, row - d, xl, xr, label, 3, -d, S.xa - 1, S.xb + 1);
-      f.kd |= kQueueOnly;
-      follow(S, f);
-    }
-  } else {
-    // sweep step: 1. the next row in the direction of travel
-    if (row + d >= 0 && row + d < N) {
+    return false;
+  }
+  W.nIns++;
+  if (xl <= 1 || xr >= N - 2) flag_point(W.A, W.gp, kFlagEdge);
+  // at most 2^26 pixels before a flush: their integers stay below 2^62
+  if (label != W.accLabel || W.accCnt >= (1u << 25)) {
+    flush_acc(W);
+    W.accLabel = label;
+  }
+  W.accCnt += cnt;
+  if (W.flags & kPtLimb) W.accBits += acc;
+  const int center = (int)(((unsigned)xl + (unsigned)xr) / 2);
+  const bool ahead = row + d >= 0 && row + d < N;
+  const bool past = row - d >= 0 && row - d < N && (xl < S.xa - 1 || xr > S.xb + 1);
+  if (__builtin_expect(kind == 0, 1)) {
+    // sweep step: the next row in the direction of travel
+    if (ahead) {
       // f2 >= 0: rows since the sweep's anchor, no scout sent yet;
       // f2 < 0: -(rows since the last scout) - 1
-      int a1 = t.f1, a2 = t.f2 >= 0 ? t.f2 + 1 : t.f2 - 1;
+      int a1 = f1, a2 = f2 >= 0 ? f2 + 1 : f2 - 1;
       const int rows = a2 >= 0 ? a2 : -a2 - 1;
-      const int J = scout_jump_for(A, xr - xl + 1);
-      const bool due = A.scoutRows > 0 && ((a2 >= 0 && rows >= A.scoutRows) ||
-                                           (a2 < 0 && rows >= J));
-      if (due) {
-        // send a scout ahead along the run's drift, then re-anchor
-        const long long rt = (long long)row + (long long)d * J;
-        if (rt >= 0 && rt < N) {
-          const long long drift = rows > 0 ? ((long long)center - a1) / rows : 0;
-          const long long pc = center + drift * J;
-          const long long adr = drift < 0 ? -drift : drift;
-          const long long hw = ((long long)xr - xl) / 2 + adr * J / 4 + 32;
-          long long sa = pc - hw, sb = pc + hw;
-          if (sa < 0) sa = 0;
-          if (sb > N - 1) sb = N - 1;
-          if (sa <= sb) {
-            // to the wave's ring (the shared queue while some wave is idle),
-            // or to the shared queue at once on the images of positions
-            // predicted heavy, whose scouts mostly land: sweeps of many
-            // small images send many scouts that miss, and queuing each of
-            // them at once makes the shared queue's head and tail the
-            // bottleneck
-            Task f = make_task(t.b, (int)rt, (int)sa, (int)sb, -1, 2, d, center, J << 16);
-            f.kd |= kQueueOnly | ((A.scoutShare || S.heavy) ? kShare : 0);
-            follow(S, f);
+      if (__builtin_expect(rows >= (a2 >= 0 ? W.scoutRows : kMinJump) && W.scoutRows > 0, 0)) {
+        const ArgPtr A = opq(W.A);
+        const int J = scout_jump_for(A, xr - xl + 1);
+        if (a2 >= 0 || rows >= J) {
+          // send a scout ahead along the run's drift, then re-anchor
+          const long long rt = (long long)row + (long long)d * J;
+          if (rt >= 0 && rt < N) {
+            const long long drift = rows > 0 ? (center - a1) / rows : 0;
+            const long long pc = center + drift * J;
+            const long long adr = drift < 0 ? -drift : drift;
+            const long long hw = ((long long)xr - xl) / 2 + adr * J / 4 + 32;
+            long long sa = pc - hw, sb = pc + hw;
+            if (sa < 0) sa = 0;
+            if (sb > N - 1) sb = N - 1;
+            if (sa <= sb) {
+              // to the wave's ring (the shared queue while some wave is idle),
+              // or to the shared queue at once on the images of positions
+              // predicted heavy, whose scouts mostly land: sweeps of many
+              // small images send many scouts that miss, and queuing each of
+              // them at once makes the shared queue's head and tail the
+              // bottleneck
+              follow(W, make_task(b, (int)rt, (int)sa, (int)sb, -1, 2, d, center, J << 16),
+                     kQueueOnly | ((A->scoutShare || (W.flags & kPtHeavy)) ? kShare : 0));
+            }
           }
-        }
-        a1 = center;
-        a2 = -1;
-      }
-      follow(S, make_task(t.b, row + d, xl, xr, label, 0, d, a1, a2));
-    }
-    // 2. the row the sweep came from, where the new run reaches past the
-    //    parent run [xa, xb] and its two bounding misses: looked at after
-    //    this scan (or queued when two look-backs are already waiting)
-    if (row - d >= 0 && row - d < N && (xl < S.xa - 1 || xr > S.xb + 1)) {
-      LookBack lb;
-      lb.row = row - d; lb.xa = xl; lb.xb = xr;
-      lb.k1 = S.xa - 1; lb.k2 = S.xb + 1; lb.dir = -d; lb.label = label;
-      if (S.nBack == 0) {
-        S.back0 = lb;
-        S.nBack = 1;
-      } else if (S.nBack == 1) {
-        S.back1 = lb;
-        S.nBack = 2;
-      } else {
-        Task f = make_task(t.b, lb.row, xl, xr, label, 3, -d, lb.k1, lb.k2);
-        f.kd |= kQueueOnly;
-        follow(S, f);
-      }
-    }
-  }
-}
-
-// The scan's next 64-pixel steps from column cb + 64 on: each step's hit
-// mask m and pixel count nb; while a step lies wholly inside the open run its
-// pixels are added to acc and cnt and the next step follows (up to column
-// hi).  Returns whether the last step taken lies inside the open run; cb is
-// left at that step's first column and val holds its lane's brightness.
-template <int MAP>
-__device__ __forceinline__ bool scan_steps(const RowCtx& R, bool open, int hi, int& cb,
-                                           unsigned long long& m, int& nb, long long& val,
-                                           long long& acc, unsigned long long& cnt,
-                                           unsigned& evals) {
-  const int ln = __lane_id();
-  bool inside;
-  while (true) {
-    if (open && cb + 192 <= hi + 1) {
-      // two whole steps inside the scan: both evaluated before either
-      // ballot (twice the independent work in flight); when the first does
-      // not lie wholly inside the run the second is dropped, and evaluated
-      // again by the caller's next step
-      const int x1 = cb + 64 + ln;
-      long long v1 = 0, v2 = 0;
-      const bool h1 = eval_px_map<MAP>(R, x1, v1);
-      const bool h2 = eval_px_map<MAP>(R, x1 + 64, v2);
-      const unsigned long long m1 = __ballot(h1), m2 = __ballot(h2);
-      evals += 128u;
-      cb += 64;
-      nb = 64;
-      if (m1 != ~0ull) {
-        m = m1;
-        val = v1;
-        return false;
-      }
-      acc += v1;
-      cnt += 64ull;
-      cb += 64;
-      m = m2;
-      val = v2;
-      if (m2 != ~0ull) return false;
-      acc += v2;
-      cnt += 64ull;
-      if (cb + 64 > hi) return true;
-      continue;
-    }
-    cb += 64;
-    const int x = cb + ln;
-    val = 0;
-    const bool hit = x <= hi && eval_px_map<MAP>(R, x, val);
-    m = __ballot(hit);
-    nb = hi - cb + 1 < 64 ? hi - cb + 1 : 64;
-    evals += (unsigned)nb;
-    const unsigned long long full = nb == 64 ? ~0ull : ((1ull << nb) - 1ull);
-    inside = open && m == full;
-    if (!inside) break;
-    acc += val;
-    cnt += (unsigned long long)nb;
-    if (cb + 64 > hi) break;
-  }
-  return inside;
-}
-
-// Maximal hit runs of the row that meet [s, e].  The row is evaluated over a
-// window that pads [s, e] to whole 64-pixel steps on the sides where runs
-// may continue (extL, extR); elsewhere the pixel next to [s, e] is a known
-// miss.  Runs inside the padding that do not reach [s, e] are ignored; a run
-// that reaches the window's right edge is followed past it in the same loop,
-// one that reaches its left edge by extend_left.  Each run is handed to
-// handle_run once both its ends are known.  A 64-pixel step that lies wholly
-// inside the open run, or wholly outside any run, costs only its ray tests.
-__device__ __forceinline__ void scan_window(const RowCtx& R, int s, int e, bool extL, bool extR,
-                                            TaskState& S) {
-  const int ln = __lane_id();
-  const int len = e - s + 1;
-  const int extra = ((len + 63) / 64) * 64 - len;
-  const int padL = extL ? (extR ? extra / 2 : extra) : 0;
-  const int padR = extR ? extra - padL : 0;
-  const int ws = s - padL < 0 ? 0 : s - padL;
-  const int we = e + padR > R.N - 1 ? R.N - 1 : e + padR;
-  int hi = we;             // last column of the scan (grows past we while a run is followed)
-  bool open = false;
-  int runL = 0, cb = ws - 64, nb = 0, pos = 0;
-  unsigned long long m = 0, cnt = 0;
-  long long acc = 0, val = 0;  // lane-local brightness of the open run, of this lane's pixel
-  for (int guard = 0;; guard++) {
-    if (guard > (1 << 27)) {
-      // more iterations than any row of 2^25 pixels needs: never expected;
-      // the point is flagged and the launch ends
-      flag_point(*S.A, S.gp, kFlagTimeout);
-      if (ln == 0) atomicExch(S.A->abortFlag, 1);
-      break;
-    }
-    bool emit = false, last = false;
-    int eR = 0;
-    if (pos >= nb) {
-      // the next 64 pixels, or the end of the scan
-      if (cb + 64 > hi) {
-        if (!open) break;
-        if (hi == we && extR && we < R.N - 1) {
-          hi = R.N - 1;  // follow the run past the window, from we + 1 on
-          cb = we + 1 - 64;
-        } else {
-          last = true;  // the run reaches the scan's last column
-          eR = hi;
-          emit = hi >= s && runL <= e;
-          if (!emit) break;
+          a1 = center;
+          a2 = -1;
         }
       }
-      if (!last) {
-        if (!open && cb + 64 > e) break;  // no later run can meet [s, e]
-        // the next steps; while each lies wholly inside the open run it is
-        // taken in without the boundary bookkeeping
-        unsigned evals = 0;
-        const bool inside =
-            R.map == kMapInRange
-                ? scan_steps<kMapInRange>(R, open, hi, cb, m, nb, val, acc, cnt, evals)
-            : R.map == kMapTriple
-                ? scan_steps<kMapTriple>(R, open, hi, cb, m, nb, val, acc, cnt, evals)
-                : scan_steps<kMapBinary>(R, open, hi, cb, m, nb, val, acc, cnt, evals);
-        S.evals += evals;
-        pos = (inside || (!open && m == 0)) ? nb : 0;
-        continue;
-      }
-    } else if (open) {
-      const unsigned long long rest = ~(m >> pos);
-      int z = rest == 0 ? 64 - pos : __builtin_ctzll(rest);
-      if (z > nb - pos) z = nb - pos;
-      if (ln >= pos && ln < pos + z) acc += val;
-      cnt += (unsigned long long)z;
-      pos += z;
-      if (pos < nb) {
-        // the run ends at cb + pos - 1
-        eR = cb + pos - 1;
-        emit = eR >= s && runL <= e;
-        if (!emit) {
-          open = false;
-          acc = 0;
-          cnt = 0;
-          if (hi > we) break;  // the followed run has ended
-        }
-      }
-    } else {
-      const unsigned long long rest = m >> pos;
-      if (rest == 0) {
-        pos = nb;
-        continue;
-      }
-      const int tz = __builtin_ctzll(rest);
-      if (cb + pos + tz > e) break;  // no later run can meet [s, e]
-      runL = cb + pos + tz;
-      open = true;
-      pos += tz;
+      follow(W, make_task(b, row + d, xl, xr, label, 0, d, a1, a2), 0);
     }
-    if (emit) {
-      if (runL == ws && extL && ws > 0) runL = extend_left(R, ws - 1, acc, cnt, S.evals);
-      handle_run(S, runL, eR, wave_sum(acc), cnt);
-      acc = 0;
-      cnt = 0;
-      open = false;
-      if (last || hi > we) break;
-    }
+    return past;
   }
+  if (kind == 1) {
+    if (row + 1 < N) follow(W, make_task(b, row + 1, xl, xr, label, 0, 1, center, 0), 0);
+    if (row - 1 >= 0) follow(W, make_task(b, row - 1, xl, xr, label, 0, -1, center, 0), 0);
+    return false;
+  }
+  if (kind == 3) {
+    // a run found looking back: sweep on away from the run it was reached
+    // from, and look back towards that run's row where this one reaches past it
+    if (ahead) follow(W, make_task(b, row + d, xl, xr, label, 0, d, center, 0), 0);
+    if (past)
+      follow(W, make_task(b, row - d, xl, xr, label, 3, -d, S.xa - 1, S.xb + 1), kQueueOnly);
+    return false;
+  }
+  // A scout landed (f1: the column of the run it was sent from, one jump
+  // back; f2: that jump's length and the scouts in its chain since the last
+  // leap).  The wave sends the next scout straight on at once, with the shift
+  // measured over the last jump, and keeps it as its next step, so that the
+  // scouts run ahead one task per jump; every leapEvery-th scout also sends a
+  // leap scout leapJumps jumps ahead to the shared queue, which starts a
+  // chain of its own, so that long images get many chains.  The two sweeps of
+  // the new class go to the shared queue for idle waves; they start as if
+  // they had just sent a scout.
+  W.nScoutRuns++;
+  const ArgPtr A = opq(W.A);
+  const int count = f2 & 0xFFFF, prevJump = (int)((unsigned)f2 >> 16);
+  const int J = scout_jump_for(A, xr - xl + 1);
+  // the shift over the last jump, rescaled to this jump
+  const long long shift = ((long long)center - f1) * J / (prevJump > 0 ? prevJump : J);
+  const long long ash = shift < 0 ? -shift : shift;
+  const int leapEvery = A->leapEvery, leapJumps = A->leapJumps;
+  const int legs = leapEvery <= 0 || (count + 1) % leapEvery != 0 ? 1 : 2;
+  for (int leap = 0; leap < legs && W.scoutRows > 0; leap++) {
+    const long long k = leap ? leapJumps : 1;
+    const long long rt = (long long)row + (long long)d * J * k;
+    if (rt < 0 || rt >= N) continue;
+    const long long pc = center + shift * k;
+    const long long hw = ((long long)xr - xl) / 2 + ash * k / 4 + 32 * k;
+    long long sa = pc - hw, sb = pc + hw;
+    if (sa < 0) sa = 0;
+    if (sb > N - 1) sb = N - 1;
+    if (sa > sb) continue;
+    // a leap's chain measures its next shift from the column expected one
+    // jump before its landing row
+    follow(W,
+           make_task(b, (int)rt, (int)sa, (int)sb, -1, 2, d,
+                     leap ? (int)(center + shift * (leapJumps - 1)) : center,
+                     (J << 16) | (leap ? 0 : (count + 1) & 0xFFFF)),
+           leap ? kQueueOnly | kShare : 0);
+  }
+  for (int e = 1; e >= -1; e -= 2)
+    if (row + e >= 0 && row + e < N)
+      follow(W, make_task(b, row + e, xl, xr, label, 0, e, center, -1), kShare);
+  return false;
 }
 
 // ---------------------------------------------------------------------------
 // Fill
 // ---------------------------------------------------------------------------
-// Processes one task and the look-backs it records, as up to six scans of one
-// row each: the task's row (one interval, or two around a known run), then
-// each look-back (the same).  The follow-up kept for this wave (if any) is
-// left in S.cont / S.haveCont.
-// The task's fields as wave-uniform values, and the constants of its source
-// position (kept while the wave stays on that position).
-__device__ __forceinline__ void load_task(TaskState& S) {
-  const FillArgs& A = *S.A;
-  S.t.b = uni(S.t.b);
-  S.t.row = uni(S.t.row);
-  S.t.xa = uni(S.t.xa);
-  S.t.xb = uni(S.t.xb);
-  S.t.label = uni(S.t.label);
-  S.t.kd = uni(S.t.kd);
-  S.t.f1 = uni(S.t.f1);
-  S.t.f2 = uni(S.t.f2);
-  S.kind = S.t.kd & 3;
-  S.dir = (S.t.kd & 4) ? -1 : 1;
-  if (S.t.b != S.curB) {
-    // constants of this source position, kept while the wave stays on it
-    S.curB = S.t.b;
-    S.gp = uni(A.batchPts[S.t.b]);
-    const CurveDev& C = A.curves[uni(A.ptCurve[S.gp])];
-    S.N = uni((int)C.N);
-    S.R.L.m1 = unid(C.L.m1); S.R.L.m2 = unid(C.L.m2); S.R.L.m3 = unid(C.L.m3);
-    S.R.L.z1 = mk(unid(C.L.z1.re), unid(C.L.z1.im));
-    S.R.L.z2 = mk(unid(C.L.z2.re), unid(C.L.z2.im));
-    S.R.L.z3 = mk(unid(C.L.z3.re), unid(C.L.z3.im));
-    S.R.blx = unid(C.blx);
-    S.R.bly = unid(C.bly);
-    S.R.step = unid(C.step);
-    S.R.rho2 = unid(C.rho2);
-    S.R.invRho2 = 1.0 / S.R.rho2;
-    S.R.ldA = unid(C.ldA);
-    S.R.ldB = unid(C.ldB);
-    S.R.sumScale = unid(C.sumScale);
-    const int bin = uni(C.binIrs);
-    S.R.inRange = bin ? 0 : uni((int)lens_in_range(S.R.L, S.R.blx, S.R.bly, S.R.step, S.N));
-    S.R.map = bin ? kMapBinary : kMapTriple;
-    S.heavy = A.shareRays > 0.0f && A.ptCost[S.gp] >= A.shareRays;
-    S.R.N = S.N;
-    const double2 pos = A.ptPos[S.gp];
-    S.R.px = unid(pos.x);
-    S.R.py = unid(pos.y);
-  }
+// The constants of batch point b, kept while the wave stays on it.
+__device__ __forceinline__ void load_position(Worker& W, int b) {
+  const ArgPtr A = opq(W.A);
+  flush_acc(W);  // under the old position's profile
+  W.accLabel = -1;
+  W.curB = b;
+  const int ln = __lane_id();
+  const double pc = A->points[(size_t)b * kPointRec + (ln < kPointRec ? ln : 0)];
+  const int g = b >> 14;
+  W.tab = A->htab + 2 * (size_t)uni64((long long)A->grpBase[g]);
+  W.tabMask = (unsigned)uni64((long long)A->grpMask[g]);
+  Ray& R = W.R;
+  R.pc = pc;
+  R.m1 = rl(pc, kPcM1); R.m2 = rl(pc, kPcM2); R.m3 = rl(pc, kPcM3);
+  R.x1 = rl(pc, kPcX1); R.x2 = rl(pc, kPcX2); R.x3 = rl(pc, kPcX3);
+  R.blx = rl(pc, kPcBlx); R.step = rl(pc, kPcStep);
+  R.px = rl(pc, kPcPx); R.inv = rl(pc, kPcInv);
+  W.gp = uni((int)rl(pc, kPcGp));
+  W.N = uni((int)rl(pc, kPcN));
+  W.flags = uni((int)rl(pc, kPcFlags));
 }
 
-__device__ __forceinline__ void process_task(TaskState& S) {
-  const FillArgs& A = *S.A;
-  S.haveCont = false;
-  S.nBack = 0;
-  load_task(S);
-  S.nScout += S.kind == 2 ? 1 : 0;
-  if (S.t.row < 0 || S.t.row >= S.N) return;
-  if (S.kind == 1 && (S.t.xa < 0 || S.t.xa > S.N - 1)) {  // seed column outside the grid
-    flag_point(A, S.gp, kFlagEdge);
-    return;
+// The rows of a sweep (the task in hand, kind 0) on a position whose rows are
+// fast: four rows at most, then the caller looks after the hand-off of waiting
+// tasks.  This is where a fill spends its time, so it is kept apart from the
+// general code: what process_task needs for scouts, seeds and look-backs would
+// be live across the row loop and spill.  Further runs go to the wave's ring;
+// look-backs end the call (process_task handles them at once: the images'
+// other branches start there).  Leaves the sweep's next row in W.t
+// (W.haveCont), for process_task (W.general) where it has to be evaluated
+// exactly.
+template <int MODE, bool LIMB>
+__device__ __forceinline__ void sweep_rows(Worker& W) {
+  const RowBase B = row_base(W.R);
+  const int N = W.N, b = W.t.b, d = (W.t.kd & 4) ? -1 : 1;
+  int row = W.t.row, xa = W.t.xa, xb = W.t.xb, label = W.t.label, f1 = W.t.f1, f2 = W.t.f2;
+  W.haveCont = false;
+  if (label != W.accLabel || W.accCnt >= (1u << 25)) {
+    flush_acc(W);
+    W.accLabel = label;
   }
-  int k1 = S.kind == 3 ? S.t.f1 : 0, k2 = S.kind == 3 ? S.t.f2 : -1;
-  S.xa = S.t.xa;
-  S.xb = S.t.xb;
-  const bool scout = S.kind == 2;
-  const int trow = S.t.row, txa = S.t.xa, txb = S.t.xb, tf1 = S.t.f1, tf2 = S.t.f2, tdir = S.dir;
-  S.landed = false;
-  for (int job = 0; job < 6; job++) {
-    if (job >= 2) {
-      const int li = (job - 2) >> 1;
-      if (li >= S.nBack) break;
-      if ((job & 1) == 0) {
-        const LookBack lb = li == 0 ? S.back0 : S.back1;
-        S.t.row = lb.row;
-        S.t.label = lb.label;
-        S.kind = 3;
-        S.dir = lb.dir;
-        S.xa = lb.xa;
-        S.xb = lb.xb;
-        k1 = lb.k1;
-        k2 = lb.k2;
+  while ((unsigned)row < (unsigned)N) {
+    if (__builtin_expect(!far_row(W.R, B, row), 0)) {
+      if (!near_row(W.R, MODE == kRowBinary)) {
+        W.general = true;
+        break;
       }
-    } else if (job == 1 && k1 > k2) {
-      continue;  // a task without a known run inside its interval scans once
     }
-    if ((job & 1) == 0) {
-      S.R.y = S.R.bly + S.R.step * (double)S.t.row;
-      if (S.R.map != kMapBinary)
-        S.R.map = S.R.inRange && uni((int)row_in_range(S.R.L, S.R.y)) ? kMapInRange : kMapTriple;
-    }
-    const int lo = S.xa < 0 ? 0 : S.xa, hi = S.xb > S.N - 1 ? S.N - 1 : S.xb;
-    int s = lo, e = hi;
-    bool extL = true, extR = true;
-    if (k1 <= k2) {
-      // two sides of the known pixels [k1, k2]
-      if ((job & 1) == 0) {
-        e = hi < k1 - 1 ? hi : k1 - 1;
-        extR = hi < k1 - 1;
+    RunScan Q;
+    Q.steps = 0;
+    scan_begin(Q, N, xa < 0 ? 0 : xa, xb > N - 1 ? N - 1 : xb, true, true);
+    // f2 >= 0: rows since the sweep's anchor, no scout sent yet;
+    // f2 < 0: -(rows since the last scout) - 1
+    int a1 = f1, a2 = f2 >= 0 ? f2 + 1 : f2 - 1;
+    bool have = false;
+    int nl = 0, nr = 0;
+    while (next_run_in<MODE, LIMB>(W.R, N, Q)) {
+      int other = 0;
+      const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, Q.xl, Q.xr, label, other);
+      if (__builtin_expect(ins != kInsNew, 0)) {
+        if (ins == kInsFull) {
+          flag_point(W.A, W.gp, kFlagHashFull);
+        } else {
+          W.nDup++;
+          unite(opq(W.A)->lparent, label, other);
+        }
+        continue;
+      }
+      W.nIns++;
+      W.accCnt += Q.cnt;
+      if (LIMB) W.accBits += Q.acc;
+      if (__builtin_expect(Q.xl <= 1 || Q.xr >= N - 2, 0)) flag_point(W.A, W.gp, kFlagEdge);
+      if (!have) {
+        have = true;
+        nl = Q.xl;
+        nr = Q.xr;
       } else {
-        s = lo > k2 + 1 ? lo : k2 + 1;
-        extL = lo > k2 + 1;
+        const int r = opq(row) + d;
+        if ((unsigned)r < (unsigned)N)
+          ring_put(W, make_task(b, r, Q.xl, Q.xr, label, 0, d, a1, a2));
+      }
+      if (__builtin_expect(Q.xl < xa - 1 || Q.xr > xb + 1, 0)) {
+        // the run reaches past its parent and the parent's bounding misses
+        const int r = opq(row) - d;
+        if ((unsigned)r < (unsigned)N)
+          put_back(W, make_task(b, r, Q.xl, Q.xr, label, 3, -d, xa - 1, xb + 1));
+      }
+      // a flush in time: at most 2^26 pixels, whose integers stay below 2^62
+      if (__builtin_expect(W.accCnt >= (1u << 25), 0)) flush_acc(W);
+      if (__builtin_expect(W.lcount > kLocalCap - kRoom, 0)) hand_off(W, 0);
+    }
+    W.steps += Q.steps;
+    W.nTasks++;
+    if (!have) break;
+    const int rows = a2 >= 0 ? a2 : -a2 - 1;
+    if (__builtin_expect(rows >= (a2 >= 0 ? W.scoutRows : kMinJump) && W.scoutRows > 0, 0)) {
+      const ArgPtr A = opq(W.A);
+      const int xl = opq(nl), xr = opq(nr), r0 = opq(row), n = opq(N);
+      const int J = scout_jump_for(A, xr - xl + 1);
+      if (a2 >= 0 || rows >= J) {
+        // send a scout ahead along the run's drift, then re-anchor
+        const int center = (int)(((unsigned)xl + (unsigned)xr) / 2);
+        const long long rt = (long long)r0 + (long long)d * J;
+        if (rt >= 0 && rt < n) {
+          const long long drift = rows > 0 ? (center - a1) / rows : 0;
+          const long long pc = center + drift * J;
+          const long long adr = drift < 0 ? -drift : drift;
+          const long long hw = ((long long)xr - xl) / 2 + adr * J / 4 + 32;
+          long long sa = pc - hw, sb = pc + hw;
+          if (sa < 0) sa = 0;
+          if (sb > n - 1) sb = n - 1;
+          // to the wave's ring (the pool while some wave is idle), or to the
+          // pool at once on the images of positions predicted heavy, whose
+          // scouts mostly land: sweeps of many small images send many scouts
+          // that miss, and queuing each of them at once makes the queues the
+          // bottleneck
+          if (sa <= sb)
+            follow(W, make_task(b, (int)rt, (int)sa, (int)sb, -1, 2, d, center, J << 16),
+                   kQueueOnly | ((A->scoutShare || (W.flags & kPtHeavy)) ? kShare : 0));
+        }
+        a1 = center;
+        a2 = -1;
       }
     }
-    if (s > e) continue;
-    scan_window(S.R, s, e, extL, extR, S);
+    row += d;
+    xa = nl;
+    xb = nr;
+    f1 = a1;
+    f2 = a2;
+    if ((W.nTasks & 3) == 0 || W.nOut + W.nBack > 0) {
+      W.haveCont = (unsigned)row < (unsigned)N;
+      break;
+    }
   }
-  S.nBack = 0;
-  if (scout && !S.landed && A.scoutRetry) {
-    // A scout that found nothing (its chain's prediction failed, or the
-    // image ends before its row): a retry from the same origin, half the
-    // jump ahead, with a window of the same width about the midpoint of the
-    // origin column and the failed window's centre.
-    const int J = (int)((unsigned)tf2 >> 16), count = tf2 & 0xFFFF;
+  W.t.row = row;
+  W.t.xa = xa;
+  W.t.xb = xb;
+  W.t.f1 = f1;
+  W.t.f2 = f2;
+}
+
+// Processes the task in hand and the look-backs recorded meanwhile (up to two;
+// the others are queued): the task's row, in one piece or in two around known
+// pixels, then each look-back the same way.  The follow-up kept for this wave
+// (if any) is left in W.t / W.haveCont.  With backsOnly, the look-backs that
+// sweep_rows recorded, leaving W.t / W.haveCont as they are (with nothing in
+// hand, the first follow-up is kept).
+__device__ __forceinline__ void process_task(Worker& W, bool backsOnly) {
+  const Task t = W.t;
+  const int kind0 = backsOnly ? 3 : t.kd & 3;
+  Scan S;
+  S.row = -1;
+  int taken = 0;
+  W.general = false;
+  W.landed = false;
+  if (!backsOnly) {
+    W.haveCont = false;
+    if (t.b != W.curB) load_position(W, t.b);
+    S.kind = kind0;
+    S.dir = (t.kd & 4) ? -1 : 1;
+    S.row = t.row;
+    S.label = t.label;
+    S.xa = t.xa;
+    S.xb = t.xb;
+    S.k1 = S.kind == 3 ? t.f1 : 0;
+    S.k2 = S.kind == 3 ? t.f2 : -1;
+    if ((unsigned)t.row >= (unsigned)W.N) return;
+    if (__builtin_expect(S.kind == 1 && (unsigned)t.xa > (unsigned)(W.N - 1), 0)) {
+      flag_point(W.A, W.gp, kFlagEdge);  // seed column outside the grid
+      return;
+    }
+  }
+  const bool limb = (W.flags & kPtLimb) != 0;
+  while (true) {
+    if (S.row < 0) {
+      if (taken >= W.nBack) break;
+      const Task lb = lanes_task(*task_int(&W.back[taken], W.spare));
+      taken++;
+      S.kind = 3;
+      S.dir = (lb.kd & 4) ? -1 : 1;
+      S.row = lb.row;
+      S.label = lb.label;
+      S.xa = lb.xa;
+      S.xb = lb.xb;
+      S.k1 = lb.f1;
+      S.k2 = lb.f2;
+    }
+    set_row(W.R, W.flags, S.row);
+    const int N = W.N;
+    const int lo = S.xa < 0 ? 0 : S.xa, hi = S.xb > N - 1 ? N - 1 : S.xb;
+    const bool known = S.k1 <= S.k2;
+    for (int side = 0; side < (known ? 2 : 1); side++) {
+      int s = lo, e = hi;
+      bool extL = true, extR = true;
+      if (__builtin_expect(known, 0)) {
+        if (side == 0) {
+          e = hi < S.k1 - 1 ? hi : S.k1 - 1;
+          extR = hi < S.k1 - 1;
+        } else {
+          s = lo > S.k2 + 1 ? lo : S.k2 + 1;
+          extL = lo > S.k2 + 1;
+        }
+      }
+      if (s > e) continue;
+      RunScan Q;
+      Q.steps = 0;
+      scan_begin(Q, N, s, e, extL, extR);
+      while (next_run(W.R, N, limb, Q)) {
+        if (__builtin_expect(W.nOut > kOutCap - 4 || W.lcount > kLocalCap - kRoom, 0))
+          hand_off(W, 0);
+        int label = 0;
+        if (__builtin_expect(handle_run(W, S, t.f1, t.f2, Q.xl, Q.xr, Q.cnt, Q.acc, label), 0)) {
+          put_back(W, make_task(W.curB, S.row - S.dir, Q.xl, Q.xr, label, 3, -S.dir, S.xa - 1,
+                                S.xb + 1));
+        }
+      }
+      W.steps += Q.steps;
+    }
+    S.row = -1;
+  }
+  W.nBack = 0;
+  if (__builtin_expect(kind0 == 2, 0)) {
+    W.nScout++;
+    const int f2 = opq(t.f2);
+    const int J = (int)((unsigned)f2 >> 16), count = f2 & 0xFFFF;
     const int J2 = J / 2;
-    if (J2 >= kMinJump) {
-      const long long rt = (long long)trow - (long long)tdir * (J - J2);
-      const long long pc = ((long long)txa + txb) / 2;
-      const long long c2 = tf1 + (pc - tf1) / 2;
-      const long long hw = ((long long)txb - txa) / 2;
+    if (!W.landed && J2 >= kMinJump && opq(W.A)->scoutRetry) {
+      // A scout that found nothing (its chain's prediction failed, or the
+      // image ends before its row): a retry from the same origin, half the
+      // jump ahead, with a window of the same width about the midpoint of the
+      // origin column and the failed window's centre.
+      const int N = opq(W.N), xa = opq(t.xa), xb = opq(t.xb);
+      const int dir = (t.kd & 4) ? -1 : 1;
+      const long long rt = (long long)t.row - (long long)dir * (J - J2);
+      const long long pc = ((long long)xa + xb) / 2;
+      const long long c2 = t.f1 + (pc - t.f1) / 2;
+      const long long hw = ((long long)xb - xa) / 2;
       long long sa = c2 - hw, sb = c2 + hw;
       if (sa < 0) sa = 0;
-      if (sb > S.N - 1) sb = S.N - 1;
-      if (rt >= 0 && rt < S.N && sa <= sb) {
-        follow(S, make_task(S.t.b, (int)rt, (int)sa, (int)sb, -1, 2, tdir, tf1,
-                            (J2 << 16) | count));
-      }
+      if (sb > N - 1) sb = N - 1;
+      if (rt >= 0 && rt < N && sa <= sb)
+        follow(W, make_task(t.b, (int)rt, (int)sa, (int)sb, -1, 2, dir, t.f1, (J2 << 16) | count),
+               0);
     }
   }
 }
@@ -2494,7 +2818,7 @@ __device__ __forceinline__ void process_task(TaskState& S) {
 // count is 0 and the ring is empty: no group then holds work, and a group
 // that starts later (its compute unit was busy with other kernels) finds
 // none and leaves.  So the groups need not all be resident at once.
-__device__ void fill_manager(const FillArgs& A, GroupPool* G, long long t0,
+__device__ __forceinline__ void fill_manager(const FillArgs& A, GroupPool* G, long long t0,
                              unsigned long long& polls) {
   const int ln = __lane_id();
   if (ln == 0) {
@@ -2620,8 +2944,11 @@ __device__ void fill_manager(const FillArgs& A, GroupPool* G, long long t0,
 __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
   __shared__ Task rings[kWorkers][kLocalCap];
   __shared__ GroupPool pool;
+  __shared__ Task outs[kWorkers][kOutCap];
+  __shared__ Task backs[kWorkers][2];
+  __shared__ int spare[kWorkers][64];
   const int ln = __lane_id();
-  const int wave = threadIdx.x / 64;
+  const int wave = uni((int)(threadIdx.x / 64));
   const long long t0 = (long long)__builtin_amdgcn_s_memrealtime();
   GroupPool* G = &pool;
   if (threadIdx.x == 0) {
@@ -2633,112 +2960,127 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
     G->hungry = 0;
   }
   __syncthreads();
-  unsigned long long nTasks = 0, busyTicks = 0, idlePolls = 0;
   if (wave == 0) {
-    fill_manager(A, G, t0, idlePolls);
-    if (ln == 0) atomicAdd(&A.stats[6], idlePolls);
+    unsigned long long polls = 0;
+    fill_manager(A, G, t0, polls);
+    if (ln == 0) atomicAdd(&A.stats[6], polls);
     return;
   }
-  TaskState S;
-  S.A = &A;
-  S.G = G;
-  S.curB = -1;
-  S.evals = 0;
-  S.nIns = 0;
-  S.nDup = 0;
-  S.insTicks = 0;
-  S.nScout = 0;
-  S.nScoutRuns = 0;
-  S.accLabel = -1;
-  S.accSum = 0;
-  S.accCnt = 0;
-  S.ring = rings[wave - 1];
-  S.lhead = 0;
-  S.lcount = 0;
+  Worker W;
+  W.A = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  W.scoutRows = A.scoutRows;
+  W.G = G;
+  W.ring = rings[wave - 1];
+  W.out = outs[wave - 1];
+  W.nOut = 0;
+  W.back = backs[wave - 1];
+  W.nBack = 0;
+  W.spare = spare[wave - 1];
+  W.lhead = 0;
+  W.lcount = 0;
+  W.general = false;
+  W.haveCont = false;
+  W.curB = -1;
+  W.gp = W.N = W.flags = 0;
+  W.tab = nullptr;
+  W.tabMask = 0;
+  W.accLabel = -1;
+  W.accCnt = 0;
+  W.accBits = 0;
+  W.nTasks = W.nIns = W.nDup = W.nScout = W.nScoutRuns = W.steps = 0;
+  const bool newest = A.poolNewest != 0;
+  unsigned idlePolls = 0;
+  unsigned long long idleTicks = 0;
   bool have = false, busy = false;
   while (true) {
-    if (!have && S.lcount > 0) {
-      S.t = ring_pop(S);
+    if (!have && W.lcount > 0) {
+      W.t = ring_pop(W);
       have = true;
     }
     if (!have && busy) {
-      // own work done: the pool's oldest task, or idle
-      flush_acc(S);
-      have = pool_take(G, S.t, true, A.poolNewest != 0);
+      // own work done: a task of the pool, or idle
+      flush_acc(W);
+      have = pool_take(G, W.t, true, newest, W.spare);
       busy = have;
     }
     if (!have) {
+      const long long ti = (long long)__builtin_amdgcn_s_memrealtime();
       bool over = false;
       while (true) {
         idlePolls++;
         __builtin_amdgcn_s_sleep(24);
-        int d = 0, c = 0;
-        if (ln == 0) {
-          d = lds_ld(&G->done);
-          c = lds_ld(&G->count);
+        if (uni(lds_ld(&G->done))) {
+          over = true;
+          break;
         }
-        if (uni(d)) { over = true; break; }
-        if (uni(c) > 0 && pool_take(G, S.t, false, A.poolNewest != 0)) break;
+        if (uni(lds_ld(&G->count)) > 0 && pool_take(G, W.t, false, newest, W.spare)) break;
         if ((idlePolls & 255) == 0 &&
-            (long long)__builtin_amdgcn_s_memrealtime() - t0 > A.timeLimitTicks + 100000000ll) {
+            (long long)__builtin_amdgcn_s_memrealtime() - t0 >
+                opq(W.A)->timeLimitTicks + 100000000ll) {
           // the manager ends the fill at the time limit; this bound only
           // guards against a manager that never does
           over = true;
           break;
         }
       }
+      idleTicks += (unsigned long long)((long long)__builtin_amdgcn_s_memrealtime() - ti);
       if (over) break;
-      have = true;
       busy = true;
     }
-    nTasks++;
-    const unsigned long long tb0 = __builtin_amdgcn_s_memrealtime();
-    process_task(S);
-    busyTicks += __builtin_amdgcn_s_memrealtime() - tb0;
-    if (S.haveCont) {
-      S.t = S.cont;
+    if ((W.t.kd & 3) == 0) {
+      if (W.t.b != W.curB) load_position(W, W.t.b);
+      const bool limb = (W.flags & kPtLimb) != 0;
+      switch (W.flags & (kPtFast | kPtBinary)) {
+        case kPtFast:
+          limb ? sweep_rows<kRowTriple, true>(W) : sweep_rows<kRowTriple, false>(W);
+          break;
+        case kPtFast | kPtBinary:
+          limb ? sweep_rows<kRowBinary, true>(W) : sweep_rows<kRowBinary, false>(W);
+          break;
+        default: W.general = true;
+      }
     } else {
-      have = false;
+      W.general = true;
     }
-    if ((nTasks & 3) == 0 && S.lcount > 0) {
-      // hand waiting tasks to idle workers of the group, and while other
-      // groups are idle keep the pool topped up for them
-      int pend = 0, cnt = 0, hungry = 0;
-      if (ln == 0) {
-        pend = lds_ld(&G->pending);
-        cnt = lds_ld(&G->count);
-        hungry = lds_ld(&G->hungry);
-      }
-      cnt = uni(cnt);
-      const int idle = kWorkers - (uni(pend) - cnt);
-      if (idle > cnt || (uni(hungry) && cnt < kPoolShare)) {
-        ring_donate(S);
-        if (S.lcount > 2) ring_donate(S);
-      }
+    if (W.general || W.nBack > 0) {
+      const bool backs = !W.general;
+      W.nTasks += backs ? 0 : 1;
+      process_task(W, backs);
     }
-    if ((nTasks & 255) == 0) {
+    have = W.haveCont;
+    // the out buffer's tasks to the pool; every fourth task, waiting ones to
+    // idle workers of the group, and while other groups are idle enough to
+    // keep the pool topped up for them
+    int give = 0;
+    if ((W.nTasks & 3) == 0 && W.lcount > 0) {
+      const int pend = uni(lds_ld(&G->pending)), cnt = uni(lds_ld(&G->count));
+      const int idle = kWorkers - (pend - cnt);
+      if (idle > cnt || (uni(lds_ld(&G->hungry)) && cnt < kPoolShare)) give = W.lcount > 2 ? 2 : 1;
+    }
+    if (W.nOut + give > 0) hand_off(W, give);
+    if ((W.nTasks & 255) == 0) {
       const long long now = (long long)__builtin_amdgcn_s_memrealtime();
-      if (now - t0 > A.timeLimitTicks) {
-        if (ln == 0) atomicExch(A.abortFlag, 1);
+      const ArgPtr a = opq(W.A);
+      if (now - t0 > a->timeLimitTicks) {
+        store32_lane0(a->abortFlag, 1);
         break;
       }
-      int ab = 0;
-      if (ln == 0) ab = aldi(A.abortFlag);
-      if (uni(ab)) break;
+      if (uni(aldi(a->abortFlag))) break;
     }
   }
-  flush_acc(S);
+  flush_acc(W);
+  const unsigned long long busyTicks =
+      (unsigned long long)((long long)__builtin_amdgcn_s_memrealtime() - t0) - idleTicks;
   if (ln == 0) {
-    atomicAdd(&A.stats[0], nTasks);
-    atomicAdd(&A.stats[1], S.evals);
-    atomicAdd(&A.stats[2], S.nIns);
-    atomicAdd(&A.stats[3], S.nDup);
+    atomicAdd(&A.stats[0], (unsigned long long)W.nTasks);
+    atomicAdd(&A.stats[1], 64ull * W.steps);
+    atomicAdd(&A.stats[2], (unsigned long long)W.nIns);
+    atomicAdd(&A.stats[3], (unsigned long long)W.nDup);
     atomicAdd(&A.stats[4], busyTicks);
-    atomicAdd(&A.stats[5], S.insTicks);
-    atomicAdd(&A.stats[6], idlePolls);
+    atomicAdd(&A.stats[6], (unsigned long long)idlePolls);
     atomicAdd(&A.stats[7], 1ull);
-    atomicAdd(&A.stats[8], S.nScout);
-    atomicAdd(&A.stats[9], S.nScoutRuns);
+    atomicAdd(&A.stats[8], (unsigned long long)W.nScout);
+    atomicAdd(&A.stats[9], (unsigned long long)W.nScoutRuns);
   }
 }
 

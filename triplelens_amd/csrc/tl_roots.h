@@ -63,7 +63,10 @@ __device__ __forceinline__ double quot_near(double a, double b, double r) {
 // s = sqrt(a) rounded to nearest and h close to 1 / (2 s), for
 // 2^-600 <= a <= 2^600: the hardware reciprocal root y, s0 = a y, h0 = y/2 with
 // h0 s0 = 1/2 - e, one third-order step (1 - 2e)^-1/2 = 1 + e + 3/2 e^2, and the
-// exact residual.
+// exact residual.  The value before the last rounding is good to 2^-104; a
+// root lies that close to a rounding boundary for about a dozen of the 2^53
+// mantissas (those next to 1 among them), where s may be the neighbouring
+// double.
 __device__ __forceinline__ void sqrt_near(double a, double& s, double& h) {
   const double y = __builtin_amdgcn_rsq(a);
   const double s0 = a * y, h0 = 0.5 * y;
@@ -88,7 +91,7 @@ __device__ __forceinline__ double hyp_near(double ax, double ay) {
   return h - quot_near(h <= 2.0 * ay ? ta : tb, w, r);
 }
 __device__ __forceinline__ bool hyp_in_range(double ax, double ay) {
-  return (ay >= 0x1p-240) & (ax <= 0x1p+240) & (ay > ax * 0x1p-54);
+  return (int(ay >= 0x1p-240) & int(ax <= 0x1p+240) & int(ay > ax * 0x1p-54)) != 0;
 }
 // csqrt_sel for re, im with hyp_in_range(max, min) of their magnitudes.
 __device__ __forceinline__ cx csqrt_near(double re, double im) {
@@ -206,14 +209,14 @@ __device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M 
     const double e2 = el * el;
     bool far = nb > e2 * 1.0001;  // nb above 1e-250 follows from lo below
     if (__builtin_expect(!all(far), 0)) {
-      if (all((nb < e2 * 0.49999) & (e2 > 1e-250))) return true;
+      if (all(nb < e2 * 0.49999 && e2 > 1e-250)) return true;
       if (any(!far)) {
         // inside the bracket: the sum with moduli from the hardware root
         double e = __builtin_amdgcn_sqrt(cnorm(b[M]));
 #pragma unroll
         for (int j = M - 1; j >= 0; j--) e = fma(ax, e, __builtin_amdgcn_sqrt(cnorm(b[j])));
         const double eh = kLagEps * e;
-        if (all((nb < eh * eh * 0.9999) & (eh * eh > 1e-250))) return true;
+        if (all(nb < eh * eh * 0.9999 && eh * eh > 1e-250)) return true;
         far = nb > eh * eh * 1.0001;
       }
     }
@@ -260,11 +263,13 @@ __device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M 
     // and den2 from below as well; f, s, g and den2 too large for the
     // quotients leave rad out of its range.)
     const double lo = min_abs(min_abs(min_abs(xf, yf), min_abs(xs, ys)), min_abs(num, num2));
-    const bool ok = far & (lo >= kTinyOp) & (fabs(den) <= kHugeOp) &
-                    hyp_in_range(max_abs(rad.re, rad.im), min_abs(rad.re, rad.im)) &
-                    (min_abs(np, nm) < max_abs(np, nm) * (1.0 - 1e-12)) &
-                    ((x.re != x1.re) | (x.im != x1.im));
-    if (__builtin_expect(all(ok), 1)) {
+    const double rx = max_abs(rad.re, rad.im), ry = min_abs(rad.re, rad.im);
+    // (ints: a chain of && would be a chain of branches)
+    const int ok = int(far) & int(lo >= kTinyOp) & int(fabs(den) <= kHugeOp) &
+                   int(hyp_in_range(rx, ry)) &
+                   int(min_abs(np, nm) < max_abs(np, nm) * (1.0 - 1e-12)) &
+                   (int(x.re != x1.re) | int(x.im != x1.im));
+    if (__builtin_expect(all(ok != 0), 1)) {
       if (__builtin_expect(i % kLagMT == 0, 0)) {
         oob |= i / kLagMT >= 8;
         x = lag_kick(x, mk(ce2 ? qa : qb, ce2 ? -qb : -qa), i);
