@@ -58,6 +58,48 @@ def test_gradients_match_oracle(S):
         o += k * n + n
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4097])
+def test_forward_row_remainders(S, n):
+    """Row counts around a workgroup's 16 rows: every row as in the oracle
+    (the tolerance of test_forward_matches_oracle) and as in a larger call."""
+    X, _ = _rand_xy(np.random.default_rng(11), 4112)
+    net = S.Net(seed=6)
+    got = net.predict_raw(X[:n])
+    want, _ = mlp.forward(net.params(), X[:n], bf16_mode=True)
+    assert got.shape == want.shape
+    assert np.max(np.abs(got - want)) <= 2e-2 * (1 + np.max(np.abs(want)))
+    assert np.array_equal(got, net.predict_raw(X)[:n])
+
+
+@pytest.mark.parametrize("n", [64, 192, 1088])
+def test_gradient_batch_remainders(S, n):
+    """Batches that end inside the weight gradients' 128 rows per step and
+    their 256-row bias sums."""
+    X, y = _rand_xy(np.random.default_rng(12), n)
+    net = S.Net(seed=9)
+    net.set_params(np.random.default_rng(13).normal(0, 0.05, S.Net.param_count())
+                   .astype(np.float32))
+    loss, g = net.grads(X, y)
+    loss_o, g_o = mlp.loss_and_grad(net.params(), X, y, bf16_mode=True)
+    assert abs(loss - loss_o) <= 1e-3 * abs(loss_o)
+    assert np.linalg.norm(g - g_o) <= 5e-2 * np.linalg.norm(g_o)
+
+
+@pytest.mark.parametrize("steps", [3, 9])
+def test_training_on_part_of_the_rows(S, steps):
+    """Steps that see only part of the rows take those along, more steps index
+    the whole set: the first three are the same either way (the losses are
+    sums of 16-row parts in any order: 64 float additions)."""
+    X, y = _rand_xy(np.random.default_rng(14), 320)
+    net = S.Net(seed=8)
+    net.fit_scaling(X, y)
+    ref = S.Net(seed=8)
+    ref.fit_scaling(X, y)
+    a = net.train(X, y, steps=steps, batch=64, lr=1e-3, seed=5)
+    b = ref.train(X, y, steps=5, batch=64, lr=1e-3, seed=5)
+    np.testing.assert_allclose(a[:3], b[:3], rtol=64 * 2.0 ** -24, atol=64 * 2.0 ** -24)
+
+
 def test_training_reduces_loss(S):
     rng = np.random.default_rng(3)
     net = S.Net(seed=4)

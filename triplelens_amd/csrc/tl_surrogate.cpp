@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <numeric>
 #include <random>
@@ -65,148 +66,47 @@ struct Mlp {
   hipStream_t stream = nullptr;
   MlpLayout L;
   Dev<float> p, g, m, v;   // FP32 master parameters, gradients, Adam moments
-  Dev<uint16_t> pb;        // BF16 copy used by the products
+  Dev<uint16_t> pbF, pbB;   // BF16 copies, in the orders the products read
   Dev<float> mean, scale;  // feature standardisation
   int t = 0;               // Adam steps taken
-  // workspaces for a batch of rows
-  int cap = 0;
-  Dev<uint16_t> h[kMlpLayers];  // h[0]: packed input, h[1..4]: hidden activations
-  Dev<float> z[kMlpLayers - 1];
-  Dev<float> out, y, xin, loss;
-  Dev<uint16_t> dzA, dzB, dz5;
+  // workspaces: inference rows; a training set and one batch of it
+  Dev<float> xin, out, y, loss, scratch;
+  Dev<int> perm;
+  Dev<uint16_t> h[kMlpLayers], dz[kMlpLayers];
 
   ~Mlp() {
-    for (auto* d : {&p, &g, &m, &v, &mean, &scale, &out, &y, &xin, &loss}) d->release();
+    for (auto* d : {&p, &g, &m, &v, &mean, &scale, &out, &y, &xin, &loss, &scratch}) d->release();
+    for (auto* d : {&pbF, &pbB}) d->release();
     for (auto& d : h) d.release();
-    for (auto& d : z) d.release();
-    pb.release();
-    dzA.release();
-    dzB.release();
-    dz5.release();
+    for (auto& d : dz) d.release();
+    perm.release();
     if (stream) (void)hipStreamDestroy(stream);
   }
 
-  void reserve(int rows) {
-    if (rows <= cap) return;
-    h[0].ensure((size_t)rows * kMlpInPad);
-    for (int l = 1; l < kMlpLayers; l++) h[l].ensure((size_t)rows * kMlpHidden);
-    for (int l = 0; l < kMlpLayers - 1; l++) z[l].ensure((size_t)rows * kMlpHidden);
-    out.ensure((size_t)rows * kMlpOutPad);
-    y.ensure(rows);
-    xin.ensure((size_t)rows * kMlpIn);
-    dzA.ensure((size_t)rows * kMlpHidden);
-    dzB.ensure((size_t)rows * kMlpHidden);
-    dz5.ensure((size_t)rows * kMlpOutPad);
-    loss.ensure(1);
-    cap = rows;
-  }
+  MlpWeights weights() const { return {pbF.p, pbB.p, p.p, mean.p, scale.p}; }
 
-  // forward pass over `rows` packed rows in h[0]; keeps the pre-activations
-  // when `keep`
-  void forward(int rows, bool keep) {
+  // a training set of n rows on the GPU and the buffers of batches of it
+  MlpTrainRows train_rows(int n, const float* x, const float* ys, int batch, int nLoss) {
+    xin.ensure((size_t)n * kMlpIn);
+    y.ensure(n);
+    loss.ensure(nLoss);
+    MCHK(hipMemcpyAsync(xin.p, x, (size_t)n * kMlpIn * sizeof(float), hipMemcpyHostToDevice,
+                        stream));
+    MCHK(hipMemcpyAsync(y.p, ys, (size_t)n * sizeof(float), hipMemcpyHostToDevice, stream));
+    MCHK(hipMemsetAsync(loss.p, 0, nLoss * sizeof(float), stream));
+    MlpTrainRows r;
+    r.x = xin.p;
+    r.y = y.p;
+    r.idx = nullptr;
+    r.rows = batch;
+    r.loss = loss.p;
     for (int l = 0; l < kMlpLayers; l++) {
-      GemmArgs a;
-      std::memset(&a, 0, sizeof(a));
-      a.A = h[l].p;
-      a.lda = L.K[l];
-      a.B = pb.p + L.w[l];
-      a.ldb = L.N[l];
-      a.M = rows;
-      a.N = L.N[l];
-      a.K = L.K[l];
-      a.bias = p.p + L.b[l];
-      if (l < kMlpLayers - 1) {
-        a.epi = kEpiGelu;
-        a.Z = keep ? z[l].p : nullptr;
-        a.ldz = kMlpHidden;
-        a.H = h[l + 1].p;
-        a.ldh = kMlpHidden;
-      } else {
-        a.epi = kEpiLinear;
-        a.C = out.p;
-        a.ldc = kMlpOutPad;
-      }
-      MCHK(launch_gemm(a, stream));
+      h[l].ensure((size_t)batch * L.K[l]);
+      dz[l].ensure((size_t)batch * L.N[l]);
+      r.h[l] = h[l].p;
+      r.dz[l] = dz[l].p;
     }
-  }
-
-  // forward pass over `rows` packed rows in h0 with caller-given buffers:
-  // the hidden layers alternate between hA and hB, the output goes to out
-  // (no pre-activations kept)
-  void forward_into(int rows, const uint16_t* h0, uint16_t* hA, uint16_t* hB, float* o) {
-    const uint16_t* in = h0;
-    uint16_t* bufs[2] = {hA, hB};
-    for (int l = 0; l < kMlpLayers; l++) {
-      GemmArgs a;
-      std::memset(&a, 0, sizeof(a));
-      a.A = in;
-      a.lda = L.K[l];
-      a.B = pb.p + L.w[l];
-      a.ldb = L.N[l];
-      a.M = rows;
-      a.N = L.N[l];
-      a.K = L.K[l];
-      a.bias = p.p + L.b[l];
-      if (l < kMlpLayers - 1) {
-        a.epi = kEpiGelu;
-        a.H = bufs[l & 1];
-        a.ldh = kMlpHidden;
-        in = a.H;
-      } else {
-        a.epi = kEpiLinear;
-        a.C = o;
-        a.ldc = kMlpOutPad;
-      }
-      MCHK(launch_gemm(a, stream));
-    }
-  }
-
-  // backward pass from the loss of targets y; gradients into g
-  void backward(int rows) {
-    MCHK(hipMemsetAsync(loss.p, 0, sizeof(float), stream));
-    MCHK(launch_nll_grad(out.p, y.p, rows, dz5.p, loss.p, stream));
-    uint16_t* dz = dz5.p;  // gradient at layer l's pre-activation
-    for (int l = kMlpLayers - 1; l >= 0; l--) {
-      const int Kl = L.K[l], Nl = L.N[l];
-      GemmArgs w;  // dW_l = H_{l-1}^T dZ_l
-      std::memset(&w, 0, sizeof(w));
-      w.A = h[l].p;
-      w.lda = Kl;
-      w.transA = 1;
-      w.B = dz;
-      w.ldb = Nl;
-      w.M = Kl;
-      w.N = Nl;
-      w.K = rows;
-      w.epi = kEpiStore;
-      w.C = g.p + L.w[l];
-      w.ldc = Nl;
-      MCHK(launch_gemm(w, stream));
-      MCHK(launch_colsum(dz, rows, Nl, g.p + L.b[l], stream));
-      if (l == 0) break;
-      GemmArgs d;  // dZ_{l-1} = (dZ_l W_l^T) * GELU'(Z_{l-1})
-      std::memset(&d, 0, sizeof(d));
-      d.A = dz;
-      d.lda = Nl;
-      d.B = pb.p + L.w[l];
-      d.ldb = Nl;
-      d.transB = 1;
-      d.M = rows;
-      d.N = Kl;
-      d.K = Nl;
-      d.epi = kEpiDGelu;
-      d.Z = z[l - 1].p;
-      d.ldz = kMlpHidden;
-      uint16_t* next = (dz == dzA.p) ? dzB.p : dzA.p;
-      d.H = next;
-      d.ldh = kMlpHidden;
-      MCHK(launch_gemm(d, stream));
-      dz = next;
-    }
-  }
-
-  void pack(const float* xdev, int rows) {
-    MCHK(launch_pack_input(xdev, rows, mean.p, scale.p, h[0].p, stream));
+    return r;
   }
 };
 
@@ -242,7 +142,7 @@ void from_logical(const MlpLayout& L, const float* in, std::vector<float>& pad) 
 
 void upload_params(Mlp& M, const std::vector<float>& pad) {
   MCHK(hipMemcpy(M.p.p, pad.data(), pad.size() * sizeof(float), hipMemcpyHostToDevice));
-  MCHK(launch_to_bf16(M.p.p, pad.size(), M.pb.p, M.stream));
+  MCHK(launch_mlp_copies(M.p.p, M.pbF.p, M.pbB.p, M.stream));
   MCHK(hipStreamSynchronize(M.stream));
 }
 
@@ -263,16 +163,15 @@ void* tl_mlp_new(unsigned long long seed) {
       throw std::runtime_error("no HIP device available: the surrogate needs a gfx950 GPU");
     M = new Mlp();
     MCHK(hipStreamCreateWithFlags(&M->stream, hipStreamNonBlocking));
-    // the allocation-free inference's scratch on this device
-    void* scratchBase = nullptr;
-    MCHK(noalloc_scratch(&scratchBase));
     M->L = mlp_layout();
     const size_t n = M->L.total;
     M->p.ensure(n);
     M->g.ensure(n);
     M->m.ensure(n);
     M->v.ensure(n);
-    M->pb.ensure(n);
+    M->pbF.ensure(n);
+    M->pbB.ensure(n);
+    M->scratch.ensure(kNoAllocRows * kMlpOut);
     M->mean.ensure(kMlpIn);
     M->scale.ensure(kMlpIn);
     MCHK(hipMemset(M->m.p, 0, n * sizeof(float)));
@@ -342,35 +241,24 @@ int tl_mlp_predict(void* h, int n, const float* x, float* out) {
     if (n < 0 || (n > 0 && (!x || !out))) throw std::invalid_argument("bad arguments");
     std::lock_guard<std::mutex> lock(M->mu);
     const int chunk = 1 << 16;
-    M->reserve(std::min(((n + 63) / 64) * 64, chunk));
-    std::vector<float> o;
+    const size_t most = (size_t)std::min(n, chunk);
+    M->xin.ensure(most * kMlpIn);
+    M->out.ensure(most * kMlpOut);
     for (int r0 = 0; r0 < n; r0 += chunk) {
       const int rows = std::min(chunk, n - r0);
-      const int padded = ((rows + 15) / 16) * 16;
       MCHK(hipMemcpyAsync(M->xin.p, x + (size_t)r0 * kMlpIn, (size_t)rows * kMlpIn * sizeof(float),
                           hipMemcpyHostToDevice, M->stream));
-      MCHK(launch_pack_input(M->xin.p, rows, M->mean.p, M->scale.p, M->h[0].p, M->stream));
-      if (padded > rows)
-        MCHK(hipMemsetAsync(M->h[0].p + (size_t)rows * kMlpInPad, 0,
-                            (size_t)(padded - rows) * kMlpInPad * sizeof(uint16_t), M->stream));
-      M->forward(padded, false);
-      o.resize((size_t)rows * kMlpOutPad);
-      MCHK(hipMemcpyAsync(o.data(), M->out.p, o.size() * sizeof(float), hipMemcpyDeviceToHost,
+      MCHK(launch_mlp_predict(M->weights(), M->xin.p, rows, M->out.p, M->stream));
+      MCHK(hipMemcpyAsync(out + (size_t)r0 * kMlpOut, M->out.p,
+                          (size_t)rows * kMlpOut * sizeof(float), hipMemcpyDeviceToHost,
                           M->stream));
       MCHK(hipStreamSynchronize(M->stream));
-      for (int i = 0; i < rows; i++) {
-        out[2 * ((size_t)r0 + i)] = o[(size_t)i * kMlpOutPad];
-        out[2 * ((size_t)r0 + i) + 1] = o[(size_t)i * kMlpOutPad + 1];
-      }
     }
     return 0;
   });
 }
 
 int tl_mlp_predict_noalloc(void* h, int n, const float* x, float* out) {
-  // one inference at a time per process: every call uses this GPU's single
-  // scratch array (tl_mlp.hip)
-  static std::mutex noallocMu;
   return mguard([&] {
     Mlp* M = checked(h);
     if (n < 0 || (size_t)n > kNoAllocRows)
@@ -378,20 +266,16 @@ int tl_mlp_predict_noalloc(void* h, int n, const float* x, float* out) {
                                   " rows; at most " + std::to_string(kNoAllocRows) +
                                   " fit its scratch array");
     if (n > 0 && (!x || !out)) throw std::invalid_argument("bad arguments");
-    std::lock_guard<std::mutex> lock(noallocMu);
-    std::lock_guard<std::mutex> lockNet(M->mu);
-    if (n == 0) return 0;
-    void* base = nullptr;
-    MCHK(noalloc_scratch(&base));
-    unsigned char* b = static_cast<unsigned char*>(base);
-    uint16_t* h0 = reinterpret_cast<uint16_t*>(b + kNaH0);
-    uint16_t* hA = reinterpret_cast<uint16_t*>(b + kNaHA);
-    uint16_t* hB = reinterpret_cast<uint16_t*>(b + kNaHB);
-    float* o = reinterpret_cast<float*>(b + kNaOut);
-    const int padded = ((n + 15) / 16) * 16;
-    MCHK(launch_pack_input_padded(x, n, padded, M->mean.p, M->scale.p, h0, M->stream));
-    M->forward_into(padded, h0, hA, hB, o);
-    MCHK(launch_unpack_output(o, n, out, M->stream));
+    std::lock_guard<std::mutex> lock(M->mu);
+    // rows are written while others are still read: a result that overlaps
+    // the input goes through the scratch array
+    const bool overlap = std::less<const float*>()(x, out + (size_t)n * kMlpOut) &&
+                         std::less<const float*>()(out, x + (size_t)n * kMlpIn);
+    float* o = overlap ? M->scratch.p : out;
+    MCHK(launch_mlp_predict(M->weights(), x, n, o, M->stream));
+    if (overlap)
+      MCHK(hipMemcpyAsync(out, o, (size_t)n * kMlpOut * sizeof(float), hipMemcpyDeviceToDevice,
+                          M->stream));
     MCHK(hipStreamSynchronize(M->stream));
     return 0;
   });
@@ -402,13 +286,9 @@ int tl_mlp_grads(void* h, int n, const float* x, const float* y, float* grads, f
     Mlp* M = checked(h);
     if (n <= 0 || n % 64 || !x || !y) throw std::invalid_argument("n must be a positive multiple of 64");
     std::lock_guard<std::mutex> lock(M->mu);
-    M->reserve(n);
-    MCHK(hipMemcpyAsync(M->xin.p, x, (size_t)n * kMlpIn * sizeof(float), hipMemcpyHostToDevice,
-                        M->stream));
-    MCHK(hipMemcpyAsync(M->y.p, y, (size_t)n * sizeof(float), hipMemcpyHostToDevice, M->stream));
-    M->pack(M->xin.p, n);
-    M->forward(n, true);
-    M->backward(n);
+    const MlpTrainRows r = M->train_rows(n, x, y, n, 1);
+    MCHK(launch_mlp_train_rows(M->weights(), r, M->stream));
+    MCHK(launch_mlp_grads(r, M->g.p, MlpAdam{}, M->stream));
     std::vector<float> pad(M->L.total);
     float l = 0.0f;
     MCHK(hipMemcpyAsync(pad.data(), M->g.p, pad.size() * sizeof(float), hipMemcpyDeviceToHost,
@@ -428,40 +308,55 @@ int tl_mlp_train(void* h, int n, const float* x, const float* y, int steps, int 
     if (n <= 0 || !x || !y || steps < 0 || batch <= 0 || batch % 64 || batch > n)
       throw std::invalid_argument("bad training arguments (batch: a multiple of 64, <= n)");
     std::lock_guard<std::mutex> lock(M->mu);
-    M->reserve(batch);
     std::mt19937_64 rng(seed ? seed : 1);
     std::vector<int> perm(n);
     std::iota(perm.begin(), perm.end(), 0);
     size_t pos = n;
-    std::vector<float> bx((size_t)batch * kMlpIn), by(batch);
-    std::vector<float> hx((size_t)n * kMlpIn);
-    std::memcpy(hx.data(), x, hx.size() * sizeof(float));
-    for (int s = 0; s < steps; s++) {
-      if (pos + batch > (size_t)n) {
-        std::shuffle(perm.begin(), perm.end(), rng);
-        pos = 0;
+    // Steps that see part of the training set only take their rows along, in
+    // order; else the whole set goes to the GPU once and batches index it.
+    const size_t used = (size_t)steps * batch;
+    const bool part = used < (size_t)n;
+    std::vector<float> px, py;
+    if (part) {
+      std::shuffle(perm.begin(), perm.end(), rng);
+      px.resize(used * kMlpIn);
+      py.resize(used);
+      for (size_t i = 0; i < used; i++) {
+        std::memcpy(&px[i * kMlpIn], x + (size_t)perm[i] * kMlpIn, kMlpIn * sizeof(float));
+        py[i] = y[perm[i]];
       }
-      for (int i = 0; i < batch; i++) {
-        const int r = perm[pos + i];
-        std::memcpy(&bx[(size_t)i * kMlpIn], &hx[(size_t)r * kMlpIn], kMlpIn * sizeof(float));
-        by[i] = y[r];
-      }
-      pos += batch;
-      MCHK(hipMemcpyAsync(M->xin.p, bx.data(), bx.size() * sizeof(float), hipMemcpyHostToDevice,
-                          M->stream));
-      MCHK(hipMemcpyAsync(M->y.p, by.data(), by.size() * sizeof(float), hipMemcpyHostToDevice,
-                          M->stream));
-      M->pack(M->xin.p, batch);
-      M->forward(batch, true);
-      M->backward(batch);
-      M->t++;
-      MCHK(launch_adam(M->p.p, M->g.p, M->m.p, M->v.p, M->pb.p, M->L.total, lr, 0.9f, 0.999f,
-                       1e-8f, M->t, M->stream));
-      if (losses) {
-        MCHK(hipMemcpyAsync(&losses[s], M->loss.p, sizeof(float), hipMemcpyDeviceToHost,
-                            M->stream));
-      }
+      x = px.data();
+      y = py.data();
+    } else {
+      M->perm.ensure(n);
     }
+    MlpTrainRows r = M->train_rows(part ? (int)used : n, x, y, batch, std::max(1, steps));
+    for (int s = 0; s < steps; s++) {
+      if (part) {
+        r.x = M->xin.p + (size_t)s * batch * kMlpIn;
+        r.y = M->y.p + (size_t)s * batch;
+      } else {
+        if (pos + batch > (size_t)n) {
+          std::shuffle(perm.begin(), perm.end(), rng);
+          MCHK(hipMemcpyAsync(M->perm.p, perm.data(), (size_t)n * sizeof(int),
+                              hipMemcpyHostToDevice, M->stream));
+          // the next shuffle may not touch perm before this copy has read it
+          MCHK(hipStreamSynchronize(M->stream));
+          pos = 0;
+        }
+        r.idx = M->perm.p + pos;
+        pos += batch;
+      }
+      r.loss = M->loss.p + s;
+      M->t++;
+      MlpAdam a = {M->p.p, M->m.p, M->v.p, M->pbF.p, M->pbB.p, lr, 0.9f, 0.999f, 1e-8f,
+                   1.0f - powf(0.9f, (float)M->t), 1.0f - powf(0.999f, (float)M->t)};
+      MCHK(launch_mlp_train_rows(M->weights(), r, M->stream));
+      MCHK(launch_mlp_grads(r, nullptr, a, M->stream));
+    }
+    if (losses && steps > 0)
+      MCHK(hipMemcpyAsync(losses, M->loss.p, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost,
+                          M->stream));
     MCHK(hipStreamSynchronize(M->stream));
     return 0;
   });
