@@ -13,6 +13,7 @@ brightness in fixed point, the reference in double in fill order) and within
 from __future__ import annotations
 
 import ctypes
+from dataclasses import replace
 
 import numpy as np
 import pytest
@@ -197,6 +198,38 @@ def test_speculative_chain_equals_serial_chain(E):
         _check_against_fixture(E, g, [res])
         assert np.array_equal(ns, ns0), name
         assert np.array_equal(pix, pix0), name
+
+
+@pytest.mark.parametrize("piece,overlap,segment", [(32, 16, 1), (8, 4, 7), (3, 16, 100000),
+                                                   (1, 1, 64)])
+def test_speculative_chain_in_segments(E, piece, overlap, segment):
+    """Repair chains in segments of one solve, of a few and unbounded, with
+    the fill in stages of the pieces known so far: seeds, ray counts and the
+    chain's final state are the serial chain's (two curves of different
+    lengths, two runs on the same objects)."""
+    g = golden("c2_ppr20.npz")
+    c = curve_from_params(g["params"])
+    cs = [replace(c, n_points=1501), replace(c, n_points=300, sx=c.ex, sy=c.ey, ex=c.sx, ey=c.sy)]
+    opts = {"spec_piece": piece, "spec_overlap": overlap, "spec_segment": segment}
+    runs = []
+    try:
+        for o in ({"spec_piece": 0}, opts):
+            for k, v in o.items():
+                E.set_option(k, v)
+            lcs = [_new(E, x) for x in cs]
+            runs.append([])
+            for _ in range(2):
+                res = E.batch_irs(lcs, np.array([x.traj() for x in cs]))
+                runs[-1].append(([r[1] for r in res], [lc.seeds() for lc in lcs], E.last_stats()))
+    finally:
+        for k, v in {"spec_piece": 32, "spec_overlap": 16, "spec_segment": 192}.items():
+            E.set_option(k, v)
+    for (rays0, seeds0, _), (rays, seeds, st) in zip(*runs):
+        assert st["spec_fallback"] == 0 and st["spec_pieces"] > 0
+        for k in range(2):
+            assert np.array_equal(rays[k], rays0[k])
+            assert np.array_equal(seeds[k][0], seeds0[k][0])
+            assert np.array_equal(seeds[k][1], seeds0[k][1])
 
 
 def test_c2_window_full_resolution_golden(E):

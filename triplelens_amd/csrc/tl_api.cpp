@@ -205,12 +205,16 @@ template <class T>
 struct DBuf {
   T* p = nullptr;
   size_t n = 0;
-  void ensure(size_t k) {
+  // A buffer that has to grow does so by a quarter at least (the sizes of a
+  // fill's stages vary a little from run to run).  Giving the old one back
+  // waits for the whole device: with `later`, that is left to the caller.
+  void ensure(size_t k, std::vector<void*>* later = nullptr) {
     if (k <= n) return;
-    if (p) HIPCHK(hipFree(p));
+    size_t want = std::max<size_t>(n ? std::max(k, n + n / 4) : k, 16);
+    if (p && later) later->push_back(p);
+    else if (p) HIPCHK(hipFree(p));
     p = nullptr;
     n = 0;
-    size_t want = std::max<size_t>(k, 16);
     HIPCHK(hipMalloc(&p, want * sizeof(T)));
     n = want;
   }
@@ -242,6 +246,7 @@ struct Options {
   int specDepth = 4096;     // ... piece boundaries a repair chain may cross (at most the
                             // batch's largest piece count is used: a repair chain can then
                             // always run to its curve's end)
+  int specSegment = 192;    // ... solves a repair chain runs between two looks at what is known
 };
 
 struct Stats {
@@ -323,10 +328,22 @@ struct Engine {
   DBuf<CccTable> dCccTab;
   DBuf<cx> dCcOut, dCaOut;
   // verified speculative chain (SpecArgs)
-  DBuf<int> dSpecBase, dSpecMerged, dSpecTarget, dSpecFailed;
-  DBuf<cx> dSpecOwn, dSpecExt, dSpecRep, dSpecStart;
+  DBuf<int> dSpecBase, dSpecMerged, dSpecTarget, dSpecInfo;
+  DBuf<int2> dSpecPos, dSpecActive, dSpecFront, dSpecList;
+  DBuf<cx> dSpecOwn, dSpecExt, dSpecRep, dSpecChain, dSpecStart;
   std::vector<int> specCalls;  // per curve: the chain's solve count after the run
-  int specPieces = 0;
+  // the segments in flight: what each leaves in SpecArgs::info, copied to a
+  // slot of a ring in pinned memory, and the event behind the copy
+  static constexpr int kSpecFlight = 16;
+  int* hSpecInfo = nullptr;
+  size_t hSpecCap = 0;  // ints a slot holds
+  hipEvent_t specEvents[kSpecFlight] = {};
+  SpecArgs specArgs{};
+  SeedArgs specSeed{};
+  int specQueued = 0, specSeen = -1;  // last segment launched, last one looked at
+  std::vector<int> specBase, specKnown;  // per curve: first global piece; pieces known
+  int specActive = 0;
+  bool specFailed = false;
   // pinned host staging for the large device-to-host copies (pageable
   // copies run at a fraction of the link's rate)
   void* hstage = nullptr;
@@ -429,7 +446,11 @@ struct Engine {
   }
 
   void run(Job& job);
-  bool run_spec(std::vector<CurveDev>& hc, const std::vector<int>& pointBase, SeedArgs& sa);
+  void spec_start(std::vector<CurveDev>& hc, const std::vector<int>& pointBase, SeedArgs& sa);
+  void spec_copy_info();
+  void spec_queue();
+  bool spec_look(bool wait);
+  bool spec_done() const;
   void point_lc(Curve& c, cx s, cx e);
   void collect_amoebae(const Job& job, const std::vector<int>& ptCurve,
                        const std::vector<int>& batchPts,
@@ -517,84 +538,152 @@ CurveDev to_dev(const Curve& c, cx s, cx e, int pointBase, int causticBase) {
   return d;
 }
 
-// The verified speculative chain's rounds on the seed stream (after the
-// solve pool is built): cuts every curve into pieces of about
-// opt.specPiece positions, runs rounds 1 and 2 and the resolution, and on
-// success leaves the piece start states in `sa` for seed_kernel (and the
-// pieces in the uploaded curves).  Returns false, with the curves restored
-// to one piece, when some curve could not be resolved within
-// opt.specDepth piece boundaries.
-bool Engine::run_spec(std::vector<CurveDev>& hc, const std::vector<int>& pointBase,
-                      SeedArgs& sa) {
+// The verified speculative chain on the seed stream (after the solve pool is
+// built): cuts every curve into pieces of about opt.specPiece positions, runs
+// round 1 and the agreement, and leaves the pieces' start states in `sa` for
+// seed_kernel as they become known.
+void Engine::spec_start(std::vector<CurveDev>& hc, const std::vector<int>& pointBase,
+                        SeedArgs& sa) {
   const int nc = (int)hc.size();
   const int nPts = pointBase[nc];
-  std::vector<int> base(nc + 1, 0);
+  specBase.assign(nc + 1, 0);
   int maxP = 1;
   for (int k = 0; k < nc; k++) {
     const int n = pointBase[k + 1] - pointBase[k];
     const int P = std::max(1, n / opt.specPiece);
     hc[k].split = P;
-    base[k + 1] = base[k] + P;
+    specBase[k + 1] = specBase[k] + P;
     maxP = std::max(maxP, P);
   }
-  const int G = base[nc];
+  const int G = specBase[nc];
   HIPCHK(hipMemcpyAsync(dCurves.p, hc.data(), nc * sizeof(CurveDev), hipMemcpyHostToDevice,
                         sstream));
   dSpecBase.ensure(nc + 1);
-  HIPCHK(hipMemcpyAsync(dSpecBase.p, base.data(), (nc + 1) * sizeof(int), hipMemcpyHostToDevice,
-                        sstream));
+  HIPCHK(hipMemcpyAsync(dSpecBase.p, specBase.data(), (nc + 1) * sizeof(int),
+                        hipMemcpyHostToDevice, sstream));
   dSpecOwn.ensure((size_t)nPts * 10);
   dSpecExt.ensure((size_t)nPts * 10);
   dSpecMerged.ensure(G);
   dSpecTarget.ensure(G);
+  dSpecPos.ensure(G);
+  dSpecActive.ensure(G);
+  dSpecList.ensure(G);
+  dSpecChain.ensure((size_t)G * 10);
   const int depth = std::max(1, std::min(opt.specDepth, maxP));
   dSpecRep.ensure((size_t)G * depth * 10);
   dSpecStart.ensure((size_t)G * 10);
-  dSpecFailed.ensure(1);
-  int zero = 0;
-  HIPCHK(hipMemcpyAsync(dSpecFailed.p, &zero, sizeof(int), hipMemcpyHostToDevice, sstream));
-  SpecArgs sp;
+  const size_t words = (size_t)kSpecInfo + nc;
+  if (hSpecCap < words) {
+    if (hSpecInfo) HIPCHK(hipHostFree(hSpecInfo));
+    hSpecInfo = nullptr;
+    hSpecCap = 0;
+    HIPCHK(hipHostMalloc((void**)&hSpecInfo, 2 * words * kSpecFlight * sizeof(int),
+                         hipHostMallocDefault));
+    hSpecCap = 2 * words;
+  }
+  for (hipEvent_t& e : specEvents)
+    if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  // piece 0 of every curve starts from a known state
+  std::vector<int> info(words, 1);
+  info[0] = info[1] = info[2] = 0;
+  std::vector<int2> front(nc, make_int2(1, 0));
+  dSpecInfo.ensure(words);
+  dSpecFront.ensure(nc);
+  HIPCHK(hipMemcpyAsync(dSpecInfo.p, info.data(), words * sizeof(int), hipMemcpyHostToDevice,
+                        sstream));
+  HIPCHK(hipMemcpyAsync(dSpecFront.p, front.data(), nc * sizeof(int2), hipMemcpyHostToDevice,
+                        sstream));
+  SpecArgs& sp = specArgs;
   sp.pieceBase = dSpecBase.p;
   sp.nPieces = G;
   sp.overlap = std::max(1, opt.specOverlap);
   sp.depth = depth;
+  sp.budget = std::max(1, opt.specSegment);
   sp.own = dSpecOwn.p;
   sp.ext = dSpecExt.p;
   sp.merged = dSpecMerged.p;
   sp.repState = dSpecRep.p;
   sp.repTarget = dSpecTarget.p;
+  sp.repChain = dSpecChain.p;
+  sp.repPos = dSpecPos.p;
   sp.start = dSpecStart.p;
-  sp.failed = dSpecFailed.p;
-  SeedArgs a = sa;
-  a.maxSplit = maxP;
-  a.chunk = 0;
-  a.nChunks = 1;
-  a.chainIn = nullptr;
-  HIPCHK((hipError_t)launch_spec(a, sp, sstream));
-  int failed = 0;
-  std::vector<int> merged(G);
-  HIPCHK(hipMemcpyAsync(&failed, dSpecFailed.p, sizeof(int), hipMemcpyDeviceToHost, sstream));
-  HIPCHK(hipMemcpyAsync(merged.data(), dSpecMerged.p, G * sizeof(int), hipMemcpyDeviceToHost,
-                        sstream));
-  HIPCHK(hipStreamSynchronize(sstream));
-  if (failed) {
-    for (auto& d : hc) d.split = 1;
-    HIPCHK(hipMemcpyAsync(dCurves.p, hc.data(), nc * sizeof(CurveDev), hipMemcpyHostToDevice,
-                          sstream));
-    stats.specFallback = 1;
-    return false;
-  }
-  int repairs = 0;
-  for (int k = 0; k < nc; k++)
-    for (int q = 1; q < hc[k].split; q++) repairs += merged[base[k] + q] ? 0 : 1;
-  stats.specRepairs = repairs;
-  specPieces = G;
+  sp.active = dSpecActive.p;
+  sp.front = dSpecFront.p;
+  sp.info = dSpecInfo.p;
   sa.maxSplit = maxP;
   sa.chunk = 0;
   sa.nChunks = 1;
   sa.chainIn = nullptr;
   sa.pieceBase = dSpecBase.p;
   sa.pieceStart = dSpecStart.p;
+  specSeed = sa;
+  specKnown.assign(nc, 0);
+  specActive = 0;
+  specFailed = false;
+  specQueued = 0;
+  specSeen = -1;
+  HIPCHK((hipError_t)launch_spec(specSeed, sp, sstream));
+  spec_copy_info();
+  spec_look(true);
+  int repairs = 0;
+  std::vector<int> merged(G);
+  HIPCHK(hipMemcpyAsync(merged.data(), dSpecMerged.p, G * sizeof(int), hipMemcpyDeviceToHost,
+                        sstream));
+  HIPCHK(hipStreamSynchronize(sstream));
+  for (int k = 0; k < nc; k++)
+    for (int q = 1; q < hc[k].split; q++) repairs += merged[specBase[k] + q] ? 0 : 1;
+  stats.specRepairs = repairs;
+  stats.specPieces = G;
+}
+
+// the copy of what segment specQueued leaves, behind it on the seed stream
+void Engine::spec_copy_info() {
+  const int slot = specQueued % kSpecFlight;
+  HIPCHK(hipMemcpyAsync(hSpecInfo + (size_t)slot * hSpecCap, dSpecInfo.p,
+                        ((size_t)kSpecInfo + specKnown.size()) * sizeof(int),
+                        hipMemcpyDeviceToHost, sstream));
+  HIPCHK(hipEventRecord(specEvents[slot], sstream));
+}
+
+// Fills the seed stream with segments (those after the last one that finds
+// anything to do end at once).  The first, which most of the repair chains
+// end in, runs alone: the others get the workgroups that the rest needs.
+void Engine::spec_queue() {
+  const int flight = specSeen > 0 ? kSpecFlight : 1;
+  const int groups = std::min(1024, std::max(1, (specActive + kWalkWaves - 1) / kWalkWaves));
+  while (!spec_done() && !specFailed && specQueued - specSeen < flight) {
+    specQueued++;
+    HIPCHK((hipError_t)launch_spec_segment(specSeed, specArgs, specQueued, groups, sstream));
+    spec_copy_info();
+  }
+}
+
+// Takes over what the segments finished since the last look have left,
+// waiting for one of them if `wait`; false if there was none.
+bool Engine::spec_look(bool wait) {
+  bool any = false;
+  while (specSeen < specQueued) {
+    const int slot = (specSeen + 1) % kSpecFlight;
+    if (wait && !any) {
+      HIPCHK(hipEventSynchronize(specEvents[slot]));
+    } else {
+      const hipError_t e = hipEventQuery(specEvents[slot]);
+      if (e == hipErrorNotReady) break;
+      HIPCHK(e);
+    }
+    specSeen++;
+    any = true;
+    const int* info = hSpecInfo + (size_t)slot * hSpecCap;
+    specFailed = info[0] != 0;
+    specActive = info[1 + (specSeen & 1)];
+    std::copy(info + kSpecInfo, info + kSpecInfo + specKnown.size(), specKnown.begin());
+  }
+  return any;
+}
+
+bool Engine::spec_done() const {
+  for (size_t k = 0; k < specKnown.size(); k++)
+    if (specKnown[k] < specBase[k + 1] - specBase[k]) return false;
   return true;
 }
 
@@ -677,6 +766,27 @@ void Engine::run(Job& job) {
   bool spec = job.runSeeds && opt.specPiece > 0 && slots.empty() &&
               (int)maxLen >= 2 * opt.specPiece;
   for (auto* c : job.curves) spec = spec && c->split == 1;
+  // however this run ends, nothing of it is left on the seed stream, and the
+  // buffers that grew beside a repair chain are given back
+  struct Drain {
+    hipStream_t s;
+    std::vector<void*> later;
+    ~Drain() {
+      (void)hipStreamSynchronize(s);
+      for (void* p : later) (void)hipFree(p);
+    }
+  } drain{sstream, {}};
+  std::vector<void*>* later = nullptr;  // drain.later while repair chains run
+  SeedArgs sa{};
+  // disk samples of the curves that asked for them, behind the seed search
+  // (and beside the fills)
+  auto launch_ring = [&]() {
+    if (!anyRing) return;
+    HIPCHK(hipEventRecord(evRing0, sstream));
+    HIPCHK((hipError_t)launch_ring_amp(dCurves.p, dPtCurve.p, dPtPos.p, dPtRoots.p, nPts, dTrig.p,
+                                       dRing.p, dRingCross.p, dPolyScratch.p, sstream));
+    HIPCHK(hipEventRecord(evRing1, sstream));
+  };
   if (job.runSeeds) {
     nChunks = std::max(1, std::min<int>(opt.seedChunks, (int)(maxLen / std::max(1, opt.seedChunkMin))));
     // a split seed search runs in parallel and needs no overlap with the
@@ -720,7 +830,6 @@ void Engine::run(Job& job) {
     HIPCHK((hipError_t)launch_solve_prep(ta, (int)used, sstream));
     HIPCHK(hipEventRecord(evTrial1, sstream));
     stats.solves = (double)used;
-    SeedArgs sa;
     sa.curves = dCurves.p;
     sa.nCurves = nc;
     sa.caustics = dCaus.p;
@@ -742,12 +851,10 @@ void Engine::run(Job& job) {
     sa.chainOut = dChain.p;
     sa.pieceBase = nullptr;
     sa.pieceStart = nullptr;
-    if (spec && run_spec(hc, pointBase, sa)) {
-      HIPCHK((hipError_t)launch_seed(sa, sstream));
-      HIPCHK(hipEventRecord(evSeed[0], sstream));
-      // the pieces' seed launch restarted its solve count at each piece:
-      // the chain's count after the run is the start count plus every
-      // solve of the curve
+    if (spec) {
+      spec_start(hc, pointBase, sa);
+      // the pieces' seed launches restart their solve counts: the chain's
+      // count after the run is the start count plus every solve of the curve
       std::vector<int> cnt(nPts);
       HIPCHK(hipMemcpyAsync(cnt.data(), dPoolCount.p, nPts * sizeof(int), hipMemcpyDeviceToHost,
                             sstream));
@@ -758,7 +865,6 @@ void Engine::run(Job& job) {
         for (int p = pointBase[k]; p < pointBase[k + 1]; p++) t += cnt[p];
         specCalls[k] = (int)t;
       }
-      stats.specPieces = specPieces;
     } else for (int ch = 0; ch < nChunks; ch++) {
       sa.chunk = ch;
       sa.nChunks = nChunks;
@@ -766,14 +872,7 @@ void Engine::run(Job& job) {
       HIPCHK((hipError_t)launch_seed(sa, sstream));
       HIPCHK(hipEventRecord(evSeed[ch], sstream));
     }
-    // disk samples of the curves that asked for them, behind the seed search
-    // (and beside the fills)
-    if (anyRing) {
-      HIPCHK(hipEventRecord(evRing0, sstream));
-      HIPCHK((hipError_t)launch_ring_amp(dCurves.p, dPtCurve.p, dPtPos.p, dPtRoots.p, nPts,
-                                         dTrig.p, dRing.p, dRingCross.p, dPolyScratch.p, sstream));
-      HIPCHK(hipEventRecord(evRing1, sstream));
-    }
+    if (!spec) launch_ring();
   } else {
     for (int p = 0; p < nPts; p++) {
       nSeeds[p] = std::min(job.nSeeds[p], kMaxSeeds);
@@ -811,27 +910,113 @@ void Engine::run(Job& job) {
   if (job.runSeeds && nChunks > 1 && opt.fillWorkgroups <= 0 && nWg > 1) nWg--;
 
   std::vector<int> order;
-  for (int ch = 0; ch < nChunks; ch++) {
+  // Stages: the chunks of the serial chain, or of the speculative chain the
+  // pieces that have become known since the last stage.  While repair chains
+  // run, they keep a few compute units (they are packed, kWalkWaves to a
+  // workgroup) and the stage's fill has the others.
+  const int nWgAll = nWg;
+  if (spec && job.runFill) {
+    later = &drain.later;
+    dBatchPts.ensure(nPts, later);
+    dPoints.ensure((size_t)nPts * kPointRec, later);
+    dPtCount.ensure(nPts, later);
+    dPtSum.ensure(2 * (size_t)nPts, later);
+    dSeedTasks.ensure((size_t)nPts * kMaxSeeds, later);
+  }
+  std::vector<int> given(nc, 0);  // pieces of earlier stages
+  bool last = false;
+  for (int ch = 0; !last; ch++) {
+  order.clear();
+  if (spec) {
+    spec_look(false);
+    while (!spec_done() && !specFailed) {
+      // a stage costs the latency of a seed and a fill launch: it waits for
+      // a sixteenth of the pieces
+      int fresh = 0;
+      for (int k = 0; k < nc; k++) fresh += specKnown[k] - given[k];
+      if (job.runFill && 16 * fresh >= specBase[nc] && specSeen > 0) break;
+      spec_queue();
+      spec_look(true);
+    }
+    if (specFailed) {
+      // some curve could not be resolved within opt.specDepth piece
+      // boundaries: the serial chain, from the start
+      HIPCHK(hipStreamSynchronize(sstream));
+      for (auto& d : hc) d.split = 1;
+      HIPCHK(hipMemcpyAsync(dCurves.p, hc.data(), nc * sizeof(CurveDev), hipMemcpyHostToDevice,
+                            sstream));
+      stats.specFallback = 1;
+      stats.specPieces = stats.specRepairs = 0;
+      specCalls.clear();
+      spec = false;
+      ch = 0;
+      later = nullptr;
+      nWg = nWgAll;
+      sa.maxSplit = 1;
+      sa.pieceBase = nullptr;
+      sa.pieceStart = nullptr;
+      sa.pieces = nullptr;
+      HIPCHK((hipError_t)launch_seed(sa, sstream));
+      HIPCHK(hipEventRecord(evSeed[0], sstream));
+      launch_ring();
+    }
+  }
+  if (spec) {
+    last = spec_done();
+    later = last ? nullptr : &drain.later;
+    nWg = nWgAll;
+    if (!last) {
+      spec_queue();
+      // workgroups are dealt to the eight XCDs, and in each to its four
+      // shader engines, in turn, and wait for room there: with a compute unit
+      // less on each XCD a launch of one workgroup still starts at once beside
+      // the fill, but the 64-workgroup resolution waited for its end (40 ms)
+      const int keep = nc == 1 && specActive <= kWalkWaves ? 8 : 32;
+      if (opt.fillWorkgroups <= 0) nWg = std::max(1, nWgAll - keep);
+    }
+    std::vector<int2> list;
+    for (int k = 0; k < nc; k++) {
+      const long long len = pointBase[k + 1] - pointBase[k];
+      const int P = specBase[k + 1] - specBase[k];
+      for (int q = given[k]; q < specKnown[k]; q++) list.push_back(make_int2(k, q));
+      for (int i = (int)(len * given[k] / P); i < (int)(len * specKnown[k] / P); i++)
+        order.push_back(pointBase[k] + i);
+      given[k] = specKnown[k];
+    }
+    HIPCHK(hipMemcpyAsync(dSpecList.p, list.data(), list.size() * sizeof(int2),
+                          hipMemcpyHostToDevice, stream));
+    sa.pieces = dSpecList.p;
+    sa.nPieces = (int)list.size();
+    HIPCHK((hipError_t)launch_seed(sa, stream));
+    HIPCHK(hipEventRecord(evSeed[0], stream));
+    if (last) {
+      HIPCHK(hipStreamWaitEvent(sstream, evSeed[0], 0));
+      launch_ring();
+    }
+  } else {
+    last = ch == nChunks - 1;
+    for (int k = 0; k < nc; k++) {
+      const long long len = pointBase[k + 1] - pointBase[k];
+      for (int i = (int)(len * ch / nChunks); i < (int)(len * (ch + 1) / nChunks); i++)
+        order.push_back(pointBase[k] + i);
+    }
+  }
   if (job.runSeeds) {
-    // this chunk's seed counts and predicted costs (the copy waits for the
-    // chunk's seed launch; later chunks are still being written)
-    HIPCHK(hipStreamWaitEvent(stream, evSeed[ch], 0));
+    // this stage's seed counts and predicted costs (the copy waits for the
+    // stage's seed launch; later ones are still being written)
+    HIPCHK(hipStreamWaitEvent(stream, evSeed[spec ? 0 : ch], 0));
     HIPCHK(hipMemcpyAsync(nSeeds.data(), dNSeeds.p, nPts * sizeof(int), hipMemcpyDeviceToHost,
                           stream));
     HIPCHK(hipMemcpyAsync(cost.data(), dCost.p, nPts * sizeof(float), hipMemcpyDeviceToHost,
                           stream));
     HIPCHK(hipStreamSynchronize(stream));
   }
-  // the chunk's positions, largest predicted cost first, in launches of
+  // the stage's positions, largest predicted cost first, in launches of
   // about kRunBudget predicted runs (groups of kGroupPoints positions with a
   // run-table slice each)
-  order.clear();
-  for (int k = 0; k < nc; k++) {
-    const long long len = pointBase[k + 1] - pointBase[k];
-    const int i0 = (int)(len * ch / nChunks), i1 = (int)(len * (ch + 1) / nChunks);
-    for (int i = i0; i < i1 && job.runFill; i++)
-      if (nSeeds[pointBase[k] + i] > 0) order.push_back(pointBase[k] + i);
-  }
+  if (!job.runFill) order.clear();
+  order.erase(std::remove_if(order.begin(), order.end(), [&](int p) { return nSeeds[p] <= 0; }),
+              order.end());
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
   // A launch holds about kRunBudget predicted runs (the run table is sized
   // from the prediction, tableLoad entries per run: up to 16 GiB).
@@ -858,11 +1043,11 @@ void Engine::run(Job& job) {
       const int gp = batchPts[b];
       for (int k = 0; k < nSeeds[gp]; k++) seedTasks.push_back(make_int2(b, k));
     }
-    dBatchPts.ensure(nb);
-    dPoints.ensure((size_t)nb * kPointRec);
-    dSeedTasks.ensure(seedTasks.size());
-    dPtCount.ensure(nb);
-    dPtSum.ensure(2 * (size_t)nb);
+    dBatchPts.ensure(nb, later);
+    dPoints.ensure((size_t)nb * kPointRec, later);
+    dSeedTasks.ensure(seedTasks.size(), later);
+    dPtCount.ensure(nb, later);
+    dPtSum.ensure(2 * (size_t)nb, later);
     HIPCHK(hipMemcpyAsync(dBatchPts.p, batchPts.data(), nb * sizeof(int), hipMemcpyHostToDevice, stream));
     HIPCHK(hipMemcpyAsync(dSeedTasks.p, seedTasks.data(), seedTasks.size() * sizeof(int2),
                           hipMemcpyHostToDevice, stream));
@@ -885,16 +1070,16 @@ void Engine::run(Job& job) {
         grpMask[g] = grpCap[g] - 1;
         hcap += grpCap[g];
       }
-      dHtab.ensure(2 * hcap);
-      dGrp.ensure(2 * (size_t)nGrp);
+      dHtab.ensure(2 * hcap, later);
+      dGrp.ensure(2 * (size_t)nGrp, later);
       HIPCHK(hipMemcpyAsync(dGrp.p, grpBase.data(), nGrp * sizeof(unsigned long long),
                             hipMemcpyHostToDevice, stream));
       HIPCHK(hipMemcpyAsync(dGrp.p + nGrp, grpMask.data(), nGrp * sizeof(unsigned long long),
                             hipMemcpyHostToDevice, stream));
-      dLParent.ensure(labelCap);
-      dLPoint.ensure(labelCap);
-      dLCount.ensure(labelCap);
-      dLSum.ensure(2 * (size_t)labelCap);
+      dLParent.ensure(labelCap, later);
+      dLPoint.ensure(labelCap, later);
+      dLCount.ensure(labelCap, later);
+      dLSum.ensure(2 * (size_t)labelCap, later);
       FillArgs fa;
       std::memset(&fa, 0, sizeof(fa));
       fa.curves = dCurves.p;
@@ -940,7 +1125,8 @@ void Engine::run(Job& job) {
       fa.leapJumps = opt.leapJumps;
       fa.pollBackoff = opt.pollBackoff;
       fa.poolNewest = opt.poolNewest;
-      if (opt.useGraph) {
+      // (a stage of several has arguments of its own: no graph)
+      if (opt.useGraph && ch == 0 && last) {
         // the launch's reset, clears, fill and resolve as one graph (kernel
         // nodes only: the resets are kernels, not memsets), captured once
         // and launched again while its arguments are the same (the next
@@ -1049,7 +1235,7 @@ void Engine::run(Job& job) {
       break;
     }
   }
-  }  // chunks
+  }  // stages
   if (job.runSeeds) {
     // the seed search's outputs are final once its last launch is done; the
     // disk samples behind it on the seed stream are waited for after the
@@ -1938,6 +2124,7 @@ int tl_set_option(const char* name, double value) {
   else if (n == "seed_chunk_min") o.seedChunkMin = std::max(1, (int)value);
   else if (n == "spec_piece") o.specPiece = std::max(0, (int)value);
   else if (n == "spec_overlap") o.specOverlap = std::min(4096, std::max(1, (int)value));
+  else if (n == "spec_segment") o.specSegment = std::min(1 << 20, std::max(1, (int)value));
   else if (n == "spec_depth") o.specDepth = std::min(4096, std::max(1, (int)value));
   else return -1;
   return 0;

@@ -138,6 +138,8 @@ struct SeedArgs {
   // fresh solve.  Null: fresh starts.
   const int* pieceBase;
   const cx* pieceStart;
+  const int2* pieces;  // (curve, piece) of the workgroups, or null: all of them
+  int nPieces;
 };
 
 // The verified speculative chain.  Every curve of n positions is cut into
@@ -146,27 +148,41 @@ struct SeedArgs {
 // the next piece for `overlap` positions, recording the state after every
 // position.  Where the next piece's own state equals the predecessor's
 // continuation at one of its first `overlap` positions, both chains agree
-// from there on.  Where none does, round 2 runs a repair chain from the
-// predecessor's end state on through the following pieces until it agrees
-// with one of them.  spec_resolve_kernel then walks each curve's pieces from
-// its first (whose start is known) and picks the true state at every piece
-// start; seed_kernel recomputes all pieces from those states in parallel.
-// A chain that has not agreed after `depth` further pieces sets `failed`,
-// and the host falls back to the serial chain.
+// from there on.  Where none does, a repair chain continues the predecessor's
+// chain through the following pieces until it agrees with one of them.
+//
+// Repair chains run in segments of `budget` solves.  After each segment
+// spec_resolve_kernel walks each curve's pieces on from the last one whose
+// start is known: seed_kernel can then run the known pieces, and the fill
+// their positions, while the next segment runs.  A repair chain sleeps while
+// another that may be the true one has run past its start without agreeing.
+// One that has not agreed after `depth` further pieces and turns out to be
+// the true one sets `failed`, and the host falls back to the serial chain.
+constexpr int kRepairEnd = -1;      // repTarget: ran to the curve's end
+constexpr int kRepairDepth = -2;    // crossed `depth` boundaries without agreeing
+constexpr int kRepairRunning = -3;
+constexpr int kSpecInfo = 4;        // words of SpecArgs::info before the curves'
+constexpr int kWalkWaves = 4;       // repair chains per workgroup: one to a SIMD
 struct SpecArgs {
   const int* pieceBase;  // [curve] first global piece
   int nPieces;           // global pieces
   int overlap;           // positions of the next piece a chain runs into (<= its length)
   int depth;             // piece boundaries a repair chain may cross
+  int budget;            // solves of one segment
   cx* own;               // [point * 10 + k] state after the point, by the piece that owns it
   cx* ext;               // [point * 10 + k] ... by the preceding piece's continuation
   int* merged;           // [piece] round 1: the piece agrees with its predecessor
   cx* repState;          // [(piece * depth + j) * 10 + k] repair chain of piece q: state
                          // before the first position of piece q + 1 + j
-  int* repTarget;        // [piece] the piece its repair chain agreed with; -1: ran to the
-                         // curve's end; -2: crossed `depth` boundaries without agreeing
+  int* repTarget;        // [piece] the piece its repair chain agreed with, or kRepair*
+  cx* repChain;          // [piece * 10 + k] the repair chain's state
+  int2* repPos;          // [piece] its next position, and the piece of the one before
   cx* start;             // [piece * 10 + k] resolved start states
-  int* failed;           // set when some curve could not be resolved
+  int2* active;          // (curve, piece) of the repair chains of the coming segment
+  int2* front;           // [curve] the true chain before piece info[kSpecInfo + curve]: the
+                         // previous piece's own (x = 1) or the repair chain of piece y
+  int* info;             // [0] failed; [1 + (s & 1)] active chains after segment s;
+                         // [kSpecInfo + curve] pieces whose start is known
 };
 
 constexpr int kPointRec = 32;    // doubles of a batch point's record
@@ -235,7 +251,12 @@ int launch_seed(const SeedArgs& a, hipStream_t s);
 // Rounds of the verified speculative chain (SpecArgs), with a.maxSplit and
 // the curves' split set to the pieces: round 1, the repair chains, and the
 // resolution of the piece start states.
+// Round 1, agreement and the resolution before the first segment (segment 0);
+// then segments 1, 2, ... of the repair chains on `groups` workgroups of
+// kWalkWaves, each followed by the resolution.
 int launch_spec(const SeedArgs& a, const SpecArgs& sp, hipStream_t s);
+int launch_spec_segment(const SeedArgs& a, const SpecArgs& sp, int segment, int groups,
+                        hipStream_t s);
 // The fill's in-range division against IEEE division on n generated operand
 // pairs (test access): adds the number of differing results to *bad (device).
 int launch_div_check(long long n, unsigned long long seed, unsigned long long* bad,

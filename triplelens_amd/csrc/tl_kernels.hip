@@ -610,7 +610,8 @@ int launch_image_poly(const Lens& L, const cx* fixedPoly, const cx* zeta, int n,
 template <bool TRACED>
 __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
   __shared__ __align__(16) double rec[64];
-  const int c = blockIdx.x / a.maxSplit, q = blockIdx.x % a.maxSplit;
+  const int c = a.pieces ? uni(a.pieces[blockIdx.x].x) : blockIdx.x / a.maxSplit;
+  const int q = a.pieces ? uni(a.pieces[blockIdx.x].y) : blockIdx.x % a.maxSplit;
   if (c >= a.nCurves) return;
   const int ln = __lane_id();
   const CurveDev& C = a.curves[c];
@@ -717,9 +718,9 @@ __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
 
 // ---- verified speculative chain (SpecArgs) ---------------------------------
 // The chain's solves of the walk's next position (centre, then caustic trial
-// points), as seed_kernel runs them, without output.
-__device__ __forceinline__ void chain_step(const Lens& L, bool binImg, const TrigTable* trig,
-                                           SolveWalk& W, double* rec, cx& chainv, int& have) {
+// points), as seed_kernel runs them, without output.  Returns their number.
+__device__ __forceinline__ int chain_step(const Lens& L, bool binImg, const TrigTable* trig,
+                                          SolveWalk& W, double* rec, cx& chainv, int& have) {
   const int nSolve = W.position();
   for (int sIdx = 0; sIdx < nSolve; sIdx++) {
     double rv;
@@ -728,6 +729,7 @@ __device__ __forceinline__ void chain_step(const Lens& L, bool binImg, const Tri
     bool oob = false;
     wl_get_images<false>(L, rv, fv, rec, false, chainv, have, trig, binImg, oob);
   }
+  return nSolve;
 }
 
 // The chain state (roots 0..9 on lanes 0..9) equals the stored one, bit for bit.
@@ -779,12 +781,9 @@ __global__ void __launch_bounds__(64) spec_round1_kernel(SeedArgs a, SpecArgs sp
   }
 }
 
-// Round 2: for a piece q > 0 that does not agree with its predecessor's
-// continuation, the repair chain from the predecessor's end state, through
-// the following pieces until its state equals a piece's own at one of that
-// piece's first sp.overlap positions.
-__global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp) {
-  __shared__ __align__(16) double rec[64];
+// Whether piece q > 0 agrees with its predecessor's continuation; if not, its
+// repair chain stands where that continuation ended.
+__global__ void __launch_bounds__(64) spec_agree_kernel(SeedArgs a, SpecArgs sp) {
   const int c = blockIdx.x / a.maxSplit, q = blockIdx.x % a.maxSplit;
   if (c >= a.nCurves) return;
   const int ln = __lane_id();
@@ -809,91 +808,186 @@ __global__ void __launch_bounds__(64) spec_repair_kernel(SeedArgs a, SpecArgs sp
     const unsigned long long m = __ballot(eq);
     for (int j = 0; j < 6; j++) agree |= ((m >> (10 * j)) & 0x3ffull) == 0x3ffull;
   }
-  if (ln == 0) sp.merged[gq] = agree ? 1 : 0;
-  if (agree) return;
-  const Lens L = uni_lens(C.L);
-  const bool binImg = uni(C.binImg) != 0;
-  cx chainv = mk(0.0, 0.0);
-  if (ln < 10) chainv = sp.own[((size_t)pointBase + b - 1) * 10 + ln];
-  int have = 1;
-  int qq = q, qb = b, qe = e;  // the piece the chain is in
-  const long long n = (long long)uni((int)C.lcLength) + 1;
-  const int split = uni(C.split);
-  if (b >= n) return;
-  SolveWalk W(a.pool, pointBase + b, pointBase + (int)n);
-  for (int i = b; i < n; i++) {
-    if (i == qe) {
-      // entering piece qq + 1: the chain's state before its first position
-      qq++;
-      qb = qe;
-      qe = (int)(n * (qq + 1) / split);
-      const int j = qq - q - 1;
-      if (j >= sp.depth) {
-        if (ln == 0) sp.repTarget[gq] = -2;
-        return;
+  if (!agree && ln < 10)
+    sp.repChain[(size_t)gq * 10 + ln] = sp.ext[((size_t)pointBase + lim - 1) * 10 + ln];
+  if (ln == 0) {
+    sp.merged[gq] = agree ? 1 : 0;
+    sp.repTarget[gq] = kRepairRunning;
+    sp.repPos[gq] = make_int2(lim, q);
+  }
+}
+
+// One segment of the active repair chains, one wavefront each.  A chain is
+// serial (its measure is the time per solve, about 20 us), so few wavefronts
+// run here for long: they are packed one to a SIMD, four to a workgroup, so
+// that they hold few compute units and the fill of the positions already
+// known has the others.  With the fill waiting for the last chain instead,
+// a 4096-point curve through a central caustic took 55 ms (repair 25, fill
+// 23) and the 64-curve batch 241 ms (130, 87).
+__global__ void __launch_bounds__(64 * kWalkWaves) spec_walk_kernel(SeedArgs a, SpecArgs sp,
+                                                                    int segment) {
+  __shared__ __align__(16) double recs[kWalkWaves][64];
+  const int ln = __lane_id(), wave = uni((int)threadIdx.x >> 6);
+  double* rec = recs[wave];
+  const int nActive = uni(sp.info[1 + ((segment - 1) & 1)]);
+  for (int w = blockIdx.x * kWalkWaves + wave; w < nActive; w += gridDim.x * kWalkWaves) {
+    const int c = uni(sp.active[w].x), q = uni(sp.active[w].y);
+    const CurveDev& C = a.curves[c];
+    const int gq = uni(sp.pieceBase[c]) + q;
+    const int pointBase = uni(C.pointBase), n = uni((int)C.lcLength) + 1, split = uni(C.split);
+    const Lens L = uni_lens(C.L);
+    const bool binImg = uni(C.binImg) != 0;
+    int i = uni(sp.repPos[gq].x), qq = uni(sp.repPos[gq].y);  // qq: the piece the chain is in
+    int qe = (int)((long long)n * (qq + 1) / split);
+    cx chainv = mk(0.0, 0.0);
+    if (ln < 10) chainv = sp.repChain[(size_t)gq * 10 + ln];
+    int have = 1, target = kRepairRunning;
+    if (i < n) {
+      SolveWalk W(a.pool, pointBase + i, pointBase + n);
+      int solves = 0;
+      for (; i < n && solves < sp.budget; i++) {
+        if (i == qe) {
+          // entering piece qq + 1: the chain's state before its first position
+          const int j = qq - q;
+          if (j >= sp.depth) {
+            target = kRepairDepth;
+            break;
+          }
+          qq++;
+          qe = (int)((long long)n * (qq + 1) / split);
+          if (ln < 10) sp.repState[((size_t)gq * sp.depth + j) * 10 + ln] = chainv;
+        }
+        // the piece's own state, loaded before the solve that it is compared with
+        cx own = mk(0.0, 0.0);
+        if (ln < 10) own = sp.own[((size_t)pointBase + i) * 10 + ln];
+        solves += chain_step(L, binImg, a.trig, W, rec, chainv, have);
+        if (state_equal(chainv, own)) {
+          target = qq;
+          break;
+        }
       }
-      if (ln < 10) sp.repState[((size_t)gq * sp.depth + j) * 10 + ln] = chainv;
     }
-    const int p = pointBase + i;
-    // the piece's own state, loaded before the solve that it is compared with
-    const bool mayJoin = qq > q && i < qb + sp.overlap;
-    cx own = mk(0.0, 0.0);
-    if (mayJoin && ln < 10) own = sp.own[(size_t)p * 10 + ln];
-    chain_step(L, binImg, a.trig, W, rec, chainv, have);
-    if (mayJoin && state_equal(chainv, own)) {
-      if (ln == 0) sp.repTarget[gq] = qq;
-      return;
+    if (target == kRepairRunning && i >= n) target = kRepairEnd;
+    if (ln < 10) sp.repChain[(size_t)gq * 10 + ln] = chainv;
+    if (ln == 0) {
+      sp.repTarget[gq] = target;
+      sp.repPos[gq] = make_int2(i, qq);
     }
   }
-  if (ln == 0) sp.repTarget[gq] = -1;
 }
 
 // The true chain's state before each piece, walking every curve's pieces in
-// order (one lane per curve): the chain known to be the true one at each
-// piece start is either the previous piece's own (it agreed with the chain
-// before it, or it is piece 0) or a repair chain that has not yet agreed.
-__global__ void spec_resolve_kernel(SeedArgs a, SpecArgs sp) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+// order from the first whose start is not known (one wavefront per curve, 64
+// pieces' records at a time): the true chain at a piece start is either the
+// previous piece's own (it agreed with the chain before it, or it is piece 0)
+// or a repair chain that has not yet agreed.  Then the repair chains of the
+// coming segment: the one the true chain waits for, and those beyond it that
+// no other chain in question has run past.
+__global__ void __launch_bounds__(64) spec_resolve_kernel(SeedArgs a, SpecArgs sp, int segment) {
+  const int c = blockIdx.x;
   if (c >= a.nCurves) return;
+  const int ln = __lane_id();
+  if (c == 0 && ln == 0) sp.info[1 + ((segment + 1) & 1)] = 0;
   const CurveDev& C = a.curves[c];
-  const int g0 = sp.pieceBase[c];
-  bool viaPiece = true;  // the true chain at the coming start is piece q - 1's own
-  int rq = 0;            // else the repair chain of piece rq
-  for (int q = 1; q < C.split; q++) {
-    int b, e;
-    piece_range(C, q, b, e);
+  const int split = uni(C.split), g0 = uni(sp.pieceBase[c]);
+  const long long n = (long long)uni((int)C.lcLength) + 1;
+  const cx* own = sp.own + (size_t)uni(C.pointBase) * 10;
+  int q = uni(sp.info[kSpecInfo + c]);
+  if (q >= split) return;
+  bool viaPiece = uni(sp.front[c].x) != 0;
+  int rq = uni(sp.front[c].y);
+  int rTarget = viaPiece ? 0 : uni(sp.repTarget[g0 + rq]);
+  int rPiece = viaPiece ? 0 : uni(sp.repPos[g0 + rq].y);
+  // it may have agreed with the piece it was in at the last resolution
+  if (!viaPiece && rTarget == q - 1) viaPiece = true;
+  bool failed = false;
+  int q0 = q, m = 0, t = 0, rp = 0;  // lane l: the records of piece q0 + l
+  auto load = [&]() {
+    const int g = g0 + (q0 + ln < split ? q0 + ln : split - 1);
+    m = sp.merged[g];
+    t = sp.repTarget[g];
+    rp = sp.repPos[g].y;
+  };
+  load();
+  for (; q < split; q++) {
+    if (q == q0 + 64) {
+      q0 = q;
+      load();
+    }
     const cx* src;
     if (viaPiece) {
-      src = sp.own + ((size_t)C.pointBase + b - 1) * 10;
-      if (!sp.merged[g0 + q]) {
+      src = own + (n * q / split - 1) * 10;
+      if (!__builtin_amdgcn_readlane(m, q - q0)) {
         viaPiece = false;
         rq = q;
+        rTarget = __builtin_amdgcn_readlane(t, q - q0);
+        rPiece = __builtin_amdgcn_readlane(rp, q - q0);
       }
     } else {
-      const int j = q - rq - 1;
-      const int tgt = sp.repTarget[g0 + rq];
-      if (j >= sp.depth || (tgt >= 0 && tgt < q)) {  // cannot happen: the chain stopped earlier
-        atomicExch(sp.failed, 1);
-        return;
+      if (rPiece < q) {
+        // the repair chain has not come here: it is running, or gave up
+        failed = rTarget != kRepairRunning;
+        break;
       }
-      src = sp.repState + ((size_t)(g0 + rq) * sp.depth + j) * 10;
-      if (tgt == q) viaPiece = true;
+      src = sp.repState + ((size_t)(g0 + rq) * sp.depth + (q - rq - 1)) * 10;
     }
-    for (int k = 0; k < 10; k++) sp.start[((size_t)g0 + q) * 10 + k] = src[k];
+    if (rTarget == q) viaPiece = true;
+    if (ln < 10) sp.start[((size_t)g0 + q) * 10 + ln] = src[ln];
   }
+  if (ln == 0) {
+    if (failed) sp.info[0] = 1;
+    sp.info[kSpecInfo + c] = q;
+    sp.front[c] = make_int2(viaPiece ? 1 : 0, rq);
+  }
+  if (q >= split || failed) return;
+  int seen = -1;  // the furthest piece that a chain in question has entered
+  for (int p0 = rq; p0 < split; p0 += 64) {
+    const int p = p0 + ln;
+    const bool there = p < split && (p == rq || p >= q) && !sp.merged[g0 + p];
+    int reach = there ? sp.repPos[g0 + p].y : -1;
+    const bool running = there && sp.repTarget[g0 + p] == kRepairRunning;
+    // the furthest of the lanes below
+    int upto = reach;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      if (ln >= o && v > upto) upto = v;
+    }
+    int before = __shfl_up(upto, 1, 64);
+    if (ln == 0 || before < seen) before = seen;
+    const bool on = running && (p == rq || before < p);
+    const unsigned long long f = __ballot(on);
+    int at = 0;
+    if (ln == 0 && f) at = atomicAdd(&sp.info[1 + (segment & 1)], __builtin_popcountll(f));
+    at = uni(at);
+    if (on) sp.active[at + __builtin_popcountll(f & ((1ull << ln) - 1ull))] = make_int2(c, p);
+    const int top = __builtin_amdgcn_readlane(upto, 63);
+    if (top > seen) seen = top;
+  }
+}
+
+static bool spec_args_ok(const SeedArgs& a, const SpecArgs& sp) {
+  return a.maxSplit >= 1 && (long long)a.nCurves * a.maxSplit <= (1ll << 30) && sp.pieceBase &&
+         sp.own && sp.ext && sp.merged && sp.repState && sp.repTarget && sp.repChain &&
+         sp.repPos && sp.start && sp.active && sp.front && sp.info && sp.overlap >= 1 &&
+         sp.depth >= 1 && sp.budget >= 1 && a.curves && a.trig && a.pool.base && a.pool.count &&
+         a.pool.rec && a.pool.fresh;
 }
 
 int launch_spec(const SeedArgs& a, const SpecArgs& sp, hipStream_t s) {
   if (a.nCurves <= 0) return 0;
-  if (a.maxSplit < 1 || (long long)a.nCurves * a.maxSplit > (1ll << 30))
-    return (int)hipErrorInvalidValue;
-  if (!sp.pieceBase || !sp.own || !sp.ext || !sp.merged || !sp.repState || !sp.repTarget ||
-      !sp.start || !sp.failed || sp.overlap < 1 || sp.depth < 1 || !a.curves || !a.trig ||
-      !a.pool.base || !a.pool.count || !a.pool.rec || !a.pool.fresh)
-    return (int)hipErrorInvalidValue;
+  if (!spec_args_ok(a, sp)) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(spec_round1_kernel, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a, sp);
-  hipLaunchKernelGGL(spec_repair_kernel, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a, sp);
-  hipLaunchKernelGGL(spec_resolve_kernel, dim3((a.nCurves + 63) / 64), dim3(64), 0, s, a, sp);
+  hipLaunchKernelGGL(spec_agree_kernel, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a, sp);
+  hipLaunchKernelGGL(spec_resolve_kernel, dim3(a.nCurves), dim3(64), 0, s, a, sp, 0);
+  return (int)hipGetLastError();
+}
+
+int launch_spec_segment(const SeedArgs& a, const SpecArgs& sp, int segment, int groups,
+                        hipStream_t s) {
+  if (a.nCurves <= 0) return 0;
+  if (!spec_args_ok(a, sp) || segment < 1 || groups < 1) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(spec_walk_kernel, dim3(groups), dim3(64 * kWalkWaves), 0, s, a, sp, segment);
+  hipLaunchKernelGGL(spec_resolve_kernel, dim3(a.nCurves), dim3(64), 0, s, a, sp, segment);
   return (int)hipGetLastError();
 }
 
@@ -1224,10 +1318,12 @@ int launch_seed(const SeedArgs& a, hipStream_t s) {
   if (a.maxSplit < 1 || (long long)a.nCurves * a.maxSplit > (1ll << 30))
     return (int)hipErrorInvalidValue;
   if (a.pieceStart && !a.pieceBase) return (int)hipErrorInvalidValue;
+  const int groups = a.pieces ? a.nPieces : a.nCurves * a.maxSplit;
+  if (groups <= 0) return 0;
   if (a.slotTrace)
-    hipLaunchKernelGGL(seed_kernel<true>, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(seed_kernel<true>, dim3(groups), dim3(64), 0, s, a);
   else
-    hipLaunchKernelGGL(seed_kernel<false>, dim3(a.nCurves * a.maxSplit), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(seed_kernel<false>, dim3(groups), dim3(64), 0, s, a);
   return (int)hipGetLastError();
 }
 
