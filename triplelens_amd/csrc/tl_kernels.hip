@@ -130,7 +130,7 @@ __device__ __forceinline__ void wl_deflate(const cx (&p)[J + 1], cx& rootv, cons
     if (ln == 9) rootv = x;
   } else {
     cx b[J + 1];
-    if (!lag_fast<J, true>(p, x, b, trig, oob)) {
+    if (!lag_wave<J, true>(p, x, b, trig, oob)) {
       x = mk(kLagEps, kLagEps);
       horner_sums<J>(p, x, b);
     }
@@ -250,7 +250,7 @@ __device__ __forceinline__ unsigned long long wl_get_images(const Lens& L, doubl
 #pragma unroll
         for (int j = 0; j <= 10; j++) c[j] = get(kRecCoef + 2 * j);
         cx x = rlc(chainv, 10), b[11];
-        if (!lag_fast<10, true>(c, x, b, trig, firstOob)) {
+        if (!lag_wave<10, true>(c, x, b, trig, firstOob)) {
           x = mk(kLagEps, kLagEps);
           horner_sums<10>(c, x, b);
         }
@@ -266,7 +266,7 @@ __device__ __forceinline__ unsigned long long wl_get_images(const Lens& L, doubl
     for (int j = 0; j <= 10; j++) c[j] = get(kRecCoef + 2 * j);
     bool laneOob = false;
     cx b[11];
-    lag_fast<10, false>(c, rootv, b, trig, laneOob);
+    lag_wave<10, false>(c, rootv, b, trig, laneOob);
     oob |= __ballot(laneOob) != 0;
     if (wl_check(c[10], c[0], rootv)) {
       const bool ok = wl_img_check(L, rootv, get(kRecZeta)) && ln < 10;
@@ -505,7 +505,7 @@ __device__ __forceinline__ void lane_deflate(const cx (&p)[J + 1], const cx* ini
     roots[DEG - 1] = x;
   } else {
     cx b[J + 1];
-    if (!lag_fast<J, false>(p, x, b, trig, oob) && withInit) {
+    if (!lag_lane<J>(p, x, b, trig, oob) && withInit) {
       x = mk(kLagEps, kLagEps);
       horner_sums<J>(p, x, b);
     }
@@ -525,7 +525,7 @@ __device__ __forceinline__ void lane_solve(const cx (&c)[11], const cx* init, bo
 #pragma unroll 1
   for (int j = 0; j < 10; j++) {
     cx x = roots[0], b[11];
-    lag_fast<10, false>(c, x, b, trig, oob);
+    lag_lane<10>(c, x, b, trig, oob);
 #pragma unroll
     for (int k = 0; k < 9; k++) roots[k] = roots[k + 1];
     roots[9] = x;
@@ -546,7 +546,7 @@ __global__ void __launch_bounds__(64) solve_prep_kernel(TrialArgs a, int nSolves
   const cx zeta = rec[kRecZeta / 2];
   cx x = mk(0.0, 0.0), b[11];
   bool oob = false;
-  if (!lag_fast<10, false>(c, x, b, a.trig, oob)) {
+  if (!lag_lane<10>(c, x, b, a.trig, oob)) {
     x = mk(kLagEps, kLagEps);
     horner_sums<10>(c, x, b);
   }
@@ -1260,7 +1260,7 @@ __global__ void __launch_bounds__(64) ccc_kernel(const Lens* lenses, int n, int 
     ccc_poly(L, st, tab->e[j], p);
     bool fresh = j == 0;
     if (!fresh) {
-      lag_fast<6, false>(p, x, b, trig, oob);
+      lag_lane<6>(p, x, b, trig, oob);
       // Laguerre::checkRoots (laguerre.cc:188-198): the product of the roots,
       // taken in any order where it decides (see wl_check), else in root order
       cx v = r < 6 ? x : mk(1.0, 0.0);
@@ -1287,7 +1287,7 @@ __global__ void __launch_bounds__(64) ccc_kernel(const Lens* lenses, int n, int 
 #pragma unroll
       for (int k = 1; k < 6; k++)
         if (r == k) y = roots[k];
-      lag_fast<6, false>(p, y, b, trig, oob);
+      lag_lane<6>(p, y, b, trig, oob);
       if (fresh) x = y;
     }
     if (mine) out[j] = x;

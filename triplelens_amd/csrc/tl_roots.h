@@ -174,105 +174,131 @@ __device__ __forceinline__ bool lag_general(const cx (&b)[M + 1], cx& x, int i,
   return false;
 }
 
-// Laguerre::laguerre for a polynomial of degree M >= 2 held in registers.
-// Every lane runs its own x, or all lanes run the same one (UNI: the branches
-// are then taken on the whole wave).  Leaves the Horner sums at the returned
-// x in b, which are the coefficients of the deflated polynomial
-// (b[j + 1] = coefficient j, laguerre.cc:133-139).
+// One iteration of Laguerre::laguerre at x, in the parts that its two drivers
+// below share.
 //
-// An iteration first runs the b recurrence alone: the one that accepts x (one
-// in two to three) needs no derivative.  The error bound sum |b_j| |x|^j is
-// bracketed by its 1-norm form E1: E1 / sqrt 2 <= E <= E1 (|x| from the
-// hardware root, good to 1e-7; the bracket is widened by 1e-5).  One
-// evaluation in a hundred falls inside it and gets moduli from the hardware
-// root, which leave a bracket of 1e-4.
-template <int M, bool UNI>
-__device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M + 1],
-                                         const TrigTable* trig, bool& oob) {
+// An iteration first runs the b recurrence alone (lag_eval): the one that
+// accepts x (one in two to three) needs no derivative.  The error bound
+// sum |b_j| |x|^j is bracketed by its 1-norm form E1: E1 / sqrt 2 <= E <= E1
+// (|x| from the hardware root, good to 1e-7; the bracket is widened by 1e-5).
+// One evaluation in a hundred falls inside it and gets moduli from the
+// hardware root, which leave a bracket of 1e-4 (lag_narrow).
+struct LagEval {
+  double ax;      // |x|, or NaN (which leaves every comparison undecided) where
+                  // its square may have lost digits
+  double nb, e2;  // |p(x)|^2 and the square of the bound on which x is accepted
+};
+template <int M>
+__device__ __forceinline__ LagEval lag_eval(const cx (&p)[M + 1], cx x, cx (&b)[M + 1]) {
+  LagEval v;
+  const double n = cnorm(x);
+  v.ax = n > 1e-280 ? __builtin_amdgcn_sqrt(n) : __builtin_nan("");
+  b[M] = p[M];
+  double e1 = fabs(p[M].re) + fabs(p[M].im);
+#pragma unroll
+  for (int j = M - 1; j >= 0; j--) {
+    b[j] = cadd(cmul(x, b[j + 1]), p[j]);
+    e1 = fma(v.ax, e1, fabs(b[j].re) + fabs(b[j].im));
+  }
+  v.nb = cnorm(b[0]);
+  const double el = kLagEps * e1;
+  v.e2 = el * el;
+  return v;
+}
+// not accepted (nb above 1e-250 follows from lag_step's lower bound)
+__device__ __forceinline__ bool lag_far(const LagEval& v) { return v.nb > v.e2 * 1.0001; }
+__device__ __forceinline__ bool lag_near(const LagEval& v) {
+  return (int(v.nb < v.e2 * 0.49999) & int(v.e2 > 1e-250)) != 0;
+}
+// inside the bracket: the sum with moduli from the hardware root
+template <int M>
+__device__ __forceinline__ void lag_narrow(const LagEval& v, const cx (&b)[M + 1], bool& far,
+                                           bool& near) {
+  double e = __builtin_amdgcn_sqrt(cnorm(b[M]));
+#pragma unroll
+  for (int j = M - 1; j >= 0; j--) e = fma(v.ax, e, __builtin_amdgcn_sqrt(cnorm(b[j])));
+  const double eh = kLagEps * e;
+  near = (int(v.nb < eh * eh * 0.9999) & int(eh * eh > 1e-250)) != 0;
+  far = v.nb > eh * eh * 1.0001;
+}
+
+// The step from x: the next point x1 and x - x1 = step.  Returns whether
+// everything is in range, every comparison decided and x1 another point; else
+// the iteration is lag_general's.
+template <int M>
+__device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx& step) {
   constexpr double md = (double)M;
-  auto all = [](bool c) { return UNI ? __ballot(!c) == 0 : c; };
-  auto any = [](bool c) { return UNI ? __ballot(c) != 0 : c; };
+  // the recurrences' first two steps, from s = f = 0, leave s = b[M] and
+  // f = x b[M] + b[M - 1] (up to the sign of a zero, which the range check
+  // below sends to lag_general wherever it could matter)
+  cx s = b[M], f = cadd(cmul(x, b[M]), b[M - 1]);
+#pragma unroll
+  for (int j = M - 3; j >= 0; j--) {
+    s = cadd(cmul(x, s), f);
+    f = cadd(cmul(x, f), b[j + 1]);
+  }
+  // g = f / b and 2 s / b by Smith's quotient over one denominator
+  const cx B = b[0];
+  const bool ce = fabs(B.re) < fabs(B.im);
+  const double num = ce ? B.re : B.im, den = ce ? B.im : B.re;
+  const double ratio = quot_near(num, den, rcp_near(den));
+  const double denom = (num * ratio) + den;
+  const double rd = rcp_near(denom);
+  const cx s2 = cscale(s, 2.0);
+  const double far_ = f.re * ratio, fbr = f.im * ratio;
+  const double sar = s2.re * ratio, sbr = s2.im * ratio;
+  const double xf = ce ? far_ + f.im : fbr + f.re, yf = ce ? fbr - f.re : f.im - far_;
+  const double xs = ce ? sar + s2.im : sbr + s2.re, ys = ce ? sbr - s2.re : s2.im - sar;
+  const cx g = mk(quot_near(xf, denom, rd), quot_near(yf, denom, rd));
+  const cx g2 = cmul(g, g);
+  const cx h = csub(g2, mk(quot_near(xs, denom, rd), quot_near(ys, denom, rd)));
+  const cx rad = cscale(csub(cscale(h, md), g2), md - 1.0);
+  const cx sq = csqrt_near(rad.re, rad.im);
+  const cx gp = cadd(g, sq), gm = csub(g, sq);
+  const double np = cnorm(gp), nm = cnorm(gm);
+  const bool minus = np < nm;
+  const cx d = mk(minus ? gm.re : gp.re, minus ? gm.im : gp.im);
+  // the step m / d: Smith's quotient of a real numerator
+  const bool ce2 = fabs(d.re) < fabs(d.im);
+  const double num2 = ce2 ? d.re : d.im, den2 = ce2 ? d.im : d.re;
+  const double ratio2 = quot_near(num2, den2, rcp_near(den2));
+  const double denom2 = (num2 * ratio2) + den2;
+  const double rd2 = rcp_near(denom2);
+  const double mr = md * ratio2;
+  const double qa = quot_near(mr, denom2, rd2), qb = quot_near(md, denom2, rd2);
+  step = mk(ce2 ? qa : qb, ce2 ? -qb : -qa);
+  x1 = mk(x.re - (ce2 ? qa : qb), x.im + (ce2 ? qb : qa));
+  // (lo bounds den and den2 from below as well; f, s, g and den2 too large for
+  // the quotients leave rad out of its range)
+  const double lo = min_abs(min_abs(min_abs(xf, yf), min_abs(xs, ys)), min_abs(num, num2));
+  const double rx = max_abs(rad.re, rad.im), ry = min_abs(rad.re, rad.im);
+  // (ints: a chain of && would be a chain of branches)
+  return (int(lo >= kTinyOp) & int(fabs(den) <= kHugeOp) & int(hyp_in_range(rx, ry)) &
+          int(min_abs(np, nm) < max_abs(np, nm) * (1.0 - 1e-12)) &
+          (int(x.re != x1.re) | int(x.im != x1.im))) != 0;
+}
+
+// Laguerre::laguerre for a polynomial of degree M >= 2 held in registers,
+// every lane on its own x.  Leaves the Horner sums at the returned x in b,
+// which are the coefficients of the deflated polynomial (b[j + 1] =
+// coefficient j, laguerre.cc:133-139).
+template <int M>
+__device__ __forceinline__ bool lag_lane(const cx (&p)[M + 1], cx& x, cx (&b)[M + 1],
+                                         const TrigTable* trig, bool& oob) {
   for (int i = 1; i <= kLagMaxIt; i++) {
-    const double n = cnorm(x);
-    // |x|, or NaN (which leaves every comparison undecided) where its square
-    // may have lost digits
-    const double ax = n > 1e-280 ? __builtin_amdgcn_sqrt(n) : __builtin_nan("");
-    b[M] = p[M];
-    double e1 = fabs(p[M].re) + fabs(p[M].im);
-#pragma unroll
-    for (int j = M - 1; j >= 0; j--) {
-      b[j] = cadd(cmul(x, b[j + 1]), p[j]);
-      e1 = fma(ax, e1, fabs(b[j].re) + fabs(b[j].im));
+    const LagEval v = lag_eval<M>(p, x, b);
+    bool far = lag_far(v);
+    if (__builtin_expect(!far, 0)) {
+      bool near = lag_near(v);
+      if (!near) lag_narrow<M>(v, b, far, near);
+      if (near) return true;
     }
-    const double nb = cnorm(b[0]);
-    const double el = kLagEps * e1;
-    const double e2 = el * el;
-    bool far = nb > e2 * 1.0001;  // nb above 1e-250 follows from lo below
-    if (__builtin_expect(!all(far), 0)) {
-      if (all(nb < e2 * 0.49999 && e2 > 1e-250)) return true;
-      if (any(!far)) {
-        // inside the bracket: the sum with moduli from the hardware root
-        double e = __builtin_amdgcn_sqrt(cnorm(b[M]));
-#pragma unroll
-        for (int j = M - 1; j >= 0; j--) e = fma(ax, e, __builtin_amdgcn_sqrt(cnorm(b[j])));
-        const double eh = kLagEps * e;
-        if (all(nb < eh * eh * 0.9999 && eh * eh > 1e-250)) return true;
-        far = nb > eh * eh * 1.0001;
-      }
-    }
-    // the recurrences' first two steps, from s = f = 0, leave s = b[M] and
-    // f = x b[M] + b[M - 1] (up to the sign of a zero, which the range check
-    // below sends to lag_general wherever it could matter)
-    cx s = b[M], f = cadd(cmul(x, b[M]), b[M - 1]);
-#pragma unroll
-    for (int j = M - 3; j >= 0; j--) {
-      s = cadd(cmul(x, s), f);
-      f = cadd(cmul(x, f), b[j + 1]);
-    }
-    // g = f / b and 2 s / b by Smith's quotient over one denominator
-    const cx B = b[0];
-    const bool ce = fabs(B.re) < fabs(B.im);
-    const double num = ce ? B.re : B.im, den = ce ? B.im : B.re;
-    const double ratio = quot_near(num, den, rcp_near(den));
-    const double denom = (num * ratio) + den;
-    const double rd = rcp_near(denom);
-    const cx s2 = cscale(s, 2.0);
-    const double far_ = f.re * ratio, fbr = f.im * ratio;
-    const double sar = s2.re * ratio, sbr = s2.im * ratio;
-    const double xf = ce ? far_ + f.im : fbr + f.re, yf = ce ? fbr - f.re : f.im - far_;
-    const double xs = ce ? sar + s2.im : sbr + s2.re, ys = ce ? sbr - s2.re : s2.im - sar;
-    const cx g = mk(quot_near(xf, denom, rd), quot_near(yf, denom, rd));
-    const cx g2 = cmul(g, g);
-    const cx h = csub(g2, mk(quot_near(xs, denom, rd), quot_near(ys, denom, rd)));
-    const cx rad = cscale(csub(cscale(h, md), g2), md - 1.0);
-    const cx sq = csqrt_near(rad.re, rad.im);
-    const cx gp = cadd(g, sq), gm = csub(g, sq);
-    const double np = cnorm(gp), nm = cnorm(gm);
-    const bool minus = np < nm;
-    const cx d = mk(minus ? gm.re : gp.re, minus ? gm.im : gp.im);
-    // the step m / d: Smith's quotient of a real numerator
-    const bool ce2 = fabs(d.re) < fabs(d.im);
-    const double num2 = ce2 ? d.re : d.im, den2 = ce2 ? d.im : d.re;
-    const double ratio2 = quot_near(num2, den2, rcp_near(den2));
-    const double denom2 = (num2 * ratio2) + den2;
-    const double rd2 = rcp_near(denom2);
-    const double mr = md * ratio2;
-    const double qa = quot_near(mr, denom2, rd2), qb = quot_near(md, denom2, rd2);
-    const cx x1 = mk(x.re - (ce2 ? qa : qb), x.im + (ce2 ? qb : qa));
-    // everything in range, every comparison decided, x moved.  (lo bounds den
-    // and den2 from below as well; f, s, g and den2 too large for the
-    // quotients leave rad out of its range.)
-    const double lo = min_abs(min_abs(min_abs(xf, yf), min_abs(xs, ys)), min_abs(num, num2));
-    const double rx = max_abs(rad.re, rad.im), ry = min_abs(rad.re, rad.im);
-    // (ints: a chain of && would be a chain of branches)
-    const int ok = int(far) & int(lo >= kTinyOp) & int(fabs(den) <= kHugeOp) &
-                   int(hyp_in_range(rx, ry)) &
-                   int(min_abs(np, nm) < max_abs(np, nm) * (1.0 - 1e-12)) &
-                   (int(x.re != x1.re) | int(x.im != x1.im));
-    if (__builtin_expect(all(ok != 0), 1)) {
+    cx x1, step;
+    const int ok = int(lag_step<M>(b, x, x1, step)) & int(far);
+    if (__builtin_expect(ok, 1)) {
       if (__builtin_expect(i % kLagMT == 0, 0)) {
         oob |= i / kLagMT >= 8;
-        x = lag_kick(x, mk(ce2 ? qa : qb, ce2 ? -qb : -qa), i);
+        x = lag_kick(x, step, i);
       } else {
         x = x1;
       }
@@ -283,6 +309,67 @@ __device__ __forceinline__ bool lag_fast(const cx (&p)[M + 1], cx& x, cx (&b)[M 
     if (lag_general<M>(b, x, i, trig, oob)) return true;
   }
   horner_sums<M>(p, x, b);  // not converged: the sums where it stopped
+  return false;
+}
+
+// The same on a whole wavefront whose branches are all taken by the whole
+// wave: SAME: every lane holds the same p and x; else each lane its own x
+// (b is then not the sums at x, and the result means nothing: a lane that is
+// done keeps x until the others are).  One wavefront alone on its SIMD waits
+// 20 to 50 cycles at every branch; with lag_lane's returns the compiler made
+// nine of an iteration, of which four were taken, one in four cycles of the
+// chain.
+template <int M, bool SAME>
+__device__ __forceinline__ bool lag_wave(const cx (&p)[M + 1], cx& x, cx (&b)[M + 1],
+                                         const TrigTable* trig, bool& oob) {
+  unsigned long long run = ~0ull;  // lanes not done
+  const unsigned long long me = 1ull << __lane_id();
+  auto settle = [&](unsigned long long done) {
+    run &= ~done;
+    return SAME ? done != 0 : run == 0;
+  };
+  for (int i = 1; i <= kLagMaxIt; i++) {
+    const LagEval v = lag_eval<M>(p, x, b);
+    unsigned long long open = __ballot(!lag_far(v)) & run;
+    if (__builtin_expect(open != 0, 0)) {
+      unsigned long long done = __ballot(lag_near(v)) & open;
+      if (open != done) {
+        bool far, near;
+        lag_narrow<M>(v, b, far, near);
+        done |= __ballot(near) & open;
+        open &= ~__ballot(far);
+      }
+      if (settle(done)) return true;
+      open &= ~done;
+    }
+    cx x1, step;
+    const bool ok = lag_step<M>(b, x, x1, step);
+    const unsigned long long gen = (__ballot(!ok) | open) & run;
+    if (__builtin_expect(i % kLagMT == 0, 0)) {
+      const unsigned long long kick = run & ~gen;
+      x1 = lag_kick(x, step, i);
+      if (i / kLagMT >= 8) oob |= (kick & me) != 0;
+    }
+    if (__builtin_expect(gen != 0, 0)) {
+      keep(x.re);  // the general iteration shares nothing with the code above
+      keep(x.im);
+      bool done = false;
+      cx y = x;
+      if (gen & me) done = lag_general<M>(b, y, i, trig, oob);
+      if (gen & me) x1 = y;
+      // (a lane that lag_general accepts keeps its x)
+      const unsigned long long d = __ballot(done);
+      if (SAME && d != 0) return true;
+      if (run & me) x = x1;
+      if (settle(d)) return true;
+    } else if (SAME) {
+      x = x1;
+    } else {
+      const bool mine = (run & me) != 0;
+      x = mk(mine ? x1.re : x.re, mine ? x1.im : x.im);
+    }
+  }
+  if (SAME) horner_sums<M>(p, x, b);  // not converged: the sums where it stopped
   return false;
 }
 
