@@ -240,9 +240,10 @@ struct Options {
   double timeLimitS = 60.0;
   int seedChunks = 3;       // the seed search is cut into this many chunks of positions
   int seedChunkMin = 64;    // ... of at least this many positions per curve
-  int specPiece = 32;       // verified speculative chain: positions per piece (0: the
-                            // serial chain in chunks)
-  int specOverlap = 16;     // ... positions a piece's chain runs into the next piece
+  int specPiece = 32;       // verified speculative chain: positions per piece, at most (0:
+                            // the serial chain in chunks)
+  int specOverlap = 16;     // ... positions a piece's chain runs into the next piece, at most
+                            // half of the piece length
   int specDepth = 4096;     // ... piece boundaries a repair chain may cross (at most the
                             // batch's largest piece count is used: a repair chain can then
                             // always run to its curve's end)
@@ -332,6 +333,7 @@ struct Engine {
   DBuf<int2> dSpecPos, dSpecActive, dSpecFront, dSpecList;
   DBuf<cx> dSpecOwn, dSpecExt, dSpecRep, dSpecChain, dSpecStart;
   std::vector<int> specCalls;  // per curve: the chain's solve count after the run
+  int specLen = 32;            // positions per piece of this run
   // the segments in flight: what each leaves in SpecArgs::info, copied to a
   // slot of a ring in pinned memory, and the event behind the copy
   static constexpr int kSpecFlight = 16;
@@ -539,7 +541,7 @@ CurveDev to_dev(const Curve& c, cx s, cx e, int pointBase, int causticBase) {
 }
 
 // The verified speculative chain on the seed stream (after the solve pool is
-// built): cuts every curve into pieces of about opt.specPiece positions, runs
+// built): cuts every curve into pieces of about specLen positions, runs
 // round 1 and the agreement, and leaves the pieces' start states in `sa` for
 // seed_kernel as they become known.
 void Engine::spec_start(std::vector<CurveDev>& hc, const std::vector<int>& pointBase,
@@ -550,7 +552,7 @@ void Engine::spec_start(std::vector<CurveDev>& hc, const std::vector<int>& point
   int maxP = 1;
   for (int k = 0; k < nc; k++) {
     const int n = pointBase[k + 1] - pointBase[k];
-    const int P = std::max(1, n / opt.specPiece);
+    const int P = std::max(1, n / specLen);
     hc[k].split = P;
     specBase[k + 1] = specBase[k] + P;
     maxP = std::max(maxP, P);
@@ -596,7 +598,7 @@ void Engine::spec_start(std::vector<CurveDev>& hc, const std::vector<int>& point
   SpecArgs& sp = specArgs;
   sp.pieceBase = dSpecBase.p;
   sp.nPieces = G;
-  sp.overlap = std::max(1, opt.specOverlap);
+  sp.overlap = std::max(1, std::min(opt.specOverlap, specLen / 2));
   sp.depth = depth;
   sp.budget = std::max(1, opt.specSegment);
   sp.own = dSpecOwn.p;
@@ -763,6 +765,15 @@ void Engine::run(Job& job) {
   // the verified speculative chain: the single chain's seeds, computed in
   // pieces in parallel (not with a split search, and not where the chain
   // replays recorded slot values)
+  // A run of few positions has shorter pieces, down to 8: round 1 and the seed
+  // launch take the time of one piece, and a chip that a hundred wavefronts
+  // leave idle has room for more pieces and repair chains.  (8 positions
+  // instead of 32: 777 points 4.9 -> 3.7 ms, eight curves of 256 points 10.8 ->
+  // 9.7, the planetary binary's 200 43 -> 36.5; but 140,000 points of 64 curves
+  // 137 -> 147.)  Curves of fewer than two full pieces keep the serial chain:
+  // at 33 positions the pieces are faster where they agree (1.6 ms instead of
+  // 1.8), slower where the whole curve is one repair chain (2.4 instead of 2.1).
+  specLen = std::min(opt.specPiece, std::max(8, nPts / 128));
   bool spec = job.runSeeds && opt.specPiece > 0 && slots.empty() &&
               (int)maxLen >= 2 * opt.specPiece;
   for (auto* c : job.curves) spec = spec && c->split == 1;
