@@ -114,7 +114,7 @@ struct SeedArgs {
   int nCurves;
   const cx* caustics;
   const TrigTable* trig;
-  SolvePool pool;      // filled by trial_kernel
+  SolvePool pool;      // filled by launch_trials and launch_solve_prep
   const double* ptCausD2;
   const cx* slotTrace; // recorded tempRoots[10] values (CurveDev::slotBase), may be null
   int2* seeds;        // [point][kMaxSeeds] pixel (nx, ny)

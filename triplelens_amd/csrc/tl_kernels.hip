@@ -1,6 +1,6 @@
 // HIP kernels of the IRS engine (gfx950).
 //
-//  trial_kernel   per light-curve point, all at once: source position, caustic
+//  trial_*_kernel per light-curve point, all at once: source position, caustic
 //                 trial points (src/LightCurves/lcirs.cc:131-165) and the
 //                 image polynomial of every solve (tl_coeffs.h).
 //  seed_kernel    per light curve, the reference's seed sequence: point images
@@ -8,6 +8,8 @@
 //                 points (src/LightCurves/lcirs.cc:116-165), as pixel seeds.
 //  solve_prep_kernel  what a solve of the chain needs that does not depend on
 //                 the chain (its first deflation step, its fresh solve).
+//  spec_*_kernel  the chain in pieces in parallel, verified, with repair chains
+//                 that run beside the fill of the pieces already known.
 //  fill_kernel    one persistent, work-stealing launch that grows the image
 //                 "amoebae" of a batch of source positions: wavefronts pop
 //                 row-check tasks, evaluate 64 pixels per step with the FP64
@@ -605,7 +607,7 @@ int launch_image_poly(const Lens& L, const cx* fixedPoly, const cx* zeta, int n,
 // split = S > 1 the chunk's positions are cut into S contiguous pieces that
 // run in parallel; piece 0 continues the chain, the others start from a
 // fresh solve.  Each position's solves (centre, then caustic trial points)
-// and their polynomials come from trial_kernel's pool, so the chain itself
+// and their polynomials come from the pool, so the chain itself
 // only runs the root solves, the image tests and the seed output.
 template <bool TRACED>
 __global__ void __launch_bounds__(64) seed_kernel(SeedArgs a) {
