@@ -206,8 +206,9 @@ int lcirs_batch_fill_positions(int n, void** lcs, const int* counts, const int* 
                                uint32_t* flags);
 
 /* Engine counters of the last run: out[0] fill tasks, out[1] evaluated
- * pixels, out[2] runs inserted, out[3] duplicate runs, out[4] seed-kernel
- * milliseconds, out[5] fill milliseconds (sum over launches), out[6] fill
+ * pixels, out[2] runs inserted, out[3] duplicate runs, out[4]
+ * milliseconds from the solve lists to the last seed launch (with the fills
+ * that ran beside the seed search), out[5] fill milliseconds (sum over launches), out[6] fill
  * launches, out[7] total milliseconds of the last run, out[8] summed busy
  * time of the fill's wavefronts (ms), out[9] of that, time in run-table
  * inserts (ms), out[10] idle polls, out[11] wavefronts of the last launch,

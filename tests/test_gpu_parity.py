@@ -232,6 +232,29 @@ def test_speculative_chain_in_segments(E, piece, overlap, segment):
             assert np.array_equal(seeds[k][1], seeds0[k][1])
 
 
+@pytest.mark.parametrize("opts", [{"spec_segment": 7}, {"spec_segment": 7, "spec_depth": 1}],
+                         ids=["stages", "fallback_after_stages"])
+def test_amoebae_of_a_fill_in_stages(E, tmp_path, opts):
+    """The amoeba files of a curve filled in stages, and of one whose serial
+    chain fills every position again after some stages, are the serial
+    chain's."""
+    from triplelens_amd.ctypes_classes import LC_irs
+    c = replace(curve_from_params(golden("c2_ppr20.npz")["params"]), n_points=400)
+    texts = []
+    try:
+        for name, o in (("serial", {"spec_piece": 0}), ("staged", {"spec_piece": 32, **opts})):
+            for k, v in o.items():
+                E.set_option(k, v)
+            lc = LC_irs(*c.lens(), c.rho, c.lc_len, c.ppr)
+            lc.set_amoeba_printout(str(tmp_path / name), str(tmp_path / ("par_" + name)))
+            lc.get_lc_irs(*c.traj())
+            texts.append([(tmp_path / f"{name}{i}").read_text() for i in range(c.n_points)])
+    finally:
+        for k, v in {"spec_piece": 32, "spec_segment": 192, "spec_depth": 4096}.items():
+            E.set_option(k, v)
+    assert texts[0] == texts[1]
+
+
 def test_c2_window_full_resolution_golden(E):
     """A 65-point curve around the C2 magnification peak at pixel rho/200."""
     g = golden("c2_window.npz")

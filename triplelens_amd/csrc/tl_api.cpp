@@ -693,6 +693,7 @@ void Engine::run(Job& job) {
   init();
   auto tStart = std::chrono::steady_clock::now();
   stats = Stats();
+  specCalls.clear();
   const int nc = (int)job.curves.size();
   std::vector<CurveDev> hc(nc);
   std::vector<int> pointBase(nc + 1, 0);
@@ -935,6 +936,7 @@ void Engine::run(Job& job) {
     dSeedTasks.ensure((size_t)nPts * kMaxSeeds, later);
   }
   std::vector<int> given(nc, 0);  // pieces of earlier stages
+  std::vector<int2> list;         // pieces of this one
   bool last = false;
   for (int ch = 0; !last; ch++) {
   order.clear();
@@ -959,6 +961,7 @@ void Engine::run(Job& job) {
       stats.specFallback = 1;
       stats.specPieces = stats.specRepairs = 0;
       specCalls.clear();
+      for (auto& a : amoebae) a.clear();
       spec = false;
       ch = 0;
       later = nullptr;
@@ -985,7 +988,7 @@ void Engine::run(Job& job) {
       const int keep = nc == 1 && specActive <= kWalkWaves ? 8 : 32;
       if (opt.fillWorkgroups <= 0) nWg = std::max(1, nWgAll - keep);
     }
-    std::vector<int2> list;
+    list.clear();
     for (int k = 0; k < nc; k++) {
       const long long len = pointBase[k + 1] - pointBase[k];
       const int P = specBase[k + 1] - specBase[k];
