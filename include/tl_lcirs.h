@@ -260,12 +260,20 @@ int tl_image_poly(double a, double b, double th, double m2, double m3, int n, co
  * whose results differ in any bit.  No counterpart in the reference. */
 int tl_math_selftest(int n, unsigned long long seed);
 
-/* GPU self-test of the fill's in-range division (the IEEE double division
- * sequence without operand pre-scaling, used for the ray test's quotients
- * m_k / |z - z_k|^2 when both lie in its range) against IEEE division on n
- * generated operand pairs; returns the number whose results differ in any
- * bit, or -1 on error.  No counterpart in the reference. */
+/* GPU self-test of the root solver's in-range quotient (and square root)
+ * against the IEEE operations on n generated operand pairs; returns the number
+ * whose results differ in any bit, or -1 on error.  No counterpart in the
+ * reference. */
 int tl_div_selftest(long long n, unsigned long long seed);
+
+/* GPU self-test of the in-range forms the root solver runs against the
+ * general ones, to the bit, on n generated operands each over the ranges the
+ * solver admits: bad[0] quotients, bad[1] square roots, bad[2] moduli, bad[3]
+ * complex square roots whose results differ.  Among the operands are the
+ * quotients and roots that lie closest to a rounding boundary.  Operands that
+ * the solver leaves to its general iteration (a few that lie just below a power of two)
+ * are left out; bad[4] is their number among the random ones.  Returns 0, or -1 with tl_last_error().  No counterpart in the reference. */
+int tl_roots_selftest(long long n, unsigned long long seed, long long bad[5]);
 
 /* Engine settings: name/value pairs ("fill_workgroups", "probe_limit",
  * "queue_log2", "scout_rows", "scout_jump", "scout_retry", "scout_width",

@@ -377,6 +377,22 @@ def test_in_range_division_equals_ieee_division(E):
         assert lib.tl_div_selftest(1 << 26, seed) == 0
 
 
+def test_root_solver_arithmetic_equals_general_forms(E):
+    """tl_roots_selftest: the in-range quotient, square root, modulus and
+    complex square root the root solver runs equal the general ones to the
+    bit over the ranges it admits, at the hardest operands too."""
+    lib = E.load()
+    lib.tl_roots_selftest.argtypes = [ctypes.c_longlong, ctypes.c_ulonglong,
+                                      ctypes.POINTER(ctypes.c_longlong)]
+    lib.tl_roots_selftest.restype = ctypes.c_int
+    bad = (ctypes.c_longlong * 5)()
+    for seed in (1, 0x5DEECE66D):
+        assert lib.tl_roots_selftest(1 << 24, seed, bad) == 0
+        assert list(bad)[:4] == [0, 0, 0, 0]
+        # four operands each, one in 2^16 of them below a power of two
+        assert bad[4] < 2 * (4 << 24) / 2 ** 16
+
+
 def test_full_c2_curve_properties(E, oracle):
     """The full benchmark curve (4096 points, pixel rho/200): no status
     flags, bitwise-identical repeat runs, every point's seed set equal to the

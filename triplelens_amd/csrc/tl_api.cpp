@@ -2060,6 +2060,57 @@ int tl_div_selftest(long long n, unsigned long long seed) {
   });
 }
 
+int tl_roots_selftest(long long n, unsigned long long seed, long long* bad) {
+  return guarded([&] {
+    if (n < 0 || !bad) throw std::invalid_argument("bad arguments");
+    // The arguments in [1, 4) whose square roots lie closest to a rounding
+    // boundary: with M an odd 54-bit integer (a midpoint of two doubles) and
+    // A 2^s - M^2 = -j, s = 54 for roots below sqrt 2 and 55 beyond, j small.
+    // M^2 = j modulo 2^s has four solutions for j = 1 modulo 8 and none else.
+    std::vector<double> hard;
+    typedef unsigned __int128 u128;
+    for (long long j = -63; j <= 65; j += 8) {
+      unsigned long long x = 1;  // x^2 = j modulo 2^k
+      for (int k = 3; k < 62; k++)
+        if ((x * x - (unsigned long long)j) >> k & 1ull) x += 1ull << (k - 1);
+      for (int s = 54; s <= 55; s++)
+        for (int v = 0; v < 4; v++) {
+          unsigned long long M = (v & 1 ? 0ull - x : x) + (v & 2 ? 1ull << (s - 1) : 0ull);
+          M &= (1ull << s) - 1;
+          if (M >> 54 || !(M >> 53)) continue;
+          const unsigned long long A = (unsigned long long)(((u128)M * M - (u128)(__int128)j) >> s);
+          if (A >> 53 || !(A >> 52)) continue;
+          hard.push_back(ldexp((double)A, s - 106));
+        }
+    }
+    Engine& E = engine();
+    std::lock_guard<std::mutex> lock(E.mu);
+    E.init();
+    unsigned long long cnt[5] = {0, 0, 0, 0, 0};
+    unsigned long long* d = nullptr;
+    double* dh = nullptr;
+    auto release = [&] {
+      (void)hipFree(d);
+      (void)hipFree(dh);
+    };
+    try {
+      HIPCHK(hipMalloc(&d, sizeof cnt));
+      HIPCHK(hipMalloc(&dh, hard.size() * sizeof(double)));
+      HIPCHK(hipMemcpy(d, cnt, sizeof cnt, hipMemcpyHostToDevice));
+      HIPCHK(hipMemcpy(dh, hard.data(), hard.size() * sizeof(double), hipMemcpyHostToDevice));
+      HIPCHK((hipError_t)launch_roots_check(n, seed, dh, (int)hard.size(), d, E.stream));
+      HIPCHK(hipStreamSynchronize(E.stream));
+      HIPCHK(hipMemcpy(cnt, d, sizeof cnt, hipMemcpyDeviceToHost));
+    } catch (...) {
+      release();
+      throw;
+    }
+    release();
+    for (int k = 0; k < 5; k++) bad[k] = (long long)cnt[k];
+    return 0;
+  });
+}
+
 int tl_math_selftest(int n, unsigned long long seed) {
   // the branch-free complex helpers against the general ones, on the host
   unsigned long long st = seed ? seed : 1;

@@ -1599,12 +1599,12 @@ __device__ __forceinline__ void afaddi(int* p, int v) {
   __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, AGENT);
 }
 
-// Self-test of the in-range quotient (quot_near) and square root (sqrt_near)
-// against the IEEE operations on n operand pairs drawn from their range: random sign, exponent and mantissa (one pair in two), the
-// ends of the range, and numerators built as the rounded product of the
-// denominator and a quotient half an ulp above a random double (the
-// quotients nearest a rounding boundary).  bad counts the pairs whose
-// results differ in any bit.
+// Self-test of the in-range quotient (quot_near) and square root (sqrt_near,
+// where lag_step takes it) against the IEEE operations on n operand pairs:
+// random sign, exponent and mantissa (one pair in two), the ends of the
+// range, and numerators built as the rounded product of the denominator and
+// a quotient half an ulp above a random double (roots_check_kernel draws the
+// hardest ones).  bad counts the pairs whose results differ in any bit.
 __global__ void div_check_kernel(long long n, unsigned long long seed, unsigned long long* bad) {
   const long long stride = (long long)gridDim.x * blockDim.x;
   unsigned long long cnt = 0;
@@ -1643,8 +1643,7 @@ __global__ void div_check_kernel(long long n, unsigned long long seed, unsigned 
     }
     const double x = quot_near(a, b, rcp_near(b)), y = a / b;
     cnt += __double_as_longlong(x) != __double_as_longlong(y) ? 1 : 0;
-    if (kind < 4) {
-      // the ends of the range hold the two mantissas sqrt_near leaves out
+    if (edge(b) < kEdge) {
       double r, h;
       sqrt_near(fabs(b), r, h);
       cnt += __double_as_longlong(r) != __double_as_longlong(sqrt(fabs(b))) ? 1 : 0;
@@ -1660,6 +1659,117 @@ int launch_div_check(long long n, unsigned long long seed, unsigned long long* b
   const long long blocks = (n + 255) / 256;
   hipLaunchKernelGGL(div_check_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256),
                      0, s, n, seed, bad);
+  return (int)hipGetLastError();
+}
+
+// Self-test of the in-range forms the root solver runs (tl_roots.h) against
+// the general ones, to the bit, over the ranges lag_step admits.  Operands that
+// it leaves to the general iteration for their mantissas are left out; bad[4]
+// counts those among the random ones.
+//   bad[0] quot_near: operands 2^-300 .. 2^300, random, and the quotients
+//          closest to a rounding boundary: A 2^s = M B -+ j for a denominator
+//          B, an odd 54-bit M and j = 1, 3, 5 (one B in four within 2^20
+//          units below a power of two, one in eight as far above);
+//   bad[1] sqrt_near: 2^-600 .. 2^600, random, and the `nHard` mantissas in
+//          hard, whose roots lie closest to a rounding boundary;
+//   bad[2] hyp_near against hyp_sel, bad[3] csqrt_near against csqrt_sel:
+//          random signs, magnitudes 2^-240 .. 2^240, less than 2^54 apart.
+__global__ void roots_check_kernel(long long n, unsigned long long seed, const double* hard,
+                                   int nHard, unsigned long long* bad) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  unsigned long long cnt[4] = {0, 0, 0, 0}, skipped = 0;
+  auto differ = [](double x, double y) {
+    return __double_as_longlong(x) != __double_as_longlong(y) ? 1ull : 0ull;
+  };
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (unsigned long long)(i + 1);
+    auto next = [&z]() {
+      z += 0x9E3779B97F4A7C15ull;
+      unsigned long long x = z;
+      x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+      x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+      return x ^ (x >> 31);
+    };
+    // random sign and mantissa, exponent elo .. ehi
+    auto make = [&next](int elo, int ehi) {
+      const unsigned long long r = next(), e = next();
+      const unsigned long long at = (unsigned long long)(1023 + elo) +
+                                    e % (unsigned long long)(ehi - elo + 1);
+      return __longlong_as_double(
+          (long long)((r & 0x800FFFFFFFFFFFFFull) | (at << 52)));
+    };
+    {
+      const double a = make(-300, 299), b = make(-300, 299);
+      if (edge(b) < kEdge) cnt[0] += differ(quot_near(a, b, rcp_near(b)), a / b);
+      else skipped++;
+      const unsigned long long r = next(), kind = next() & 7;
+      unsigned long long B = (r & ((1ull << 52) - 1)) | (1ull << 52) | 1ull;
+      if (kind < 2) B = (1ull << 53) - ((r & ((1ull << 20) - 1)) | 1ull);
+      else if (kind == 2) B = (1ull << 52) + ((r & ((1ull << 20) - 1)) | 1ull);
+      unsigned long long inv = B;  // 1 / B modulo 2^64 (Newton)
+      for (int k = 0; k < 6; k++) inv *= 2ull - B * inv;
+      const int eb = (int)(next() % 500) - 250;
+      for (int j = -5; j <= 5; j += 2) {
+        const unsigned long long t = (unsigned long long)(long long)j * inv;
+        for (int s = 53; s <= 54; s++) {
+          const unsigned long long M =
+              s == 53 ? (t & ((1ull << 53) - 1)) | (1ull << 53) : t & ((1ull << 54) - 1);
+          if (!(M >> 53)) continue;
+          // (M B - j) >> s
+          unsigned long long lo = M * B, hi = __umul64hi(M, B);
+          const unsigned long long d = (unsigned long long)(long long)j;
+          hi -= (j < 0 ? ~0ull : 0ull) + (lo < d ? 1ull : 0ull);
+          lo -= d;
+          const unsigned long long A = (hi << (64 - s)) | (lo >> s);
+          if (A >> 53 || !(A >> 52) || (s == 53) != (A >= B)) continue;
+          const double x = (double)A, y = ldexp((double)B, eb);
+          if (edge(y) < kEdge) cnt[0] += differ(quot_near(x, y, rcp_near(y)), x / y);
+        }
+      }
+    }
+    {
+      double r, h;
+      const double a = fabs(make(-600, 599));
+      sqrt_near(a, r, h);
+      if (edge(a) < kEdge) cnt[1] += differ(r, sqrt(a));
+      else skipped++;
+      if (nHard > 0) {
+        const double c = ldexp(hard[next() % (unsigned long long)nHard],
+                               2 * ((int)(next() % 596) - 298));
+        sqrt_near(c, r, h);
+        if (edge(c) < kEdge) cnt[1] += differ(r, sqrt(c));
+      }
+    }
+    {
+      const double x = make(-240, 239);
+      const int e = ilogb(x);
+      const int lo = e - 53 < -240 ? -240 : e - 53, hi = e + 53 > 239 ? 239 : e + 53;
+      // magnitudes near each other in one pair of two (a radicand's usual case)
+      const double y = next() & 1 ? make(lo, hi) : make(e - 1 < -240 ? -240 : e - 1,
+                                                        e + 1 > 239 ? 239 : e + 1);
+      const double ax = max_abs(x, y), ay = min_abs(x, y);
+      if (hyp_in_range(ax, ay)) {
+        Edge em = 0;
+        const double h = hyp_near(ax, ay, em);
+        if (em < kEdge) cnt[2] += differ(h, hyp_sel(x, y));
+        const cx c0 = csqrt_near(x, y, em), c1 = csqrt_sel(mk(x, y));
+        if (em < kEdge) cnt[3] += differ(c0.re, c1.re) | differ(c0.im, c1.im);
+        else skipped++;
+      }
+    }
+  }
+  for (int k = 0; k < 4; k++)
+    if (cnt[k]) atomicAdd(&bad[k], cnt[k]);
+  if (skipped) atomicAdd(&bad[4], skipped);
+}
+
+int launch_roots_check(long long n, unsigned long long seed, const double* hard, int nHard,
+                       unsigned long long* bad, hipStream_t s) {
+  if (n <= 0) return 0;
+  if (!bad || nHard < 0 || (nHard > 0 && !hard)) return (int)hipErrorInvalidValue;
+  const long long blocks = (n + 255) / 256;
+  hipLaunchKernelGGL(roots_check_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256),
+                     0, s, n, seed, hard, nHard, bad);
   return (int)hipGetLastError();
 }
 

@@ -18,8 +18,8 @@
 // Quotients and square roots of operands in a safe range are taken without
 // the pre-scaling and special-value fix-up of the IEEE sequences, and a
 // square root hands its reciprocal on to the divisions by it (modulus
-// correction, csqrt).  Operands outside the range, signed zeros, kicks and
-// everything else unusual go through the general iteration.
+// correction, csqrt).  Operands outside the range or just below a power of two,
+// signed zeros and everything else unusual go through the general iteration.
 #pragma once
 
 #include "tl_math.h"
@@ -45,9 +45,22 @@ __device__ __forceinline__ double max_abs(double a, double b) {
 __device__ __forceinline__ void keep(double& a) { asm volatile("" : "+v"(a)); }
 
 // ---- in-range arithmetic ---------------------------------------------------
-// Reciprocal of b within about half a unit in the last place, for
-// 2^-900 <= |b| <= 2^900: the hardware estimate r0 (e = 1 - b r0, |e| below
-// 2^-22) and one third-order correction r0 (1 + e + e^2).
+// The forms below round as the IEEE operations do, except for a few operands
+// that all lie just below a power of two (see quot_near and sqrt_near).  So an
+// iteration with an operand whose mantissa bits 32 to 47 are all ones (one
+// iteration in 10^4) is left to the general form: edge(a) holds these bits,
+// and the largest of several operands' is kEdge where one of them has them.
+// (The maximum of 16-bit halves takes one instruction for three operands: a
+// 200-point chain takes 4.06 ms instead of 3.95 without the check, and 4.12
+// with a shift and both sides of a power of two.)
+typedef unsigned short Edge;
+constexpr Edge kEdge = 0xFFFF;
+__device__ __forceinline__ Edge edge(double a) { return (Edge)__double2hiint(a); }
+__device__ __forceinline__ Edge edge_max(Edge a, Edge b) { return a > b ? a : b; }
+
+// Reciprocal of b for 2^-900 <= |b| <= 2^900: the hardware estimate r0
+// (e = 1 - b r0, |e| below 2^-22) and one third-order correction
+// r0 (1 + e + e^2), within 2^-66 of 1/b before the last rounding.
 __device__ __forceinline__ double rcp_near(double b) {
   const double r0 = __builtin_amdgcn_rcp(b);
   const double e = fma(-b, r0, 1.0);
@@ -55,7 +68,12 @@ __device__ __forceinline__ double rcp_near(double b) {
   return fma(r0, p, r0);
 }
 // a / b rounded to nearest from r = rcp_near(b), one correction by the exact
-// residual (Markstein), for operands and quotients within 2^-900 .. 2^900.
+// residual, for operands and quotients within 2^-900 .. 2^900.  With r the
+// nearest double to 1/b the result is rounded to nearest (Markstein).  For
+// b = 2 - k 2^-52, k odd, 1/b lies k^2 2^-107 above a midpoint: where the
+// estimate does not resolve that (k below 2^20), r is the double below, and
+// for k >= 3 the quotients next to a midpoint may come out one unit off.
+// These b have edge(b) == kEdge.
 __device__ __forceinline__ double quot_near(double a, double b, double r) {
   const double q = a * r;
   return fma(fma(-b, q, a), r, q);
@@ -63,10 +81,10 @@ __device__ __forceinline__ double quot_near(double a, double b, double r) {
 // s = sqrt(a) rounded to nearest and h close to 1 / (2 s), for
 // 2^-600 <= a <= 2^600: the hardware reciprocal root y, s0 = a y, h0 = y/2 with
 // h0 s0 = 1/2 - e, one third-order step (1 - 2e)^-1/2 = 1 + e + 3/2 e^2, and the
-// exact residual.  The value before the last rounding is good to 2^-104; a
-// root lies that close to a rounding boundary for about a dozen of the 2^53
-// mantissas (those next to 1 among them), where s may be the neighbouring
-// double.
+// exact residual.  The value before the last rounding is good to 3.4 2^-106 of
+// the root: enough for all mantissas but the dozen whose roots lie closer to a
+// midpoint.  Of those (enumerated: A 2^s = M^2 - j, |j| <= 27) the only one
+// that comes out as the neighbouring double is 4 - 2^-51, edge(a) == kEdge.
 __device__ __forceinline__ void sqrt_near(double a, double& s, double& h) {
   const double y = __builtin_amdgcn_rsq(a);
   const double s0 = a * y, h0 = 0.5 * y;
@@ -76,10 +94,15 @@ __device__ __forceinline__ void sqrt_near(double a, double& s, double& h) {
   h = fma(h0, p, h0);
   s = fma(fma(-s1, s1, a), h, s1);
 }
-// hyp_sel for 2^-240 <= ay <= ax <= 2^240 and ay > ax 2^-54.
-__device__ __forceinline__ double hyp_near(double ax, double ay) {
+// hyp_sel for 2^-240 <= ay <= ax <= 2^240 and ay > ax 2^-54, if `em` (raised to
+// the edge of the root's operand) stays below kEdge.  (1/w and, in
+// csqrt_near, 1/q come from a root's reciprocal by a second-order step, good
+// to 2^-103: of the b of quot_near only k = 1 is left, which is harmless.)
+__device__ __forceinline__ double hyp_near(double ax, double ay, Edge& em) {
   double h, hi;
-  sqrt_near(ax * ax + ay * ay, h, hi);
+  const double n = ax * ax + ay * ay;
+  em = edge_max(em, edge(n));
+  sqrt_near(n, h, hi);
   const double w = 2.0 * h;
   const double r = fma(hi, fma(-w, hi, 1.0), hi);  // 1 / w
   const double d1 = h - ay;
@@ -93,12 +116,15 @@ __device__ __forceinline__ double hyp_near(double ax, double ay) {
 __device__ __forceinline__ bool hyp_in_range(double ax, double ay) {
   return (int(ay >= 0x1p-240) & int(ax <= 0x1p+240) & int(ay > ax * 0x1p-54)) != 0;
 }
-// csqrt_sel for re, im with hyp_in_range(max, min) of their magnitudes.
-__device__ __forceinline__ cx csqrt_near(double re, double im) {
+// csqrt_sel for re, im with hyp_in_range(max, min) of their magnitudes, if
+// `em` stays below kEdge.
+__device__ __forceinline__ cx csqrt_near(double re, double im, Edge& em) {
   const double fr = fabs(re);
-  const double d = hyp_near(max_abs(re, im), min_abs(re, im));
+  const double d = hyp_near(max_abs(re, im), min_abs(re, im), em);
   double q, h;
-  sqrt_near(0.5 * (d + fr), q, h);
+  const double n = 0.5 * (d + fr);
+  em = edge_max(em, edge(n));
+  sqrt_near(n, q, h);
   h = 2.0 * h;
   const double w = 0.5 * quot_near(im, q, fma(h, fma(-q, h, 1.0), h));
   const bool pos = re > 0.0;
@@ -253,7 +279,8 @@ __device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx&
   const cx g2 = cmul(g, g);
   const cx h = csub(g2, mk(quot_near(xs, denom, rd), quot_near(ys, denom, rd)));
   const cx rad = cscale(csub(cscale(h, md), g2), md - 1.0);
-  const cx sq = csqrt_near(rad.re, rad.im);
+  Edge em = edge_max(edge(den), edge(denom));
+  const cx sq = csqrt_near(rad.re, rad.im, em);
   const cx gp = cadd(g, sq), gm = csub(g, sq);
   const double np = cnorm(gp), nm = cnorm(gm);
   const bool minus = np < nm;
@@ -263,6 +290,7 @@ __device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx&
   const double num2 = ce2 ? d.re : d.im, den2 = ce2 ? d.im : d.re;
   const double ratio2 = quot_near(num2, den2, rcp_near(den2));
   const double denom2 = (num2 * ratio2) + den2;
+  em = edge_max(em, edge_max(edge(den2), edge(denom2)));
   const double rd2 = rcp_near(denom2);
   const double mr = md * ratio2;
   const double qa = quot_near(mr, denom2, rd2), qb = quot_near(md, denom2, rd2);
@@ -274,6 +302,7 @@ __device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx&
   const double rx = max_abs(rad.re, rad.im), ry = min_abs(rad.re, rad.im);
   // (ints: a chain of && would be a chain of branches)
   return (int(lo >= kTinyOp) & int(fabs(den) <= kHugeOp) & int(hyp_in_range(rx, ry)) &
+          int(em < kEdge) &
           int(min_abs(np, nm) < max_abs(np, nm) * (1.0 - 1e-12)) &
           (int(x.re != x1.re) | int(x.im != x1.im))) != 0;
 }
