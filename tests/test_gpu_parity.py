@@ -393,6 +393,104 @@ def test_root_solver_arithmetic_equals_general_forms(E):
         assert bad[4] < 2 * (4 << 24) / 2 ** 16
 
 
+@pytest.mark.parametrize("u", [0.0, 0.5])
+@pytest.mark.parametrize("lens,like", [((1.1, 1.0, 1.0, 0.05, 1e-70), (1.1, 1.0, 1.0, 0.05, 0.0)),
+                                       ((1.1, 1.0, 1.0, 1e-70, 0.0), (1.1, 1.0, 1.0, 1e-6, 0.0))],
+                         ids=["triple", "binary"])
+def test_fill_without_fast_rows(E, oracle, lens, like, u):
+    """A mass below 2^-200 leaves every row of the fill to the reference's own
+    operations (kRowExact): ray counts and magnifications from the images of
+    the lens without that mass equal the oracle's."""
+    rho, ppr = 1e-2, 40
+    lc = E.LightCurve(*lens, rho, 8, ppr)
+    lc.set_limb_darkening("linear", u)
+    lo = oracle.new(*lens, rho, 8, ppr, u)
+    g = lo.grid()
+    pos = np.array([[0.05, 0.02], [-0.01, 0.004], [0.3, -0.2], [0.006, -0.002]])
+    roots, is_img, _ = oracle.images(*like, pos[:, 0] + 1j * pos[:, 1])
+    ns = is_img.sum(axis=1)
+    pix = np.zeros((len(pos), E.MAX_SEEDS, 2), np.int32)
+    for i in range(len(pos)):
+        r = roots[i][is_img[i]]
+        px, py = pixel_seeds(g, np.stack([r.real, r.imag], axis=1))
+        pix[i, :ns[i], 0], pix[i, :ns[i], 1] = px, py
+    amp, rays, flags = lc.fill_seeds(pos, ns, pix)
+    _assert_no_status(E, flags)
+    for i in range(len(pos)):
+        sxy = np.stack([g[3] + pix[i, :ns[i], 0] * (g[1] / g[0]),
+                        g[4] + pix[i, :ns[i], 1] * (g[1] / g[0])], axis=1)
+        r, b, _ = lo.fill_point(*pos[i], sxy)
+        assert r > 0 and rays[i] == r, i
+        assert abs(amp[i] - b * g[7]) <= AMP_RTOL * abs(b * g[7]), i
+
+
+@pytest.mark.parametrize("u", [0.0, 0.5])
+@pytest.mark.parametrize("lens,ppr", [((1.0, 2.0, 0.0, 0.1, 0.05), 42),
+                                      ((1.1, 1.0, 1.0, 0.02, 0.0), 40)], ids=["triple", "binary"])
+def test_sweep_across_a_row_through_the_lenses(E, oracle, lens, ppr, u):
+    """Lenses on the real axis and a grid whose middle row is that axis: a
+    sweep leaves the fast rows there (the row lies on the lenses) and comes
+    back to them on the other side; the whole curve equals the oracle's."""
+    traj = (-0.04, 0.004, 0.05, 0.012)
+    lc = E.LightCurve(*lens, 1e-2, 8, ppr)
+    lc.set_limb_darkening("linear", u)
+    lo = oracle.new(*lens, 1e-2, 8, ppr, u)
+    g = lo.grid()
+    N = int(g[0])
+    mid = (N - 1) // 2
+    assert N % 2 == 1 and abs(g[4] + g[2] * mid) < 2.0 ** -50
+    amp, rays, flags = lc.lc_irs(*traj)
+    amp_o, rays_o, _ = lo.lc_irs(*traj)
+    _assert_no_status(E, flags)
+    assert np.array_equal(rays, rays_o)
+    assert _rel(amp, amp_o) < AMP_RTOL
+    xy, ns, _ = lo.seeds(*traj)
+    lo.fill_point(traj[0], traj[1], xy[0, :ns[0]])
+    rows = set(lo.last_segments()[:, 0].tolist())
+    assert {mid - 1, mid, mid + 1} <= rows
+
+
+def test_small_source_pixels_inside_the_undecided_band(E, oracle):
+    """A source of 1e-5: a boundary pixel in a few thousand lies closer to
+    rho than the fused ray is good for, and the reference's operations
+    decide it."""
+    from triplelens_amd import workloads as W
+    c = W.c1()
+    rho, ppr, n = 1e-5, 40, 40
+    lc = E.LightCurve(*c.lens(), rho, n, ppr)
+    lc.set_limb_darkening("linear", 0.3)
+    lo = oracle.new(*c.lens(), rho, n, ppr, 0.3)
+    amp, rays, flags = lc.lc_irs(*c.traj())
+    amp_o, rays_o, _ = lo.lc_irs(*c.traj())
+    _assert_no_status(E, flags)
+    assert np.array_equal(rays, rays_o)
+    assert _rel(amp, amp_o) < AMP_RTOL
+
+
+def test_staged_fill_with_too_small_tables(E):
+    """A fill in stages beside the repair chains whose run tables overflow:
+    each stage is run again with larger ones, and the curve is the one of
+    tables that fit."""
+    c = replace(curve_from_params(golden("c2_ppr20.npz")["params"]), ppr=200, n_points=600)
+    runs = []
+    try:
+        E.set_option("spec_segment", 7)
+        for o in ({}, {"run_pixels": 65536, "table_load": 1.5, "probe_limit": 64}):
+            for k, v in o.items():
+                E.set_option(k, v)
+            res = _new(E, c).lc_irs(*c.traj())
+            runs.append((res, E.last_stats()))
+    finally:
+        for k, v in {"spec_segment": 192, "run_pixels": 128, "table_load": 4,
+                     "probe_limit": 4096}.items():
+            E.set_option(k, v)
+    (a, st0), (b, st) = runs
+    assert st0["spec_repairs"] > 0 and st0["fill_launches"] > 1
+    assert st["runs"] > st0["runs"] * 1.1  # some launches were repeated
+    _assert_no_status(E, b[2])
+    assert np.array_equal(a[1], b[1]) and np.array_equal(a[0], b[0])
+
+
 def test_full_c2_curve_properties(E, oracle):
     """The full benchmark curve (4096 points, pixel rho/200): no status
     flags, bitwise-identical repeat runs, every point's seed set equal to the

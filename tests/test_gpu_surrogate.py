@@ -100,6 +100,51 @@ def test_training_on_part_of_the_rows(S, steps):
     np.testing.assert_allclose(a[:3], b[:3], rtol=64 * 2.0 ** -24, atol=64 * 2.0 ** -24)
 
 
+def _batches(S, n, steps, batch, seed):
+    """The rows of every training step: with lr = 0 and equal rows, the steps
+    whose loss a single row's target raises are those that hold the row."""
+    X = np.zeros((n, 14), np.float32)
+    hit = np.zeros((steps, n), bool)
+    for r in range(n):
+        y = np.zeros(n, np.float32)
+        y[r] = 50.0
+        net = S.Net(seed=8) if r == 0 else net
+        hit[:, r] = net.train(X, y, steps=steps, batch=batch, lr=0.0, seed=seed) > 5.0
+    return hit
+
+
+@pytest.mark.parametrize("steps", [4, 12])
+def test_training_steps_equal_single_batches(S, steps):
+    """A call of several steps leaves the parameters of as many calls of one
+    step each on the same rows: 4 steps take their rows along, 12 index the
+    whole set through two reshuffles (330 rows, 5 batches of 64 an epoch).
+    Only the order of the rows' sums differs, which flips the sign of the
+    first Adam updates where a gradient is rounding noise (one in 1e5), below 2% of
+    the total change; a wrong row would change it by tens of percent."""
+    n, batch = 330, 64
+    hit = _batches(S, n, steps, batch, 5)
+    assert (hit.sum(axis=1) == batch).all()
+    for e in range(0, steps, 5):
+        assert hit[e:e + 5].sum(axis=0).max() == 1
+    X, y = _rand_xy(np.random.default_rng(15), n)
+    net, ref = S.Net(seed=8), S.Net(seed=8)
+    p0 = net.params()
+    losses = net.train(X, y, steps=steps, batch=batch, lr=1e-3, seed=5)
+    one = [ref.train(X[h], y[h], steps=1, batch=batch, lr=1e-3, seed=1)[0] for h in hit]
+    np.testing.assert_allclose(losses, one, rtol=1e-3, atol=1e-3)
+    p, q = net.params(), ref.params()
+    assert np.linalg.norm(p - q) <= 2e-2 * np.linalg.norm(p - p0)
+
+
+def test_training_without_steps(S):
+    """No steps: nothing changes, nothing is copied."""
+    X, y = _rand_xy(np.random.default_rng(16), 128)
+    net = S.Net(seed=8)
+    p0 = net.params()
+    assert len(net.train(X, y, steps=0, batch=64)) == 0
+    assert np.array_equal(net.params(), p0)
+
+
 def test_training_reduces_loss(S):
     rng = np.random.default_rng(3)
     net = S.Net(seed=4)

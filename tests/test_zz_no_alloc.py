@@ -62,3 +62,28 @@ def test_noalloc_inference_equals_predict(hip):
     finally:
         hip.hipFree(dx)
         hip.hipFree(dout)
+
+
+def test_noalloc_result_over_its_input(hip):
+    """A result array that overlaps the rows in any way holds what one of its
+    own would: in place, behind the first rows, and in front of them."""
+    from triplelens_amd import surrogate as S
+    lib = S._lib()
+    lib.tl_mlp_predict_noalloc.argtypes = [_P, ctypes.c_int, _P, _P]
+    net = S.Net(seed=6)
+    n, F = 3001, S.N_FEATURES
+    x = np.random.default_rng(8).normal(size=(n, F)).astype(np.float32)
+    want = np.zeros((n, 2), np.float32)
+    assert lib.tl_mlp_predict(net.h, n, x.ctypes.data, want.ctypes.data) == 0
+    pad = 2 * n * 4
+    buf = _dev(hip, x.nbytes + 2 * pad)
+    try:
+        for shift in (0, 4, 5 * F * 4 + 8, x.nbytes - 8, -8, 8 - pad, -pad, x.nbytes):
+            rows = buf.value + pad
+            assert hip.hipMemcpy(rows, x.ctypes.data, x.nbytes, 1) == 0
+            assert lib.tl_mlp_predict_noalloc(net.h, n, rows, rows + shift) == 0
+            got = np.zeros((n, 2), np.float32)
+            assert hip.hipMemcpy(got.ctypes.data, rows + shift, got.nbytes, 2) == 0
+            assert np.array_equal(got, want), shift
+    finally:
+        hip.hipFree(buf)
