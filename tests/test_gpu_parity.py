@@ -520,6 +520,23 @@ def test_full_c2_curve_properties(E, oracle):
         assert abs(amp[i] - s * g[7]) <= AMP_RTOL * abs(s * g[7]), i
 
 
+def test_counters_of_a_fill(E):
+    """The last run's counters: every wavefront's tasks and runs, and of its
+    busy time a share in run-table inserts."""
+    c = curve_from_params(golden("c1.npz")["params"])
+    lc = _new(E, c)
+    for groups in (0, 3):
+        E.set_option("fill_workgroups", groups)
+        try:
+            lc.lc_irs(*c.traj())
+        finally:
+            E.set_option("fill_workgroups", 0)
+        st = E.last_stats()
+        assert st["waves"] == 15 * (groups or E.device_info()[1])
+        assert st["tasks"] >= st["runs"] > 10000 and st["evals"] >= 64 * st["runs"]
+        assert 0 < st["insert_ms"] < st["busy_ms"]
+
+
 def test_scout_options_keep_results(E):
     """Scouts only add labels that merge: without them, with the retry of
     missed scouts off, with the jump shortened on wide runs and with the

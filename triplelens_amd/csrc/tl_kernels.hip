@@ -2155,6 +2155,7 @@ __device__ __forceinline__ bool next_run(const Ray& R, int N, bool limb, RunScan
 // wave are performed in program order; the unlock waits for the wave's LDS
 // operations before it releases the word.
 constexpr int kWorkers = kFillWaves - 1;
+constexpr int kFillStats = 10;   // FillArgs::stats
 constexpr int kFeedMax = 16;     // tasks the manager brings in at a time
 constexpr int kDonateMax = 8;    // tasks the manager queues for other groups at a time
 constexpr int kPoolShare = 16;   // while other groups are idle, workers keep the pool at
@@ -2176,6 +2177,10 @@ struct GroupPool {
 __device__ __forceinline__ int lds_ld(int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, WGS); }
 __device__ __forceinline__ void lds_st(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, WGS);
+}
+template <class T>
+__device__ __forceinline__ T lds_add(T* p, T v) {
+  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, WGS);
 }
 // Waits until the wave's LDS (and scalar) memory operations are done.
 __device__ __forceinline__ void lds_wait() {
@@ -2492,6 +2497,7 @@ struct Worker {
   unsigned accCnt;
   long long accBits;        // (lane) brightness bits, kMagicBits included per pixel
   unsigned nTasks, nIns, nDup, nScout, nScoutRuns, steps;
+  unsigned insTicks;        // in run-table inserts, of one task in kTimedTasks
   bool landed;              // the scout task found a run (new or known)
 };
 
@@ -2614,6 +2620,20 @@ __device__ __forceinline__ int scout_jump_for(ArgPtr A, int w) {
   return j < lo ? lo : (int)j;
 }
 
+// insert_run for the wave's position.  The inserts of one task in kTimedTasks
+// are timed.
+constexpr unsigned kTimedTasks = 64;
+__device__ __forceinline__ int insert_timed(Worker& W, int b, int row, int xl, int xr, int label,
+                                            int& other) {
+  const bool timed = W.nTasks % kTimedTasks == 0;
+  unsigned t0 = 0;
+  if (__builtin_expect(timed, 0)) t0 = (unsigned)__builtin_amdgcn_s_memrealtime();
+  const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, xl, xr, label, other);
+  if (__builtin_expect(timed, 0))
+    W.insTicks += (unsigned)__builtin_amdgcn_s_memrealtime() - t0;
+  return ins;
+}
+
 // What a task scans: a row between columns, in one or two pieces around known
 // pixels.
 struct Scan {
@@ -2648,7 +2668,7 @@ __device__ __forceinline__ bool handle_run(Worker& W, const Scan& S, int f1, int
   }
   labelOut = label;
   int other = 0;
-  const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, xl, xr, label, other);
+  const int ins = insert_timed(W, b, row, xl, xr, label, other);
   if (__builtin_expect(ins != kInsNew, 0)) {
     if (ins == kInsFull) {
       flag_point(W.A, W.gp, kFlagHashFull);
@@ -2826,7 +2846,7 @@ __device__ __forceinline__ void sweep_rows(Worker& W) {
     int nl = 0, nr = 0;
     while (next_run_in<MODE, LIMB>(W.R, N, Q)) {
       int other = 0;
-      const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, Q.xl, Q.xr, label, other);
+      const int ins = insert_timed(W, b, row, Q.xl, Q.xr, label, other);
       if (__builtin_expect(ins != kInsNew, 0)) {
         if (ins == kInsFull) {
           flag_point(W.A, W.gp, kFlagHashFull);
@@ -3155,6 +3175,8 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
   __shared__ Task outs[kWorkers][kOutCap];
   __shared__ Task backs[kWorkers][2];
   __shared__ int spare[kWorkers][64];
+  __shared__ unsigned long long sums[kFillStats];
+  __shared__ int left;  // workers that have not added theirs
   const int ln = __lane_id();
   const int wave = uni((int)(threadIdx.x / 64));
   const long long t0 = (long long)__builtin_amdgcn_s_memrealtime();
@@ -3166,7 +3188,9 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
     G->count = 0;
     G->done = 0;
     G->hungry = 0;
+    left = kWorkers;
   }
+  if (threadIdx.x < kFillStats) sums[threadIdx.x] = 0;
   __syncthreads();
   if (wave == 0) {
     unsigned long long polls = 0;
@@ -3195,7 +3219,7 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
   W.accLabel = -1;
   W.accCnt = 0;
   W.accBits = 0;
-  W.nTasks = W.nIns = W.nDup = W.nScout = W.nScoutRuns = W.steps = 0;
+  W.nTasks = W.nIns = W.nDup = W.nScout = W.nScoutRuns = W.steps = W.insTicks = 0;
   const bool newest = A.poolNewest != 0;
   unsigned idlePolls = 0;
   unsigned long long idleTicks = 0;
@@ -3279,16 +3303,16 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
   flush_acc(W);
   const unsigned long long busyTicks =
       (unsigned long long)((long long)__builtin_amdgcn_s_memrealtime() - t0) - idleTicks;
+  // The workgroup's counters go to the launch's from its last worker: 3840
+  // waves that add to one address take turns (a 17-point curve 1.62 -> 1.37 ms
+  // with ten counters added by 256).
   if (ln == 0) {
-    atomicAdd(&A.stats[0], (unsigned long long)W.nTasks);
-    atomicAdd(&A.stats[1], 64ull * W.steps);
-    atomicAdd(&A.stats[2], (unsigned long long)W.nIns);
-    atomicAdd(&A.stats[3], (unsigned long long)W.nDup);
-    atomicAdd(&A.stats[4], busyTicks);
-    atomicAdd(&A.stats[6], (unsigned long long)idlePolls);
-    atomicAdd(&A.stats[7], 1ull);
-    atomicAdd(&A.stats[8], (unsigned long long)W.nScout);
-    atomicAdd(&A.stats[9], (unsigned long long)W.nScoutRuns);
+    const unsigned long long v[kFillStats] = {W.nTasks, 64ull * W.steps, W.nIns, W.nDup, busyTicks,
+                                              (unsigned long long)W.insTicks * kTimedTasks,
+                                              idlePolls, 1, W.nScout, W.nScoutRuns};
+    for (int k = 0; k < kFillStats; k++) lds_add(&sums[k], v[k]);
+    if (lds_add(&left, -1) == 1)
+      for (int k = 0; k < kFillStats; k++) atomicAdd(&A.stats[k], lds_add(&sums[k], 0ull));
   }
 }
 
@@ -3349,7 +3373,7 @@ __global__ void fill_reset_kernel(FillArgs A) {
     *A.seedNext = 0;
     *A.labelNext = A.nBatch;
     *A.abortFlag = 0;
-    for (int k = 0; k < 10; k++) A.stats[k] = 0;
+    for (int k = 0; k < kFillStats; k++) A.stats[k] = 0;
   }
 }
 
