@@ -207,8 +207,8 @@ int lcirs_batch_fill_positions(int n, void** lcs, const int* counts, const int* 
 
 /* Engine counters of the last run: out[0] fill tasks, out[1] evaluated
  * pixels, out[2] runs inserted, out[3] duplicate runs, out[4]
- * milliseconds from the solve lists to the last seed launch (with the fills
- * that ran beside the seed search), out[5] fill milliseconds (sum over launches), out[6] fill
+ * milliseconds of the seed search's launches behind the solve lists (in a
+ * chunked serial search with the gaps between them), out[5] fill milliseconds (sum over launches), out[6] fill
  * launches, out[7] total milliseconds of the last run, out[8] summed busy
  * time of the fill's wavefronts (ms), out[9] of that, time in run-table
  * inserts (ms, from one task in 64), out[10] idle polls, out[11] wavefronts of the last launch,

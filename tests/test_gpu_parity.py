@@ -537,6 +537,27 @@ def test_counters_of_a_fill(E):
         assert 0 < st["insert_ms"] < st["busy_ms"]
 
 
+def test_seed_time_without_the_fills(E, oracle):
+    """The seed search's time in a run whose fills go on between its launches
+    is that of the seed search alone (which the fills beside it slow down by a
+    third), not the time until its last launch (twice that)."""
+    from triplelens_amd import workloads as W
+    c = replace(W.c2(seed=2, ca_fn=lambda *p: oracle.ccc(*p)[1]), n_points=400)
+    lc = _new(E, c)
+    E.set_option("spec_segment", 7)
+    try:
+        alone, both = [], []
+        for _ in range(5):
+            lc.find_seeds(*c.traj())
+            alone.append(E.last_stats()["seed_ms"])
+            lc.lc_irs(*c.traj())
+            both.append(E.last_stats()["seed_ms"])
+    finally:
+        E.set_option("spec_segment", 192)
+    assert E.last_stats()["fill_launches"] > 1
+    assert np.median(both) < 1.6 * np.median(alone)
+
+
 def test_scout_options_keep_results(E):
     """Scouts only add labels that merge: without them, with the retry of
     missed scouts off, with the jump shortened on wide runs and with the

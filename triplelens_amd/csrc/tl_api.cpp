@@ -298,6 +298,7 @@ struct Engine {
   std::vector<hipEvent_t> seedEvents;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evTrial0 = nullptr, evTrial1 = nullptr, evRing0 = nullptr, evRing1 = nullptr;
+  hipEvent_t evSeed0 = nullptr;   // before a seed launch on its own
   DBuf<TrigTable> dTrig;
   DBuf<CurveDev> dCurves;
   DBuf<cx> dCaus;
@@ -339,7 +340,7 @@ struct Engine {
   static constexpr int kSpecFlight = 16;
   int* hSpecInfo = nullptr;
   size_t hSpecCap = 0;  // ints a slot holds
-  hipEvent_t specEvents[kSpecFlight] = {};
+  hipEvent_t specBegin[kSpecFlight] = {}, specEvents[kSpecFlight] = {};
   SpecArgs specArgs{};
   SeedArgs specSeed{};
   int specQueued = 0, specSeen = -1;  // last segment launched, last one looked at
@@ -416,15 +417,16 @@ struct Engine {
     HIPCHK(hipStreamCreateWithFlags(&sstream, hipStreamNonBlocking));
     HIPCHK(hipEventCreate(&ev0));
     HIPCHK(hipEventCreate(&ev1));
-    for (hipEvent_t* e : {&evTrial0, &evTrial1, &evRing0, &evRing1}) HIPCHK(hipEventCreate(e));
+    for (hipEvent_t* e : {&evTrial0, &evTrial1, &evRing0, &evRing1, &evSeed0})
+      HIPCHK(hipEventCreate(e));
     dTrig.ensure(1);
     HIPCHK(hipMemcpy(dTrig.p, &trig(), sizeof(TrigTable), hipMemcpyHostToDevice));
     ready = true;
   }
 
-  float elapsed() {
+  static float elapsed(hipEvent_t from, hipEvent_t to) {
     float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, ev0, ev1));
+    HIPCHK(hipEventElapsedTime(&ms, from, to));
     return ms;
   }
 
@@ -583,8 +585,9 @@ void Engine::spec_start(std::vector<CurveDev>& hc, const std::vector<int>& point
                          hipHostMallocDefault));
     hSpecCap = 2 * words;
   }
-  for (hipEvent_t& e : specEvents)
-    if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  for (int k = 0; k < kSpecFlight; k++)
+    for (hipEvent_t* e : {&specBegin[k], &specEvents[k]})
+      if (!*e) HIPCHK(hipEventCreate(e));
   // piece 0 of every curve starts from a known state
   std::vector<int> info(words, 1);
   info[0] = info[1] = info[2] = 0;
@@ -624,6 +627,7 @@ void Engine::spec_start(std::vector<CurveDev>& hc, const std::vector<int>& point
   specFailed = false;
   specQueued = 0;
   specSeen = -1;
+  HIPCHK(hipEventRecord(specBegin[0], sstream));
   HIPCHK((hipError_t)launch_spec(specSeed, sp, sstream));
   spec_copy_info();
   spec_look(true);
@@ -655,6 +659,7 @@ void Engine::spec_queue() {
   const int groups = std::min(1024, std::max(1, (specActive + kWalkWaves - 1) / kWalkWaves));
   while (!spec_done() && !specFailed && specQueued - specSeen < flight) {
     specQueued++;
+    HIPCHK(hipEventRecord(specBegin[specQueued % kSpecFlight], sstream));
     HIPCHK((hipError_t)launch_spec_segment(specSeed, specArgs, specQueued, groups, sstream));
     spec_copy_info();
   }
@@ -675,6 +680,7 @@ bool Engine::spec_look(bool wait) {
     }
     specSeen++;
     any = true;
+    stats.seedMs += elapsed(specBegin[slot], specEvents[slot]);
     const int* info = hSpecInfo + (size_t)slot * hSpecCap;
     specFailed = info[0] != 0;
     specActive = info[1 + (specSeen & 1)];
@@ -970,6 +976,7 @@ void Engine::run(Job& job) {
       sa.pieceBase = nullptr;
       sa.pieceStart = nullptr;
       sa.pieces = nullptr;
+      HIPCHK(hipEventRecord(evSeed0, sstream));
       HIPCHK((hipError_t)launch_seed(sa, sstream));
       HIPCHK(hipEventRecord(evSeed[0], sstream));
       launch_ring();
@@ -1001,6 +1008,7 @@ void Engine::run(Job& job) {
                           hipMemcpyHostToDevice, stream));
     sa.pieces = dSpecList.p;
     sa.nPieces = (int)list.size();
+    HIPCHK(hipEventRecord(evSeed0, stream));
     HIPCHK((hipError_t)launch_seed(sa, stream));
     HIPCHK(hipEventRecord(evSeed[0], stream));
     if (last) {
@@ -1024,6 +1032,7 @@ void Engine::run(Job& job) {
     HIPCHK(hipMemcpyAsync(cost.data(), dCost.p, nPts * sizeof(float), hipMemcpyDeviceToHost,
                           stream));
     HIPCHK(hipStreamSynchronize(stream));
+    if (spec) stats.seedMs += elapsed(evSeed0, evSeed[0]);
   }
   // the stage's positions, largest predicted cost first, in launches of
   // about kRunBudget predicted runs (groups of kGroupPoints positions with a
@@ -1192,7 +1201,7 @@ void Engine::run(Job& job) {
         HIPCHK((hipError_t)launch_resolve(fa, labelCap, dPtCount.p, dPtSum.p, stream));
         HIPCHK(hipStreamSynchronize(stream));
       }
-      stats.fillMs += elapsed();
+      stats.fillMs += elapsed(ev0, ev1);
       stats.fillLaunches += 1;
       std::vector<unsigned long long> sync(7 * kLine);
       HIPCHK(hipMemcpy(sync.data(), dSync.p, sync.size() * sizeof(unsigned long long),
@@ -1255,11 +1264,9 @@ void Engine::run(Job& job) {
     // disk samples behind it on the seed stream are waited for after the
     // other results are copied back
     HIPCHK(hipEventSynchronize(evSeed[nChunks - 1]));
-    float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, evTrial1, evSeed[nChunks - 1]));
-    stats.seedMs = ms;
-    HIPCHK(hipEventElapsedTime(&ms, evTrial0, evTrial1));
-    stats.trialMs = ms;
+    if (!spec)
+      stats.seedMs += elapsed(stats.specFallback ? evSeed0 : evTrial1, evSeed[nChunks - 1]);
+    stats.trialMs = elapsed(evTrial0, evTrial1);
     std::vector<RootChain> chains(nc);
     HIPCHK(hipMemcpy(chains.data(), dChain.p, nc * sizeof(RootChain), hipMemcpyDeviceToHost));
     for (int k = 0; k < nc; k++) {
@@ -1339,9 +1346,7 @@ void Engine::run(Job& job) {
   // curves that asked for them
   HIPCHK(hipStreamSynchronize(sstream));
   if (anyRing) {
-    float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, evRing0, evRing1));
-    stats.ringMs = ms;
+    stats.ringMs = elapsed(evRing0, evRing1);
     ringHost.resize((size_t)nPts * kRingSamples);
     crossHost.resize(nPts);
     rootsHost.resize((size_t)nPts * 10);
