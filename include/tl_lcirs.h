@@ -275,6 +275,11 @@ int tl_div_selftest(long long n, unsigned long long seed);
  * are left out; bad[4] is their number among the random ones.  Returns 0, or -1 with tl_last_error().  No counterpart in the reference. */
 int tl_roots_selftest(long long n, unsigned long long seed, long long bad[5]);
 
+/* Workgroups a fill has on a device of `cus` compute units while repair chains
+ * of the seed search run beside it, the chains in one workgroup (oneGroup) or
+ * in several.  No counterpart in the reference (test access). */
+int tl_fill_groups_beside(int cus, int oneGroup);
+
 /* Engine settings: name/value pairs ("fill_workgroups", "probe_limit",
  * "queue_log2", "scout_rows", "scout_jump", "scout_retry", "scout_width",
  * "scout_share", "share_rays", "use_graph", "leap_every", "leap_jumps", "poll_backoff",

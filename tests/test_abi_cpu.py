@@ -111,6 +111,18 @@ def test_branch_free_complex_routines_match_general_ones():
         assert lib.tl_math_selftest(300000, seed) == 0
 
 
+@pytest.mark.parametrize("cus", [1, 2, 8, 16, 20, 32, 38, 64, 128, 256, 304])
+def test_fill_beside_repair_chains_keeps_most_of_the_device(lib, cus):
+    """The compute units left to the repair chains are a share of the device:
+    a partition of a few dozen units still fills with most of them."""
+    for one in (0, 1):
+        groups = lib.tl_fill_groups_beside(cus, one)
+        assert max(1, cus // 2) <= groups <= max(1, cus - 1)
+        assert groups >= 0.8 * cus or cus < 16
+    if cus == 256:
+        assert (lib.tl_fill_groups_beside(cus, 1), lib.tl_fill_groups_beside(cus, 0)) == (248, 224)
+
+
 def test_new_entry_points_reject_bad_arguments(lib):
     """The clone, batched seed search and fills of chosen positions check
     their arguments before any GPU work and report through tl_last_error."""

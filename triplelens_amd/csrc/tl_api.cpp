@@ -988,12 +988,8 @@ void Engine::run(Job& job) {
     nWg = nWgAll;
     if (!last) {
       spec_queue();
-      // workgroups are dealt to the eight XCDs, and in each to its four
-      // shader engines, in turn, and wait for room there: with a compute unit
-      // less on each XCD a launch of one workgroup still starts at once beside
-      // the fill, but the 64-workgroup resolution waited for its end (40 ms)
-      const int keep = nc == 1 && specActive <= kWalkWaves ? 8 : 32;
-      if (opt.fillWorkgroups <= 0) nWg = std::max(1, nWgAll - keep);
+      if (opt.fillWorkgroups <= 0)
+        nWg = fill_groups_beside(nWgAll, nc == 1 && specActive <= kWalkWaves);
     }
     list.clear();
     for (int k = 0; k < nc; k++) {
@@ -2155,6 +2151,8 @@ int tl_math_selftest(int n, unsigned long long seed) {
   }
   return bad;
 }
+
+int tl_fill_groups_beside(int cus, int oneGroup) { return fill_groups_beside(cus, oneGroup != 0); }
 
 int tl_last_stats(double* out) {
   g_err.clear();

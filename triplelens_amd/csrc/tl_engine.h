@@ -242,6 +242,18 @@ struct FillArgs {
                               // cycles
 };
 
+// Workgroups (one per compute unit) of a fill beside running repair chains.
+// Workgroups are dealt to the XCDs, and in each to its shader engines, in turn,
+// and wait for room there: on 256 compute units, eight to a shader engine and
+// 32 to an XCD, a launch of one workgroup still started at once beside a fill
+// that left a unit of each XCD, but the resolution of 64 workgroups waited for
+// the fill's end (40 ms) unless it left one of each shader engine.  A smaller
+// device keeps the same shares.
+inline int fill_groups_beside(int cus, bool oneGroup) {
+  const int keep = oneGroup ? (cus + 31) / 32 : (cus + 7) / 8;
+  return cus - keep > 1 ? cus - keep : 1;
+}
+
 // Host-side launchers (tl_kernels.hip).  All return hipError_t as int.
 int launch_trials(const TrialArgs& a, hipStream_t s);
 // The records and fresh roots of the first nSolves solves of the pool (after
