@@ -51,6 +51,7 @@ struct Dev {
     if (k <= n) return;
     if (p) MCHK(hipFree(p));
     p = nullptr;
+    n = 0;  // (should the allocation fail)
     MCHK(hipMalloc(&p, std::max<size_t>(k, 1) * sizeof(T)));
     n = k;
   }
@@ -60,6 +61,10 @@ struct Dev {
     n = 0;
   }
 };
+
+// Rows whose device buffers a network keeps between calls: those of one piece
+// of an inference, 4 MiB.
+constexpr int kKeepRows = 1 << 16;
 
 struct Mlp {
   std::mutex mu;
@@ -81,6 +86,14 @@ struct Mlp {
     for (auto& d : dz) d.release();
     perm.release();
     if (stream) (void)hipStreamDestroy(stream);
+  }
+
+  // Gives back the rows of a training set beyond what an inference keeps.
+  void drop_rows() {
+    if (xin.n > (size_t)kKeepRows * kMlpIn) xin.release();
+    if (y.n > (size_t)kKeepRows) y.release();
+    if (perm.n > (size_t)kKeepRows) perm.release();
+    if (loss.n > (size_t)kKeepRows) loss.release();
   }
 
   MlpWeights weights() const { return {pbF.p, pbB.p, p.p, mean.p, scale.p}; }
@@ -240,7 +253,7 @@ int tl_mlp_predict(void* h, int n, const float* x, float* out) {
     Mlp* M = checked(h);
     if (n < 0 || (n > 0 && (!x || !out))) throw std::invalid_argument("bad arguments");
     std::lock_guard<std::mutex> lock(M->mu);
-    const int chunk = 1 << 16;
+    const int chunk = kKeepRows;
     const size_t most = (size_t)std::min(n, chunk);
     M->xin.ensure(most * kMlpIn);
     M->out.ensure(most * kMlpOut);
@@ -358,6 +371,7 @@ int tl_mlp_train(void* h, int n, const float* x, const float* y, int steps, int 
       MCHK(hipMemcpyAsync(losses, M->loss.p, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost,
                           M->stream));
     MCHK(hipStreamSynchronize(M->stream));
+    M->drop_rows();
     return 0;
   });
 }
