@@ -200,6 +200,30 @@ __device__ __forceinline__ bool lag_general(const cx (&b)[M + 1], cx& x, int i,
   return false;
 }
 
+// A polynomial whose constant term is NaN in both parts (a source position
+// that is not finite) has NaN sums at every x: no comparison accepts x, and
+// lag_general's step is that of a vanishing denominator.  The iterations from i
+// to the last, with its results (the fresh solves of one such position took
+// 26.7 ms by lag_general, and take 9.8).  lag_wave goes on by lag_general: its
+// code with this branch cost every chain 2%.
+__device__ __forceinline__ bool lag_is_lost(cx p0) {
+  return p0.re != p0.re && p0.im != p0.im;
+}
+__device__ inline bool lag_lost(cx& x, int i, const TrigTable* trig, bool& oob) {
+  for (; i <= kLagMaxIt; i++) {
+    const cx dx = cscale(mk(trig->c[i], trig->s[i]), 1.0 + cabs_(x));
+    const cx x1 = csub(x, dx);
+    if (x.re == x1.re && x.im == x1.im) return true;
+    if (i % kLagMT) {
+      x = x1;
+    } else {
+      oob |= i / kLagMT >= 8;
+      x = lag_kick(x, dx, i);
+    }
+  }
+  return false;
+}
+
 // One iteration of Laguerre::laguerre at x, in the parts that its two drivers
 // below share.
 //
@@ -335,6 +359,11 @@ __device__ __forceinline__ bool lag_lane(const cx (&p)[M + 1], cx& x, cx (&b)[M 
     }
     keep(x.re);  // the general iteration shares nothing with the code above
     keep(x.im);
+    if (lag_is_lost(p[0])) {
+      const bool done = lag_lost(x, i, trig, oob);
+      horner_sums<M>(p, x, b);
+      return done;
+    }
     if (lag_general<M>(b, x, i, trig, oob)) return true;
   }
   horner_sums<M>(p, x, b);  // not converged: the sums where it stopped
