@@ -275,6 +275,11 @@ int tl_div_selftest(long long n, unsigned long long seed);
  * are left out; bad[4] is their number among the random ones.  Returns 0, or -1 with tl_last_error().  No counterpart in the reference. */
 int tl_roots_selftest(long long n, unsigned long long seed, long long bad[5]);
 
+/* Elements of `elementBytes` bytes that a device buffer of `have` elements is
+ * given when it has to hold `need` > have.  No counterpart in the reference
+ * (test access). */
+long long tl_grown_elements(long long have, long long need, long long elementBytes);
+
 /* Workgroups a fill has on a device of `cus` compute units while repair chains
  * of the seed search run beside it, the chains in one workgroup (oneGroup) or
  * in several.  No counterpart in the reference (test access). */

@@ -123,6 +123,23 @@ def test_fill_beside_repair_chains_keeps_most_of_the_device(lib, cus):
         assert (lib.tl_fill_groups_beside(cus, 1), lib.tl_fill_groups_beside(cus, 0)) == (248, 224)
 
 
+@pytest.mark.parametrize("size", [4, 16, 160])
+def test_device_buffers_grow_by_a_bounded_share(lib, size):
+    """A buffer's first size is the one asked for; one that grows gets a
+    quarter more than it had, at most 64 MiB more than it needs."""
+    lib.tl_grown_elements.argtypes = [ctypes.c_longlong] * 3
+    lib.tl_grown_elements.restype = ctypes.c_longlong
+    for have in (0, 1, 7, 1000, 10 ** 6, 10 ** 9, 2 * 10 ** 9):
+        for need in (have + 1, have + have // 8 + 1, 2 * have + 5):
+            got = lib.tl_grown_elements(have, need, size)
+            assert need <= got <= max(need, have + have // 4)
+            assert (got - need) * size <= 64 << 20
+            if have == 0:
+                assert got == need
+            elif have < 10 ** 5:
+                assert got == max(need, have + have // 4)
+
+
 def test_new_entry_points_reject_bad_arguments(lib):
     """The clone, batched seed search and fills of chosen positions check
     their arguments before any GPU work and report through tl_last_error."""

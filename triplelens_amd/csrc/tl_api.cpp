@@ -205,12 +205,11 @@ template <class T>
 struct DBuf {
   T* p = nullptr;
   size_t n = 0;
-  // A buffer that has to grow does so by a quarter at least (the sizes of a
-  // fill's stages vary a little from run to run).  Giving the old one back
-  // waits for the whole device: with `later`, that is left to the caller.
+  // Giving the old buffer back waits for the whole device: with `later`, that
+  // is left to the caller.
   void ensure(size_t k, std::vector<void*>* later = nullptr) {
     if (k <= n) return;
-    size_t want = std::max<size_t>(n ? std::max(k, n + n / 4) : k, 16);
+    const size_t want = std::max<size_t>(grown_elements(n, k, sizeof(T)), 16);
     if (p && later) later->push_back(p);
     else if (p) HIPCHK(hipFree(p));
     p = nullptr;
@@ -2150,6 +2149,10 @@ int tl_math_selftest(int n, unsigned long long seed) {
       bad++;
   }
   return bad;
+}
+
+long long tl_grown_elements(long long have, long long need, long long elementBytes) {
+  return (long long)grown_elements((size_t)have, (size_t)need, (size_t)elementBytes);
 }
 
 int tl_fill_groups_beside(int cus, int oneGroup) { return fill_groups_beside(cus, oneGroup != 0); }

@@ -242,6 +242,17 @@ struct FillArgs {
                               // cycles
 };
 
+// Elements of a buffer of `have` that has to hold `need` > have: a buffer that
+// grows does so by a quarter (the sizes of a fill's stages vary a little from
+// run to run, and giving a buffer back waits for the device), at most 64 MiB
+// beyond the need.
+inline size_t grown_elements(size_t have, size_t need, size_t elementBytes) {
+  const size_t spare = (64u << 20) / elementBytes;
+  const size_t quarter = have + have / 4;
+  if (quarter <= need) return need;
+  return quarter - need < spare ? quarter : need + spare;
+}
+
 // Workgroups (one per compute unit) of a fill beside running repair chains.
 // Workgroups are dealt to the XCDs, and in each to its shader engines, in turn,
 // and wait for room there: on 256 compute units, eight to a shader engine and
