@@ -305,7 +305,7 @@ int tl_device_info(char* name, int len, int* cus);
 #define TL_FLAG_LABEL_FULL 8u
 #define TL_FLAG_QUEUE_FULL 16u
 #define TL_FLAG_TIMEOUT 32u
-#define TL_FLAG_ROW_OVERFLOW 64u
+#define TL_FLAG_ROW_OVERFLOW 64u /* not set any more */
 /* Informational: a Laguerre iteration of the point's solves reached step 64,
  * where the reference reads its 8-entry fractional-step table past the end
  * (laguerre.cc:22,92), i.e. heap memory: the reference's result at this point

@@ -12,7 +12,6 @@ constexpr int kCccLen = 500;       // critical-curve samples per branch (lcirs.c
 constexpr int kMaxSeeds = 64;      // seeds kept per source position
 constexpr int kGroupPoints = 16384;  // source positions per run-table group (14-bit key
                                      // field); a fill launch holds any number of groups
-constexpr int kMaxCover = 16;      // known runs read per row lookup
 constexpr int kFillWaves = 16;     // waves per fill workgroup: 1 manager + 15 workers, four
                                    // waves per SIMD
 constexpr int kFillThreads = 64 * kFillWaves;
@@ -29,7 +28,7 @@ enum : uint32_t {
   kFlagLabelFull = 8u,     // label table full
   kFlagQueueFull = 16u,    // task queue full
   kFlagTimeout = 32u,      // the fill launch hit its time limit
-  kFlagRowOverflow = 64u,  // more than kMaxCover runs in one row (work repeated, result exact)
+                           // (64: TL_FLAG_ROW_OVERFLOW, which nothing sets any more)
   kFlagKickTable = 128u,   // a Laguerre iteration of the point's solves reached step 64, where
                            // the reference reads its 8-entry fractional-step table past the
                            // end (laguerre.cc:22,92): heap memory, so the reference's result

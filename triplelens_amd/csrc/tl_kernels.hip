@@ -71,14 +71,8 @@ __device__ __forceinline__ double unid(double v) {
 }
 
 // ---------------------------------------------------------------------------
-// Pixel <-> plane mapping (lcirs.cc:355-378)
+// Plane -> pixel mapping (lcirs.cc:367-378; pixel -> plane is a row's own, Ray)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double nx_to_x(const CurveDev& C, long long nx) {
-  return C.blx + C.step * (double)nx;
-}
-__device__ __forceinline__ double ny_to_y(const CurveDev& C, long long ny) {
-  return C.bly + C.step * (double)ny;
-}
 // (long)((x - BL) * N / L + 0.5), with the operand clamped so that the
 // conversion is defined for any root.
 __device__ __forceinline__ int to_pixel(double v, double bl, double Nd, double L) {
@@ -341,11 +335,6 @@ struct SolveWalk {
     fetch();
   }
 };
-
-__device__ __forceinline__ double wave_sum_d(double v) {
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // Seed pixels of the images in `m` (root order), appended at out[cnt..].
 __device__ __forceinline__ void emit_seeds(const CurveDev& C, const cx& chainv,

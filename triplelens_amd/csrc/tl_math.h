@@ -137,7 +137,6 @@ TL_HD double hyp_sel(double x, double y) {
   h -= (t1 + t2) / (2.0 * h);
   return h;
 }
-TL_HD double cabs_sel(cx a) { return hyp_sel(a.re, a.im); }
 
 // Complex square root, glibc csqrt algorithm for finite operands.
 TL_HD cx csqrt_(cx z) {
