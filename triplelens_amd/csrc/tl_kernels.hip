@@ -71,7 +71,7 @@ __device__ __forceinline__ double unid(double v) {
 }
 
 // ---------------------------------------------------------------------------
-// Plane -> pixel mapping (lcirs.cc:367-378; pixel -> plane is a row's own, Ray)
+// Plane -> pixel mapping (lcirs.cc:355-378; pixel -> plane is formed where a row is scanned)
 // ---------------------------------------------------------------------------
 // (long)((x - BL) * N / L + 0.5), with the operand clamped so that the
 // conversion is defined for any root.
@@ -486,7 +486,7 @@ __global__ void __launch_bounds__(64) trial_poly_kernel(TrialArgs a, int nSolves
 // degree is a template argument).
 // The deflation steps J..1 of Laguerre::solveRoots (laguerre.cc:103-167) for a
 // polynomial of degree DEG: the root found at step J goes to roots[DEG - J].
-template <int DEG, int J>
+template <int DEG, int J, bool LOST = false>
 __device__ __forceinline__ void lane_deflate(const cx (&p)[J + 1], const cx* init, bool withInit,
                                              cx* roots, const TrigTable* trig, bool& oob) {
   cx x = withInit ? init[J] : mk(kLagEps, kLagEps);
@@ -496,7 +496,7 @@ __device__ __forceinline__ void lane_deflate(const cx (&p)[J + 1], const cx* ini
     roots[DEG - 1] = x;
   } else {
     cx b[J + 1];
-    if (!lag_lane<J>(p, x, b, trig, oob) && withInit) {
+    if (!lag_lane<J, LOST>(p, x, b, trig, oob) && withInit) {
       x = mk(kLagEps, kLagEps);
       horner_sums<J>(p, x, b);
     }
@@ -504,19 +504,20 @@ __device__ __forceinline__ void lane_deflate(const cx (&p)[J + 1], const cx* ini
     cx q[J];
 #pragma unroll
     for (int j = 0; j < J; j++) q[j] = b[j + 1];
-    lane_deflate<DEG, J - 1>(q, init, withInit, roots, trig, oob);
+    lane_deflate<DEG, J - 1, LOST>(q, init, withInit, roots, trig, oob);
   }
 }
 // solveRoots: the deflation, then each root polished on the full polynomial
 // in root order (the roots rotate through roots[0], so one copy of the
 // polishing code serves all of them).
+template <bool LOST = false>
 __device__ __forceinline__ void lane_solve(const cx (&c)[11], const cx* init, bool withInit,
                                            cx* roots, const TrigTable* trig, bool& oob) {
-  lane_deflate<10, 10>(c, init, withInit, roots, trig, oob);
+  lane_deflate<10, 10, LOST>(c, init, withInit, roots, trig, oob);
 #pragma unroll 1
   for (int j = 0; j < 10; j++) {
     cx x = roots[0], b[11];
-    lag_lane<10>(c, x, b, trig, oob);
+    lag_lane<10, LOST>(c, x, b, trig, oob);
 #pragma unroll
     for (int k = 0; k < 9; k++) roots[k] = roots[k + 1];
     roots[9] = x;
@@ -537,7 +538,7 @@ __global__ void __launch_bounds__(64) solve_prep_kernel(TrialArgs a, int nSolves
   const cx zeta = rec[kRecZeta / 2];
   cx x = mk(0.0, 0.0), b[11];
   bool oob = false;
-  if (!lag_lane<10>(c, x, b, a.trig, oob)) {
+  if (!lag_lane<10, true>(c, x, b, a.trig, oob)) {
     x = mk(kLagEps, kLagEps);
     horner_sums<10>(c, x, b);
   }
@@ -547,7 +548,7 @@ __global__ void __launch_bounds__(64) solve_prep_kernel(TrialArgs a, int nSolves
   int fl = oob ? kRecOobFirst : 0;
   cx roots[10];
   oob = false;
-  lane_solve(c, nullptr, false, roots, a.trig, oob);
+  lane_solve<true>(c, nullptr, false, roots, a.trig, oob);
   if (oob) fl |= kRecOobFresh;
 #pragma unroll
   for (int k = 0; k < 10; k++) {

@@ -204,8 +204,8 @@ __device__ __forceinline__ bool lag_general(const cx (&b)[M + 1], cx& x, int i,
 // that is not finite) has NaN sums at every x: no comparison accepts x, and
 // lag_general's step is that of a vanishing denominator.  The iterations from i
 // to the last, with its results (the fresh solves of one such position took
-// 26.7 ms by lag_general, and take 9.8).  lag_wave goes on by lag_general: its
-// code with this branch cost every chain 2%.
+// 26.7 ms by lag_general, and take 9.8).  The chains and the critical curves go
+// on by lag_general: this branch in their code cost every one of them 2%.
 __device__ __forceinline__ bool lag_is_lost(cx p0) {
   return p0.re != p0.re && p0.im != p0.im;
 }
@@ -334,8 +334,9 @@ __device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx&
 // Laguerre::laguerre for a polynomial of degree M >= 2 held in registers,
 // every lane on its own x.  Leaves the Horner sums at the returned x in b,
 // which are the coefficients of the deflated polynomial (b[j + 1] =
-// coefficient j, laguerre.cc:133-139).
-template <int M>
+// coefficient j, laguerre.cc:133-139).  LOST: a polynomial of NaNs is left to
+// lag_lost.
+template <int M, bool LOST = false>
 __device__ __forceinline__ bool lag_lane(const cx (&p)[M + 1], cx& x, cx (&b)[M + 1],
                                          const TrigTable* trig, bool& oob) {
   for (int i = 1; i <= kLagMaxIt; i++) {
@@ -359,7 +360,7 @@ __device__ __forceinline__ bool lag_lane(const cx (&p)[M + 1], cx& x, cx (&b)[M 
     }
     keep(x.re);  // the general iteration shares nothing with the code above
     keep(x.im);
-    if (lag_is_lost(p[0])) {
+    if (LOST && lag_is_lost(p[0])) {
       const bool done = lag_lost(x, i, trig, oob);
       horner_sums<M>(p, x, b);
       return done;
