@@ -1739,11 +1739,11 @@ __global__ void roots_check_kernel(long long n, unsigned long long seed, const d
                                                         e + 1 > 239 ? 239 : e + 1);
       const double ax = max_abs(x, y), ay = min_abs(x, y);
       if (hyp_in_range(ax, ay)) {
-        Edge em = 0;
-        const double h = hyp_near(ax, ay, em);
-        if (em < kEdge) cnt[2] += differ(h, hyp_sel(x, y));
-        const cx c0 = csqrt_near(x, y, em), c1 = csqrt_sel(mk(x, y));
-        if (em < kEdge) cnt[3] += differ(c0.re, c1.re) | differ(c0.im, c1.im);
+        double n1, n2;
+        const double h = hyp_near(ax, ay, n1);
+        if (edge(n1) < kEdge) cnt[2] += differ(h, hyp_sel(x, y));
+        const cx c0 = csqrt_near(x, y, n1, n2), c1 = csqrt_sel(mk(x, y));
+        if (edge(n1) < kEdge && edge(n2) < kEdge) cnt[3] += differ(c0.re, c1.re) | differ(c0.im, c1.im);
         else skipped++;
       }
     }

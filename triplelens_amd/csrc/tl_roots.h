@@ -50,13 +50,19 @@ __device__ __forceinline__ void keep(double& a) { asm volatile("" : "+v"(a)); }
 // iteration with an operand whose mantissa bits 32 to 47 are all ones (one
 // iteration in 10^4) is left to the general form: edge(a) holds these bits,
 // and the largest of several operands' is kEdge where one of them has them.
-// (The maximum of 16-bit halves takes one instruction for three operands: a
-// 200-point chain takes 4.06 ms instead of 3.95 without the check, and 4.12
-// with a shift and both sides of a power of two.)
-typedef unsigned short Edge;
-constexpr Edge kEdge = 0xFFFF;
-__device__ __forceinline__ Edge edge(double a) { return (Edge)__double2hiint(a); }
-__device__ __forceinline__ Edge edge_max(Edge a, Edge b) { return a > b ? a : b; }
+// (Three maxima of 16-bit halves and a sign in lag_step: a 200-point chain
+// takes 3.95 ms instead of 3.91 without the check; with the compiler's packed
+// maxima and a comparison of its own 4.06, with a shift per operand and both
+// sides of a power of two 4.12.)
+constexpr unsigned kEdge = 0xFFFF;
+__device__ __forceinline__ unsigned edge_bits(double a) { return (unsigned)__double2hiint(a); }
+__device__ __forceinline__ unsigned edge(double a) { return edge_bits(a) & 0xFFFFu; }
+// (the lower halves' maximum, its upper half not defined)
+__device__ __forceinline__ unsigned edge_max(unsigned a, unsigned b, unsigned c) {
+  unsigned r;
+  asm("v_max3_u16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
 
 // Reciprocal of b for 2^-900 <= |b| <= 2^900: the hardware estimate r0
 // (e = 1 - b r0, |e| below 2^-22) and one third-order correction
@@ -94,14 +100,13 @@ __device__ __forceinline__ void sqrt_near(double a, double& s, double& h) {
   h = fma(h0, p, h0);
   s = fma(fma(-s1, s1, a), h, s1);
 }
-// hyp_sel for 2^-240 <= ay <= ax <= 2^240 and ay > ax 2^-54, if `em` (raised to
-// the edge of the root's operand) stays below kEdge.  (1/w and, in
+// hyp_sel for 2^-240 <= ay <= ax <= 2^240 and ay > ax 2^-54, if the root's
+// operand n (set here) has edge(n) != kEdge.  (1/w and, in
 // csqrt_near, 1/q come from a root's reciprocal by a second-order step, good
 // to 2^-103: of the b of quot_near only k = 1 is left, which is harmless.)
-__device__ __forceinline__ double hyp_near(double ax, double ay, Edge& em) {
+__device__ __forceinline__ double hyp_near(double ax, double ay, double& n) {
   double h, hi;
-  const double n = ax * ax + ay * ay;
-  em = edge_max(em, edge(n));
+  n = ax * ax + ay * ay;
   sqrt_near(n, h, hi);
   const double w = 2.0 * h;
   const double r = fma(hi, fma(-w, hi, 1.0), hi);  // 1 / w
@@ -116,15 +121,14 @@ __device__ __forceinline__ double hyp_near(double ax, double ay, Edge& em) {
 __device__ __forceinline__ bool hyp_in_range(double ax, double ay) {
   return (int(ay >= 0x1p-240) & int(ax <= 0x1p+240) & int(ay > ax * 0x1p-54)) != 0;
 }
-// csqrt_sel for re, im with hyp_in_range(max, min) of their magnitudes, if
-// `em` stays below kEdge.
-__device__ __forceinline__ cx csqrt_near(double re, double im, Edge& em) {
+// csqrt_sel for re, im with hyp_in_range(max, min) of their magnitudes, if the
+// operands n1, n2 of its roots have an edge other than kEdge.
+__device__ __forceinline__ cx csqrt_near(double re, double im, double& n1, double& n2) {
   const double fr = fabs(re);
-  const double d = hyp_near(max_abs(re, im), min_abs(re, im), em);
+  const double d = hyp_near(max_abs(re, im), min_abs(re, im), n1);
   double q, h;
-  const double n = 0.5 * (d + fr);
-  em = edge_max(em, edge(n));
-  sqrt_near(n, q, h);
+  n2 = 0.5 * (d + fr);
+  sqrt_near(n2, q, h);
   h = 2.0 * h;
   const double w = 0.5 * quot_near(im, q, fma(h, fma(-q, h, 1.0), h));
   const bool pos = re > 0.0;
@@ -303,8 +307,9 @@ __device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx&
   const cx g2 = cmul(g, g);
   const cx h = csub(g2, mk(quot_near(xs, denom, rd), quot_near(ys, denom, rd)));
   const cx rad = cscale(csub(cscale(h, md), g2), md - 1.0);
-  Edge em = edge_max(edge(den), edge(denom));
-  const cx sq = csqrt_near(rad.re, rad.im, em);
+  double n1, n2;
+  const cx sq = csqrt_near(rad.re, rad.im, n1, n2);
+  unsigned em = edge_max(edge_bits(den), edge_bits(denom), edge_bits(n1));
   const cx gp = cadd(g, sq), gm = csub(g, sq);
   const double np = cnorm(gp), nm = cnorm(gm);
   const bool minus = np < nm;
@@ -314,7 +319,8 @@ __device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx&
   const double num2 = ce2 ? d.re : d.im, den2 = ce2 ? d.im : d.re;
   const double ratio2 = quot_near(num2, den2, rcp_near(den2));
   const double denom2 = (num2 * ratio2) + den2;
-  em = edge_max(em, edge_max(edge(den2), edge(denom2)));
+  em = edge_max(em, edge_bits(n2), edge_bits(den2));
+  em = edge_max(em, edge_bits(denom2), 0);
   const double rd2 = rcp_near(denom2);
   const double mr = md * ratio2;
   const double qa = quot_near(mr, denom2, rd2), qb = quot_near(md, denom2, rd2);
@@ -322,11 +328,12 @@ __device__ __forceinline__ bool lag_step(const cx (&b)[M + 1], cx x, cx& x1, cx&
   x1 = mk(x.re - (ce2 ? qa : qb), x.im + (ce2 ? qb : qa));
   // (lo bounds den and den2 from below as well; f, s, g and den2 too large for
   // the quotients leave rad out of its range)
-  const double lo = min_abs(min_abs(min_abs(xf, yf), min_abs(xs, ys)), min_abs(num, num2));
+  double lo = min_abs(min_abs(min_abs(xf, yf), min_abs(xs, ys)), min_abs(num, num2));
+  // (negative where the maximum is kEdge: a sign costs no comparison)
+  lo = __builtin_copysign(lo, __hiloint2double((int)(((em & 0xFFFFu) + 1u) << 15), 0));
   const double rx = max_abs(rad.re, rad.im), ry = min_abs(rad.re, rad.im);
   // (ints: a chain of && would be a chain of branches)
   return (int(lo >= kTinyOp) & int(fabs(den) <= kHugeOp) & int(hyp_in_range(rx, ry)) &
-          int(em < kEdge) &
           int(min_abs(np, nm) < max_abs(np, nm) * (1.0 - 1e-12)) &
           (int(x.re != x1.re) | int(x.im != x1.im))) != 0;
 }
