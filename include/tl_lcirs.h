@@ -269,11 +269,13 @@ int tl_div_selftest(long long n, unsigned long long seed);
 /* GPU self-test of the in-range forms the root solver runs against the
  * general ones, to the bit, on n generated operands each over the ranges the
  * solver admits: bad[0] quotients, bad[1] square roots, bad[2] moduli, bad[3]
- * complex square roots whose results differ.  Among the operands are the
- * quotients and roots that lie closest to a rounding boundary.  Operands that
- * the solver leaves to its general iteration (a few that lie just below a power of two)
- * are left out; bad[4] is their number among the random ones.  Returns 0, or -1 with tl_last_error().  No counterpart in the reference. */
-int tl_roots_selftest(long long n, unsigned long long seed, long long bad[5]);
+ * complex square roots, bad[4] Laguerre steps whose results differ.  Among the
+ * operands are the quotients and roots that lie closest to a rounding
+ * boundary.  Operands that the solver leaves to its general iteration (a few
+ * that lie just below a power of two) are left out; bad[5] is their number
+ * among the random ones, and bad[6] that of the steps compared.  Returns 0, or
+ * -1 with tl_last_error().  No counterpart in the reference. */
+int tl_roots_selftest(long long n, unsigned long long seed, long long bad[7]);
 
 /* Elements of `elementBytes` bytes that a device buffer of `have` elements is
  * given when it has to hold `need` > have.  No counterpart in the reference

@@ -378,19 +378,22 @@ def test_in_range_division_equals_ieee_division(E):
 
 
 def test_root_solver_arithmetic_equals_general_forms(E):
-    """tl_roots_selftest: the in-range quotient, square root, modulus and
-    complex square root the root solver runs equal the general ones to the
-    bit over the ranges it admits, at the hardest operands too."""
+    """tl_roots_selftest: the in-range quotient, square root, modulus, complex
+    square root and Laguerre step the root solver runs equal the general ones
+    to the bit over the ranges it admits, at the hardest operands too, and a
+    step does not divide by a mantissa it leaves to the general iteration."""
     lib = E.load()
     lib.tl_roots_selftest.argtypes = [ctypes.c_longlong, ctypes.c_ulonglong,
                                       ctypes.POINTER(ctypes.c_longlong)]
     lib.tl_roots_selftest.restype = ctypes.c_int
-    bad = (ctypes.c_longlong * 5)()
+    bad = (ctypes.c_longlong * 7)()
     for seed in (1, 0x5DEECE66D):
         assert lib.tl_roots_selftest(1 << 24, seed, bad) == 0
-        assert list(bad)[:4] == [0, 0, 0, 0]
+        assert list(bad)[:5] == [0, 0, 0, 0, 0]
+        # three steps each, one in four left out
+        assert bad[6] > 1.5 * (1 << 24)
         # four operands each, one in 2^16 of them below a power of two
-        assert bad[4] < 2 * (4 << 24) / 2 ** 16
+        assert bad[5] < 2 * (4 << 24) / 2 ** 16
 
 
 @pytest.mark.parametrize("u", [0.0, 0.5])

@@ -2086,7 +2086,7 @@ int tl_roots_selftest(long long n, unsigned long long seed, long long* bad) {
     Engine& E = engine();
     std::lock_guard<std::mutex> lock(E.mu);
     E.init();
-    unsigned long long cnt[5] = {0, 0, 0, 0, 0};
+    unsigned long long cnt[7] = {0, 0, 0, 0, 0, 0, 0};
     unsigned long long* d = nullptr;
     double* dh = nullptr;
     auto release = [&] {
@@ -2098,7 +2098,7 @@ int tl_roots_selftest(long long n, unsigned long long seed, long long* bad) {
       HIPCHK(hipMalloc(&dh, hard.size() * sizeof(double)));
       HIPCHK(hipMemcpy(d, cnt, sizeof cnt, hipMemcpyHostToDevice));
       HIPCHK(hipMemcpy(dh, hard.data(), hard.size() * sizeof(double), hipMemcpyHostToDevice));
-      HIPCHK((hipError_t)launch_roots_check(n, seed, dh, (int)hard.size(), d, E.stream));
+      HIPCHK((hipError_t)launch_roots_check(n, seed, dh, (int)hard.size(), E.dTrig.p, d, E.stream));
       HIPCHK(hipStreamSynchronize(E.stream));
       HIPCHK(hipMemcpy(cnt, d, sizeof cnt, hipMemcpyDeviceToHost));
     } catch (...) {
@@ -2106,7 +2106,7 @@ int tl_roots_selftest(long long n, unsigned long long seed, long long* bad) {
       throw;
     }
     release();
-    for (int k = 0; k < 5; k++) bad[k] = (long long)cnt[k];
+    for (int k = 0; k < 7; k++) bad[k] = (long long)cnt[k];
     return 0;
   });
 }

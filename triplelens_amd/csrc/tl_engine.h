@@ -283,11 +283,12 @@ int launch_spec_segment(const SeedArgs& a, const SpecArgs& sp, int segment, int 
 // n generated operand pairs (test access): adds the number of differing results to *bad (device).
 int launch_div_check(long long n, unsigned long long seed, unsigned long long* bad,
                      hipStream_t s);
-// The root solver's in-range quotient, root, modulus and complex root against
-// the general ones (test access): adds the differing results to bad[0..3] and
-// the operands left out to bad[4] (device).  hard: nHard arguments of the root in [1, 4) (device).
+// The root solver's in-range quotient, root, modulus, complex root and step
+// against the general ones (test access): adds the differing results to
+// bad[0..4], the operands left out to bad[5], the steps compared to bad[6]
+// (device).  hard: nHard arguments of the root in [1, 4) (device).
 int launch_roots_check(long long n, unsigned long long seed, const double* hard, int nHard,
-                       unsigned long long* bad, hipStream_t s);
+                       const TrigTable* trig, unsigned long long* bad, hipStream_t s);
 // image_poly for n source positions of one lens on the GPU (test access):
 // zeta[n] in, coef[11 n] out (device pointers).
 int launch_image_poly(const Lens& L, const cx* fixedPoly, const cx* zeta, int n, cx* coef,

@@ -1654,7 +1654,7 @@ int launch_div_check(long long n, unsigned long long seed, unsigned long long* b
 
 // Self-test of the in-range forms the root solver runs (tl_roots.h) against
 // the general ones, to the bit, over the ranges lag_step admits.  Operands that
-// it leaves to the general iteration for their mantissas are left out; bad[4]
+// it leaves to the general iteration for their mantissas are left out; bad[5]
 // counts those among the random ones.
 //   bad[0] quot_near: operands 2^-300 .. 2^300, random, and the quotients
 //          closest to a rounding boundary: A 2^s = M B -+ j for a denominator
@@ -1663,11 +1663,46 @@ int launch_div_check(long long n, unsigned long long seed, unsigned long long* b
 //   bad[1] sqrt_near: 2^-600 .. 2^600, random, and the `nHard` mantissas in
 //          hard, whose roots lie closest to a rounding boundary;
 //   bad[2] hyp_near against hyp_sel, bad[3] csqrt_near against csqrt_sel:
-//          random signs, magnitudes 2^-240 .. 2^240, less than 2^54 apart.
+//          random signs, magnitudes 2^-240 .. 2^240, less than 2^54 apart;
+//   bad[4] lag_step's next point, where it gives one, against lag_general's
+//          from the same Horner sums, and points it gives although a part of
+//          the sums' b[0] that it divides by has edge kEdge (one draw in
+//          four); bad[6] counts the points compared.
+template <int M>
+__device__ __noinline__ void step_check(unsigned long long z, const TrigTable* trig,
+                                        unsigned long long& differing,
+                                        unsigned long long& compared) {
+  auto next = [&z]() {
+    z += 0x9E3779B97F4A7C15ull;
+    unsigned long long x = z;
+    x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+    x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+    return x ^ (x >> 31);
+  };
+  auto val = [&next]() { return ((double)(long long)next()) * 0x1p-63 * (double)(1 << (next() & 7)); };
+  cx b[M + 1];
+  for (int j = 0; j <= M; j++) b[j] = mk(val(), val());
+  const cx x = mk(val(), val());
+  const bool edged = (next() & 3) == 0;
+  if (edged) {
+    // the larger part is the first divisor
+    double& d = fabs(b[0].re) < fabs(b[0].im) ? b[0].im : b[0].re;
+    d = __hiloint2double(__double2hiint(d) | 0xFFFF, __double2loint(d));
+  }
+  cx x1, step, y = x;
+  if (!lag_step<M>(b, x, x1, step)) return;
+  bool oob = false;
+  if (!edged && lag_general<M>(b, y, 1, trig, oob)) return;
+  compared++;
+  if (edged || __double_as_longlong(y.re) != __double_as_longlong(x1.re) ||
+      __double_as_longlong(y.im) != __double_as_longlong(x1.im))
+    differing++;
+}
+
 __global__ void roots_check_kernel(long long n, unsigned long long seed, const double* hard,
-                                   int nHard, unsigned long long* bad) {
+                                   int nHard, const TrigTable* trig, unsigned long long* bad) {
   const long long stride = (long long)gridDim.x * blockDim.x;
-  unsigned long long cnt[4] = {0, 0, 0, 0}, skipped = 0;
+  unsigned long long cnt[5] = {0, 0, 0, 0, 0}, skipped = 0, steps = 0;
   auto differ = [](double x, double y) {
     return __double_as_longlong(x) != __double_as_longlong(y) ? 1ull : 0ull;
   };
@@ -1747,19 +1782,23 @@ __global__ void roots_check_kernel(long long n, unsigned long long seed, const d
         else skipped++;
       }
     }
+    step_check<10>(next(), trig, cnt[4], steps);
+    step_check<5>(next(), trig, cnt[4], steps);
+    step_check<2>(next(), trig, cnt[4], steps);
   }
-  for (int k = 0; k < 4; k++)
+  for (int k = 0; k < 5; k++)
     if (cnt[k]) atomicAdd(&bad[k], cnt[k]);
-  if (skipped) atomicAdd(&bad[4], skipped);
+  if (skipped) atomicAdd(&bad[5], skipped);
+  if (steps) atomicAdd(&bad[6], steps);
 }
 
 int launch_roots_check(long long n, unsigned long long seed, const double* hard, int nHard,
-                       unsigned long long* bad, hipStream_t s) {
+                       const TrigTable* trig, unsigned long long* bad, hipStream_t s) {
   if (n <= 0) return 0;
-  if (!bad || nHard < 0 || (nHard > 0 && !hard)) return (int)hipErrorInvalidValue;
+  if (!bad || !trig || nHard < 0 || (nHard > 0 && !hard)) return (int)hipErrorInvalidValue;
   const long long blocks = (n + 255) / 256;
   hipLaunchKernelGGL(roots_check_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256),
-                     0, s, n, seed, hard, nHard, bad);
+                     0, s, n, seed, hard, nHard, trig, bad);
   return (int)hipGetLastError();
 }
 
