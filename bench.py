@@ -27,8 +27,9 @@ only the plain loop runs and its rate is the value.
 Roofline figures are those of the fill kernel, where the path's arithmetic
 is (43 FP64 operations per counted ray): its launch durations come from HIP
 events around it on the engine's stream, over the plain-IRS timed loop, and
-its HBM traffic per launch from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE
-summary under profiles/.
+its HBM traffic per launch is that of a curve's launches in the committed
+rocprofv3 FETCH_SIZE/WRITE_SIZE summary under profiles/, over their number in
+the timed loop.
 
 The CPU baseline is the reference LightCurveIRS compiled from its own
 sources (oracle/_ref: the parity flags -O2 -ffp-contract=off -mavx, and, as
@@ -131,14 +132,15 @@ def _split(c, parts):
     return out
 
 
-def measured_traffic():
-    """HBM bytes per fill launch from the committed rocprofv3 FETCH_SIZE /
-    WRITE_SIZE summary (scaled by a plain copy kernel's readings), or None."""
+def measured_traffic(launches_per_curve):
+    """HBM bytes per fill launch: those of one curve's fill launches in the
+    committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary (scaled by a plain copy
+    kernel's readings) over the launches of a curve; None without it."""
     path = os.path.join(HERE, "profiles", "fill_kernel_c2_traffic.txt")
     try:
         for line in open(path):
-            if line.startswith("traffic_bytes_per_launch:"):
-                return float(line.split(":")[1])
+            if line.startswith("traffic_bytes_per_curve:"):
+                return float(line.split(":")[1]) / launches_per_curve
     except OSError:
         pass
     return None
@@ -561,7 +563,7 @@ def main(argv=None):
             "peak": FP64_PEAK_TFLOPS,
             "unit": "TFLOP/s",
             "frac": achieved / FP64_PEAK_TFLOPS,
-            "traffic": measured_traffic(),
+            "traffic": measured_traffic(launches / args.steps),
             "kernel": "fill_kernel",
             "kernel_ms": fill_launch_ms,
             "flop_per_ray": FLOP_PER_RAY,

@@ -11,3 +11,12 @@ def test_multi_gpu_refused():
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 2
     assert "one GPU" in r.stderr
+
+
+def test_fill_traffic_is_a_curves_share_per_launch():
+    """The roofline's bytes per launch are the measured bytes of one curve's
+    fill launches over their number."""
+    import bench
+    one = bench.measured_traffic(1)
+    assert one > 1e8
+    assert bench.measured_traffic(3.4) == one / 3.4
