@@ -254,10 +254,11 @@ int lcirs_set_slot_trace(void* lc, const double* xy, long n);
 int tl_image_poly(double a, double b, double th, double m2, double m3, int n, const double* zeta,
                   double* out, int onDevice);
 
-/* Host self-test of the branch-free complex routines the kernels use (modulus,
- * division, square root) against the general ones on n random operand pairs,
- * normal, tiny, huge, zero, infinite and NaN; returns the number of pairs
- * whose results differ in any bit.  No counterpart in the reference. */
+/* Host self-test of the branch-free complex routines (modulus, division, square
+ * root: the kernels' division, and what tl_roots_selftest compares the root
+ * solver's modulus and square root with) against the general ones on n random
+ * operand pairs, normal, tiny, huge, zero, infinite and NaN; returns the number
+ * of pairs whose results differ in any bit.  No counterpart in the reference. */
 int tl_math_selftest(int n, unsigned long long seed);
 
 /* GPU self-test of the root solver's in-range quotient (and square root)
