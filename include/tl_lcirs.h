@@ -211,7 +211,7 @@ int lcirs_batch_fill_positions(int n, void** lcs, const int* counts, const int* 
  * chunked serial search with the gaps between them), out[5] fill milliseconds (sum over launches), out[6] fill
  * launches, out[7] total milliseconds of the last run, out[8] summed busy
  * time of the fill's wavefronts (ms), out[9] of that, time in run-table
- * inserts (ms, from one task in 64), out[10] idle polls, out[11] wavefronts of the last launch,
+ * inserts (ms, from those of one sweep in 16), out[10] idle polls, out[11] wavefronts of the last launch,
  * out[12] scout tasks, out[13] runs found by scouts, out[14] milliseconds
  * of the solve lists and their polynomials (trial kernels), out[15] of the
  * disk samples, out[16] solves (centre and caustic-trial positions),

@@ -1201,7 +1201,7 @@ void Engine::run(Job& job) {
       std::vector<unsigned long long> sync(7 * kLine);
       HIPCHK(hipMemcpy(sync.data(), dSync.p, sync.size() * sizeof(unsigned long long),
                        hipMemcpyDeviceToHost));
-      const unsigned long long* st = sync.data() + 6 * kLine - 2;  // st[2..11] = stats[0..9]
+      const unsigned long long* st = sync.data() + 6 * kLine - 2;  // st[2..12] = stats[0..10]
       const bool aborted = *reinterpret_cast<const int*>(sync.data() + 5 * kLine) != 0;
       std::vector<uint32_t> bflags(nPts);
       HIPCHK(hipMemcpy(bflags.data(), dFlags.p, nPts * sizeof(uint32_t), hipMemcpyDeviceToHost));
@@ -1218,7 +1218,8 @@ void Engine::run(Job& job) {
       stats.ins += (double)st[4];
       stats.dup += (double)st[5];
       stats.busyMs += (double)st[6] * 1e-5;
-      stats.insertMs += (double)st[7] * 1e-5;
+      if (st[12] > 0)
+        stats.insertMs += (double)st[7] * 1e-5 * (double)(st[4] + st[5]) / (double)st[12];
       stats.idlePolls += (double)st[8];
       stats.waves = (double)st[9];
       stats.scouts += (double)st[10];

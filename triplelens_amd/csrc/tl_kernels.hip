@@ -2184,7 +2184,7 @@ __device__ __forceinline__ bool next_run(const Ray& R, int N, bool limb, RunScan
 // wave are performed in program order; the unlock waits for the wave's LDS
 // operations before it releases the word.
 constexpr int kWorkers = kFillWaves - 1;
-constexpr int kFillStats = 10;   // FillArgs::stats
+constexpr int kFillStats = 11;   // FillArgs::stats
 constexpr int kFeedMax = 16;     // tasks the manager brings in at a time
 constexpr int kDonateMax = 8;    // tasks the manager queues for other groups at a time
 constexpr int kPoolShare = 16;   // while other groups are idle, workers keep the pool at
@@ -2526,7 +2526,7 @@ struct Worker {
   unsigned accCnt;
   long long accBits;        // (lane) brightness bits, kMagicBits included per pixel
   unsigned nTasks, nIns, nDup, nScout, nScoutRuns, steps;
-  unsigned insTicks;        // in run-table inserts, of one task in kTimedTasks
+  unsigned insTicks, nTimed;  // time of the timed inserts, and their number
   bool landed;              // the scout task found a run (new or known)
 };
 
@@ -2649,20 +2649,6 @@ __device__ __forceinline__ int scout_jump_for(ArgPtr A, int w) {
   return j < lo ? lo : (int)j;
 }
 
-// insert_run for the wave's position.  The inserts of one task in kTimedTasks
-// are timed.
-constexpr unsigned kTimedTasks = 64;
-__device__ __forceinline__ int insert_timed(Worker& W, int b, int row, int xl, int xr, int label,
-                                            int& other) {
-  const bool timed = W.nTasks % kTimedTasks == 0;
-  unsigned t0 = 0;
-  if (__builtin_expect(timed, 0)) t0 = (unsigned)__builtin_amdgcn_s_memrealtime();
-  const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, xl, xr, label, other);
-  if (__builtin_expect(timed, 0))
-    W.insTicks += (unsigned)__builtin_amdgcn_s_memrealtime() - t0;
-  return ins;
-}
-
 // What a task scans: a row between columns, in one or two pieces around known
 // pixels.
 struct Scan {
@@ -2697,7 +2683,7 @@ __device__ __forceinline__ bool handle_run(Worker& W, const Scan& S, int f1, int
   }
   labelOut = label;
   int other = 0;
-  const int ins = insert_timed(W, b, row, xl, xr, label, other);
+  const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, xl, xr, label, other);
   if (__builtin_expect(ins != kInsNew, 0)) {
     if (ins == kInsFull) {
       flag_point(W.A, W.gp, kFlagHashFull);
@@ -2847,8 +2833,9 @@ __device__ __forceinline__ void load_position(Worker& W, int b) {
 // look-backs end the call (process_task handles them at once: the images'
 // other branches start there).  Leaves the sweep's next row in W.t
 // (W.haveCont), for process_task (W.general) where it has to be evaluated
-// exactly.
-template <int MODE, bool LIMB>
+// exactly.  TIMED: the inserts are timed (by a call in 16; a branch at every
+// insert of the one loop cost each task 1%).
+template <int MODE, bool LIMB, bool TIMED>
 __device__ __forceinline__ void sweep_rows(Worker& W) {
   const RowBase B = row_base(W.R);
   const int N = W.N, b = W.t.b, d = (W.t.kd & 4) ? -1 : 1;
@@ -2875,7 +2862,12 @@ __device__ __forceinline__ void sweep_rows(Worker& W) {
     int nl = 0, nr = 0;
     while (next_run_in<MODE, LIMB>(W.R, N, Q)) {
       int other = 0;
-      const int ins = insert_timed(W, b, row, Q.xl, Q.xr, label, other);
+      const unsigned t0 = TIMED ? (unsigned)__builtin_amdgcn_s_memrealtime() : 0u;
+      const int ins = insert_run(W.tab, W.tabMask, W.A, b, row, Q.xl, Q.xr, label, other);
+      if (TIMED) {
+        W.insTicks += (unsigned)__builtin_amdgcn_s_memrealtime() - t0;
+        W.nTimed++;
+      }
       if (__builtin_expect(ins != kInsNew, 0)) {
         if (ins == kInsFull) {
           flag_point(W.A, W.gp, kFlagHashFull);
@@ -2956,6 +2948,15 @@ __device__ __forceinline__ void sweep_rows(Worker& W) {
   W.t.xb = xb;
   W.t.f1 = f1;
   W.t.f2 = f2;
+}
+
+template <int MODE>
+__device__ __forceinline__ void sweep_call(Worker& W) {
+  const bool limb = (W.flags & kPtLimb) != 0;
+  if (__builtin_expect(W.nTasks % 64 < 4, 0))
+    limb ? sweep_rows<MODE, true, true>(W) : sweep_rows<MODE, false, true>(W);
+  else
+    limb ? sweep_rows<MODE, true, false>(W) : sweep_rows<MODE, false, false>(W);
 }
 
 // Processes the task in hand and the look-backs recorded meanwhile (up to two;
@@ -3248,7 +3249,8 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
   W.accLabel = -1;
   W.accCnt = 0;
   W.accBits = 0;
-  W.nTasks = W.nIns = W.nDup = W.nScout = W.nScoutRuns = W.steps = W.insTicks = 0;
+  W.nTasks = W.nIns = W.nDup = W.nScout = W.nScoutRuns = W.steps = 0;
+  W.insTicks = W.nTimed = 0;
   const bool newest = A.poolNewest != 0;
   unsigned idlePolls = 0;
   unsigned long long idleTicks = 0;
@@ -3290,13 +3292,12 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
     }
     if ((W.t.kd & 3) == 0) {
       if (W.t.b != W.curB) load_position(W, W.t.b);
-      const bool limb = (W.flags & kPtLimb) != 0;
       switch (W.flags & (kPtFast | kPtBinary)) {
         case kPtFast:
-          limb ? sweep_rows<kRowTriple, true>(W) : sweep_rows<kRowTriple, false>(W);
+          sweep_call<kRowTriple>(W);
           break;
         case kPtFast | kPtBinary:
-          limb ? sweep_rows<kRowBinary, true>(W) : sweep_rows<kRowBinary, false>(W);
+          sweep_call<kRowBinary>(W);
           break;
         default: W.general = true;
       }
@@ -3337,8 +3338,8 @@ __global__ void __launch_bounds__(kFillThreads) fill_kernel(FillArgs A) {
   // with ten counters added by 256).
   if (ln == 0) {
     const unsigned long long v[kFillStats] = {W.nTasks, 64ull * W.steps, W.nIns, W.nDup, busyTicks,
-                                              (unsigned long long)W.insTicks * kTimedTasks,
-                                              idlePolls, 1, W.nScout, W.nScoutRuns};
+                                              W.insTicks, idlePolls, 1, W.nScout,
+                                              W.nScoutRuns, W.nTimed};
     for (int k = 0; k < kFillStats; k++) lds_add(&sums[k], v[k]);
     if (lds_add(&left, -1) == 1)
       for (int k = 0; k < kFillStats; k++) atomicAdd(&A.stats[k], lds_add(&sums[k], 0ull));
